@@ -173,3 +173,27 @@ def test_pertoken_quant_division_is_exact_over_many_values(qd, kind):
     got = y.view(torch.uint8).cpu().numpy()
     bad = np.argwhere(got != want_y.view(np.uint8))
     assert len(bad) == 0, (len(bad), bad[:5].tolist())
+
+
+# one wavefront per row (short rows, many of them) and four; register-resident rows of one, two and four vectors a thread, and
+# rows with a tail behind them; row counts that leave the last workgroup partly filled
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("m,k", [(1, 8), (3, 2040), (3, 2048), (2, 2056), (5, 4104), (2, 8192), (2, 8200), (2051, 512), (2050, 1016), (2049, 1032), (2050, 2048)])
+def test_pertoken_quant_row_splits_bit_exact(dt, m, k):
+    from flydsl_amd import quant, quant_device
+
+    g = torch.Generator().manual_seed(m * 7 + k)
+    x = torch.randn(m, k, generator=g) * torch.exp2(torch.randint(-6, 7, (m, 1), generator=g).float())
+    if dt == torch.float32:  # scales outside the range of the short division, where rows take the full one
+        x[0] *= 2.0 ** -100
+        x[-1] *= 2.0 ** 110
+    x = x.to(dt)
+    x[:, 0] = -0.0  # the sign of a zero reaches the fp8 code
+    if m > 2:
+        x[m // 2] = 0
+        x[m - 2, k // 2], x[m - 2, k - 1], x[m - 2, 1] = float("nan"), float("-inf"), float("inf")
+    for qd in (torch.int8, torch.float8_e4m3fn):
+        want, ws = quant.pertoken_quant(x, quant_dtype=qd)
+        y, s = quant_device.pertoken_quant(x.cuda(), quant_dtype=qd)
+        assert torch.equal(s.cpu(), ws)
+        assert torch.equal(y.view(torch.uint8).cpu(), want.view(torch.uint8))
