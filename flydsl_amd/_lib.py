@@ -27,6 +27,9 @@ EXPORTS = (
     "psg_gemm_mxfp4_acc",
     "psg_quant_pertoken",
     "psg_quant_mxfp4",
+    "psg_moe_rows_workspace_bytes",
+    "psg_moe_gemm_rows",
+    "psg_moe_mx_gemm_rows",
     "psg_init",
     "psg_static_scratch_bytes",
     "psg_gemm_a8w8_static",
@@ -246,6 +249,12 @@ def lib() -> ctypes.CDLL:
         fn = getattr(handle, name)
         fn.restype = ctypes.c_int
         fn.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    handle.psg_moe_rows_workspace_bytes.restype = ctypes.c_uint64
+    handle.psg_moe_rows_workspace_bytes.argtypes = [ctypes.c_int32] * 6
+    handle.psg_moe_gemm_rows.restype = ctypes.c_int
+    handle.psg_moe_gemm_rows.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p]
+    handle.psg_moe_mx_gemm_rows.restype = ctypes.c_int
+    handle.psg_moe_mx_gemm_rows.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p]
     for name in ("psg_gemm_a8w8_acc", "psg_gemm_mxfp4_acc"):
         fn = getattr(handle, name)
         fn.restype = ctypes.c_int
@@ -360,6 +369,21 @@ def workspace(device, nbytes: int, stream=0, owner="shared"):
     d = torch.device(device)
     index = d.index if d.index is not None else torch.cuda.current_device()
     return _pool.get(owner, index, int(stream), int(nbytes))
+
+
+def call_scratch(device, nbytes: int, stream: int):
+    """Scratch for the launches of ONE call: a tensor from torch's caching allocator, which hands its memory on in the order of
+    the stream it was allocated on, so it may be dropped as soon as the launches are queued.  That holds for the current
+    stream of ``device`` only; for a launch on another stream, while the stream is being captured (nothing is allocated then), and
+    when memory is short, the answer is ``None`` and the caller takes its way without scratch."""
+    import torch
+
+    if nbytes <= 0 or torch.cuda.current_stream(device).cuda_stream != stream or _torch_capturing():
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def check_operand(name, t, *, min_elems, elem_sizes, device=None):

@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p) {
             const int t = (int)(sid & 0xFFFFFFu), slot = (int)(sid >> 24);
             if (t < p.tokens && slot < p.topk && n < p.n_out) {
                 const uint8_t* src = stage + r * row_bytes + ((((cb >> 4) ^ r) & gmask) << 4) + (cb & 15);
-                const size_t orow = atomic ? (size_t)t : (size_t)t * p.topk + slot;
+                const size_t orow = atomic ? (size_t)t : p.by_position ? (size_t)(blk * BLK + r) : (size_t)t * p.topk + slot;
                 uint8_t* o = static_cast<uint8_t*>(p.out) + (orow * (size_t)p.n_out + n) * esize;
                 if (!atomic) {
                     *reinterpret_cast<v4i*>(o) = *reinterpret_cast<const v4i*>(src);

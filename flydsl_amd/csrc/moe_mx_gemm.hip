@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
             }
         }
         __syncthreads();
-        if (p.atomic) {
+        if (p.atomic == 1) {
             for (int q = tid; q < TM * 128; q += 256) {
                 const int r = q >> 7, cb = (q & 127) * 4;
                 const int t = p.sorted_ids[blk * TM + r] & 0xFFFFFF;

@@ -9,6 +9,7 @@
 
 #include "psg_common.h"
 #include "moe_gating.h"
+#include "moe_rows.h"
 #include "tile_order.h"
 
 hipError_t psg_launch_a8w8_tiled(const A8W8Params& p, int kind, int store, int tile_m, int tile_n, hipStream_t stream);
@@ -667,7 +668,18 @@ int psg_gemm_mxfp4(const psg_mxfp4_args* args, void* stream) { return mx_common(
 
 int psg_gemm_mxfp4_acc(const psg_mxfp4_args* args, void* acc, void* stream) { return mx_common(args, acc, STORE_ACC, stream); }
 
-int psg_moe_gemm(const psg_moe_args* a, void* stream) {
+// Workspace of a stage 2 that accumulates by way of rows (moe_rows.hip), or 0 where adding directly is faster.
+// The MX pair goes by rows from 12 MB of additions (tokens x topk x model_dim) on (us by rows / atomics, model 4096, inter 1536, top-8:
+// 64 tokens 28.4 / 24.2, 128 34.4 / 33.4, 256 42.7 / 53.4, 512 53.5 / 74.3, 1024 79.8 / 119.6, 4096 297 / 392; top-1 4096 x 4096 58.6 /
+// 63.1, 4096 x 1024 23.4 / 21.0; top-6 512 x 2048 26.5 / 28.2, 4096 x 1024 42.6 / 75.4).  The stages with one scale per row are bound by
+// their mainloop instead (4096 tokens 408 / 393, 512 70.3 / 70.8): they add directly.
+uint64_t psg_moe_rows_workspace_bytes(int32_t tokens, int32_t topk, int32_t sorted_size, int32_t model_dim, int32_t out_dtype, int32_t mx) {
+    if (tokens < 1 || topk < 1 || sorted_size < 1 || model_dim < 2 || (out_dtype != PSG_OUT_BF16 && out_dtype != PSG_OUT_FP16)) return 0;
+    if (!mx || (int64_t)tokens * topk * model_dim * 2 < (12ll << 20)) return 0;
+    return psg_moe_rows_bytes(tokens, topk, sorted_size, model_dim);
+}
+
+static int moe_gemm_common(const psg_moe_args* a, void* workspace, uint64_t workspace_bytes, void* stream) {
     if (!a) return fail(PSG_E_NULL, "args is NULL");
     if (!a->out || !a->x || !a->w || !a->scale_x || !a->scale_w || !a->sorted_token_ids || !a->sorted_expert_ids || !a->num_valid_ids)
         return fail(PSG_E_NULL, "out, x, w, scale_x, scale_w, sorted_token_ids, sorted_expert_ids, num_valid_ids must be non-NULL");
@@ -717,10 +729,43 @@ int psg_moe_gemm(const psg_moe_args* a, void* stream) {
     p.out_dtype = a->out_dtype;
     p.doweight = a->doweight ? 1 : 0;
     p.accumulate = a->stage == 2 && a->accumulate ? 1 : 0;
-    const hipError_t e = psg_launch_moe_gemm(p, a->in_dtype == PSG_IN_INT8 ? KIND_INT8 : a->in_dtype == PSG_IN_INT8_W4 ? KIND_INT8W4 : KIND_FP8, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
+    p.by_position = 0;
+    hipError_t e = hipSuccess;
+    const bool rows = workspace && p.accumulate && a->out_dtype != PSG_OUT_F32 && workspace_bytes >= psg_moe_rows_bytes(a->tokens, a->topk, a->sorted_size, n_out);
+    MoeRowsParams r{};
+    if (rows) {
+        r.out = static_cast<uint16_t*>(a->out);
+        r.sorted_ids = p.sorted_ids;
+        r.expert_ids = p.expert_ids;
+        r.num_valid = p.num_valid;
+        r.tokens = p.tokens;
+        r.topk = p.topk;
+        r.experts = p.experts;
+        r.dim = n_out;
+        r.sorted_size = p.sorted_size;
+        r.blocks = a->blocks;
+        r.block_m = r.granule = a->block_m;
+        r.slots = p.topk;
+        r.out_dtype = p.out_dtype;
+        psg_moe_rows_carve(r, workspace);
+        p.out = r.rows;
+        p.accumulate = 0;
+        p.by_position = 1;
+        e = psg_launch_moe_rows_index(r, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return hip_fail(e, "psg_moe_gemm launch");
+    }
+    e = psg_launch_moe_gemm(p, a->in_dtype == PSG_IN_INT8 ? KIND_INT8 : a->in_dtype == PSG_IN_INT8_W4 ? KIND_INT8W4 : KIND_FP8, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
+    if (e == hipSuccess && rows) e = psg_launch_moe_rows_add(r, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "psg_moe_gemm launch");
     g_err[0] = 0;
     return 0;
+}
+
+int psg_moe_gemm(const psg_moe_args* a, void* stream) { return moe_gemm_common(a, nullptr, 0, stream); }
+
+int psg_moe_gemm_rows(const psg_moe_args* a, void* workspace, uint64_t workspace_bytes, void* stream) {
+    if (workspace && !aligned(workspace, 16)) return fail(PSG_E_ALIGN, "workspace must be 16-byte aligned");
+    return moe_gemm_common(a, workspace, workspace_bytes, stream);
 }
 
 namespace {
@@ -754,7 +799,7 @@ int psg_moe_mx_scale_sort(const void* scale, const int32_t* sorted_token_ids, co
     return 0;
 }
 
-int psg_moe_mx_gemm(const psg_moe_mx_args* a, void* stream) {
+static int moe_mx_gemm_common(const psg_moe_mx_args* a, int32_t topk, void* workspace, uint64_t workspace_bytes, void* stream) {
     if (!a) return fail(PSG_E_NULL, "args is NULL");
     const bool inline_quant = a->stage == 1 && a->a_dtype == PSG_MX_BF16_QUANT;
     if (!a->out || !a->a || (!a->a_scale && !inline_quant) || !a->w || !a->w_scale || !a->sorted_token_ids || !a->sorted_expert_ids || !a->num_valid_ids)
@@ -807,10 +852,42 @@ int psg_moe_mx_gemm(const psg_moe_mx_args* a, void* stream) {
     p.eshift = 0;
     p.n_tiles = p.n_groups = p.by_expert = p.quad_tiles = 0;
     if (((int64_t)a->blocks << 1) * (int64_t)((n_out / 128 + 7) / 8 * 8) > 0x7FFFFFFFll) return fail(PSG_E_SHAPE, "blocks=%d times the column tiles exceed the grid", a->blocks);
-    const hipError_t e = psg_launch_moe_mx_gemm(p, a->a_dtype == PSG_MX_FP8 ? MXF_FP8 : MXF_FP4, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
+    hipError_t e = hipSuccess;
+    const bool rows = workspace && p.atomic && topk >= 1 && topk <= 255 && workspace_bytes >= psg_moe_rows_bytes(a->tokens, topk, a->sorted_size, n_out);
+    MoeRowsParams r{};
+    if (rows) {
+        r.out = static_cast<uint16_t*>(a->out);
+        r.sorted_ids = p.sorted_ids;
+        r.expert_ids = p.expert_ids;
+        r.num_valid = p.num_valid;
+        r.tokens = p.tokens;
+        r.topk = topk;
+        r.experts = p.experts;
+        r.dim = n_out;
+        r.sorted_size = p.sorted_size;
+        r.blocks = a->blocks;
+        r.block_m = a->block_m;
+        r.granule = a->block_m == 128 ? 64 : a->block_m;
+        r.slots = 256;  // this pair of stages reads the token of an id only
+        r.out_dtype = p.out_dtype;
+        psg_moe_rows_carve(r, workspace);
+        p.out = r.rows;
+        p.atomic = 2;
+        e = psg_launch_moe_rows_index(r, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return hip_fail(e, "psg_moe_mx_gemm launch");
+    }
+    e = psg_launch_moe_mx_gemm(p, a->a_dtype == PSG_MX_FP8 ? MXF_FP8 : MXF_FP4, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
+    if (e == hipSuccess && rows) e = psg_launch_moe_rows_add(r, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "psg_moe_mx_gemm launch");
     g_err[0] = 0;
     return 0;
+}
+
+int psg_moe_mx_gemm(const psg_moe_mx_args* a, void* stream) { return moe_mx_gemm_common(a, 0, nullptr, 0, stream); }
+
+int psg_moe_mx_gemm_rows(const psg_moe_mx_args* a, int32_t topk, void* workspace, uint64_t workspace_bytes, void* stream) {
+    if (workspace && !aligned(workspace, 16)) return fail(PSG_E_ALIGN, "workspace must be 16-byte aligned");
+    return moe_mx_gemm_common(a, topk, workspace, workspace_bytes, stream);
 }
 
 int psg_moe_reduce(const void* x, void* y, int32_t tokens, int32_t topk, int32_t model_dim, int32_t dtype, void* stream) {

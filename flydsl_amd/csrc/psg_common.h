@@ -184,6 +184,7 @@ struct MoeParams {
     int doweight;               // multiply by the routing weight in this stage
     int accumulate;             // stage 2: atomic add into out[token] (else one row per (token, slot))
     int x_slot_major;           // stage 1: x / sx hold one row per (slot, token) at slot*tokens + token
+    int by_position;            // stage 2 without accumulate: one row per sorted position instead of one per (token, slot)
     int pair_blocks;            // blocks of 16 / 32 rows: multiply two consecutive blocks of one expert in one workgroup
 };
 
@@ -206,7 +207,7 @@ struct MoeMxParams {
     int K;                      // model_dim (stage 1) or inter_dim (stage 2)
     int sorted_size;
     int out_dtype;              // stage 2: OUT_BF16 / OUT_FP16
-    int atomic;                 // stage 2: weighted atomic add into out[token]
+    int atomic;                 // stage 2: 1 = weighted atomic add into out[token], 2 = weighted, one row per sorted position, 0 = the same unweighted
     int eshift;                 // set by the launcher: log2(sorter block rows / rows per workgroup)
     int n_tiles, n_groups;      // set by the launcher: column tiles of the output, and groups of 8 of them
     int by_expert;              // set by the launcher: workgroup ids are mapped to XCDs by (expert, column tile)

@@ -82,7 +82,13 @@ class MoeStage:
         a.doweight, a.accumulate = int(self.doweight), int(self.accumulate)
         a.x_slot_major = int(self.slot_major)
         a.no_pairing = int(self.no_pairing)
-        rc = self._lib.psg_moe_gemm(ctypes.byref(a), _lib.stream_handle(stream))
+        h = _lib.stream_handle(stream)
+        need = self._lib.psg_moe_rows_workspace_bytes(tokens, self.topk, a.sorted_size, n_out, self.out_dtype, 0) if self.stage == 2 and self.accumulate else 0
+        ws = _lib.call_scratch(dev, need, h) if need else None
+        if ws is None:
+            rc = self._lib.psg_moe_gemm(ctypes.byref(a), h)
+        else:
+            rc = self._lib.psg_moe_gemm_rows(ctypes.byref(a), ws.data_ptr(), need, h)
         if rc:
             _lib.check(rc, "psg_moe_gemm")
 

@@ -172,7 +172,14 @@ def flydsl_mxfp4_gemm2(*, inter_sorted_quant, inter_sorted_shuffled_scale, w2_u8
     args.out_dtype = 0 if flat_out.dtype == torch.bfloat16 else 1
     args.stage, args.atomic, args.pad0 = 2, int(atomic), 0
     lib = _lib.lib()
-    _lib.check(lib.psg_moe_mx_gemm(ctypes.byref(args), _stream_handle(stream)), "psg_moe_mx_gemm (stage 2)")
+    h = _lib.stream_handle(stream)
+    need = lib.psg_moe_rows_workspace_bytes(args.tokens, int(topk), max_sorted, args.model_dim, args.out_dtype, 1) if atomic else 0
+    ws = _lib.call_scratch(flat_out.device, need, h) if need else None
+    if ws is None:
+        rc = lib.psg_moe_mx_gemm(ctypes.byref(args), h)
+    else:
+        rc = lib.psg_moe_mx_gemm_rows(ctypes.byref(args), int(topk), ws.data_ptr(), need, h)
+    _lib.check(rc, "psg_moe_mx_gemm (stage 2)")
     return flat_out
 
 

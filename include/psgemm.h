@@ -333,6 +333,16 @@ typedef struct psg_moe_mx_args {
 
 int psg_moe_mx_gemm(const psg_moe_mx_args *args, void *stream);
 
+/* Stage 2 with accumulation (accumulate = 1, or atomic = 1 of the MX pair; 16-bit output) with scratch memory: the rows are stored to
+ * the workspace and every token's sum is added into out once, which is several times cheaper than topk additions per element.
+ * psg_moe_rows_workspace_bytes: the bytes it takes, or 0 where adding directly is the better way.  Without a workspace (NULL or too
+ * small), and for anything else than such a stage 2, the calls are psg_moe_gemm / psg_moe_mx_gemm.  The workspace needs no
+ * initialisation, 16-byte alignment, and must not be used by anything else until the call's work on `stream` has ended. */
+uint64_t psg_moe_rows_workspace_bytes(int32_t tokens, int32_t topk, int32_t sorted_size, int32_t model_dim, int32_t out_dtype,
+                                      int32_t mx /* 1: the MX pair, 0: psg_moe_gemm */);
+int psg_moe_gemm_rows(const psg_moe_args *args, void *workspace, uint64_t workspace_bytes, void *stream);
+int psg_moe_mx_gemm_rows(const psg_moe_mx_args *args, int32_t topk, void *workspace, uint64_t workspace_bytes, void *stream);
+
 /* a_scale of psg_moe_mx_gemm stage 1 from the scales of the quantised activations: the reference's moe_mxfp4_sort
  * (tests/kernels/utils/gemm_common_utils.py:464-598).  scale [tokens, cols] e8m0 bytes (topk = 1) or [tokens, topk, cols] (then the
  * row of a sorted id is token * topk + slot); out: ceil(sorted_size/32)*32 rows x cols bytes in the shuffled order, row i = the scale
