@@ -360,8 +360,25 @@ hipError_t launch_kind(const MoeParams& p, int block_m, int blocks, hipStream_t 
 
 }  // namespace
 
+hipError_t psg_launch_moe_tiled(const MoeParams& p, int kind, int stage, int blocks, hipStream_t stream);
+
+// Whether the 256-row tiles (moe_gemm_tiled.hip) are the better way for blocks of 128 rows: enough rows per expert that most
+// blocks find a partner, and a tile count (on average over routings: pairs / 256, and half a tile more per expert) that fills its
+// rounds of one tile per CU to 80 %.  Measured, fp8, us k_moe_gemm / 256-row tiles: stage 1 4096 tokens x top-8 on 32 experts, 4096 x
+// 1536 (1728 tiles) 473 / 391; 4096 x top-6 on 64, 1024 x 256 (256 tiles) 34.7 / 27.4; but 1024 x top-8 (576 tiles) 168 / 179, 4096 x
+// top-2 on 8, 2048 x 1024 (288) 52.8 / 61.1.  Stage 2 without atomics: 4096 x top-8 (2304 tiles) 360 / 273, 1024 x top-8 (768) 119 /
+// 105; but 512 x top-8 (512 tiles, 128 rows per expert) 70.2 / 72.7, 4096 x top-1 on 8, 4096 x 1024 (320) 68.7 / 74.9.
+bool takes_tiled(const MoeParams& p, int stage) {
+    const long pairs = (long)p.tokens * p.topk, cus = psg_cu_count(), tn = stage == 1 ? 128 : 256;
+    if (pairs < 192L * p.experts) return false;
+    const long tiles = (pairs / 256 + p.experts / 2) * ((p.n_out + tn - 1) / tn);
+    const long rounds = (tiles + cus - 1) / cus;
+    return tiles * 10 >= rounds * cus * 8;
+}
+
 // kind: KIND_INT8 / KIND_FP8 / KIND_INT8W4; stage 1 or 2; block_m in {16, 32, 64, 128}; blocks = entries of expert_ids
 hipError_t psg_launch_moe_gemm(const MoeParams& p, int kind, int stage, int block_m, int blocks, hipStream_t stream) {
+    if (block_m == 128 && kind != KIND_INT8W4 && p.out_dtype != OUT_F32 && p.pair_blocks && takes_tiled(p, stage)) return psg_launch_moe_tiled(p, kind, stage, blocks, stream);
     if (kind == KIND_INT8) return stage == 1 ? launch_kind<KIND_INT8, 1>(p, block_m, blocks, stream) : launch_kind<KIND_INT8, 2>(p, block_m, blocks, stream);
     if (kind == KIND_INT8W4) return stage == 1 ? launch_kind<KIND_INT8W4, 1>(p, block_m, blocks, stream) : launch_kind<KIND_INT8W4, 2>(p, block_m, blocks, stream);
     return stage == 1 ? launch_kind<KIND_FP8, 1>(p, block_m, blocks, stream) : launch_kind<KIND_FP8, 2>(p, block_m, blocks, stream);

@@ -671,11 +671,13 @@ int psg_gemm_mxfp4_acc(const psg_mxfp4_args* args, void* acc, void* stream) { re
 // Workspace of a stage 2 that accumulates by way of rows (moe_rows.hip), or 0 where adding directly is faster.
 // The MX pair goes by rows from 12 MB of additions (tokens x topk x model_dim) on (us by rows / atomics, model 4096, inter 1536, top-8:
 // 64 tokens 28.4 / 24.2, 128 34.4 / 33.4, 256 42.7 / 53.4, 512 53.5 / 74.3, 1024 79.8 / 119.6, 4096 297 / 392; top-1 4096 x 4096 58.6 /
-// 63.1, 4096 x 1024 23.4 / 21.0; top-6 512 x 2048 26.5 / 28.2, 4096 x 1024 42.6 / 75.4).  The stages with one scale per row are bound by
-// their mainloop instead (4096 tokens 408 / 393, 512 70.3 / 70.8): they add directly.
+// 63.1, 4096 x 1024 23.4 / 21.0; top-6 512 x 2048 26.5 / 28.2, 4096 x 1024 42.6 / 75.4).  The stages with one scale per row go by rows from
+// 24 MB and four slots on (fp8: 333 tokens x top-9 72 / 75, 512 x top-8 70 / 72, 1024 105 / 118, 4096 330 / 371; 4096 x top-6 x 1024 53 / 60;
+// but 1024 x top-2 x 4096 41 / 35, 4096 x top-1 75 / 64).
 uint64_t psg_moe_rows_workspace_bytes(int32_t tokens, int32_t topk, int32_t sorted_size, int32_t model_dim, int32_t out_dtype, int32_t mx) {
     if (tokens < 1 || topk < 1 || sorted_size < 1 || model_dim < 2 || (out_dtype != PSG_OUT_BF16 && out_dtype != PSG_OUT_FP16)) return 0;
-    if (!mx || (int64_t)tokens * topk * model_dim * 2 < (12ll << 20)) return 0;
+    const int64_t bytes = (int64_t)tokens * topk * model_dim * 2;
+    if (bytes < (mx ? 12ll << 20 : 24ll << 20) || (!mx && topk < 4)) return 0;
     return psg_moe_rows_bytes(tokens, topk, sorted_size, model_dim);
 }
 
@@ -730,6 +732,7 @@ static int moe_gemm_common(const psg_moe_args* a, void* workspace, uint64_t work
     p.doweight = a->doweight ? 1 : 0;
     p.accumulate = a->stage == 2 && a->accumulate ? 1 : 0;
     p.by_position = 0;
+    p.blocks = p.group_m = 0;
     hipError_t e = hipSuccess;
     const bool rows = workspace && p.accumulate && a->out_dtype != PSG_OUT_F32 && workspace_bytes >= psg_moe_rows_bytes(a->tokens, a->topk, a->sorted_size, n_out);
     MoeRowsParams r{};
