@@ -27,6 +27,7 @@ bool psg_moe_gate_sort_fuses(int tokens, int topk, int experts);
 hipError_t psg_launch_moe_reduce(const void* x, void* y, int tokens, int topk, int dim, int out_dtype, const int32_t* mask,
                                  const int32_t* ids, int experts, hipStream_t stream);
 hipError_t psg_launch_mx_generic(const MxGenParams& p, int af, int bf, int store, int batch, hipStream_t stream);
+hipError_t psg_launch_mx_smallm(const MxGenParams& p, int af, int bf, int batch, hipStream_t stream);
 hipError_t psg_launch_mxfp4_smallm(const MxParams& p, int store, int nw, hipStream_t stream);
 hipError_t psg_launch_splitk_finalize(const A8W8Params& p, const void* partial, int is_int, int scaled, hipStream_t stream);
 hipError_t psg_launch_tile_order(int tiles_m, int tiles_n, int group_m, int32_t* out, hipStream_t stream);
@@ -199,6 +200,17 @@ int pick_splits(int M, int N, int kbytes, Tile t) {
         if (fits && steps / c >= min_steps && (long)c * M * 16 <= (long)kbytes * 5) s = c;
     }
     return s;
+}
+
+// Which calls of the general MX path the small-M kernel takes (the others: gemm_mx_generic.hip).
+// Up to 64 rows, while what its N / 32 workgroups read of A together stays below 160 MB with fp4 weights and 320 MB with fp8 weights (N K M
+// / 32, M in whole register tiles of 16, 32 or 64 rows), and from 1024 columns on (32 workgroups).  Measured, us small-M / general:
+// fp8 x fp4 1 x 8192 x 8192 7.7 / 12.2, 64 x 8192 x 8192 12.3 / 20.2, 64 x 4096 x 4096 6.9 / 16.0, 16 x 1024 x 2048 3.1 / 6.8, 64 x 1024 x
+// 14336 15.7 / 27.3, 64 x 16384 x 4096 (134 MB) 14.5 / 17.7, 16 x 16384 x 14336 (117 MB) 22.6 / 23.2, but 24 rows of it (235 MB) 25.9 / 24.1
+// and 64 (470 MB) 37.5 / 32.0; fp8 x fp8 32 x 16384 x 14336 (235 MB) 40.9 / 46.8, 64 rows 51.1 / 48.8; fp6 x fp4 as fp8 x fp4.
+bool mx_general_small(int M, int N, int K, bool fp8_weights) {
+    const long rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+    return M <= kStreamMaxM && N >= 1024 && (long)(N / 32) * rows * K <= (fp8_weights ? 320L : 160L) * 1000000L;
 }
 
 // Split-K for the general MX kernel: its tiles are 64x128 (32x128 for M <= 32), so decode-like shapes launch few
@@ -586,8 +598,11 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         g.sa_batch = a->scale_a_batch_stride ? a->scale_a_batch_stride : (int64_t)((uint64_t)((a->M + 31) / 32) * sa_cs);
         g.sb_batch = (int64_t)((uint64_t)(a->N / 32) * chunk);
         hipError_t ge;
-        const int splits = batch == 1 && c_rs == (uint64_t)a->N && store == STORE_C ? mx_general_splits(a->M, a->N, a->K) : 1;
-        if (splits > 1 && a->workspace && aligned(a->workspace, 16) && a->workspace_bytes >= splitk_bytes(a->M, a->N, splits)) {
+        const bool small = store == STORE_C && a->force_path == 0 && mx_general_small(a->M, a->N, a->K, a->b_dtype == PSG_MX_FP8);
+        const int splits = !small && batch == 1 && c_rs == (uint64_t)a->N && store == STORE_C ? mx_general_splits(a->M, a->N, a->K) : 1;
+        if (small) {
+            ge = psg_launch_mx_smallm(g, a->a_dtype, a->b_dtype, batch, static_cast<hipStream_t>(stream));
+        } else if (splits > 1 && a->workspace && aligned(a->workspace, 16) && a->workspace_bytes >= splitk_bytes(a->M, a->N, splits)) {
             MxGenParams part = g;
             part.c = a->workspace;
             part.splits = splits;

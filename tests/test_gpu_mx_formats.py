@@ -282,3 +282,30 @@ def test_general_kernel_large_tile(a_dtype, b_dtype):
     # the small tile through the same kernel (forced by a batch of one narrow problem) gives the same accumulators
     acc = _launch(d, M, N, K, acc=True)
     assert np.allclose(acc, ref, rtol=1e-4, atol=_acc_atol(d, ref))
+
+
+# the small-M kernel: edges of its 16-row tiles, one K step and several per wavefront, four and eight wavefronts, a wavefront without a
+# step (K = 256 * odd), N that is no multiple of the XCD count's 256 columns, two batches with rows apart
+@pytest.mark.parametrize("a_dtype,b_dtype", PAIRS)
+@pytest.mark.parametrize("M,N,K,batch", [(1, 1024, 256, 2), (15, 1056, 1280, 1), (16, 1024, 2048, 1), (17, 1184, 2304, 2), (32, 1024, 6400, 1), (33, 1024, 2560, 1), (64, 1088, 1024, 2)])
+def test_small_m_kernel_against_the_general_kernel(a_dtype, b_dtype, M, N, K, batch):
+    if (a_dtype, b_dtype) == ("fp4", "fp4") and batch == 1:
+        pytest.skip("dense fp4 x fp4 has kernels of its own")
+    from kernels.gemm.mxfp4_preshuffle import launch_gemm
+
+    d = [make_mx(M, N, K, a_dtype, b_dtype, seed=M + b, w_std=1.0) for b in range(batch)]
+    cat = lambda key: torch.cat([x[key].reshape(-1) for x in d]).cuda()
+    outs = []
+    for path, pad in ((0, 0), (0, 64), (3, 0)):
+        c = torch.full((batch, M, N + pad), SENTINEL, dtype=torch.bfloat16, device="cuda")
+        launch_gemm(c, cat("a_q"), cat("b_shuf"), cat("sa_shuf"), cat("sb_shuf"), M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, a_dtype, "bf16", b_dtype,
+                    batch, -1, -1, -1, -1, N + pad if pad else -1, M * (N + pad) * 2 if pad else -1, 0, 0, _force_path=path)
+        torch.cuda.synchronize()
+        assert (c[:, :, N:] == SENTINEL).all()
+        outs.append(c[:, :, :N].float().cpu().numpy())
+    assert np.array_equal(outs[0], outs[1])
+    # the fp32 sums differ in their order only (the bound of the accumulators above), and each side rounds once to bf16
+    for b in range(batch):
+        ref = _ref(d[b])
+        for o in (outs[0][b], outs[2][b]):
+            assert np.all(np.abs(o - ref) <= 2.0 ** -8 * np.abs(ref) + 1.01 * _acc_atol(d[b], ref) + 1e-4 * np.abs(ref))
