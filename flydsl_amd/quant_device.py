@@ -22,8 +22,9 @@ def _x_code(x):
 
 
 def _check_out(x, *outs):
+    index = x.get_device()
     for t in outs:
-        if not t.is_cuda or t.device != x.device or not t.is_contiguous():
+        if not t.is_cuda or t.get_device() != index or not t.is_contiguous():
             raise ValueError("out tensors must be contiguous and on the same device as x")
 
 
@@ -47,11 +48,10 @@ def pertoken_quant(x: torch.Tensor, quant_dtype=torch.int8, stream=None, out=Non
         _check_out(x, y, scale)
         if y.numel() != m * k or y.element_size() != 1 or scale.numel() != m or scale.dtype != torch.float32:
             raise ValueError("out must be (1-byte [M,K], fp32 [M]) tensors")
-        y = y.view(torch.uint8)
     rc = _lib.lib().psg_quant_pertoken(x.data_ptr(), code, y.data_ptr(), scale.data_ptr(), m, k, out_code, _lib.stream_handle(stream))
     if rc:
         _lib.check(rc, "psg_quant_pertoken")
-    return y.view(quant_dtype), scale.view(m, 1)
+    return y if y.dtype == quant_dtype else y.view(quant_dtype), scale if scale.shape == (m, 1) else scale.view(m, 1)
 
 
 def per_1x32_f4_quant(x: torch.Tensor, shuffle: bool = True, stream=None, out=None):
@@ -67,11 +67,13 @@ def per_1x32_f4_quant(x: torch.Tensor, shuffle: bool = True, stream=None, out=No
         scales = torch.empty((r, k // 32), dtype=torch.uint8, device=x.device)
     else:  # caller-owned outputs: no allocation, graph-capturable
         _check_out(x, *out)
-        packed, scales = (t.view(torch.uint8) for t in out)
+        packed, scales = out
+        if packed.element_size() != 1 or scales.element_size() != 1:  # counted in bytes, whatever the element type
+            packed, scales = packed.view(torch.uint8), scales.view(torch.uint8)
         if packed.numel() != m * (k // 2) or scales.numel() != r * (k // 32):
             raise ValueError("out must be (packed [M,K/2], scales [ceil(M/32)*32, K/32]) byte tensors")
     rc = _lib.lib().psg_quant_mxfp4(x.data_ptr(), code, packed.data_ptr(), scales.data_ptr(), m, k, 1 if shuffle else 0,
                                     _lib.stream_handle(stream))
     if rc:
         _lib.check(rc, "psg_quant_mxfp4")
-    return packed.view(fp4x2), scales.view(fp8_e8m0)
+    return packed if packed.dtype == fp4x2 else packed.view(fp4x2), scales if scales.dtype == fp8_e8m0 else scales.view(fp8_e8m0)
