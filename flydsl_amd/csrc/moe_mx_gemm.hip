@@ -372,16 +372,19 @@ hipError_t launch_rows(MoeMxParams p, int block_m, int blocks, hipStream_t strea
 
 }  // namespace
 
-// Scales of the sorted rows in the shuffled order stage 1 reads: one thread per output dword = the scale bytes of the rows r16 and
-// r16 + 16 of a 32-row chunk at the columns c4 and c4 + 4 of an 8-column chunk (byte = 2 * column half + row half).
+// Scales of the sorted rows in the shuffled order stage 1 reads: one thread per (32-row chunk, 8 columns, row r16 of the chunk's 16-row
+// halves): the eight bytes of the rows r16 and r16 + 16 become four output dwords, dword c4 = the bytes of both rows at the columns c4 and
+// c4 + 4 (byte = 2 * column half + row half).  WIDE: scale rows are 8-byte aligned and fetched in one load each.  One thread per dword
+// with four byte loads spent its time on addresses and ids: 36,864 sorted rows of 128 columns 10.6 -> 3.7 us, 8,192 rows 4.2 -> 2.7.
+template <bool WIDE>
 __global__ void __launch_bounds__(256) k_moe_mx_scale_sort(const uint8_t* scale, const int32_t* sorted_ids, const int32_t* num_valid, uint32_t* out,
-                                                            int tokens, int topk, int cols, int sorted_size, int dwords) {
+                                                            int tokens, int topk, int cols, int sorted_size, int threads) {
     const int d = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (d >= dwords) return;
-    const int r16 = d & 15, c4 = (d >> 4) & 3, blk = d >> 6;  // blk = chunk * (cols / 8) + column chunk
+    if (d >= threads) return;
+    const int r16 = d & 15, blk = d >> 4;  // blk = chunk * (cols / 8) + column chunk
     const int ncc = cols >> 3, chunk = blk / ncc, cc = blk % ncc;
     const int nv = num_valid[0];
-    uint32_t word = 0;
+    uint32_t lo[2] = {0, 0}, hi[2] = {0, 0};  // columns 0..3 and 4..7 of the two rows
 #pragma unroll
     for (int rh = 0; rh < 2; rh++) {
         const int i = chunk * 32 + rh * 16 + r16;
@@ -389,11 +392,24 @@ __global__ void __launch_bounds__(256) k_moe_mx_scale_sort(const uint8_t* scale,
         const uint32_t id = (uint32_t)sorted_ids[i];
         const int tok = (int)(id & 0xFFFFFFu), slot = (int)(id >> 24);
         if (tok >= tokens || (topk > 1 && slot >= topk)) continue;
-        const uint8_t* row = scale + (size_t)(topk > 1 ? tok * topk + slot : tok) * (size_t)cols + cc * 8 + c4;
-        word |= (uint32_t)row[0] << (8 * rh);
-        word |= (uint32_t)row[4] << (8 * (2 + rh));
+        const uint8_t* row = scale + (topk > 1 ? (size_t)tok * topk + slot : (size_t)tok) * (size_t)cols + cc * 8;
+        if constexpr (WIDE) {
+            const v2i w = *reinterpret_cast<const v2i*>(row);
+            lo[rh] = (uint32_t)w[0];
+            hi[rh] = (uint32_t)w[1];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                lo[rh] |= (uint32_t)row[j] << (8 * j);
+                hi[rh] |= (uint32_t)row[4 + j] << (8 * j);
+            }
+        }
     }
-    out[d] = word;
+#pragma unroll
+    for (int c4 = 0; c4 < 4; c4++) {
+        const auto byte = [c4](uint32_t w) { return w >> (8 * c4) & 0xFFu; };
+        out[(size_t)blk * 64 + c4 * 16 + r16] = byte(lo[0]) | byte(lo[1]) << 8 | byte(hi[0]) << 16 | byte(hi[1]) << 24;
+    }
 }
 
 // a_format: MXF_FP4 / MXF_FP8 (stage 1 only; stage 2 reads the fp4 rows stage 1 wrote); block_m: 32 / 64 / 128, or 16: stage 1 then
@@ -407,8 +423,13 @@ hipError_t psg_launch_moe_mx_gemm(const MoeMxParams& p, int a_format, int stage,
 // out: ceil(sorted_size / 32) * 32 rows x cols bytes, every byte written
 hipError_t psg_launch_moe_mx_scale_sort(const void* scale, const int32_t* sorted_ids, const int32_t* num_valid, void* out, int tokens, int topk, int cols,
                                         int sorted_size, hipStream_t stream) {
-    const int dwords = (sorted_size + 31) / 32 * 8 * cols;
-    hipLaunchKernelGGL(k_moe_mx_scale_sort, dim3((dwords + 255) / 256), dim3(256), 0, stream, static_cast<const uint8_t*>(scale), sorted_ids, num_valid,
-                       static_cast<uint32_t*>(out), tokens, topk, cols, sorted_size, dwords);
+    const int threads = (sorted_size + 31) / 32 * 2 * cols;
+    const dim3 grid((threads + 255) / 256);
+    if (reinterpret_cast<uintptr_t>(scale) % 8 == 0)
+        hipLaunchKernelGGL((k_moe_mx_scale_sort<true>), grid, dim3(256), 0, stream, static_cast<const uint8_t*>(scale), sorted_ids, num_valid, static_cast<uint32_t*>(out), tokens,
+                           topk, cols, sorted_size, threads);
+    else
+        hipLaunchKernelGGL((k_moe_mx_scale_sort<false>), grid, dim3(256), 0, stream, static_cast<const uint8_t*>(scale), sorted_ids, num_valid, static_cast<uint32_t*>(out), tokens,
+                           topk, cols, sorted_size, threads);
     return hipGetLastError();
 }
