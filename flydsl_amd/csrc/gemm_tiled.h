@@ -79,6 +79,23 @@ __device__ __forceinline__ void mfma_mx8(v4f& c, const v8i& a, const v8i& b, int
                  : "v"(a), "v"(b), "v"(s0), "v"(s1), "n"(LO0), "n"(LO1), "n"(HI));
 }
 
+// fp8 (v8i) or fp6 (v6i) activations against fp4 weights: one MFMA per 128-element step, HI as above; `a` is the weight fragment
+typedef int v6i __attribute__((ext_vector_type(6)));
+template <int HI, int LO0, int LO1>
+__device__ __forceinline__ void mfma_mx4w(v4f& c, const v4i& a, const v8i& b, int s0, int s1) {
+    asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%7,0] cbsz:4"
+                 : "+a"(c)
+                 : "v"(a), "v"(b), "v"(s0), "v"(s1), "n"(LO0), "n"(LO1), "n"(HI));
+}
+template <int HI, int LO0, int LO1>
+__device__ __forceinline__ void mfma_mx4w(v4f& c, const v4i& a, const v6i& b, int s0, int s1) {
+    // the six registers of a fragment are two loads' worth, so the compiler moves two of them into place: a VALU write needs two wait
+    // states in front of the MFMA that reads it, and the compiler does not know that this is one
+    asm volatile("s_nop 1\n\tv_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,%6,0] op_sel_hi:[%7,%7,0] cbsz:4 blgp:2"
+                 : "+a"(c)
+                 : "v"(a), "v"(b), "v"(s0), "v"(s1), "n"(LO0), "n"(LO1), "n"(HI));
+}
+
 // LDS byte offset of 16-byte chunk `kc` (0..7) of row `row` inside one A stage
 __device__ __forceinline__ int lds_off(int row, int kc) { return row * TK + ((kc ^ ((row >> 1) & 7)) << 4); }
 

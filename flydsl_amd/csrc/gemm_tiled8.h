@@ -93,7 +93,8 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     static_assert(NS % NB == 0 && MR % 4 == 0 && A_DMA >= 1 && A_DMA % 2 == 0 && STAGE % (1024 * WAVES) == 0, "tile geometry");
     constexpr bool IS16 = KIND == KIND_FP16 || KIND == KIND_BF16;
     constexpr bool SCALED = KIND == KIND_INT8 || KIND == KIND_FP8;
-    constexpr bool MX = KIND == KIND_MXFP4 || KIND == KIND_MXFP8;
+    constexpr bool W4 = KIND == KIND_MXA8W4 || KIND == KIND_MXA6W4;  // fp4 W against a wider A: half a row's bytes
+    constexpr bool MX = KIND == KIND_MXFP4 || KIND == KIND_MXFP8 || W4;
     static_assert(!MX || (MR == 16 && NS == 4), "MX scale slots are laid out for the 256-row tile");
 
     // LDS: the A stages; behind them NS slots of MX scale dwords (per slot 8 A-side chunks + 8 W-side chunks of 256 bytes)
@@ -125,8 +126,9 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     const uint64_t a_rows = (uint64_t)(p.M - m0);
     __amdgpu_buffer_rsrc_t ra = make_rsrc_uniform(p.a + (uint64_t)m0 * K, a_rows * (uint64_t)K);
     const int nb0 = (n0 >> 4) + wave * NR;
-    const uint64_t b_off = (uint64_t)nb0 * 16ull * (uint64_t)K;
-    const uint64_t b_total = (uint64_t)p.N * (uint64_t)K;
+    const int KW = W4 ? K >> 1 : K;  // bytes of one W row
+    const uint64_t b_off = (uint64_t)nb0 * 16ull * (uint64_t)KW;
+    const uint64_t b_total = (uint64_t)p.N * (uint64_t)KW;
     __amdgpu_buffer_rsrc_t rb = make_rsrc_uniform(p.b + (b_off < b_total ? b_off : b_total), b_off < b_total ? b_total - b_off : 0);
 
     // MX scales: per (32-row chunk, 256-element K chunk) 64 dwords, one per lane.  Wavefront w brings A-side chunk w of the
@@ -178,25 +180,26 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     auto dma_sc = [&](int kt, int slot, int which) __attribute__((always_inline)) {
         const bool has = kt < kt_end;
         const uint32_t dst = lds_base + (uint32_t)(NS * STAGE + slot * SC_SLOT + which * 2048 + wave * 256);
-        dma4(which ? rsb : rsa, dst, has ? (uint32_t)lane * 4u : 0xFFFFFFF0u, has ? (uint32_t)(KIND == KIND_MXFP8 ? (kt >> 1) : kt) * 256u : 0u);
+        dma4(which ? rsb : rsa, dst, has ? (uint32_t)lane * 4u : 0xFFFFFFF0u, has ? (uint32_t)(KIND == KIND_MXFP4 ? kt : (kt >> 1)) * 256u : 0u);
     };
     auto read_sc = [&](int slot, int q, int* sa_dst, int* sb_dst) __attribute__((always_inline)) {
         if (q < MP) sa_dst[q] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + q * 256 + lane * 4);
         else sb_dst[0] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + 2048 + wave * 256 + lane * 4);
     };
     const uint32_t b_lane_off = p.b_rowmajor ? (uint32_t)li * (uint32_t)K + (uint32_t)lg * 16u : (uint32_t)lane * 16u;
-    const uint32_t b_step = p.b_rowmajor ? 128u : 2048u, b_half = p.b_rowmajor ? 64u : 1024u;
+    const uint32_t b_step = p.b_rowmajor ? 128u : W4 ? 1024u : 2048u, b_half = p.b_rowmajor ? 64u : 1024u;
     auto load_b1 = [&](int kt, int idx, v4i* lo, v4i* hi, auto CHK) __attribute__((always_inline)) {
-        const int ni = idx >> 1;
-        const bool has = !decltype(CHK)::value || (kt < kt_end && (kt * TK + (idx & 1) * 64) < K);
-        const uint32_t voff = b_lane_off + (uint32_t)ni * 16u * (uint32_t)K;
-        const v4i v = buf_load16(rb, has ? voff : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)(idx & 1) * b_half : 0u);
-        if (idx & 1) hi[ni] = v; else lo[ni] = v;
+        const int ni = W4 ? idx : idx >> 1, half = W4 ? 0 : idx & 1;
+        const bool has = !decltype(CHK)::value || (kt < kt_end && (kt * TK + half * 64) < K);
+        const uint32_t voff = b_lane_off + (uint32_t)ni * 16u * (uint32_t)KW;
+        const v4i v = buf_load16(rb, has ? voff : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
+        if (half) hi[ni] = v; else lo[ni] = v;
     };
     // fragment (16 rows x 2 x 16 bytes of K) of m-block mi from a stage: row mi*16 + li, chunks lg and 4 + lg; the swizzle
     // term (row/2)%8 = (li/2)%8 does not depend on mi
-    const int f_lo = li * TK + ((lg ^ ((li >> 1) & 7)) << 4);
-    const int f_hi = li * TK + (((4 + lg) ^ ((li >> 1) & 7)) << 4);
+    // (fp6: the 32-byte group lg, of which the first 24 bytes hold the 32 codes)
+    const int f_lo = li * TK + (((KIND == KIND_MXA6W4 ? 2 * lg : lg) ^ ((li >> 1) & 7)) << 4);
+    const int f_hi = li * TK + (((KIND == KIND_MXA6W4 ? 2 * lg + 1 : 4 + lg) ^ ((li >> 1) & 7)) << 4);
     auto read_frag = [&](int stage, int mi, v4i& flo, v4i& fhi) __attribute__((always_inline)) {
         flo = *reinterpret_cast<const v4i*>(&lds[stage * STAGE + mi * 16 * TK + f_lo]);
         fhi = *reinterpret_cast<const v4i*>(&lds[stage * STAGE + mi * 16 * TK + f_hi]);
@@ -212,7 +215,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     // (always_inline: with many call sites the inliner would otherwise leave this lambda a function of its own, with the
     // accumulators and descriptors passed through memory)
     constexpr int N_DMA = A_DMA + (MX ? 2 : 0);  // DMAs per wavefront per step
-    constexpr int N_W = 2 * NR;                  // W fragment loads per wavefront per step
+    constexpr int N_W = W4 ? NR : 2 * NR;        // W fragment loads per wavefront per step
     constexpr int N_OPS = A_DMA + (MX ? 1 : 0) + N_W;          // slots: the two scale DMAs share one
     constexpr int OPS_PER = (N_OPS + MR - 2) / (MR - 1);       // slots per m-block (m-blocks 1 .. MR-1)
     auto step = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
@@ -266,6 +269,17 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
                     constexpr int ni = decltype(NI)::value;
                     mfma_mx<1, ni & 1, mi & 1>(acc[mi][ni], bhi[SB][ni], ahi, sbv[SS][ni / 2], sav[SS][mi / 2]);
                 });
+            } else if constexpr (W4) {
+                static_for<NR>([&](auto NI) {
+                    constexpr int ni = decltype(NI)::value;
+                    if constexpr (KIND == KIND_MXA8W4) {
+                        const v8i af = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1], ahi[2], ahi[3]};
+                        mfma_mx4w<SS, ni & 1, mi & 1>(acc[mi][ni], blo[SB][ni], af, sbv[SS][ni / 2], sav[SS][mi / 2]);
+                    } else {
+                        const v6i af = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1]};
+                        mfma_mx4w<SS, ni & 1, mi & 1>(acc[mi][ni], blo[SB][ni], af, sbv[SS][ni / 2], sav[SS][mi / 2]);
+                    }
+                });
             } else if constexpr (KIND == KIND_MXFP8) {
                 const v8i af = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1], ahi[2], ahi[3]};
                 static_for<NR>([&](auto NI) {
@@ -315,7 +329,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     static_for<PFW>([&](auto I) {
         constexpr int i = decltype(I)::value;
 #pragma unroll
-        for (int idx = 0; idx < 2 * NR; idx++) load_b1(kt_begin + i, idx, blo[i], bhi[i], std::true_type{});
+        for (int idx = 0; idx < N_W; idx++) load_b1(kt_begin + i, idx, blo[i], bhi[i], std::true_type{});
     });
     if constexpr (SCALED && STORE != STORE_ACC) {
         if (tid < TM) reinterpret_cast<float*>(lds_x)[tid] = ep_sa;

@@ -27,6 +27,7 @@ bool psg_moe_gate_sort_fuses(int tokens, int topk, int experts);
 hipError_t psg_launch_moe_reduce(const void* x, void* y, int tokens, int topk, int dim, int out_dtype, const int32_t* mask,
                                  const int32_t* ids, int experts, hipStream_t stream);
 hipError_t psg_launch_mx_generic(const MxGenParams& p, int af, int bf, int store, int batch, hipStream_t stream);
+hipError_t psg_launch_tiled_mxw4(const A8W8Params& p, bool fp6, hipStream_t stream);
 hipError_t psg_launch_mx_smallm(const MxGenParams& p, int af, int bf, int batch, hipStream_t stream);
 hipError_t psg_launch_mxfp4_smallm(const MxParams& p, int store, int nw, hipStream_t stream);
 hipError_t psg_launch_splitk_finalize(const A8W8Params& p, const void* partial, int is_int, int scaled, hipStream_t stream);
@@ -200,6 +201,15 @@ int pick_splits(int M, int N, int kbytes, Tile t) {
         if (fits && steps / c >= min_steps && (long)c * M * 16 <= (long)kbytes * 5) s = c;
     }
     return s;
+}
+
+// Whether fp8 / fp6 x fp4, and one batch of several of the fp4 and fp8 pairs too, runs on the tiles of the dense kernels: where 128x256
+// tiles would give every CU one.  There the general kernel works on 128x256 tiles, and one of those takes as long as a 256x256
+// tile does here (fp8 x fp4, us 256x256 / general: 500x16384x4096 42.9 / 48.7, 1000x8192x4096 42.6 / 47.3, 1024x16384x2048 30.4 /
+// 51.7, 1280x8192x4096 41.3 / 87.2, 4096x4096x8192 92.2 / 169.5, 8192x1024x14336 124 / 146); with fewer its 64x128 tiles and its K
+// splits are the better way (768x8192x4096 39.4 / 34.7, 1000x4096x14336 115 / 63).
+bool mx_fills_tiles(int M, int N) {
+    return M > kStreamMaxM && (long)((M + 127) / 128) * (long)((N + 255) / 256) >= psg_cu_count();
 }
 
 // Which calls of the general MX path the small-M kernel takes (the others: gemm_mx_generic.hip).
@@ -554,7 +564,15 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
     if (a->force_path == 1 && !fp4_fast && !fp8_pair)
         return fail(PSG_E_SHAPE, "force_path=1 is for dense, unbatched fp4 x fp4 or fp8 x fp8 only");
     if (a->force_path == 2 && a->M > kStreamMaxM) return fail(PSG_E_SHAPE, "small-M path needs M <= %d, got %d", kStreamMaxM, a->M);
-    if (fp8_tiled) {
+    // fp8 / fp6 x fp4, and batches of these and of the fp4 and fp8 pairs: a launch of the dense tiles per batch
+    const int64_t a_bs = a->a_batch_stride ? a->a_batch_stride : (int64_t)((uint64_t)a->M * a_rs);
+    const int64_t c_bs = a->c_batch_stride ? a->c_batch_stride : (int64_t)((uint64_t)a->M * c_rs * 2);
+    const int64_t sa_bs = a->scale_a_batch_stride ? a->scale_a_batch_stride : (int64_t)((uint64_t)((a->M + 31) / 32) * sa_cs);
+    const bool w4 = a->b_dtype == PSG_MX_FP4 && a->a_dtype != PSG_MX_FP4;
+    const bool same = a->b_dtype == a->a_dtype && batch > 1;
+    const bool per_batch = (w4 || same) && dense && store == STORE_C && a->force_path == 0 && batch <= 8 && mx_fills_tiles(a->M, a->N) && a_bs % 16 == 0 &&
+                           c_bs % 16 == 0 && sa_bs % 4 == 0;
+    if (fp8_tiled || per_batch) {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
         const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : pick_tile(a->M, a->N, true, 0, 0);
         A8W8Params q{};
@@ -572,8 +590,18 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         q.splits = 1;
         q.epi = EPI_NONE;
         q.out = a->out_dtype;
-        const hipError_t te = psg_launch_a8w8_tiled(q, KIND_MXFP8, store, t.m, t.n, static_cast<hipStream_t>(stream));
-        if (te != hipSuccess) return hip_fail(te, "psg_gemm_mxfp4 launch");
+        const bool fp4 = a->a_dtype == PSG_MX_FP4;
+        if (fp4) q.wave_layout = t.waves == 8 ? 8 : 1;
+        for (int z = 0; z < batch; z++) {
+            const hipError_t te = w4 ? psg_launch_tiled_mxw4(q, a->a_dtype == PSG_MX_FP6, static_cast<hipStream_t>(stream))
+                                     : psg_launch_a8w8_tiled(q, fp4 ? KIND_MXFP4 : KIND_MXFP8, store, t.m, t.n, static_cast<hipStream_t>(stream));
+            if (te != hipSuccess) return hip_fail(te, "psg_gemm_mxfp4 launch");
+            q.c = static_cast<uint8_t*>(q.c) + c_bs;
+            q.a += a_bs;
+            q.b += (uint64_t)a->N * b_row;
+            q.mx_sa += sa_bs;
+            q.mx_sb += (uint64_t)(a->N / 32) * chunk;
+        }
         g_err[0] = 0;
         return 0;
     }
@@ -592,10 +620,10 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         g.a_row_stride = (int64_t)a_rs;
         g.c_row_stride = (int64_t)c_rs;
         g.sa_chunk_stride = (int64_t)sa_cs;
-        g.a_batch = a->a_batch_stride ? a->a_batch_stride : (int64_t)((uint64_t)a->M * a_rs);
+        g.a_batch = a_bs;
         g.b_batch = (int64_t)((uint64_t)a->N * b_row);
-        g.c_batch = store == STORE_ACC ? (int64_t)a->M * a->N * 4 : (a->c_batch_stride ? a->c_batch_stride : (int64_t)((uint64_t)a->M * c_rs * 2));
-        g.sa_batch = a->scale_a_batch_stride ? a->scale_a_batch_stride : (int64_t)((uint64_t)((a->M + 31) / 32) * sa_cs);
+        g.c_batch = store == STORE_ACC ? (int64_t)a->M * a->N * 4 : c_bs;
+        g.sa_batch = sa_bs;
         g.sb_batch = (int64_t)((uint64_t)(a->N / 32) * chunk);
         hipError_t ge;
         const bool small = store == STORE_C && a->force_path == 0 && mx_general_small(a->M, a->N, a->K, a->b_dtype == PSG_MX_FP8);

@@ -309,3 +309,32 @@ def test_small_m_kernel_against_the_general_kernel(a_dtype, b_dtype, M, N, K, ba
         ref = _ref(d[b])
         for o in (outs[0][b], outs[2][b]):
             assert np.all(np.abs(o - ref) <= 2.0 ** -8 * np.abs(ref) + 1.01 * _acc_atol(d[b], ref) + 1e-4 * np.abs(ref))
+
+
+# the dense 256x256 tiles behind fp8 / fp6 x fp4 and behind batches: ragged last tiles, the shortest K, K steps that are no multiple of the
+# pipeline's stages, batches apart from each other; the general kernel adds in the same order, so the bits agree
+@pytest.mark.parametrize("a_dtype,b_dtype", [("fp8", "fp4"), ("fp6", "fp4"), ("fp4", "fp4"), ("fp8", "fp8")])
+@pytest.mark.parametrize("M,N,K,batch,apart", [(8000, 1056, 256, 1, 0), (129, 32768, 768, 1, 0), (1000, 8224, 1280, 2, 0), (2056, 4096, 512, 3, 64)])
+def test_dense_tiles_against_the_general_kernel(a_dtype, b_dtype, M, N, K, batch, apart):
+    from kernels.gemm.mxfp4_preshuffle import launch_gemm
+
+    if a_dtype == b_dtype and batch == 1:
+        batch = 2
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    byte = lambda *s, hi=256: torch.randint(0, hi, s, generator=g, device="cuda", dtype=torch.uint8)
+    row = lambda f: K // 2 if f == "fp4" else K
+    fp8 = lambda t: t & 0xB7  # clears bits 6 and 3: no NaN code, magnitudes below 2
+    a_bs, m32 = M * row(a_dtype) + apart * 16, (M + 31) // 32 * 32
+    a, b = byte(batch * a_bs), byte(batch * N * row(b_dtype))
+    a, b = (fp8(a) if a_dtype == "fp8" else a), (fp8(b) if b_dtype == "fp8" else b)
+    sa_bs = m32 * (K // 32) + apart * 4
+    sa, sb = byte(batch * sa_bs, hi=4) + 124, byte(batch * N * (K // 32), hi=4) + 124
+    c_bs = M * N * 2 + apart * 16
+    outs = []
+    for path in (0, 3):
+        c = torch.zeros(batch * c_bs // 2, dtype=torch.bfloat16, device="cuda")
+        launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, a_dtype, "bf16", b_dtype, batch, -1, a_bs, -1, sa_bs, -1, c_bs, 0, 0, _force_path=path)
+        outs.append(c)
+    torch.cuda.synchronize()
+    assert outs[1].count_nonzero() > 0.9 * batch * M * N
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
