@@ -1,4 +1,4 @@
-// Small-M (M <= 64) MX preshuffle GEMM for every format the general kernel takes: A in fp4 / fp6 / fp8, W in fp4 / fp8, strided
+// Small-M MX preshuffle GEMM (64 rows a workgroup) for every format the general kernel takes: A in fp4 / fp6 / fp8, W in fp4 / fp8, strided
 // rows, batches over blockIdx.z.  Operand and scale layouts: gemm_mx_generic.hip.
 //
 // Bound: the bytes of W and, from 32 rows on, of A, which every workgroup reads whole.  A workgroup owns 32 columns and splits K over
@@ -52,6 +52,7 @@ __global__ void __launch_bounds__(NW * 64) k_mx_smallm(MxGenParams p) {
     // neighbours share are completed in one L2
     const int np = (gridDim.x & 7) == 0 ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
     const uint64_t z = blockIdx.z;
+    const int m0 = (int)blockIdx.y * (16 * MB), M = p.M - m0;  // rows of this workgroup: up to 16 MB from m0 on (MB = 4 beyond 64 rows)
     const int KT = p.K >> 8;
     const int per = (KT + NW - 1) / NW;
     const int s_begin = wave * per;
@@ -60,9 +61,9 @@ __global__ void __launch_bounds__(NW * 64) k_mx_smallm(MxGenParams p) {
     const uint32_t a_row_bytes = AF == MXF_FP4 ? (uint32_t)p.K >> 1 : (uint32_t)p.K;
     const uint32_t a_rs = (uint32_t)p.a_row_stride, sa_cs = (uint32_t)p.sa_chunk_stride, chunk_bytes = (uint32_t)KT * 256u;
 
-    __amdgpu_buffer_rsrc_t ra = make_rsrc_uniform(p.a + z * (uint64_t)p.a_batch, (uint64_t)(p.M - 1) * a_rs + a_row_bytes);  // rows >= M read as zero
+    __amdgpu_buffer_rsrc_t ra = make_rsrc_uniform(p.a + z * (uint64_t)p.a_batch + (uint64_t)m0 * a_rs, (uint64_t)(M - 1) * a_rs + a_row_bytes);  // rows >= M read as zero
     __amdgpu_buffer_rsrc_t rb = make_rsrc(p.b + z * (uint64_t)p.b_batch + (uint64_t)np * 32ull * b_row_bytes, 32ull * b_row_bytes);
-    __amdgpu_buffer_rsrc_t rsa = make_rsrc(p.sa + z * (uint64_t)p.sa_batch, (uint64_t)(((p.M + 31) >> 5) - 1) * sa_cs + chunk_bytes);
+    __amdgpu_buffer_rsrc_t rsa = make_rsrc(p.sa + z * (uint64_t)p.sa_batch + (uint64_t)(m0 >> 5) * sa_cs, (uint64_t)(((M + 31) >> 5) - 1) * sa_cs + chunk_bytes);
     __amdgpu_buffer_rsrc_t rsb = make_rsrc(p.sb + z * (uint64_t)p.sb_batch + (uint64_t)np * chunk_bytes, chunk_bytes);
     // the lane's 16-byte pieces of a 128-element step of its A row: fp4 g; fp6 2g, 2g + 1; fp8 g, 4 + g
     const uint32_t a_voff = (uint32_t)li * a_rs + (uint32_t)lg * 16u;
@@ -180,16 +181,17 @@ __global__ void __launch_bounds__(NW * 64) k_mx_smallm(MxGenParams p) {
 #pragma unroll
         for (int j = 1; j < NW; j++) sum += part[j];
         const int m = mb * 16 + li, n = np * 32 + nb * 16 + lg * 4;
-        if (m < p.M) *reinterpret_cast<v2i*>(c + (int64_t)m * p.c_row_stride + n) = p.out == OUT_BF16 ? pack4_out16<OUT_BF16>(sum[0], sum[1], sum[2], sum[3]) : pack4_out16<OUT_FP16>(sum[0], sum[1], sum[2], sum[3]);
+        if (m < M) *reinterpret_cast<v2i*>(c + (int64_t)(m0 + m) * p.c_row_stride + n) = p.out == OUT_BF16 ? pack4_out16<OUT_BF16>(sum[0], sum[1], sum[2], sum[3]) : pack4_out16<OUT_FP16>(sum[0], sum[1], sum[2], sum[3]);
     }
 }
 
 template <int AF, int BF>
 hipError_t launch_fmt(const MxGenParams& p, int batch, hipStream_t stream) {
+    const int groups = (p.M + 63) / 64;  // of 64 rows
     const bool wide = p.K >= 2048;  // eight wavefronts once each has a whole step
 #define PSG_GO(MB_)                                                                                                                     \
-    if (wide) hipLaunchKernelGGL((k_mx_smallm<AF, BF, MB_, 8>), dim3(p.N / 32, 1, batch), dim3(512), 0, stream, p);                      \
-    else hipLaunchKernelGGL((k_mx_smallm<AF, BF, MB_, 4>), dim3(p.N / 32, 1, batch), dim3(256), 0, stream, p);
+    if (wide) hipLaunchKernelGGL((k_mx_smallm<AF, BF, MB_, 8>), dim3(p.N / 32, groups, batch), dim3(512), 0, stream, p);                      \
+    else hipLaunchKernelGGL((k_mx_smallm<AF, BF, MB_, 4>), dim3(p.N / 32, groups, batch), dim3(256), 0, stream, p);
     if (p.M <= 16) { PSG_GO(1) } else if (p.M <= 32) { PSG_GO(2) } else { PSG_GO(4) }
 #undef PSG_GO
     return hipGetLastError();
@@ -197,7 +199,7 @@ hipError_t launch_fmt(const MxGenParams& p, int batch, hipStream_t stream) {
 
 }  // namespace
 
-// 16-bit output, 1 <= M <= 64; af: MXF_FP4 / MXF_FP6 / MXF_FP8; bf: MXF_FP4 / MXF_FP8; batch >= 1 (grid.z <= 65535)
+// 16-bit output, M >= 1 (meant for up to a few hundred rows, 64 a workgroup); af: MXF_FP4 / MXF_FP6 / MXF_FP8; bf: MXF_FP4 / MXF_FP8; batch >= 1 (grid.z <= 65535)
 hipError_t psg_launch_mx_smallm(const MxGenParams& p, int af, int bf, int batch, hipStream_t stream) {
     if (bf == MXF_FP4) {
         if (af == MXF_FP4) return launch_fmt<MXF_FP4, MXF_FP4>(p, batch, stream);

@@ -218,9 +218,16 @@ bool mx_fills_tiles(int M, int N) {
 // fp8 x fp4 1 x 8192 x 8192 7.7 / 12.2, 64 x 8192 x 8192 12.3 / 20.2, 64 x 4096 x 4096 6.9 / 16.0, 16 x 1024 x 2048 3.1 / 6.8, 64 x 1024 x
 // 14336 15.7 / 27.3, 64 x 16384 x 4096 (134 MB) 14.5 / 17.7, 16 x 16384 x 14336 (117 MB) 22.6 / 23.2, but 24 rows of it (235 MB) 25.9 / 24.1
 // and 64 (470 MB) 37.5 / 32.0; fp8 x fp8 32 x 16384 x 14336 (235 MB) 40.9 / 46.8, 64 rows 51.1 / 48.8; fp6 x fp4 as fp8 x fp4.
-bool mx_general_small(int M, int N, int K, bool fp8_weights) {
+// Beyond 64 rows a workgroup takes 64 of them, and the kernel is the better one while its workgroups make one round of one per CU, or two on
+// rows of up to 8192 elements (fp8 x fp4, 128 x 2048 x 4096 6.7 / 16.1, 256 x 1024 x 14336 16.6 / 46.8, 128 x 4096 x 4096 7.2 / 16.2; two
+// rounds 256 x 4096 x 4096 12.8 / 16.5, 128 x 8192 x 8192 22.8 / 29.0; three 192 x 8192 x 8192 32.8 / 29.1, four 128 x 16384 x 4096 26 / 18).
+bool mx_general_small(int M, int N, int K, bool fp8_weights, int batch) {
+    if (M > kStreamMaxM) {
+        const long wgs = (long)(N / 32) * ((M + 63) / 64) * batch, cus = psg_cu_count();
+        return N >= 1024 && wgs <= (K <= 8192 ? 2 : 1) * cus;
+    }
     const long rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
-    return M <= kStreamMaxM && N >= 1024 && (long)(N / 32) * rows * K <= (fp8_weights ? 320L : 160L) * 1000000L;
+    return N >= 1024 && (long)(N / 32) * rows * K <= (fp8_weights ? 320L : 160L) * 1000000L;
 }
 
 // Split-K for the general MX kernel: its tiles are 64x128 (32x128 for M <= 32), so decode-like shapes launch few
@@ -626,7 +633,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         g.sa_batch = sa_bs;
         g.sb_batch = (int64_t)((uint64_t)(a->N / 32) * chunk);
         hipError_t ge;
-        const bool small = store == STORE_C && a->force_path == 0 && mx_general_small(a->M, a->N, a->K, a->b_dtype == PSG_MX_FP8);
+        const bool small = store == STORE_C && a->force_path == 0 && mx_general_small(a->M, a->N, a->K, a->b_dtype == PSG_MX_FP8, batch);
         const int splits = !small && batch == 1 && c_rs == (uint64_t)a->N && store == STORE_C ? mx_general_splits(a->M, a->N, a->K) : 1;
         if (small) {
             ge = psg_launch_mx_smallm(g, a->a_dtype, a->b_dtype, batch, static_cast<hipStream_t>(stream));

@@ -287,7 +287,7 @@ def test_general_kernel_large_tile(a_dtype, b_dtype):
 # the small-M kernel: edges of its 16-row tiles, one K step and several per wavefront, four and eight wavefronts, a wavefront without a
 # step (K = 256 * odd), N that is no multiple of the XCD count's 256 columns, two batches with rows apart
 @pytest.mark.parametrize("a_dtype,b_dtype", PAIRS)
-@pytest.mark.parametrize("M,N,K,batch", [(1, 1024, 256, 2), (15, 1056, 1280, 1), (16, 1024, 2048, 1), (17, 1184, 2304, 2), (32, 1024, 6400, 1), (33, 1024, 2560, 1), (64, 1088, 1024, 2)])
+@pytest.mark.parametrize("M,N,K,batch", [(1, 1024, 256, 2), (15, 1056, 1280, 1), (16, 1024, 2048, 1), (17, 1184, 2304, 2), (32, 1024, 6400, 1), (33, 1024, 2560, 1), (64, 1088, 1024, 2), (65, 1024, 768, 2), (200, 1056, 2048, 1)])
 def test_small_m_kernel_against_the_general_kernel(a_dtype, b_dtype, M, N, K, batch):
     if (a_dtype, b_dtype) == ("fp4", "fp4") and batch == 1:
         pytest.skip("dense fp4 x fp4 has kernels of its own")
