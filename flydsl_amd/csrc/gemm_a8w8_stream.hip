@@ -1,4 +1,4 @@
-// Memory-bound small-M (M <= 32) path of the 8-bit / 16-bit preshuffle GEMM for gfx950.
+// Memory-bound small-M path (64 rows a workgroup) of the 8-bit / 16-bit preshuffle GEMM for gfx950.
 //
 // The whole cost is streaming W once (N*K bytes), so the launch is shaped by the memory system, not by the MFMAs:
 //   * The columns are dealt out in units of 8 (half a preshuffled 16-row block), evenly over one workgroup per CU:
@@ -91,6 +91,9 @@ __global__ void __launch_bounds__(NWAVES * 64) k_a8w8_stream(A8W8Params p) {
     // C that neighbouring workgroups share are merged in one L2 instead of being written back from several.
     const int bid = (gridDim.x & 7) == 0 ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
     const int grp = bid * gpw + (wave >> ksh);
+    // rows of this workgroup: up to ROWS from m0 on.  Only the 64-row build has more than one group (in the 16-row build the two extra
+    // scalar operations in front of the loads cost 0.08 of 6.15 us)
+    const int m0 = MB == 4 ? (int)blockIdx.y * ROWS : 0, M = p.M - m0;
     const int steps = (K + 127) >> 7;
     const int per = (steps + ks - 1) >> ksh;
     const int s_begin = my_ks * per;
@@ -121,7 +124,7 @@ __global__ void __launch_bounds__(NWAVES * 64) k_a8w8_stream(A8W8Params p) {
         const int ne = gq < tg ? unit_begin(gq + 1) << 3 : 0;
         m = (frag % MB) * 16 + li;
         n = nb + (frag / MB) * 16 + lg * 4;
-        live = g < gpw && n < ne && m < p.M;
+        live = g < gpw && n < ne && m < M;
     };
     auto fetch_scales = [&]() {
         if constexpr (STORE != STORE_ACC && !IS16) {
@@ -131,7 +134,7 @@ __global__ void __launch_bounds__(NWAVES * 64) k_a8w8_stream(A8W8Params p) {
                 bool live;
                 item_coords(tid + f * NWAVES * 64, g, frag, m, n, live);
                 // clamp the ADDRESS of dead items instead of selecting the loaded value (a select would wait here)
-                fin_sa[f] = p.sa[live ? m : 0];
+                fin_sa[f] = p.sa[m0 + (live ? m : 0)];
                 fin_sb[f] = *reinterpret_cast<const v4f*>(p.sb + (live ? n : 0));
             }
         }
@@ -139,7 +142,8 @@ __global__ void __launch_bounds__(NWAVES * 64) k_a8w8_stream(A8W8Params p) {
 
     if (nchunks > 0 && n_end > n_begin) {
         __amdgpu_buffer_rsrc_t rb = make_rsrc(p.b, (uint64_t)p.N * (uint64_t)K);
-        __amdgpu_buffer_rsrc_t ra = ADMA ? make_rsrc_uniform(p.a, (uint64_t)p.M * (uint64_t)K) : make_rsrc(p.a, (uint64_t)p.M * (uint64_t)K);
+        const uint8_t* a = p.a + (uint64_t)m0 * (uint64_t)K;
+        __amdgpu_buffer_rsrc_t ra = ADMA ? make_rsrc_uniform(a, (uint64_t)M * (uint64_t)K) : make_rsrc(a, (uint64_t)M * (uint64_t)K);
         v4i* my_patch = patch[wave];
         const uint32_t patch_lds = (uint32_t)(uintptr_t)my_patch;
         // per-window W offset of this lane: row n of the window, 16-byte K group lg of a 1 KB block
@@ -318,7 +322,7 @@ __global__ void __launch_bounds__(NWAVES * 64) k_a8w8_stream(A8W8Params p) {
 #pragma unroll
             for (int j = 1; j < NWAVES; j++)
                 if (j < ks) sum += part[j];
-            const size_t idx = (size_t)m * (size_t)p.N + (size_t)n;
+            const size_t idx = (size_t)(m0 + m) * (size_t)p.N + (size_t)n;
             if constexpr (STORE == STORE_ACC) {
                 *reinterpret_cast<acc_t*>(reinterpret_cast<uint8_t*>(p.c) + idx * 4) = sum;
             } else {
@@ -339,10 +343,10 @@ __global__ void __launch_bounds__(NWAVES * 64) k_a8w8_stream(A8W8Params p) {
 
 template <int KIND, int NWAVES, int CH, int STORE>
 hipError_t launch_kind(const A8W8Params& p, int nwin, int grid, hipStream_t stream) {
-    const int mb = (p.M + 15) / 16;
+    const int mb = p.M > 48 ? 4 : (p.M + 15) / 16, groups = (p.M + 63) / 64;
 #define PSG_GO(MB_, NWIN_)                                                                                                   \
     {                                                                                                                        \
-        hipLaunchKernelGGL((k_a8w8_stream<KIND, MB_, NWIN_, NWAVES, CH, STORE>), dim3(grid), dim3(NWAVES * 64), 0, stream, p); \
+        hipLaunchKernelGGL((k_a8w8_stream<KIND, MB_, NWIN_, NWAVES, CH, STORE>), dim3(grid, groups), dim3(NWAVES * 64), 0, stream, p); \
         return hipGetLastError();                                                                                            \
     }
     if (mb == 1) {
@@ -369,7 +373,8 @@ hipError_t launch_planned(const A8W8Params& p0, int kbytes, hipStream_t stream) 
     while (ks > 1 && ks * 2 > steps) ks >>= 1;
     const int gpw = nwaves / ks;
     const long units = p.N / 8;
-    const long cus = psg_cu_count();
+    // beyond 64 rows the workgroups of all 64-row groups together are dealt out over the CUs
+    const long groups = (p.M + 63) / 64, cus = psg_cu_count() > groups ? psg_cu_count() / groups : 1;
     const long rounds = (units + 4 * cus * gpw - 1) / (4 * cus * gpw);
     long tg = cus * gpw * rounds;  // column groups: a whole number of workgroups per CU ...
     if (tg > units) tg = units;    // ... but never less than one 8-column unit per group
@@ -385,7 +390,7 @@ hipError_t launch_planned(const A8W8Params& p0, int kbytes, hipStream_t stream) 
 
 }  // namespace
 
-// Host entry used by the C-ABI layer.  Requires 1 <= M <= 64.  Plans the launch: wavefronts per workgroup by the
+// Host entry used by the C-ABI layer.  Requires M >= 1 (64 rows a workgroup).  Plans the launch: wavefronts per workgroup by the
 // row length, K slices per workgroup so that a slice holds at least two K steps, then column groups dealt out
 // evenly over a multiple of the CU count (at most four 8-column units per group, at least one).
 hipError_t psg_launch_a8w8_stream(const A8W8Params& p, int kind, int store, hipStream_t stream) {

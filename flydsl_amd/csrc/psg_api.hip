@@ -98,9 +98,13 @@ bool mx_takes_small(int M, int N, int K) {
 // 4.3 / 8.0, 6144x4096 9.2 / 14.1, 8192x8192 15.3 / 19.6, 28672x4096 31.7 / 32.3, 2048x16384 15.5 / 16.0; M=48 9.7 / 14.4,
 // 16.5 / 20.4, 33.0 / 31.3, 17.3 / 16.3; M=64 1024x2048 5.5 / 8.2, 6144x4096 11.3 / 15.0, 8192x8192 18.3 / 22.2,
 // 5120x8192 15.8 / 19.0, 28672x4096 37.5 / 32.7, 2048x16384 20.0 / 15.6).
+// Beyond 64 rows a workgroup takes 64 of them, and the kernel is the better one while 32 columns a workgroup make one round of the CUs (N
+// times the 64-row groups up to 8192) on rows of 2 to 4 KB (us streaming / tiled plan: fp8 80x1024x4096 6.6 / 9.5, 256x1024x4096 7.2 /
+// 10.1, 128x2048x2048 4.8 / 7.3, 128x4096x4096 9.9 / 11.9, 192x2048x2048 7.2 / 7.4; bf16 256x1024x1024 4.8 / 6.8, 128x2048x2048 7.4 /
+// 10.4; but fp8 128x4096x1024 6.2 / 5.5, 192x2048x8192 17.4 / 14.7, 192x4096x4096 19.4 / 11.5).
 bool takes_stream(int M, int N, int kbytes) {
     if (M <= kSmallM) return true;
-    if (M > kStreamMaxM) return false;
+    if (M > kStreamMaxM) return M <= 256 && kbytes >= 2048 && kbytes <= 4096 && (long)N * ((M + 63) / 64) <= 8192;
     const long w = (long)N * kbytes, a = (long)M * kbytes;
     return a <= (512L << 10) && w <= (80L << 20);
 }

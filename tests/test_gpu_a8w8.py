@@ -272,3 +272,24 @@ def test_fp8_eight_wavefront_tile(epilogue):
         ref = O.apply_bias_act(ref, bias.float().numpy(), "silu")
     c = _launch(d, M, N, K, force_path=1, tile=(256, 256), epilogue=epilogue, bias=bias, wave_layout=8)
     _check_fp(c[:M].float().cpu().numpy(), ref)
+
+
+# the streaming kernel beyond 64 rows: last 64-row groups of 1, 16, 36 and 64 rows, columns that do not divide evenly, a K tail of 64 bytes,
+# four and eight wavefronts; int8 sums are exact, so the scaled and rounded output is too
+@pytest.mark.parametrize("M,N,K", [(65, 4096, 2048), (80, 1040, 4096), (100, 4080, 2112), (192, 2720, 4032), (256, 2048, 2048), (256, 1024, 4096)])
+def test_streaming_kernel_beyond_64_rows(M, N, K):
+    from flydsl_amd import _lib, layout
+    from kernels.gemm.preshuffle_gemm import compile_preshuffle_gemm
+
+    assert _lib.lib().psg_workspace_bytes(M, N, K, 0) == 0  # the streaming kernel is what takes it
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    a = torch.randint(-127, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
+    w = torch.randint(-127, 128, (N, K), generator=g, device="cuda", dtype=torch.int8)
+    sa, sb = torch.rand(M, generator=g, device="cuda") + 0.5, torch.rand(N, generator=g, device="cuda") + 0.5
+    c = torch.full((M + 3, N), -8192.0, dtype=torch.bfloat16, device="cuda")
+    fn = compile_preshuffle_gemm(N=N, K=K, tile_m=64, tile_n=128, tile_k=64, in_dtype="int8")
+    fn(c, a, layout.shuffle_weight(w).contiguous(), sa, sb, torch.empty(0, dtype=torch.bfloat16, device="cuda"), M, N, torch.cuda.current_stream())
+    acc = (a.double() @ w.double().T).float()  # whole numbers below 2^53, then the int32 -> fp32 rounding
+    want = ((acc * sa[:, None]) * sb[None, :]).bfloat16()
+    assert torch.equal(c[:M], want)
+    assert (c[M:] == -8192.0).all()
