@@ -173,7 +173,8 @@ def flydsl_mxfp4_gemm2(*, inter_sorted_quant, inter_sorted_shuffled_scale, w2_u8
     args.stage, args.atomic, args.pad0 = 2, int(atomic), 0
     lib = _lib.lib()
     h = _lib.stream_handle(stream)
-    need = lib.psg_moe_rows_workspace_bytes(args.tokens, int(topk), max_sorted, args.model_dim, args.out_dtype, 1) if atomic else 0
+    # (the stage itself has no use for topk; without a number it adds directly)
+    need = lib.psg_moe_rows_workspace_bytes(args.tokens, int(topk), max_sorted, args.model_dim, args.out_dtype, 1) if atomic and topk else 0
     ws = _lib.call_scratch(flat_out.device, need, h) if need else None
     if ws is None:
         rc = lib.psg_moe_mx_gemm(ctypes.byref(args), h)
