@@ -43,15 +43,22 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc_uniform(const void* 
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((uintptr_t)(((uint64_t)hi << 32) | lo)), 0, (int)n, 0x00020000);
 }
 
-// one DMA instruction: 64 lanes x 16 bytes from (descriptor, voff + soff) to LDS [lds_addr, lds_addr + 1024)
+// One DMA instruction: 64 lanes x 16 bytes from (descriptor, voff + soff) to LDS [lds_addr, lds_addr + 1024).
+// A vector memory instruction must stay five wait states behind a vector instruction that wrote one of its scalar operands, and the compiler
+// does not know that this statement is one: where scalar registers run short it fetched `soff` back from a vector register (v_readlane)
+// directly in front.  So the offset goes through a scalar move, which waits by itself and is at the same time the wait state behind
+// the write of M0 (the s_nop it replaces: the statement is no longer than before).  The descriptor must come from make_rsrc_uniform and
+// stay in scalar registers; tests/test_wait_states.py looks at what was built.
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane((int)soff))
+    int so;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b32 %0, %4\n\tbuffer_load_dwordx4 %2, %3, %0 offen lds" : "=&s"(so) : "s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane((int)soff))
                  : "memory");
 }
 
 // 4 bytes per lane: 64 lanes x 4 bytes to LDS [lds_addr, lds_addr + 256)
 __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane((int)soff))
+    int so;
+    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b32 %0, %4\n\tbuffer_load_dword %2, %3, %0 offen lds" : "=&s"(so) : "s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane((int)soff))
                  : "memory");
 }
 
