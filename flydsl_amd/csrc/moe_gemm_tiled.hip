@@ -10,6 +10,8 @@
 // k_moe_gemm (128 rows x 64 or 128 columns) are bound by their operand traffic: 128 flop per byte against 256 here.  Measured, 4096
 // tokens x top-8 on 32 experts, 4096 x 1536, fp8: stage 1 473 -> 391 us, stage 2 (one row per sorted position) 360 -> 273; int8 528 ->
 // 423.  Of the 56 us of a stage-1 tile 43 are the loop, 7 the epilogue and the rest its start.  The bits are those of k_moe_gemm.
+// Registers: all 256 vector registers a lane are in use; 4 to 20 of them and about 40 scalar registers spill, none inside the unchecked
+// loop (scratch stores between the loops and the epilogue, scalars into lanes of a vector register around the prologue).
 //
 // The tiles: blocks pair up from the start of each run of equal expert ids; the last block of an odd run is a tile of its own, for
 // which only the lower eight 16-row blocks are multiplied.  How many tiles there are is only known on the device, so every
@@ -169,9 +171,11 @@ __global__ void __launch_bounds__(512, 1) k_moe_tiled(MoeParams p) {
     constexpr int FRAG_AHEAD = 2, FRAG_BUFS = 4;
     v4i flo[FRAG_BUFS], fhi[FRAG_BUFS];
 
-    // one K step over ML 16-row blocks (all sixteen, or the lower eight of a tile without a second block)
+    // one K step over ML 16-row blocks (all sixteen, or the lower eight of a tile without a second block).  END: it may be the last one, so
+    // the wait states between its last MFMA and the first ordinary read of an accumulator stand in the statement that ends it: behind
+    // the loops the compiler may spill accumulators before it comes to any statement of ours (it stores up to 20 registers there)
     constexpr int N_W = 2 * NR;
-    auto step = [&](int kt, auto SP, auto CHK, auto MLP) __attribute__((always_inline)) {
+    auto step = [&](int kt, auto SP, auto CHK, auto MLP, auto END) __attribute__((always_inline)) {
         constexpr int S = decltype(SP)::value, ML = decltype(MLP)::value;
         constexpr int SB = S % NB, SN = (SB + 1) % NB;
         constexpr int N_OPS = A_DMA + N_W, OPS_PER = (N_OPS + ML - 2) / (ML - 1);
@@ -206,7 +210,8 @@ __global__ void __launch_bounds__(512, 1) k_moe_tiled(MoeParams p) {
             }
             __builtin_amdgcn_sched_barrier(0);
         });
-        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N_W + (NS - 3) * (A_DMA + N_W)) : "memory");
+        if constexpr (decltype(END)::value) asm volatile("s_nop 15\n\ts_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N_W + (NS - 3) * (A_DMA + N_W)) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(N_W + (NS - 3) * (A_DMA + N_W)) : "memory");
     };
 
     // prologue: the epilogue's factors, A(0..2) by DMA, W(0)
@@ -237,17 +242,17 @@ __global__ void __launch_bounds__(512, 1) k_moe_tiled(MoeParams p) {
     auto mainloop = [&](auto MLP) __attribute__((always_inline)) {
         int kt = 0;
         for (; kt + 2 * NS - 1 <= KT; kt += NS)
-            static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::false_type{}, MLP); });
+            static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::false_type{}, MLP, std::false_type{}); });
         for (; kt + NS <= KT; kt += NS)
-            static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::true_type{}, MLP); });
+            static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::true_type{}, MLP, std::bool_constant<decltype(I)::value == NS - 1>{}); });
         static_for<NS - 1>([&](auto I) {
-            if (kt + decltype(I)::value < KT) step(kt + decltype(I)::value, I, std::true_type{}, MLP);
+            if (kt + decltype(I)::value < KT) step(kt + decltype(I)::value, I, std::true_type{}, MLP, std::true_type{});
         });
     };
     if (paired) mainloop(std::integral_constant<int, 16>{});
     else mainloop(std::integral_constant<int, 8>{});
-    // wait states behind the last MFMA, and every DMA still on its way must land before the stages are reused
-    asm volatile("s_nop 15\n\ts_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    // every DMA still on its way must land before the stages are reused
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 
     // ---- epilogue: 16-bit rows through LDS (16-byte granules XOR-swizzled by the row), then out row by row ----
     int lane_e;

@@ -10,7 +10,9 @@ the built code itself is looked at.  From every producer all paths are followed 
   * a register written by an MFMA and used by anything but an MFMA that takes exactly it as SrcC: 8 for 4 passes, 12 for 8
   * a vector register written by a vector instruction and read by an MFMA: 2
 
-Every instruction is one wait state, s_nop N is N + 1.
+Every instruction is one wait state, s_nop N is N + 1.  In the kernels whose MFMAs are inline assembly the accumulators must besides be
+separated from whatever reads them by an s_nop that is long enough by itself: instructions that happen to stand there would do as
+well, until they don't.
 """
 
 import re
@@ -107,13 +109,14 @@ def _passes(i):
     return 4
 
 
-def hazards(code):
-    """Messages for one kernel: [Ins] -> [str]."""
+def hazards(code, explicit=False):
+    """Messages for one kernel: [Ins] -> [str].  `explicit`: an MFMA's result needs an s_nop, looked for over 32 wait states."""
     at = {i.addr: n for n, i in enumerate(code)}
     found = []
 
-    def follow(n, need, regs, hit):
-        """All paths behind instruction n until `need` states have passed or `regs` are written again: where hit() holds, report."""
+    def follow(n, need, regs, hit, nop=None):
+        """All paths behind instruction n until `need` states have passed (or an s_nop of `nop` states) or `regs` are written again: where
+        hit() holds, report."""
         todo, seen = [(n + 1, 0, frozenset(regs))], set()
         while todo:
             k, states, live = todo.pop()
@@ -126,7 +129,7 @@ def hazards(code):
                     found.append(f"{code[n]}  ->  {i}  ({states} of {need} wait states)")
                     break
                 states += i.states
-                if i.op == "s_endpgm":
+                if i.op == "s_endpgm" or (nop and i.states >= nop):
                     break
                 if i.target is not None and i.target in at:
                     if i.op == "s_branch":
@@ -147,7 +150,8 @@ def hazards(code):
                 # exactly the result as SrcC: the hardware waits
                 return bool((j.ops[1] | j.ops[2]).union(*j.ops[4:]) & live) or (j.ops[3] != d and bool(j.ops[3] & live))
 
-            follow(n, 12 if _passes(i) == 8 else 8, d, early)
+            need = 12 if _passes(i) == 8 else 8
+            follow(n, 32 if explicit else need, d, (lambda j, live: not j.mfma and bool(j.used() & live)) if explicit else early, need if explicit else None)
         elif i.valu:
             d = set().union(*i.ops[:2]) if i.op.startswith(("v_add_co", "v_addc_co", "v_sub_co", "v_subb_co", "v_mad_u64", "v_mad_i64", "v_div_scale")) else i.ops[0]
             sregs = {r for r in d if r >= _BASE["s"]}
@@ -203,7 +207,7 @@ def test_the_check_itself(text, bad):
 
 def _scan(blob):
     text = subprocess.run([str(OBJDUMP), "-d", "--no-leading-addr", "/dev/stdin"], input=blob, capture_output=True, check=True).stdout.decode()
-    return {name: bad for name, code in parse(text).items() if (bad := hazards(code))}
+    return {name: bad for name, code in parse(text).items() if (bad := hazards(code) + (hazards(code, True) if "_tiled" in name else []))}
 
 
 @pytest.mark.skipif(not LIB.exists() or not OBJDUMP.exists(), reason="needs the built library and llvm-objdump")
