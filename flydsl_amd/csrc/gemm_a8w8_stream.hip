@@ -21,6 +21,7 @@
 //     s_waitcnt vmcnt(number of W loads) is the wait for A.
 // Operands are swapped like in the tiled kernel (src0 = W fragment, src1 = A fragment): a lane holds
 // C[m = lane%16][n = window + (lane/16)*4 + 0..3].
+#include "lds_dma.h"
 #include "psg_common.h"
 
 namespace {
@@ -35,23 +36,6 @@ template <>
 struct Acc<KIND_INT8> {
     using type = v4i;
 };
-
-// descriptor built from values forced into scalar registers (an inline-asm "s" operand must not end up in vector registers)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc_uniform(const void* base, uint64_t bytes) {
-    const uint64_t b = (uint64_t)(uintptr_t)base;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)(bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes));
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((uintptr_t)(((uint64_t)hi << 32) | lo)), 0, (int)n, 0x00020000);
-}
-
-// one DMA instruction: 64 lanes x 16 bytes from (descriptor, voff) to LDS [lds_addr, lds_addr + 1024).  Issued from inline
-// assembly: the compiler does not know that it writes LDS (it would put a full vmcnt wait in front of every LDS read that
-// follows), so the kernel waits for it itself.
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t lds_addr, uint32_t voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(r)
-                 : "memory");
-}
 
 // MB = 16-row blocks of A (1 to 4); NWIN = 16-column windows per wavefront group (1 or 2).
 // CH = 128-byte K steps per chunk; NWAVES = wavefronts per workgroup.
@@ -184,7 +168,7 @@ __global__ void __launch_bounds__(NWAVES * 64) k_a8w8_stream(A8W8Params p) {
                     // redirected there too: both write zeros
                     const uint32_t kb = kbyte0 + ((((uint32_t)(lane % CPR)) ^ (uint32_t)(((ps % NVAR) * RPP + lane / CPR) & 15)) << 4);
                     const bool a_ok = c < nchunks && kb < slice_end;
-                    dma16(ra, patch_lds + (uint32_t)ps * 1024u, a_ok ? src + kbyte0 : OOB);
+                    dma16(ra, patch_lds + (uint32_t)ps * 1024u, a_ok ? src + kbyte0 : OOB, 0u);
                 }
             } else {
                 const uint32_t kbyte = kbyte0 + (uint32_t)st_c * 16u;

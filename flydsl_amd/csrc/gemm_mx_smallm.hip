@@ -6,25 +6,10 @@
 // fixed order, and there is neither a partials buffer nor a second launch.  The 64 x 128 tiles of the general kernel gave such
 // calls N / 128 workgroups per K split and a finalising launch: fp8 x fp4, 64 x 8192 x 8192, 20.2 -> 12.3 us (37 MB, 7.2 at the rate of
 // a large copy), one row of it 12.2 -> 7.7.  Of the 12.3 about 5 go into reading the 512 KB of A through every CU.
+#include "lds_dma.h"
 #include "psg_common.h"
 
 namespace {
-
-// descriptor built from values forced into scalar registers (an inline-asm "s" operand must not end up in vector registers)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc_uniform(const void* base, uint64_t bytes) {
-    const uint64_t b = (uint64_t)(uintptr_t)base;
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)(bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes));
-    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((uintptr_t)(((uint64_t)hi << 32) | lo)), 0, (int)n, 0x00020000);
-}
-
-// one DMA instruction: 64 lanes x 16 bytes from (descriptor, voff + soff) to LDS [lds_addr, lds_addr + 1024).  Issued from inline
-// assembly: the compiler does not know that it writes LDS, so the kernel waits for it itself.
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t lds_addr, uint32_t voff, uint32_t soff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane((int)lds_addr)), "v"(voff), "s"(r), "s"(__builtin_amdgcn_readfirstlane((int)soff))
-                 : "memory");
-}
 
 template <int F>
 struct MxCode {  // cbsz / blgp format code of the MFMA
