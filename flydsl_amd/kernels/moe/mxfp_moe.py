@@ -41,14 +41,6 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr())
 
 
-def _stream_handle(stream):
-    if stream is None:
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    if isinstance(stream, int):
-        return ctypes.c_void_p(stream)
-    return ctypes.c_void_p(stream.cuda_stream)
-
-
 def _need(t, name, dtype=None, itemsize=None):
     """A pointer is all the library gets: refuse tensors whose element type, device or layout it would misread."""
     if not isinstance(t, torch.Tensor) or not t.is_cuda or not t.is_contiguous():
@@ -121,7 +113,7 @@ def flydsl_mxfp4_gemm1(*, a_quant, a_scale_sorted_shuffled, w1_u8, w1_scale_u8, 
     if inter_sorted_shuffled_scale.numel() < (sorted_size + 31) // 32 * 32 * (D_INTER // 32):
         raise ValueError("inter_sorted_shuffled_scale is smaller than ceil(sorted rows / 32) * 32 * D_INTER/32 bytes")
     lib = _lib.lib()
-    _lib.check(lib.psg_moe_mx_gemm(ctypes.byref(args), _stream_handle(stream)), "psg_moe_mx_gemm (stage 1)")
+    _lib.check(lib.psg_moe_mx_gemm(ctypes.byref(args), _lib.stream_handle(stream)), "psg_moe_mx_gemm (stage 1)")
     return inter_sorted_quant, inter_sorted_shuffled_scale
 
 
@@ -208,5 +200,5 @@ def moe_mxfp4_sort(blockscale_e8m0, sorted_ids, num_valid_ids, token_num, block_
         raise ValueError(f"out holds {out.numel() * out.element_size()} bytes, {rows * cols} are written")
     lib = _lib.lib()
     _lib.check(lib.psg_moe_mx_scale_sort(_ptr(s), _ptr(sorted_ids), _ptr(num_valid_ids), _ptr(out), int(token_num), topk, cols, int(sorted_ids.numel()),
-                                         _stream_handle(stream)), "psg_moe_mx_scale_sort")
+                                         _lib.stream_handle(stream)), "psg_moe_mx_scale_sort")
     return out
