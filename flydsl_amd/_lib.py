@@ -371,18 +371,33 @@ def workspace(device, nbytes: int, stream=0, owner="shared"):
     return _pool.get(owner, index, int(stream), int(nbytes))
 
 
+_REFUSED_CALLS = 256  # calls that go without scratch before the allocator is asked again
+_refused = {}         # device index -> [smallest number of bytes refused, calls left]
+
+
 def call_scratch(device, nbytes: int, stream: int):
     """Scratch for the launches of ONE call: a tensor from torch's caching allocator, which hands its memory on in the order of
     the stream it was allocated on, so it may be dropped as soon as the launches are queued.  That holds for the current
     stream of ``device`` only; for a launch on another stream, while the stream is being captured (nothing is allocated then), and
-    when memory is short, the answer is ``None`` and the caller takes its way without scratch."""
+    when memory is short, the answer is ``None`` and the caller takes its way without scratch.
+
+    An allocation that fails is expensive (the allocator gives back every cached block, which waits for the device, and tries
+    again), so after one the next calls that want as much go without scratch unasked."""
     import torch
 
     if nbytes <= 0 or torch.cuda.current_stream(device).cuda_stream != stream or _torch_capturing():
         return None
+    index = torch.device(device).index
+    refused = _refused.get(index)
+    if refused is not None and nbytes >= refused[0]:
+        if refused[1] > 0:
+            refused[1] -= 1
+            return None
+        _refused.pop(index, None)
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
     except torch.cuda.OutOfMemoryError:
+        _refused[index] = [nbytes, _REFUSED_CALLS]
         return None
 
 
