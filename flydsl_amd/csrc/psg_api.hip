@@ -225,12 +225,19 @@ bool mx_fills_tiles(int M, int N) {
 // Beyond 64 rows a workgroup takes 64 of them, and the kernel is the better one while its workgroups make one round of one per CU, or two on
 // rows of up to 8192 elements (fp8 x fp4, 128 x 2048 x 4096 6.7 / 16.1, 256 x 1024 x 14336 16.6 / 46.8, 128 x 4096 x 4096 7.2 / 16.2; two
 // rounds 256 x 4096 x 4096 12.8 / 16.5, 128 x 8192 x 8192 22.8 / 29.0; three 192 x 8192 x 8192 32.8 / 29.1, four 128 x 16384 x 4096 26 / 18).
-bool mx_general_small(int M, int N, int K, bool fp8_weights, int batch) {
+// Batches multiply the workgroups, and the general kernel, which cannot split K over them, gets the workgroups it lacked.  So up to 64 rows
+// batches also have to make at most two rounds of 64-row workgroups (one with fp4 activations, which are read in fragment order), fewer
+// rows counting for as much less (768 points of 2 to 8 batches: the other kernel more than 5 % faster at 53 of them, at 198 without this
+// bound; us small-M / general: fp8 x fp4 64 x 4096 x 4096 2 batches 7.6 / 16.4, 4 (two rounds) 13.8 / 17.3, 8 27.1 / 21.8; 64 x 16384 x 4096 2
+// batches 27.3 / 21.5; fp4 x fp4 64 x 4096 x 4096 2 (one round) 8.0 / 11.7, 4 14.3 / 13.4, 8 27.6 / 19.1; 16 x 4096 x 4096 8 14.0 / 15.7; fp8 x
+// fp8 64 x 8192 x 8192 2 (two rounds) 32.0 / 33.0, 4 65.0 / 47.8).
+bool mx_general_small(int M, int N, int K, bool fp4_acts, bool fp8_weights, int batch) {
     if (M > kStreamMaxM) {
         const long wgs = (long)(N / 32) * ((M + 63) / 64) * batch, cus = psg_cu_count();
         return N >= 1024 && wgs <= (K <= 8192 ? 2 : 1) * cus;
     }
     const long rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+    if (batch > 1 && (long)(N / 32) * batch * rows > (fp4_acts ? 1 : 2) * 64L * psg_cu_count()) return false;
     return N >= 1024 && (long)(N / 32) * rows * K <= (fp8_weights ? 320L : 160L) * 1000000L;
 }
 
@@ -637,7 +644,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         g.sa_batch = sa_bs;
         g.sb_batch = (int64_t)((uint64_t)(a->N / 32) * chunk);
         hipError_t ge;
-        const bool small = store == STORE_C && a->force_path == 0 && mx_general_small(a->M, a->N, a->K, a->b_dtype == PSG_MX_FP8, batch);
+        const bool small = store == STORE_C && a->force_path == 0 && mx_general_small(a->M, a->N, a->K, a->a_dtype == PSG_MX_FP4, a->b_dtype == PSG_MX_FP8, batch);
         const int splits = !small && batch == 1 && c_rs == (uint64_t)a->N && store == STORE_C ? mx_general_splits(a->M, a->N, a->K) : 1;
         if (small) {
             ge = psg_launch_mx_smallm(g, a->a_dtype, a->b_dtype, batch, static_cast<hipStream_t>(stream));

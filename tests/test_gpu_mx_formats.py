@@ -311,6 +311,31 @@ def test_small_m_kernel_against_the_general_kernel(a_dtype, b_dtype, M, N, K, ba
             assert np.all(np.abs(o - ref) <= 2.0 ** -8 * np.abs(ref) + 1.01 * _acc_atol(d[b], ref) + 1e-4 * np.abs(ref))
 
 
+# batches of up to 64 rows on both sides of the line between the small-M and the general kernel (256 CUs: 16384 rows of workgroups with fp4
+# activations, 32768 with the others, e.g. 64 rows x 32 column blocks x 8 batches), against the general kernel
+@pytest.mark.parametrize("a_dtype,b_dtype", PAIRS)
+@pytest.mark.parametrize("M,N,K,batch", [(64, 1024, 512, 8), (50, 1024, 512, 9), (64, 2080, 256, 8), (33, 1024, 768, 16), (40, 1056, 256, 17), (32, 2048, 256, 9), (9, 4096, 256, 9)])
+def test_batches_around_the_small_m_line(a_dtype, b_dtype, M, N, K, batch):
+    from kernels.gemm.mxfp4_preshuffle import launch_gemm
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    m32 = (M + 31) // 32 * 32
+    # multiples of one step up to 60 of it (fp8 codes from the lowest two binades) and two scale bytes: a product takes 10 bits, two scales 2 and
+    # 768 of them 10 more, so every sum is exact in fp32 whatever its order and the bits agree
+    byte = lambda f, rows: torch.randint(0, 256, (rows * (K // 2 if f == "fp4" else K),), generator=g, device="cuda", dtype=torch.uint8) & (0x8F if f == "fp8" else 0xFF)
+    a, b = byte(a_dtype, batch * M), byte(b_dtype, batch * N)
+    scale = lambda rows: torch.randint(126, 128, (rows * (K // 32),), generator=g, device="cuda", dtype=torch.uint8)
+    sa, sb = scale(batch * m32), scale(batch * N)
+    outs = []
+    for path in (0, 3):
+        c = torch.full((batch, M, N), SENTINEL, dtype=torch.bfloat16, device="cuda")
+        launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, a_dtype, "bf16", b_dtype, batch, -1, -1, -1, -1, -1, -1, 0, 0, _force_path=path)
+        outs.append(c)
+    torch.cuda.synchronize()
+    assert not (outs[1] == SENTINEL).any()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 # the dense 256x256 tiles behind fp8 / fp6 x fp4 and behind batches: ragged last tiles, the shortest K, K steps that are no multiple of the
 # pipeline's stages, batches apart from each other; the general kernel adds in the same order, so the bits agree
 @pytest.mark.parametrize("a_dtype,b_dtype", [("fp8", "fp4"), ("fp6", "fp4"), ("fp4", "fp4"), ("fp8", "fp8")])
