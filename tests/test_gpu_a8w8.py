@@ -293,3 +293,48 @@ def test_streaming_kernel_beyond_64_rows(M, N, K):
     want = ((acc * sa[:, None]) * sb[None, :]).bfloat16()
     assert torch.equal(c[:M], want)
     assert (c[M:] == -8192.0).all()
+
+
+# the other kinds of it, with every fused epilogue.  Operands are multiples of 1/4 up to 2, so the fp32 sums are exact in any order, and so is
+# everything up to the bias; silu and gelu go through __expf (2^-20 relative is ample) and both sides round once to 16 bits
+@pytest.mark.parametrize("out,half", [("bf16", 2.0 ** -8), ("fp16", 2.0 ** -11)])
+@pytest.mark.parametrize("kind,M,N,kbytes,epilogue", [
+    ("fp8", 65, 4096, 2048, "none"), ("fp8", 100, 4080, 2112, "bias_silu"), ("fp8", 192, 2720, 4032, "bias_gelu"), ("fp8", 256, 1024, 4096, "bias"),
+    ("bf16", 65, 4096, 2048, "bias_relu"), ("bf16", 192, 2720, 4032, "none"), ("fp16", 100, 4080, 2112, "bias_gelu"), ("fp16", 256, 1024, 4096, "bias_silu"),
+    ("int8", 80, 1040, 4096, "bias_relu"), ("int8", 129, 2048, 2048, "bias_silu")])
+def test_streaming_kernel_beyond_64_rows_kinds_and_epilogues(kind, M, N, kbytes, epilogue, out, half):
+    from flydsl_amd import _lib, layout
+    from kernels.gemm.preshuffle_gemm import compile_preshuffle_gemm
+
+    wide = kind in ("bf16", "fp16")
+    K = kbytes // 2 if wide else kbytes
+    assert _lib.lib().psg_workspace_bytes(M, N, K, _lib.IN_DTYPE[kind]) == 0
+    td = {"fp8": torch.float8_e4m3fn, "int8": torch.int8, "bf16": torch.bfloat16, "fp16": torch.float16}[kind]
+    tout = torch.bfloat16 if out == "bf16" else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    step = 1.0 if kind == "int8" else 0.25
+    a, w = (torch.randint(-8, 9, (r, K), generator=g, device="cuda").float() * step for r in (M, N))
+    scale = lambda n: 2.0 ** torch.randint(-5, -2, (n,), generator=g, device="cuda").float()
+    sa, sb = (None, None) if wide else (scale(M), scale(N))
+    bias = torch.randn(N, generator=g, device="cuda").to(tout)
+    c = torch.full((M + 3, N), -8192.0, dtype=tout, device="cuda")
+    wq = w.to(td)
+    fn = compile_preshuffle_gemm(N=N, K=K, tile_m=64, tile_n=128, tile_k=32 if wide else 64, in_dtype=kind, out_dtype=out, epilogue=epilogue)
+    fn(c, a.to(td), layout.shuffle_weight(wq.view(torch.int8) if kind == "fp8" else wq).view(td).contiguous(), sa, sb, bias, M, N, torch.cuda.current_stream())
+    v = a.double() @ w.double().T
+    if not wide:
+        v = v * sa.double()[:, None] * sb.double()[None, :]
+    if epilogue != "none":
+        v = (v.float() + bias.float()).double()  # the one rounding in front of the activation
+    if epilogue == "bias_relu":
+        v = v.clamp(min=0)
+    if epilogue == "bias_silu":
+        v = v / (1 + torch.exp(-v))
+    if epilogue == "bias_gelu":
+        v = 0.5 * v * (1 + torch.tanh(0.7978845608 * (v + 0.044715 * v ** 3)))
+    assert (c[M:] == -8192.0).all()
+    if epilogue in ("bias_silu", "bias_gelu"):
+        # half a unit in the last place of the output on top of the fp32 error; below the normal range of fp16 the spacing is 2^-24
+        assert ((c[:M].double() - v).abs() <= (half + 2.0 ** -19) * v.abs() + 2.0 ** -24 + 1e-6).all()
+    else:
+        assert torch.equal(c[:M], v.to(tout))

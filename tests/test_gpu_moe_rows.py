@@ -88,3 +88,26 @@ def test_stage2_by_rows_equals_the_exact_sum(monkeypatch, kind, tokens, topk, bl
         want.index_add_(0, t[ok], (x[src].double() @ w[e].double().T) * wts[pos[ok]].double()[:, None])
     assert want.abs().max() <= 256
     assert torch.equal(out.cpu().double(), want)
+
+
+class _RealRule:
+    """In place of monkeypatch above: the library's own rule and size, watched instead of replaced."""
+
+    def __init__(self, monkeypatch):
+        self.monkeypatch = monkeypatch
+
+    def setattr(self, obj, name, seen):
+        real = getattr(obj, name)
+
+        def rule(*args):
+            seen(*args)
+            need = real(*args)
+            assert need > 0, "the rule does not take this call by rows"
+            return need
+
+        self.monkeypatch.setattr(obj, name, rule)
+
+
+@pytest.mark.parametrize("kind,tokens,topk,block,model,inter", [("mx", 410, 8, 64, 2048, 256), ("fp8", 515, 6, 128, 4096, 128), ("int8", 813, 4, 32, 4096, 128), ("int4", 410, 8, 64, 4096, 128)])
+def test_stage2_by_rows_where_the_library_takes_it(monkeypatch, kind, tokens, topk, block, model, inter):
+    test_stage2_by_rows_equals_the_exact_sum(_RealRule(monkeypatch), kind, tokens, topk, block, model, inter, torch.bfloat16)

@@ -363,3 +363,26 @@ def test_dense_tiles_against_the_general_kernel(a_dtype, b_dtype, M, N, K, batch
     torch.cuda.synchronize()
     assert outs[1].count_nonzero() > 0.9 * batch * M * N
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+# fp16 output of the dense tiles with fp4 weights (builds of their own: the general epilogue) and of the small-M kernel.  The sums are exact as in
+# test_batches_around_the_small_m_line (a K of 2048 takes 13 bits on top of 10), so the bits of the general kernel are expected
+@pytest.mark.parametrize("a_dtype,b_dtype", PAIRS)
+@pytest.mark.parametrize("M,N,K,batch", [(129, 32768, 768, 1), (2056, 4096, 512, 2), (1, 1024, 256, 2), (17, 1184, 2048, 2), (64, 1088, 1024, 2), (200, 1056, 512, 2)])
+def test_fp16_output(a_dtype, b_dtype, M, N, K, batch):
+    from kernels.gemm.mxfp4_preshuffle import launch_gemm
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    m32 = (M + 31) // 32 * 32
+    byte = lambda f, rows: torch.randint(0, 256, (rows * (K // 2 if f == "fp4" else K),), generator=g, device="cuda", dtype=torch.uint8) & (0x8F if f == "fp8" else 0xFF)
+    a, b = byte(a_dtype, batch * M), byte(b_dtype, batch * N)
+    scale = lambda rows, lo: torch.randint(lo, lo + 2, (rows * (K // 32),), generator=g, device="cuda", dtype=torch.uint8)
+    sa, sb = scale(batch * m32, 130 if a_dtype == "fp8" else 126), scale(batch * N, 130 if b_dtype == "fp8" else 126)
+    outs = []
+    for path in (0, 3):
+        c = torch.full((batch, M, N), SENTINEL, dtype=torch.float16, device="cuda")
+        launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, a_dtype, "fp16", b_dtype, batch, -1, -1, -1, -1, -1, -1, 0, 0, _force_path=path)
+        outs.append(c)
+    torch.cuda.synchronize()
+    assert outs[1].isfinite().all() and not (outs[1] == SENTINEL).any() and outs[1].count_nonzero() > 0.9 * outs[1].numel()
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
