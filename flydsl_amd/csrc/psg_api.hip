@@ -737,13 +737,16 @@ int psg_gemm_mxfp4_acc(const psg_mxfp4_args* args, void* acc, void* stream) { re
 // but 1024 x top-2 x 4096 41 / 35, 4096 x top-1 75 / 64).
 // The scratch is bounded: 1 GiB with one scale per row, where it stops being faster anyway (fp8, model 7168, inter 2048, top-8 on 32
 // experts: 8192 tokens, 0.95 GB, 1355 / 1412; 16384 tokens, 1.85 GB, 2791 / 2768; 32768 tokens, 3.6 GB, 6046 / 5882), and 4 GiB, one and a
-// half per cent of the device, for the MX pair, which still gains there (1042 / 1395, 2040 / 2947, 4013 / 6383).
-uint64_t psg_moe_rows_workspace_bytes(int32_t tokens, int32_t topk, int32_t sorted_size, int32_t model_dim, int32_t out_dtype, int32_t mx) {
+// half per cent of the device, for the MX pair, which still gains there (1042 / 1395, 2040 / 2947, 4013 / 6383).  With int4 weights, whose
+// tiles run two workgroups a CU and hide more of the additions, 256 MB, what the last-level cache holds of the rows (model 4096, inter 1536,
+// top-8 on 32 experts: 1024 tokens 120 / 134, 2048, 160 MB, 213 / 224, but 4096, 288 MB, 446 / 402; 2048 x 7168 x 2048, 280 MB, 461 / 442).
+uint64_t psg_moe_rows_workspace_bytes(int32_t tokens, int32_t topk, int32_t sorted_size, int32_t model_dim, int32_t out_dtype, int32_t kind) {
     if (tokens < 1 || topk < 1 || sorted_size < 1 || model_dim < 2 || (out_dtype != PSG_OUT_BF16 && out_dtype != PSG_OUT_FP16)) return 0;
     const int64_t bytes = (int64_t)tokens * topk * model_dim * 2;
+    const bool mx = kind == 1;
     if (bytes < (mx ? 12ll << 20 : 24ll << 20) || (!mx && topk < 4)) return 0;
     const uint64_t need = psg_moe_rows_bytes(tokens, topk, sorted_size, model_dim);
-    return need <= (mx ? 4ull << 30 : 1ull << 30) ? need : 0;
+    return need <= (mx ? 4ull << 30 : kind == 2 ? 256ull << 20 : 1ull << 30) ? need : 0;
 }
 
 static int moe_gemm_common(const psg_moe_args* a, void* workspace, uint64_t workspace_bytes, void* stream) {

@@ -83,7 +83,7 @@ class MoeStage:
         a.x_slot_major = int(self.slot_major)
         a.no_pairing = int(self.no_pairing)
         h = _lib.stream_handle(stream)
-        need = self._lib.psg_moe_rows_workspace_bytes(tokens, self.topk, a.sorted_size, n_out, self.out_dtype, 0) if self.stage == 2 and self.accumulate else 0
+        need = self._lib.psg_moe_rows_workspace_bytes(tokens, self.topk, a.sorted_size, n_out, self.out_dtype, 2 if self.w4 else 0) if self.stage == 2 and self.accumulate else 0
         ws = _lib.call_scratch(dev, need, h) if need else None
         if ws is None:
             rc = self._lib.psg_moe_gemm(ctypes.byref(a), h)

@@ -11,6 +11,7 @@ BF16, FP16, F32 = 0, 1, 2
 
 
 def _bytes(tokens, topk, sorted_size, model, out=BF16, mx=0):
+    """mx: 0 one scale per row, 1 the MX pair, 2 int4 weights."""
     return _lib.lib().psg_moe_rows_workspace_bytes(tokens, topk, sorted_size, model, out, mx)
 
 
@@ -28,7 +29,7 @@ def test_scratch_holds_the_rows_and_the_lists(tokens, topk, model, mx):
 
 def test_scratch_starts_and_ends_where_the_rule_says():
     mb = 1 << 20
-    for mx, least, most in ((1, 12 * mb, 4 << 30), (0, 24 * mb, 1 << 30)):
+    for mx, least, most in ((1, 12 * mb, 4 << 30), (0, 24 * mb, 1 << 30), (2, 24 * mb, 256 * mb)):
         # topk * model * 2 = 64 KiB of additions a token
         least_tokens = least >> 16
         assert _bytes(least_tokens, 8, least_tokens * 8, 4096, mx=mx) > 0
