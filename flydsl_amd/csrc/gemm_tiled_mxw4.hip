@@ -1,4 +1,4 @@
-// Instantiations of the 256x256 tile (gemm_tiled8.h) for fp8 and fp6 activations against fp4 weights, dense and unbatched.
+// Instantiations of the 256x256 tile (gemm_tiled8.h) for fp8 and fp6 activations against fp4 weights, dense; batches are a launch each.
 // Against the 128x256 tile of the general MX kernel, whose A goes through registers and whose steps wait for LDS behind their
 // barrier: fp8 x fp4 4096x4096x8192 169 -> 92 us (2.98 PFLOP/s), 8192x4096x2048 102 -> 57; the bits are the same.
 #include "gemm_tiled8.h"

@@ -368,6 +368,10 @@ hipError_t psg_launch_moe_tiled(const MoeParams& p, int kind, int stage, int blo
 // 1536 (1728 tiles) 473 / 391; 4096 x top-6 on 64, 1024 x 256 (256 tiles) 34.7 / 27.4; but 1024 x top-8 (576 tiles) 168 / 179, 4096 x
 // top-2 on 8, 2048 x 1024 (288) 52.8 / 61.1.  Stage 2 without atomics: 4096 x top-8 (2304 tiles) 360 / 273, 1024 x top-8 (768) 119 /
 // 105; but 512 x top-8 (512 tiles, 128 rows per expert) 70.2 / 72.7, 4096 x top-1 on 8, 4096 x 1024 (320) 68.7 / 74.9.
+// Where stage 2 adds directly (no scratch, fewer than four slots, under capture) the rule holds as well, though one workgroup a CU leaves
+// nothing to run beside the additions: 4096 x top-8 405 / 388, 2048 x top-8 220 / 203, 2048 tokens x top-3 on 8 experts, 4096 x 1024, 83 /
+// 75, x 2048 110 / 98; on two or three slots and short rows it is a few per cent the other way (4096 x top-3 on 16, 4096 x 768 127 / 131, x 256
+// 102 / 111; but 2048 x 512 70 / 64), which no size of the call tells apart.
 bool takes_tiled(const MoeParams& p, int stage) {
     const long pairs = (long)p.tokens * p.topk, cus = psg_cu_count(), tn = stage == 1 ? 128 : 256;
     if (pairs < 192L * p.experts) return false;

@@ -9,7 +9,7 @@
 // Bound: MFMA, at the clock the power limit leaves (1.87 GHz in the loop, 2,490 cycles a K step of 2,048 issue cycles).  The tiles of
 // k_moe_gemm (128 rows x 64 or 128 columns) are bound by their operand traffic: 128 flop per byte against 256 here.  Measured, 4096
 // tokens x top-8 on 32 experts, 4096 x 1536, fp8: stage 1 473 -> 391 us, stage 2 (one row per sorted position) 360 -> 273; int8 528 ->
-// 423.  Of the 56 us of a stage-1 tile 43 are the loop, 7 the epilogue and the rest its start.  The bits are those of k_moe_gemm.
+// 423 (loops of launches; under the profiler, on other boxes, 394 to 414 and 274 to 293).  Of the 56 us of a stage-1 tile 43 are the loop, 7 the epilogue and the rest its start.  The bits are those of k_moe_gemm.
 // Registers: all 256 vector registers a lane are in use; 4 to 20 of them and about 40 scalar registers spill, none inside the unchecked
 // loop (scratch stores between the loops and the epilogue, scalars into lanes of a vector register around the prologue).
 //

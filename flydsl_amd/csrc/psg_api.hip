@@ -101,7 +101,9 @@ bool mx_takes_small(int M, int N, int K) {
 // Beyond 64 rows a workgroup takes 64 of them, and the kernel is the better one while 32 columns a workgroup make one round of the CUs (N
 // times the 64-row groups up to 8192) on rows of 2 to 4 KB (us streaming / tiled plan: fp8 80x1024x4096 6.6 / 9.5, 256x1024x4096 7.2 /
 // 10.1, 128x2048x2048 4.8 / 7.3, 128x4096x4096 9.9 / 11.9, 192x2048x2048 7.2 / 7.4; bf16 256x1024x1024 4.8 / 6.8, 128x2048x2048 7.4 /
-// 10.4; but fp8 128x4096x1024 6.2 / 5.5, 192x2048x8192 17.4 / 14.7, 192x4096x4096 19.4 / 11.5).
+// 10.4; but fp8 128x4096x1024 6.2 / 5.5, 192x4096x4096, one and a half rounds, 19.2 / 11.9).  On rows of 4 to 8 KB it is the better one
+// in the same range of columns too (fp8 128x2048x6144 9.8 / 15.7, 128x2048x8192 11.7 / 18.8, 192x2048x8192 16.6 / 19.1, 128x4096x5120 12.1 /
+// 14.0; bf16 128x2048x4096 11.5 / 19.6): the line at 4 KB is a cautious one, which leaves those calls their split-K plan.
 bool takes_stream(int M, int N, int kbytes) {
     if (M <= kSmallM) return true;
     if (M > kStreamMaxM) return M <= 256 && kbytes >= 2048 && kbytes <= 4096 && (long)N * ((M + 63) / 64) <= 8192;
@@ -176,7 +178,7 @@ Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
     return t;
 }
 
-// Split-K for the regime between the streaming kernel (M <= 32) and problems with enough tiles to fill the GPU:
+// Split-K for the regime between the streaming kernel (takes_stream) and problems with enough tiles to fill the GPU:
 // with few tiles every workgroup walks all of K behind a one-step prefetch and the launch is latency-bound.
 // Splitting K over `splits` workgroups per tile multiplies the loads in flight; the price is one fp32 slice of
 // [M,N] per split written and read back, so the split count is capped where that traffic reaches 1.25 W, and where the
@@ -211,7 +213,11 @@ int pick_splits(int M, int N, int kbytes, Tile t) {
 // tiles would give every CU one.  There the general kernel works on 128x256 tiles, and one of those takes as long as a 256x256
 // tile does here (fp8 x fp4, us 256x256 / general: 500x16384x4096 42.9 / 48.7, 1000x8192x4096 42.6 / 47.3, 1024x16384x2048 30.4 /
 // 51.7, 1280x8192x4096 41.3 / 87.2, 4096x4096x8192 92.2 / 169.5, 8192x1024x14336 124 / 146); with fewer its 64x128 tiles and its K
-// splits are the better way (768x8192x4096 39.4 / 34.7, 1000x4096x14336 115 / 63).
+// splits are the better way (768x8192x4096 39.4 / 34.7, 1000x4096x14336 115 / 63).  Batches, one launch each against the general kernel's one
+// over all: fp8 x fp8 2 x 1024x8192x4096 78 / 104, 8 324 / 497, 12 473 / 744, 4 x 1280x8192x2048 139 / 139; fp4 x fp4 2 x 512x16384x2048
+// 34.8 / 45.7, 8 x 2048x4096x4096 194 / 277; fp8 x fp4 2 x 2048x4096x4096 88 / 93, 8 327 / 371; fp6 x fp4 2 x 512x16384x2048 53.6 / 52.6, 8
+// 205 / 216; with half as many tiles fp8 x fp4 8 x 512x8192x2048 183 / 104.  More batches gain as much; the limit of eight (mx_common) is
+// what one call may queue as launches of its own.
 bool mx_fills_tiles(int M, int N) {
     return M > kStreamMaxM && (long)((M + 127) / 128) * (long)((N + 255) / 256) >= psg_cu_count();
 }

@@ -139,7 +139,9 @@ def launch_gemm(
     """Launch ``C[b] = A_mx[b] @ W_mx[b]^T`` (``[M,K] x [N,K]``) for every batch ``b`` on ``stream``.  The reference's
     constraints are kept: ``tile_k in {128, 256}``, ``tile_n % 128 == 0``, ``K % tile_k == 0``
     (mxfp4_preshuffle.py:122,316).  Dense unbatched fp4 x fp4 runs on the tuned fp4 kernels (``tile_*`` are hints the
-    planner may override); every other combination runs on the general MX kernel, which has a fixed tile."""
+    planner may override).  Every other combination is planned from its sizes alone, whatever ``tile_*`` say: few rows run on the small-M
+    MX kernel, dense fp8 x fp8 and fp8 / fp6 x fp4 problems that fill the GPU on the dense tiles (their batches, and those of fp4 x fp4,
+    one launch each), the rest on the general MX kernel."""
     # (anything but plain numbers and texts is worked out anew: other types may hash by identity)
     plain = type(N) is type(K) is type(tile_m) is type(tile_n) is type(tile_k) is int and type(a_dtype) is type(b_dtype) is type(out_dtype) is str
     plan = _plan if plain else _plan.__wrapped__
