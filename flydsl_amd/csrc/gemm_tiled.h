@@ -410,6 +410,14 @@ k_a8w8_tiled(A8W8Params p) {
             sb_v[ni] = *reinterpret_cast<const v4f*>(p.sb + (n < p.N ? n : 0));
         }
     }
+    v4f bias_v[NR] = {};
+    if constexpr (STORE == STORE_C_GENERIC && !MX) {
+#pragma unroll
+        for (int ni = 0; ni < NR; ni++) {
+            const int n = n0 + (wn * NR + ni) * 16 + lg * 4;
+            bias_v[ni] = load_bias4(p.bias + (n < p.N ? n : 0), p.out, p.epi);
+        }
+    }
 
     // epilogue: lane owns C[m0 + mi*16 + li][n0 + (wave*NR + ni)*16 + lg*4 + 0..3].  Compile-time indices only,
     // so the accumulators are never addressed dynamically.
@@ -447,37 +455,34 @@ k_a8w8_tiled(A8W8Params p) {
         uint8_t* stage = &lds[0][0];
         static_for<NCH>([&](auto CI) {
             constexpr int ci = decltype(CI)::value;
-            static_for<MR>([&](auto MI) {
-                constexpr int mi = decltype(MI)::value;
-                const int blk = wm * MR + mi;             // 16-row block of the tile (uniform over the wavefront)
-                if (blk / CH_BLK == ci) {
-                    const int rl = (blk - ci * CH_BLK) * 16 + li;  // row within the pass
-                    float sa = 0.f;
-                    if constexpr (SCALED) sa = sa_v[mi];
-                    static_for<NR>([&](auto NI) {
-                        constexpr int ni = decltype(NI)::value;
-                        const int n = n0 + (wn * NR + ni) * 16 + lg * 4;
-                        if (n < p.N) {
-                            const acc_t r = acc[mi][ni];
-                            v4f x;
-                            if constexpr (!SCALED) {
-                                x = (v4f){(float)r[0], (float)r[1], (float)r[2], (float)r[3]};  // no epilogue scales (MX: applied by the MFMA)
-                            } else {
-                                const v4f sb = sb_v[ni];
-                                x = (v4f){((float)r[0] * sa) * sb[0], ((float)r[1] * sa) * sb[1], ((float)r[2] * sa) * sb[2],
-                                          ((float)r[3] * sa) * sb[3]};
+            epi_dispatch<STORE, MX>(p.out, p.epi, [&](auto finish4) __attribute__((always_inline)) {
+                static_for<MR>([&](auto MI) {
+                    constexpr int mi = decltype(MI)::value;
+                    const int blk = wm * MR + mi;             // 16-row block of the tile (uniform over the wavefront)
+                    if (blk / CH_BLK == ci) {
+                        const int rl = (blk - ci * CH_BLK) * 16 + li;  // row within the pass
+                        float sa = 0.f;
+                        if constexpr (SCALED) sa = sa_v[mi];
+                        static_for<NR>([&](auto NI) {
+                            constexpr int ni = decltype(NI)::value;
+                            const int n = n0 + (wn * NR + ni) * 16 + lg * 4;
+                            if (n < p.N) {
+                                const acc_t r = acc[mi][ni];
+                                v4f x;
+                                if constexpr (!SCALED) {
+                                    x = (v4f){(float)r[0], (float)r[1], (float)r[2], (float)r[3]};  // no epilogue scales (MX: applied by the MFMA)
+                                } else {
+                                    const v4f sb = sb_v[ni];
+                                    x = (v4f){((float)r[0] * sa) * sb[0], ((float)r[1] * sa) * sb[1], ((float)r[2] * sa) * sb[2],
+                                              ((float)r[3] * sa) * sb[3]};
+                                }
+                                const int g = (wn * NR + ni) * 2 + (lg >> 1);
+                                *reinterpret_cast<v2i*>(stage + rl * ROWB + ((g ^ (rl & XM)) << 4) + (lg & 1) * 8) =
+                                    finish4(x, bias_v[ni]);
                             }
-                            v2i out;
-                            if constexpr (STORE == STORE_C) {
-                                out = finish4<OUT_BF16, EPI_NONE>(x, nullptr);
-                            } else {
-                                out = p.out == OUT_BF16 ? finish4_rt<OUT_BF16>(x, p.bias + n, p.epi) : finish4_rt<OUT_FP16>(x, p.bias + n, p.epi);
-                            }
-                            const int g = (wn * NR + ni) * 2 + (lg >> 1);
-                            *reinterpret_cast<v2i*>(stage + rl * ROWB + ((g ^ (rl & XM)) << 4) + (lg & 1) * 8) = out;
-                        }
-                    });
-                }
+                        });
+                    }
+                });
             });
             __syncthreads();
 #pragma unroll

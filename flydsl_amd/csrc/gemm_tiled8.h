@@ -78,9 +78,10 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     static_assert(!MX || (MR == 16 && NS == 4), "MX scale slots are laid out for the 256-row tile");
 
     // LDS: the A stages; behind them NS slots of MX scale dwords (per slot 8 A-side chunks + 8 W-side chunks of 256 bytes)
-    // or the per-token / per-channel scales of the epilogue (TM + TN floats)
+    // or the per-token / per-channel scales of the epilogue (TM + TN floats) and its bias (TN 16-bit values)
     constexpr int SC_SLOT = 4096;
-    constexpr int LDS_EXTRA = MX ? NS * SC_SLOT : (TM + TN) * 4;
+    constexpr bool BIAS = STORE == STORE_C_GENERIC && !MX;
+    constexpr int LDS_EXTRA = MX ? NS * SC_SLOT : (TM + TN) * 4 + (BIAS ? TN * 2 : 0);
     __shared__ __attribute__((aligned(1024))) uint8_t lds[NS * STAGE + LDS_EXTRA];
     uint8_t* const lds_x = lds + NS * STAGE;
 
@@ -297,6 +298,13 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
             ep_sb = p.sb[n < p.N ? n : p.N - 1];
         }
     }
+    uint16_t ep_bias = 0;
+    if constexpr (BIAS) {
+        if (tid < TN && p.epi != EPI_NONE) {
+            const int n = n0 + tid;
+            ep_bias = p.bias[n < p.N ? n : p.N - 1];
+        }
+    }
 #pragma unroll
     for (int s = 0; s < NS - 1; s++) {
 #pragma unroll
@@ -314,6 +322,9 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     if constexpr (SCALED && STORE != STORE_ACC) {
         if (tid < TM) reinterpret_cast<float*>(lds_x)[tid] = ep_sa;
         if (tid < TN) reinterpret_cast<float*>(lds_x)[TM + tid] = ep_sb;
+    }
+    if constexpr (BIAS) {
+        if (tid < TN) reinterpret_cast<uint16_t*>(lds_x + (TM + TN) * 4)[tid] = ep_bias;
     }
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(PFW * N_W) : "memory");
     static_for<FRAG_AHEAD>([&](auto I) {
@@ -401,31 +412,31 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
         const uint32_t c_off = ((uint32_t)r0 * (uint32_t)p.N + (uint32_t)n_st) * 2u;
         const uint32_t c_step = 16u * (uint32_t)p.N * 2u;
         const uint8_t* src = lds + r0 * ROWB + ((g ^ (r0 & XM)) << 4);
+        v4f bias_v[NR] = {};
+        if constexpr (BIAS) {
+#pragma unroll
+            for (int ni = 0; ni < NR; ni++)
+                bias_v[ni] = load_bias4(reinterpret_cast<const uint16_t*>(lds_x + (TM + TN) * 4) + (wave * NR + ni) * 16 + lg_e * 4, p.out, p.epi);
+        }
         static_for<2>([&](auto HALF) {
             constexpr int half = decltype(HALF)::value;
-            static_for<MR / 2>([&](auto MI) {
-                constexpr int mi = half * (MR / 2) + decltype(MI)::value;
-                float sa = 0.f;
-                if constexpr (SCALED) sa = sa_v[mi];
-                static_for<NR>([&](auto NI) {
-                    constexpr int ni = decltype(NI)::value;
-                    const acc_t r = acc[mi][ni];
-                    v4f x;
-                    if constexpr (!SCALED) {
-                        x = (v4f){(float)r[0], (float)r[1], (float)r[2], (float)r[3]};
-                    } else {
-                        const v4f sb = sb_v[ni];
-                        x = (v4f){((float)r[0] * sa) * sb[0], ((float)r[1] * sa) * sb[1], ((float)r[2] * sa) * sb[2], ((float)r[3] * sa) * sb[3]};
-                    }
-                    v2i out;
-                    if constexpr (STORE == STORE_C) {
-                        out = finish4<OUT_BF16, EPI_NONE>(x, nullptr);
-                    } else {
-                        const int n = n0 + (wave * NR + ni) * 16 + lg_e * 4;
-                        const uint16_t* bias_n = p.bias + (n < p.N ? n : 0);
-                        out = p.out == OUT_BF16 ? finish4_rt<OUT_BF16>(x, bias_n, p.epi) : finish4_rt<OUT_FP16>(x, bias_n, p.epi);
-                    }
-                    *reinterpret_cast<v2i*>(st_base[ni] + mi * 16 * ROWB) = out;
+            epi_dispatch<STORE, MX>(p.out, p.epi, [&](auto finish4) __attribute__((always_inline)) {
+                static_for<MR / 2>([&](auto MI) {
+                    constexpr int mi = half * (MR / 2) + decltype(MI)::value;
+                    float sa = 0.f;
+                    if constexpr (SCALED) sa = sa_v[mi];
+                    static_for<NR>([&](auto NI) {
+                        constexpr int ni = decltype(NI)::value;
+                        const acc_t r = acc[mi][ni];
+                        v4f x;
+                        if constexpr (!SCALED) {
+                            x = (v4f){(float)r[0], (float)r[1], (float)r[2], (float)r[3]};
+                        } else {
+                            const v4f sb = sb_v[ni];
+                            x = (v4f){((float)r[0] * sa) * sb[0], ((float)r[1] * sa) * sb[1], ((float)r[2] * sa) * sb[2], ((float)r[3] * sa) * sb[3]};
+                        }
+                        *reinterpret_cast<v2i*>(st_base[ni] + mi * 16 * ROWB) = finish4(x, bias_v[ni]);
+                    });
                 });
             });
             if constexpr (half == 1) T8_STAMP(4);

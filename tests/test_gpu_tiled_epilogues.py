@@ -1,0 +1,58 @@
+"""Fused epilogues and both output types on every tile of the tiled kernels, forced on ragged sizes (rows past M, columns past N).
+
+Operands are multiples of 1/4 up to 2 and the scales powers of two, so the sums are exact in any order, and so is everything up to the bias;
+silu and gelu add the error of an fp32 exponential and reciprocal, and every side rounds once to 16 bits."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TILES = [((256, 256), 8), ((256, 256), 0), ((128, 256), 0), ((64, 256), 0), ((128, 128), 0), ((64, 64), 0)]
+KINDS = {"fp8": torch.float8_e4m3fn, "int8": torch.int8, "bf16": torch.bfloat16, "fp16": torch.float16}
+
+
+@pytest.mark.parametrize("out,half", [("bf16", 2.0 ** -8), ("fp16", 2.0 ** -11)])
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("epilogue", ["none", "bias", "bias_relu", "bias_silu", "bias_gelu"])
+def test_every_tile(kind, epilogue, out, half):
+    from flydsl_amd import layout
+    from kernels.gemm.preshuffle_gemm import compile_preshuffle_gemm
+
+    M, N, K = 277, 272, 416
+    wide = kind in ("bf16", "fp16")
+    td, tout = KINDS[kind], torch.bfloat16 if out == "bf16" else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(len(epilogue))
+    step = 1.0 if kind == "int8" else 0.25
+    a, w = (torch.randint(-8, 9, (r, K), generator=g, device="cuda").float() * step for r in (M, N))
+    if not wide:
+        a, w = a[:, :384], w[:, :384]
+    K = a.shape[1]
+    scale = lambda n: 2.0 ** torch.randint(-5, -2, (n,), generator=g, device="cuda").float()
+    sa, sb = (None, None) if wide else (scale(M), scale(N))
+    bias = torch.randn(N, generator=g, device="cuda").to(tout)
+    bias[:6] = torch.tensor([-0.0, 300.0, -300.0, 30000.0, -30000.0, -12.0], device="cuda").to(tout)  # both tails of the activations
+    wq = w.to(td)
+    shuffled = layout.shuffle_weight(wq.view(torch.int8) if kind == "fp8" else wq).view(td).contiguous()
+    fn = compile_preshuffle_gemm(N=N, K=K, tile_m=64, tile_n=128, tile_k=32 if wide else 64, in_dtype=kind, out_dtype=out, epilogue=epilogue)
+    v = a.double() @ w.double().T
+    if not wide:
+        v = v * sa.double()[:, None] * sb.double()[None, :]
+    if epilogue != "none":
+        v = (v.float() + bias.float()).double()  # the one rounding in front of the activation
+    if epilogue == "bias_relu":
+        v = v.clamp(min=0)
+    if epilogue == "bias_silu":
+        v = v / (1 + torch.exp(-v))
+    if epilogue == "bias_gelu":
+        v = 0.5 * v * (1 + torch.tanh(0.7978845608 * (v + 0.044715 * v ** 3)))
+    for tile, layout_ in TILES:
+        c = torch.full((M + 3, N), -8192.0, dtype=tout, device="cuda")
+        fn.launch_forced(c, a.to(td).contiguous(), shuffled, sa, sb, bias, M, N, torch.cuda.current_stream(), force_path=1, tile=tile, wave_layout=layout_)
+        assert (c[M:] == -8192.0).all(), tile
+        if epilogue in ("bias_silu", "bias_gelu"):
+            # half a unit in the last place of the output on top of the fp32 error (the exponent of exp2 is rounded to 24 bits: 2^-24 times
+            # its size, at most 128); below the normal range of fp16 the spacing is 2^-24
+            assert ((c[:M].double() - v).abs() <= (half + 2.0 ** -16) * v.abs() + 2.0 ** -24 + 1e-6).all(), tile
+        else:
+            assert torch.equal(c[:M], v.to(tout)), tile
