@@ -15,6 +15,7 @@
 // (v_j & 15) | (v_{j+4} << 4) (tests/kernels/test_moe_gemm_2stage.py:64-80 of the reference), so a lane's 16-byte piece
 // of a fragment is 8 bytes at half the offset; it is unpacked with the reference's sign-extending mask-and-multiply
 // (kernels/common/mma/mfma_preshuffle_pipeline.py:225-238) into the same int8 fragment and multiplied by the int8 MFMA.
+#include "moe_rows.h"
 #include "psg_common.h"
 
 namespace {
@@ -57,7 +58,7 @@ __device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g));
 // from the start of each run of equal expert ids: the workgroup of the second block of a pair ends at once, and the
 // first one treats the second half of its tile as padding when the run ends there.
 template <int KIND, int MR, int NR, int STAGE, int CO = 1>
-__global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p) {
+__global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, MoeRowsParams rows) {
     using acc_t = typename MoeAcc<KIND>::type;
     constexpr int BM = 16 * MR, TN = 64 * NR;
     constexpr int BLK = BM / CO;                        // rows of one block of the sorted list
@@ -72,7 +73,13 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p) {
     const int tid = threadIdx.x;
     const int wave = wave_id();
     const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
-    const int blk = (int)blockIdx.y;
+    if constexpr (STAGE == 2) {
+        if ((int)blockIdx.y < rows.wgs) {
+            moe_rows_index_share(rows, (int)(blockIdx.y * gridDim.x + blockIdx.x), rows.wgs * (int)gridDim.x, reinterpret_cast<int*>(lds), BM * 64);
+            return;
+        }
+    }
+    const int blk = (int)blockIdx.y - (STAGE == 2 ? rows.wgs : 0);
     const int n0 = (int)blockIdx.x * TN;
     const int used = p.num_valid[0];
     if (blk * BLK >= used) return;                     // uniform: blocks past the sorted rows in use
@@ -323,11 +330,22 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p) {
 }
 
 template <int KIND, int STAGE, int NR>
-hipError_t launch_nr(const MoeParams& p, int block_m, int blocks, bool pair, hipStream_t stream) {
-    const dim3 grid((p.n_out + 64 * NR - 1) / (64 * NR), blocks, 1);
+hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int blocks, bool pair, hipStream_t stream) {
+    const unsigned nx = (unsigned)((p.n_out + 64 * NR - 1) / (64 * NR));
+    rows.wgs = 0;
+    if (p.by_position) {
+        // rows of the grid for the lists, as far as it has any left (65535 of them)
+        rows.wgs = (int)((ROWS_INDEX_WGS + nx - 1) / nx);
+        if (blocks + rows.wgs > 65535) {
+            rows.wgs = 0;
+            const hipError_t e = psg_launch_moe_rows_index(rows, stream);
+            if (e != hipSuccess) return e;
+        }
+    }
+    const dim3 grid(nx, blocks + rows.wgs, 1);
 #define PSG_MOE(MR_, CO_)                                                                                \
     {                                                                                                    \
-        hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_>), grid, dim3(256), 0, stream, p);     \
+        hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_>), grid, dim3(256), 0, stream, p, rows);     \
         return hipGetLastError();                                                                        \
     }
     if (pair && block_m == 16) PSG_MOE(2, 2)
@@ -341,7 +359,7 @@ hipError_t launch_nr(const MoeParams& p, int block_m, int blocks, bool pair, hip
 }
 
 template <int KIND, int STAGE>
-hipError_t launch_kind(const MoeParams& p, int block_m, int blocks, hipStream_t stream) {
+hipError_t launch_kind(const MoeParams& p, const MoeRowsParams& rows, int block_m, int blocks, hipStream_t stream) {
     // Stage 1 with one-byte weights multiplies blocks of 16 and 32 rows two at a time where they share an expert (64 tokens x
     // top-8 on 32 experts, blocks of 16: 107 -> 92 us).  Measured and left alone: stage 2 (34 -> 37 us: its second pass over an
     // expert's smaller slab already hits in L2, and pairing halves the workgroups in flight) and packed int4 weights (49 -> 50).
@@ -354,13 +372,13 @@ hipError_t launch_kind(const MoeParams& p, int block_m, int blocks, hipStream_t 
     // flight allow, so a decode-sized stage 1 (64 tokens x top-8 on 32 experts: at most 63 blocks x 12 column tiles) is faster
     // with twice as many workgroups of half the width
     const long wgs128 = (long)blocks / (pair ? 2 : 1) * (long)(p.n_out / 128);
-    if (p.n_out % 128 == 0 && (STAGE == 2 || (tile_m <= 32 && wgs128 >= 1024))) return launch_nr<KIND, STAGE, 2>(p, block_m, blocks, pair, stream);
-    return launch_nr<KIND, STAGE, 1>(p, block_m, blocks, pair, stream);
+    if (p.n_out % 128 == 0 && (STAGE == 2 || (tile_m <= 32 && wgs128 >= 1024))) return launch_nr<KIND, STAGE, 2>(p, rows, block_m, blocks, pair, stream);
+    return launch_nr<KIND, STAGE, 1>(p, rows, block_m, blocks, pair, stream);
 }
 
 }  // namespace
 
-hipError_t psg_launch_moe_tiled(const MoeParams& p, int kind, int stage, int blocks, hipStream_t stream);
+hipError_t psg_launch_moe_tiled(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int blocks, hipStream_t stream);
 
 // Whether the 256-row tiles (moe_gemm_tiled.hip) are the better way for blocks of 128 rows: enough rows per expert that most
 // blocks find a partner, and a tile count (on average over routings: pairs / 256, and half a tile more per expert) that fills its
@@ -380,12 +398,12 @@ bool takes_tiled(const MoeParams& p, int stage) {
     return tiles * 10 >= rounds * cus * 8;
 }
 
-// kind: KIND_INT8 / KIND_FP8 / KIND_INT8W4; stage 1 or 2; block_m in {16, 32, 64, 128}; blocks = entries of expert_ids
-hipError_t psg_launch_moe_gemm(const MoeParams& p, int kind, int stage, int block_m, int blocks, hipStream_t stream) {
-    if (block_m == 128 && kind != KIND_INT8W4 && p.out_dtype != OUT_F32 && p.pair_blocks && takes_tiled(p, stage)) return psg_launch_moe_tiled(p, kind, stage, blocks, stream);
-    if (kind == KIND_INT8) return stage == 1 ? launch_kind<KIND_INT8, 1>(p, block_m, blocks, stream) : launch_kind<KIND_INT8, 2>(p, block_m, blocks, stream);
-    if (kind == KIND_INT8W4) return stage == 1 ? launch_kind<KIND_INT8W4, 1>(p, block_m, blocks, stream) : launch_kind<KIND_INT8W4, 2>(p, block_m, blocks, stream);
-    return stage == 1 ? launch_kind<KIND_FP8, 1>(p, block_m, blocks, stream) : launch_kind<KIND_FP8, 2>(p, block_m, blocks, stream);
+// kind: KIND_INT8 / KIND_FP8 / KIND_INT8W4; stage 1 or 2; rows: where p.by_position is set; block_m in {16, 32, 64, 128}; blocks = entries of expert_ids
+hipError_t psg_launch_moe_gemm(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int block_m, int blocks, hipStream_t stream) {
+    if (block_m == 128 && kind != KIND_INT8W4 && p.out_dtype != OUT_F32 && p.pair_blocks && takes_tiled(p, stage)) return psg_launch_moe_tiled(p, rows, kind, stage, blocks, stream);
+    if (kind == KIND_INT8) return stage == 1 ? launch_kind<KIND_INT8, 1>(p, rows, block_m, blocks, stream) : launch_kind<KIND_INT8, 2>(p, rows, block_m, blocks, stream);
+    if (kind == KIND_INT8W4) return stage == 1 ? launch_kind<KIND_INT8W4, 1>(p, rows, block_m, blocks, stream) : launch_kind<KIND_INT8W4, 2>(p, rows, block_m, blocks, stream);
+    return stage == 1 ? launch_kind<KIND_FP8, 1>(p, rows, block_m, blocks, stream) : launch_kind<KIND_FP8, 2>(p, rows, block_m, blocks, stream);
 }
 
 // sum over the topk slots: y[t, :] = sum_s x[t, s, :] (bf16, fp16 or fp32, the same type in and out; fp32 sum in slot order)

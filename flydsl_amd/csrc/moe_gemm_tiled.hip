@@ -18,6 +18,7 @@
 // workgroup scans the expert ids (64 a ballot), takes its tile in the XCD-aware order of the GEMM tiles over the real count, and
 // leaves when its id is past that.
 #include "gemm_tiled8.h"
+#include "moe_rows.h"
 
 namespace {
 
@@ -327,10 +328,14 @@ __global__ void __launch_bounds__(512, 1) k_moe_tiled(MoeParams p) {
 }
 
 template <int KIND, int STAGE>
-hipError_t go(MoeParams p, int blocks, hipStream_t stream) {
+hipError_t go(MoeParams p, const MoeRowsParams& rows, int blocks, hipStream_t stream) {
     constexpr int TN = STAGE == 1 ? 128 : 256;
     p.blocks = blocks;
     p.group_m = 8;
+    if (p.by_position) {
+        const hipError_t e = psg_launch_moe_rows_index(rows, stream);
+        if (e != hipSuccess) return e;
+    }
     // a list grouped by expert has at most one tile per two blocks and half a tile more per expert
     const long runs = (blocks + (long)p.experts + 1) / 2;
     const unsigned units = (unsigned)(runs < blocks ? runs : blocks);
@@ -340,7 +345,7 @@ hipError_t go(MoeParams p, int blocks, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t psg_launch_moe_tiled(const MoeParams& p, int kind, int stage, int blocks, hipStream_t stream) {
-    if (kind == KIND_INT8) return stage == 1 ? go<KIND_INT8, 1>(p, blocks, stream) : go<KIND_INT8, 2>(p, blocks, stream);
-    return stage == 1 ? go<KIND_FP8, 1>(p, blocks, stream) : go<KIND_FP8, 2>(p, blocks, stream);
+hipError_t psg_launch_moe_tiled(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int blocks, hipStream_t stream) {
+    if (kind == KIND_INT8) return stage == 1 ? go<KIND_INT8, 1>(p, rows, blocks, stream) : go<KIND_INT8, 2>(p, rows, blocks, stream);
+    return stage == 1 ? go<KIND_FP8, 1>(p, rows, blocks, stream) : go<KIND_FP8, 2>(p, rows, blocks, stream);
 }

@@ -14,6 +14,7 @@
 // Operands are swapped (src0 = W, src1 = A) so a lane ends up with 4 consecutive columns of one row.  Four wavefronts side
 // by side along N; each covers 64 W rows: in stage 1 32 gate rows and the 32 up rows of the same columns, so a wavefront
 // owns whole 32-column quantisation groups.
+#include "moe_rows.h"
 #include "psg_common.h"
 
 namespace {
@@ -83,7 +84,7 @@ __device__ __forceinline__ int quant_silu_mul(const v4f g0, const v4f g1, const 
 // that first quantised all K elements of the 16 rows into LDS and then ran the K loop without barriers measured slower: 16 tokens
 // x top-8 on 32 experts 38.9 us against 35.4, 64 tokens 42.2 against 41.)
 template <int AF, int MR, int STAGE, bool IQ = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 4 ? 2 : 1))) k_moe_mx(MoeMxParams p) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 4 ? 2 : 1))) k_moe_mx(MoeMxParams p, MoeRowsParams rows) {
     static_assert(MR % 2 == 0 || MR == 1, "scale chunks cover 32 rows; a single 16-row block picks its half at run time");
     static_assert(!IQ || (MR == 1 && STAGE == 1 && AF == MXF_FP4), "inline quantisation: 16-row blocks of stage 1");
     constexpr int NR = 4;
@@ -100,30 +101,37 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     __shared__ uint8_t iq_scale[2][IQ ? 64 : 1];   // IQ: scale byte of (row, 32-element group) of each LDS stage
     uint8_t(*lds)[TM * AB] = reinterpret_cast<uint8_t(*)[TM * AB]>(lds_raw);
 
+    if constexpr (STAGE == 2) {
+        if ((int)blockIdx.x < rows.wgs) {
+            moe_rows_index_share(rows, (int)blockIdx.x, rows.wgs, reinterpret_cast<int*>(lds_raw), LDS_BYTES / 4);
+            return;
+        }
+    }
+    const int wg = (int)blockIdx.x - (STAGE == 2 ? rows.wgs : 0);
     // Workgroup id -> (row block, column tile).  Consecutive ids go to the 8 XCDs in turn, each with an L2 of its own.
     // by_expert: slice (expert e, column tile t) of the weights belongs to XCD (e * n_tiles + t) % 8, so the few row blocks of an
     // expert read it through the same L2 (ids whose column tile does not exist leave at once); else ids simply count the tiles
     // row block by row block (a slice then alternates between 8 / gcd(8, n_tiles) XCDs).
     int blk, n_tile;
     if (p.by_expert) {
-        const int wg_slot = (int)blockIdx.x >> 3;
+        const int wg_slot = wg >> 3;
         blk = wg_slot / p.n_groups;
         n_tile = wg_slot % p.n_groups * 8;
     } else if (p.quad_tiles) {
         // XCD x = id % 8 takes the row blocks of parity x / 4 and the column tiles t with t % 4 == x % 4: the tiles of a block meet in
         // four L2s instead of eight, a slice of the weights alternates between two
-        const int x = (int)blockIdx.x & 7, s = (int)blockIdx.x >> 3, nq = p.n_tiles >> 2;
+        const int x = wg & 7, s = wg >> 3, nq = p.n_tiles >> 2;
         blk = 2 * (s / nq) + (x >> 2);
         n_tile = (x & 3) + 4 * (s % nq);
     } else {
-        blk = (int)blockIdx.x / p.n_tiles;  // block of TM sorted rows; the sorter's blocks hold TM << eshift rows
-        n_tile = (int)blockIdx.x % p.n_tiles;
+        blk = wg / p.n_tiles;  // block of TM sorted rows; the sorter's blocks hold TM << eshift rows
+        n_tile = wg % p.n_tiles;
     }
     // the quad order rounds the row blocks up to an even number: the odd one out has no entry in expert_ids
     if ((blk >> p.eshift) >= p.blocks || blk * TM >= p.num_valid[0]) return;
     const int e = p.expert_ids[blk >> p.eshift];
     if ((unsigned)e >= (unsigned)p.experts) return;
-    if (p.by_expert) n_tile += ((int)blockIdx.x - e * p.n_tiles) & 7;
+    if (p.by_expert) n_tile += (wg - e * p.n_tiles) & 7;
     if (n_tile >= p.n_tiles) return;
     const int tid = threadIdx.x;
     const int wave = wave_id();
@@ -349,8 +357,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
 // tokens x top-8 on 32 experts, 4096 x 1536, operands three steps ahead in both: stage 1 364 us with 128-row tiles against 292 with
 // 64-row tiles, stage 2 with the atomic epilogue 655 against 393, one row per sorted position 271 against 225).
 template <int AF, int STAGE>
-hipError_t launch_rows(MoeMxParams p, int block_m, int blocks, hipStream_t stream) {
+hipError_t launch_rows(MoeMxParams p, MoeRowsParams rows, int block_m, int blocks, hipStream_t stream) {
     p.eshift = block_m == 128 ? 1 : 0;
+    rows.wgs = p.atomic == 2 ? ROWS_INDEX_WGS : 0;
     p.blocks = blocks;
     p.n_tiles = p.n_out / (STAGE == 1 ? 128 : 256);
     p.n_groups = (p.n_tiles + 7) / 8;
@@ -360,13 +369,13 @@ hipError_t launch_rows(MoeMxParams p, int block_m, int blocks, hipStream_t strea
     p.by_expert = p.n_tiles % 8 != 0 && (long)p.sorted_size <= 192L * p.experts;
     p.quad_tiles = !p.by_expert && p.n_tiles % 4 == 0 && p.n_tiles % 8 != 0;
     const unsigned row_blocks = (unsigned)(blocks << p.eshift);
-    const dim3 grid((unsigned)(p.by_expert ? p.n_groups * 8 : p.n_tiles) * (p.quad_tiles ? (row_blocks + 1) / 2 * 2 : row_blocks));
+    const dim3 grid((unsigned)(p.by_expert ? p.n_groups * 8 : p.n_tiles) * (p.quad_tiles ? (row_blocks + 1) / 2 * 2 : row_blocks) + (unsigned)rows.wgs);
     if (block_m == 16) {
-        if constexpr (STAGE == 2) hipLaunchKernelGGL((k_moe_mx<MXF_FP4, 1, 2>), grid, dim3(256), 0, stream, p);
-        else if constexpr (AF == MXF_FP4) hipLaunchKernelGGL((k_moe_mx<MXF_FP4, 1, 1, true>), grid, dim3(256), 0, stream, p);
+        if constexpr (STAGE == 2) hipLaunchKernelGGL((k_moe_mx<MXF_FP4, 1, 2>), grid, dim3(256), 0, stream, p, rows);
+        else if constexpr (AF == MXF_FP4) hipLaunchKernelGGL((k_moe_mx<MXF_FP4, 1, 1, true>), grid, dim3(256), 0, stream, p, rows);
         else return hipErrorInvalidValue;
-    } else if (block_m == 32) hipLaunchKernelGGL((k_moe_mx<AF, 2, STAGE>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((k_moe_mx<AF, 4, STAGE>), grid, dim3(256), 0, stream, p);
+    } else if (block_m == 32) hipLaunchKernelGGL((k_moe_mx<AF, 2, STAGE>), grid, dim3(256), 0, stream, p, rows);
+    else hipLaunchKernelGGL((k_moe_mx<AF, 4, STAGE>), grid, dim3(256), 0, stream, p, rows);
     return hipGetLastError();
 }
 
@@ -415,9 +424,9 @@ __global__ void __launch_bounds__(256) k_moe_mx_scale_sort(const uint8_t* scale,
 // a_format: MXF_FP4 / MXF_FP8 (stage 1 only; stage 2 reads the fp4 rows stage 1 wrote); block_m: 32 / 64 / 128, or 16: stage 1 then
 // takes bf16 activations in p.a and quantises them itself (a_format MXF_FP4); blocks: blocks of
 // block_m sorted rows the launch covers (blocks past num_valid[0] exit at once)
-hipError_t psg_launch_moe_mx_gemm(const MoeMxParams& p, int a_format, int stage, int block_m, int blocks, hipStream_t stream) {
-    if (stage == 1) return a_format == MXF_FP8 ? launch_rows<MXF_FP8, 1>(p, block_m, blocks, stream) : launch_rows<MXF_FP4, 1>(p, block_m, blocks, stream);
-    return launch_rows<MXF_FP4, 2>(p, block_m, blocks, stream);
+hipError_t psg_launch_moe_mx_gemm(const MoeMxParams& p, const MoeRowsParams& rows, int a_format, int stage, int block_m, int blocks, hipStream_t stream) {
+    if (stage == 1) return a_format == MXF_FP8 ? launch_rows<MXF_FP8, 1>(p, rows, block_m, blocks, stream) : launch_rows<MXF_FP4, 1>(p, rows, block_m, blocks, stream);
+    return launch_rows<MXF_FP4, 2>(p, rows, block_m, blocks, stream);
 }
 
 // out: ceil(sorted_size / 32) * 32 rows x cols bytes, every byte written

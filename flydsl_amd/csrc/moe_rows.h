@@ -6,19 +6,79 @@
 struct MoeRowsParams {
     uint16_t* out;              // [tokens, dim] 16-bit, added into
     uint16_t* rows;             // [sorted_size, dim] weighted rows of the stage
-    int* count;                 // [tokens] rows of each token, then the number of entries of `extra`
+    int* count;                 // [tokens] rows of each token
     int* list;                  // [tokens, topk] sorted positions of a token's rows
-    int* extra;                 // sorted positions of rows past topk
+    int* next;                  // [sorted_size] behind the last entry of a full list: the token's rows past topk, chained, -1 at the end
     const int32_t* sorted_ids;
     const int32_t* expert_ids;
     const int32_t* num_valid;
-    int tokens, topk, experts, dim, sorted_size, blocks, block_m;
+    int tokens, topk, experts, dim, sorted_size, blocks;
+    int block_m;                // a power of two
     int slots;                  // ids with a slot number from here on are padding
     int granule;                // rows of the tiles the stage computes up to num_valid in
     int out_dtype;
+    int wgs;                    // workgroups (k_moe_gemm: rows of the grid) in front of a stage's tiles that make the lists; 0 = none
 };
+
+// Workgroups that make the lists above.  The stages of k_moe_gemm and k_moe_mx spend them in front of their own tiles, where they work beside the
+// tiles and cost no time of their own; the 256-row tiles (one workgroup a CU, not a register to spare: with the lists in the same kernel
+// it spilled 28 instead of 18 of them and lost 20 us) have them in a launch in front.  (One launch that cleared the counts and
+// another that entered the rows took 9.5 us, 1024 or 4096 tokens x top-8; as one launch it is 8.  Whole layers, us before / now: int4 1052 tokens x
+// top-8, 1536 x 1024, 128 / 124; int8 813 x top-4, 4096 x 512, 140 / 135; MX 410 x top-8, 4096 x 1536, 140.6 / 134.6; 1500 x top-6, 2048 x 768, 99 /
+// 93; 4096 x top-8 602 / 596; fp8 on 256-row tiles, which the power limit bounds, 807 / 809.)  A multiple of 8 leaves every tile on its XCD.
+constexpr int ROWS_INDEX_WGS = 32;
 
 uint64_t psg_moe_rows_bytes(int64_t tokens, int64_t topk, int64_t sorted_size, int64_t dim);
 void psg_moe_rows_carve(MoeRowsParams& p, void* workspace);
 hipError_t psg_launch_moe_rows_index(const MoeRowsParams& p, hipStream_t stream);
 hipError_t psg_launch_moe_rows_add(const MoeRowsParams& p, hipStream_t stream);
+
+// Share `wg` of `wgs` of the lists: a range of tokens, for which it looks through the whole sorted list (16 to 600 KB out of L2).  The counts stay in
+// LDS (`lds`, two ints a token, `lds_ints` in all), so nothing has to be cleared before.
+__device__ __forceinline__ void moe_rows_index_share(const MoeRowsParams& p, int wg, int wgs, int* lds, int lds_ints) {
+    const int tid = (int)threadIdx.x, nt = (int)blockDim.x;
+    const int per = (p.tokens + wgs - 1) / wgs, first = wg * per, last = first + per < p.tokens ? first + per : p.tokens;
+    const int cap = lds_ints / 2;
+    int* cnt = lds;
+    int* head = lds + cap;
+    // the rows the stage computes: whole tiles up to num_valid, in blocks that are in the list
+    const int nv = p.num_valid[0];
+    int limit = nv >= p.sorted_size ? p.sorted_size : nv <= 0 ? 0 : (nv + p.granule - 1) / p.granule * p.granule;
+    if (limit > p.sorted_size) limit = p.sorted_size;
+    if ((int64_t)p.blocks * p.block_m < limit) limit = p.blocks * p.block_m;
+    const int sh = __builtin_ctz(p.block_m);
+    constexpr int B = 16;  // ids, and experts of their blocks, that a thread asks for at a time
+    for (int t0 = first; t0 < last; t0 += cap) {
+        const int n = last - t0 < cap ? last - t0 : cap;
+        for (int i = tid; i < n; i += nt) {
+            cnt[i] = 0;
+            head[i] = -1;
+        }
+        __syncthreads();
+        for (int i0 = 0; i0 < limit; i0 += nt * B) {
+            uint32_t id[B];
+            int e[B];
+#pragma unroll
+            for (int j = 0; j < B; j++) {
+                const int i = i0 + j * nt + tid, at = i < limit ? i : 0;
+                id[j] = (uint32_t)p.sorted_ids[at];
+                e[j] = p.expert_ids[at >> sh];
+            }
+#pragma unroll
+            for (int j = 0; j < B; j++) {
+                const int i = i0 + j * nt + tid, t = (int)(id[j] & 0xFFFFFFu), at = t - t0;
+                if (i >= limit || (unsigned)at >= (unsigned)n || (int)(id[j] >> 24) >= p.slots) continue;
+                if ((unsigned)e[j] >= (unsigned)p.experts) continue;  // a block without an expert
+                const int k = atomicAdd(&cnt[at], 1);
+                if (k < p.topk - 1) p.list[(size_t)t * p.topk + k] = i;
+                else p.next[i] = atomicExch(&head[at], i);
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < n; i += nt) {
+            p.count[t0 + i] = cnt[i];
+            if (cnt[i] >= p.topk) p.list[(size_t)(t0 + i) * p.topk + p.topk - 1] = head[i];
+        }
+        __syncthreads();
+    }
+}

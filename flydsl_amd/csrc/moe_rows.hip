@@ -5,9 +5,9 @@
 // model 4096, i.e. 268 MB of additions: fp8 stage 2 434 us, MX-FP4 436), a store and a read of the same rows at 5.  So `topk`
 // additions per output element become one; that one stays atomic, because launches on other streams may be adding into `out` too.
 //
-// Which sorted rows belong to a token is found on the device, so any sorted list the atomic epilogue accepts works here: rows are
-// entered into a list of `topk` places per token, and rows that do not fit (a list that names a token more often than topk
-// times) go to a list of their own and are added one by one.
+// Which sorted rows belong to a token is found on the device, by workgroups in front of the stage's tiles (moe_rows_index_share), so any sorted
+// list the atomic epilogue accepts works here: rows are entered into a list of `topk` places per token, and rows that do not fit (a
+// list that names a token more often than topk times) are chained behind its last entry.
 #include "psg_common.h"
 #include "moe_rows.h"
 
@@ -16,7 +16,6 @@ namespace {
 typedef __fp16 v2h_t __attribute__((ext_vector_type(2)));
 typedef __bf16 v2b_t __attribute__((ext_vector_type(2)));
 
-constexpr int EXTRA_WGS = 8;    // workgroups per column chunk that add the rows beyond topk
 constexpr int DWORDS = 4;       // dword columns per thread: 256 threads cover 2048 16-bit columns
 
 __device__ __forceinline__ void add_packed(uint32_t* o, int bits, int out_dtype) {
@@ -24,24 +23,9 @@ __device__ __forceinline__ void add_packed(uint32_t* o, int bits, int out_dtype)
     else __builtin_amdgcn_global_atomic_fadd_v2f16((__attribute__((address_space(1))) v2h_t*)o, __builtin_bit_cast(v2h_t, bits));
 }
 
-__global__ void __launch_bounds__(256) k_moe_rows_clear(int* count, int n) {
-    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (i < n) count[i] = 0;
-}
-
-__global__ void __launch_bounds__(256) k_moe_rows_index(MoeRowsParams p) {
-    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (i >= p.sorted_size) return;
-    // the rows the stage computes: whole workgroup tiles up to num_valid, in blocks that have an expert
-    const int blk = i / p.block_m;
-    if (blk >= p.blocks || i / p.granule * p.granule >= p.num_valid[0]) return;
-    if ((unsigned)p.expert_ids[blk] >= (unsigned)p.experts) return;
-    const uint32_t sid = (uint32_t)p.sorted_ids[i];
-    const int t = (int)(sid & 0xFFFFFFu);
-    if (t >= p.tokens || (int)(sid >> 24) >= p.slots) return;
-    const int k = atomicAdd(&p.count[t], 1);
-    if (k < p.topk) p.list[(size_t)t * p.topk + k] = i;
-    else p.extra[atomicAdd(&p.count[p.tokens], 1)] = i;
+__global__ void __launch_bounds__(1024) k_moe_rows_index(MoeRowsParams p) {
+    __shared__ int lds[4096];
+    moe_rows_index_share(p, (int)blockIdx.x, (int)gridDim.x, lds, 4096);
 }
 
 template <int OUT>
@@ -51,29 +35,16 @@ __global__ void __launch_bounds__(256) k_moe_rows_add(MoeRowsParams p, int chunk
     const int c0 = ((int)blockIdx.x % chunks) * (256 * DWORDS) + (int)threadIdx.x;
     const uint32_t* rows = reinterpret_cast<const uint32_t*>(p.rows);
     uint32_t* out = reinterpret_cast<uint32_t*>(p.out);
-    if (unit >= p.tokens) {
-        const int n = p.count[p.tokens];
-        for (int q = unit - p.tokens; q < n; q += EXTRA_WGS) {
-            const int pos = p.extra[q];
-            const size_t t = (size_t)(p.sorted_ids[pos] & 0xFFFFFF);
-#pragma unroll
-            for (int j = 0; j < DWORDS; j++) {
-                const int c = c0 + j * 256;
-                if (c < dws) add_packed(out + t * dws + c, (int)rows[(size_t)pos * dws + c], OUT);
-            }
-        }
-        return;
-    }
-    const int n = p.count[unit] < p.topk ? p.count[unit] : p.topk;
-    if (n == 0) return;
+    const int count = p.count[unit], n = count < p.topk ? count : p.topk;
+    if (n <= 0) return;
     const int* list = p.list + (size_t)unit * p.topk;
     float lo[DWORDS] = {}, hi[DWORDS] = {};
-    auto add4 = [&](int k0, auto CNT) {
+    auto add4 = [&](const int* list, auto CNT) {
         constexpr int N = decltype(CNT)::value;
         uint32_t v[N][DWORDS];
 #pragma unroll
         for (int k = 0; k < N; k++) {
-            const size_t base = (size_t)__builtin_amdgcn_readfirstlane(list[k0 + k]) * dws;
+            const size_t base = (size_t)__builtin_amdgcn_readfirstlane(list[k]) * dws;
 #pragma unroll
             for (int j = 0; j < DWORDS; j++) {
                 const int c = c0 + j * 256;
@@ -89,9 +60,11 @@ __global__ void __launch_bounds__(256) k_moe_rows_add(MoeRowsParams p, int chunk
             }
     };
     int k = 0;
-    for (; k + 8 <= n; k += 8) add4(k, std::integral_constant<int, 8>{});
-    for (; k + 2 <= n; k += 2) add4(k, std::integral_constant<int, 2>{});
-    if (k < n) add4(k, std::integral_constant<int, 1>{});
+    for (; k + 8 <= n; k += 8) add4(list + k, std::integral_constant<int, 8>{});
+    for (; k + 2 <= n; k += 2) add4(list + k, std::integral_constant<int, 2>{});
+    if (k < n) add4(list + k, std::integral_constant<int, 1>{});
+    if (count > p.topk)  // uniform
+        for (int pos = p.next[list[p.topk - 1]], left = count - p.topk; left > 0; pos = p.next[pos], left--) add4(&pos, std::integral_constant<int, 1>{});
 #pragma unroll
     for (int j = 0; j < DWORDS; j++) {
         const int c = c0 + j * 256;
@@ -115,18 +88,18 @@ void psg_moe_rows_carve(MoeRowsParams& p, void* workspace) {
     w += up16((uint64_t)(p.tokens + 1) * 4);
     p.list = reinterpret_cast<int*>(w);
     w += up16((uint64_t)p.tokens * p.topk * 4);
-    p.extra = reinterpret_cast<int*>(w);
+    p.next = reinterpret_cast<int*>(w);
 }
 
+// the lists in a launch of their own, for the stages that do not make them beside their tiles
 hipError_t psg_launch_moe_rows_index(const MoeRowsParams& p, hipStream_t stream) {
-    hipLaunchKernelGGL(k_moe_rows_clear, dim3((p.tokens + 256) / 256), dim3(256), 0, stream, p.count, p.tokens + 1);
-    hipLaunchKernelGGL(k_moe_rows_index, dim3((p.sorted_size + 255) / 256), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(k_moe_rows_index, dim3(ROWS_INDEX_WGS), dim3(1024), 0, stream, p);
     return hipGetLastError();
 }
 
 hipError_t psg_launch_moe_rows_add(const MoeRowsParams& p, hipStream_t stream) {
     const int chunks = (p.dim / 2 + 256 * DWORDS - 1) / (256 * DWORDS);
-    const dim3 grid((unsigned)(p.tokens + EXTRA_WGS) * (unsigned)chunks);
+    const dim3 grid((unsigned)p.tokens * (unsigned)chunks);
     if (p.out_dtype == OUT_BF16) hipLaunchKernelGGL((k_moe_rows_add<OUT_BF16>), grid, dim3(256), 0, stream, p, chunks);
     else hipLaunchKernelGGL((k_moe_rows_add<OUT_FP16>), grid, dim3(256), 0, stream, p, chunks);
     return hipGetLastError();

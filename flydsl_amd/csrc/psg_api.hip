@@ -14,8 +14,8 @@
 
 hipError_t psg_launch_a8w8_tiled(const A8W8Params& p, int kind, int store, int tile_m, int tile_n, hipStream_t stream);
 hipError_t psg_launch_a8w8_stream(const A8W8Params& p, int kind, int store, hipStream_t stream);
-hipError_t psg_launch_moe_gemm(const MoeParams& p, int kind, int stage, int block_m, int blocks, hipStream_t stream);
-hipError_t psg_launch_moe_mx_gemm(const MoeMxParams& p, int a_format, int stage, int block_m, int blocks, hipStream_t stream);
+hipError_t psg_launch_moe_gemm(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int block_m, int blocks, hipStream_t stream);
+hipError_t psg_launch_moe_mx_gemm(const MoeMxParams& p, const MoeRowsParams& rows, int a_format, int stage, int block_m, int blocks, hipStream_t stream);
 hipError_t psg_launch_moe_mx_scale_sort(const void* scale, const int32_t* sorted_ids, const int32_t* num_valid, void* out, int tokens, int topk, int cols,
                                         int sorted_size, hipStream_t stream);
 hipError_t psg_launch_moe_sort(const MoeSortParams& p, void* workspace, uint64_t workspace_bytes, hipStream_t stream);
@@ -828,10 +828,8 @@ static int moe_gemm_common(const psg_moe_args* a, void* workspace, uint64_t work
         p.out = r.rows;
         p.accumulate = 0;
         p.by_position = 1;
-        e = psg_launch_moe_rows_index(r, static_cast<hipStream_t>(stream));
-        if (e != hipSuccess) return hip_fail(e, "psg_moe_gemm launch");
     }
-    e = psg_launch_moe_gemm(p, a->in_dtype == PSG_IN_INT8 ? KIND_INT8 : a->in_dtype == PSG_IN_INT8_W4 ? KIND_INT8W4 : KIND_FP8, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
+    e = psg_launch_moe_gemm(p, r, a->in_dtype == PSG_IN_INT8 ? KIND_INT8 : a->in_dtype == PSG_IN_INT8_W4 ? KIND_INT8W4 : KIND_FP8, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
     if (e == hipSuccess && rows) e = psg_launch_moe_rows_add(r, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "psg_moe_gemm launch");
     g_err[0] = 0;
@@ -928,7 +926,7 @@ static int moe_mx_gemm_common(const psg_moe_mx_args* a, int32_t topk, void* work
     p.atomic = a->stage == 2 && a->atomic ? 1 : 0;
     p.eshift = 0;
     p.n_tiles = p.n_groups = p.by_expert = p.quad_tiles = 0;
-    if (((int64_t)a->blocks << 1) * (int64_t)((n_out / 128 + 7) / 8 * 8) > 0x7FFFFFFFll) return fail(PSG_E_SHAPE, "blocks=%d times the column tiles exceed the grid", a->blocks);
+    if (((int64_t)a->blocks << 1) * (int64_t)((n_out / 128 + 7) / 8 * 8) > 0x7FFFFFFFll - ROWS_INDEX_WGS) return fail(PSG_E_SHAPE, "blocks=%d times the column tiles exceed the grid", a->blocks);
     hipError_t e = hipSuccess;
     const bool rows = workspace && p.atomic && topk >= 1 && topk <= 255 && workspace_bytes >= psg_moe_rows_bytes(a->tokens, topk, a->sorted_size, n_out);
     MoeRowsParams r{};
@@ -950,10 +948,8 @@ static int moe_mx_gemm_common(const psg_moe_mx_args* a, int32_t topk, void* work
         psg_moe_rows_carve(r, workspace);
         p.out = r.rows;
         p.atomic = 2;
-        e = psg_launch_moe_rows_index(r, static_cast<hipStream_t>(stream));
-        if (e != hipSuccess) return hip_fail(e, "psg_moe_mx_gemm launch");
     }
-    e = psg_launch_moe_mx_gemm(p, a->a_dtype == PSG_MX_FP8 ? MXF_FP8 : MXF_FP4, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
+    e = psg_launch_moe_mx_gemm(p, r, a->a_dtype == PSG_MX_FP8 ? MXF_FP8 : MXF_FP4, a->stage, a->block_m, a->blocks, static_cast<hipStream_t>(stream));
     if (e == hipSuccess && rows) e = psg_launch_moe_rows_add(r, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "psg_moe_mx_gemm launch");
     g_err[0] = 0;
