@@ -57,8 +57,10 @@ __device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g));
 // of 16 or 32 rows: an expert with 17 to 32 routed rows would otherwise stream its weights once per block).  Blocks pair up
 // from the start of each run of equal expert ids: the workgroup of the second block of a pair ends at once, and the
 // first one treats the second half of its tile as padding when the run ends there.
-template <int KIND, int MR, int NR, int STAGE, int CO = 1>
-__global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, MoeRowsParams rows) {
+// ROWS = MoeRowsParams: the down stage by rows, whose first `rows.wgs` rows of the grid make the lists of the tokens' rows.  A build of
+// its own: the decode layers, which add directly, lost 0.4 to 0.8 us of 55 to 140 to the longer arguments and the branch.
+template <int KIND, int MR, int NR, int STAGE, int CO, class... ROWS>
+__global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     using acc_t = typename MoeAcc<KIND>::type;
     constexpr int BM = 16 * MR, TN = 64 * NR;
     constexpr int BLK = BM / CO;                        // rows of one block of the sorted list
@@ -73,13 +75,15 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, MoeRowsParams row
     const int tid = threadIdx.x;
     const int wave = wave_id();
     const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
-    if constexpr (STAGE == 2) {
-        if ((int)blockIdx.y < rows.wgs) {
-            moe_rows_index_share(rows, (int)(blockIdx.y * gridDim.x + blockIdx.x), rows.wgs * (int)gridDim.x, reinterpret_cast<int*>(lds), BM * 64);
+    int blk = (int)blockIdx.y;
+    if constexpr (sizeof...(ROWS) == 1) {
+        const MoeRowsParams& r = (rows, ...);
+        if (blk < r.wgs) {
+            moe_rows_index_share<4>(r, (int)(blockIdx.y * gridDim.x + blockIdx.x), r.wgs * (int)gridDim.x, reinterpret_cast<int*>(lds), BM * 64);
             return;
         }
+        blk -= r.wgs;
     }
-    const int blk = (int)blockIdx.y - (STAGE == 2 ? rows.wgs : 0);
     const int n0 = (int)blockIdx.x * TN;
     const int used = p.num_valid[0];
     if (blk * BLK >= used) return;                     // uniform: blocks past the sorted rows in use
@@ -333,11 +337,13 @@ template <int KIND, int STAGE, int NR>
 hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int blocks, bool pair, hipStream_t stream) {
     const unsigned nx = (unsigned)((p.n_out + 64 * NR - 1) / (64 * NR));
     rows.wgs = 0;
-    if (p.by_position) {
+    bool lists = STAGE == 2 && p.by_position;
+    if (lists) {
         // rows of the grid for the lists, as far as it has any left (65535 of them)
         rows.wgs = (int)((ROWS_INDEX_WGS + nx - 1) / nx);
         if (blocks + rows.wgs > 65535) {
             rows.wgs = 0;
+            lists = false;
             const hipError_t e = psg_launch_moe_rows_index(rows, stream);
             if (e != hipSuccess) return e;
         }
@@ -345,7 +351,12 @@ hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int bl
     const dim3 grid(nx, blocks + rows.wgs, 1);
 #define PSG_MOE(MR_, CO_)                                                                                \
     {                                                                                                    \
-        hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_>), grid, dim3(256), 0, stream, p, rows);     \
+        if constexpr (STAGE == 2)                                                                        \
+            if (lists) {                                                                                 \
+                hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
+                return hipGetLastError();                                                                \
+            }                                                                                            \
+        hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_>), grid, dim3(256), 0, stream, p);     \
         return hipGetLastError();                                                                        \
     }
     if (pair && block_m == 16) PSG_MOE(2, 2)

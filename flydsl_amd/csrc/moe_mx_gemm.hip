@@ -103,7 +103,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
 
     if constexpr (STAGE == 2) {
         if ((int)blockIdx.x < rows.wgs) {
-            moe_rows_index_share(rows, (int)blockIdx.x, rows.wgs, reinterpret_cast<int*>(lds_raw), LDS_BYTES / 4);
+            moe_rows_index_share<16>(rows, (int)blockIdx.x, rows.wgs, reinterpret_cast<int*>(lds_raw), LDS_BYTES / 4);
             return;
         }
     }

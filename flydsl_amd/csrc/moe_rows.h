@@ -20,9 +20,10 @@ struct MoeRowsParams {
     int wgs;                    // workgroups (k_moe_gemm: rows of the grid) in front of a stage's tiles that make the lists; 0 = none
 };
 
-// Workgroups that make the lists above.  The stages of k_moe_gemm and k_moe_mx spend them in front of their own tiles, where they work beside the
-// tiles and cost no time of their own; the 256-row tiles (one workgroup a CU, not a register to spare: with the lists in the same kernel
-// it spilled 28 instead of 18 of them and lost 20 us) have them in a launch in front.  (One launch that cleared the counts and
+// Workgroups that make the lists above.  The stages of k_moe_gemm and k_moe_mx have them in front of their own tiles, where they work beside
+// these and cost no time of their own (behind the tiles their own 15 us are the end of the launch: MX stage 2, 4096 tokens x top-8, 242 us against
+// 231); the 256-row tiles (one workgroup a CU, not a register to spare: with the lists in the same kernel it spilled 28 instead of 18 of
+// them and lost 20 us) have them in a launch in front.  (One launch that cleared the counts and
 // another that entered the rows took 9.5 us, 1024 or 4096 tokens x top-8; as one launch it is 8.  Whole layers, us before / now: int4 1052 tokens x
 // top-8, 1536 x 1024, 128 / 124; int8 813 x top-4, 4096 x 512, 140 / 135; MX 410 x top-8, 4096 x 1536, 140.6 / 134.6; 1500 x top-6, 2048 x 768, 99 /
 // 93; 4096 x top-8 602 / 596; fp8 on 256-row tiles, which the power limit bounds, 807 / 809.)  A multiple of 8 leaves every tile on its XCD.
@@ -35,6 +36,9 @@ hipError_t psg_launch_moe_rows_add(const MoeRowsParams& p, hipStream_t stream);
 
 // Share `wg` of `wgs` of the lists: a range of tokens, for which it looks through the whole sorted list (16 to 600 KB out of L2).  The counts stay in
 // LDS (`lds`, two ints a token, `lds_ints` in all), so nothing has to be cleared before.
+// B = ids, and experts of their blocks, that a thread asks for at a time (few enough that the stage keeps its registers: 16 of them in the 16-row down
+// stage, 64 registers without, cost it two wavefronts a SIMD and the decode layer of 64 tokens 3 us)
+template <int B>
 __device__ __forceinline__ void moe_rows_index_share(const MoeRowsParams& p, int wg, int wgs, int* lds, int lds_ints) {
     const int tid = (int)threadIdx.x, nt = (int)blockDim.x;
     const int per = (p.tokens + wgs - 1) / wgs, first = wg * per, last = first + per < p.tokens ? first + per : p.tokens;
@@ -47,7 +51,6 @@ __device__ __forceinline__ void moe_rows_index_share(const MoeRowsParams& p, int
     if (limit > p.sorted_size) limit = p.sorted_size;
     if ((int64_t)p.blocks * p.block_m < limit) limit = p.blocks * p.block_m;
     const int sh = __builtin_ctz(p.block_m);
-    constexpr int B = 16;  // ids, and experts of their blocks, that a thread asks for at a time
     for (int t0 = first; t0 < last; t0 += cap) {
         const int n = last - t0 < cap ? last - t0 : cap;
         for (int i = tid; i < n; i += nt) {

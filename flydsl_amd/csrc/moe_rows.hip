@@ -5,7 +5,7 @@
 // model 4096, i.e. 268 MB of additions: fp8 stage 2 434 us, MX-FP4 436), a store and a read of the same rows at 5.  So `topk`
 // additions per output element become one; that one stays atomic, because launches on other streams may be adding into `out` too.
 //
-// Which sorted rows belong to a token is found on the device, by workgroups in front of the stage's tiles (moe_rows_index_share), so any sorted
+// Which sorted rows belong to a token is found on the device, by workgroups beside the stage's tiles (moe_rows_index_share), so any sorted
 // list the atomic epilogue accepts works here: rows are entered into a list of `topk` places per token, and rows that do not fit (a
 // list that names a token more often than topk times) are chained behind its last entry.
 #include "psg_common.h"
@@ -25,7 +25,7 @@ __device__ __forceinline__ void add_packed(uint32_t* o, int bits, int out_dtype)
 
 __global__ void __launch_bounds__(1024) k_moe_rows_index(MoeRowsParams p) {
     __shared__ int lds[4096];
-    moe_rows_index_share(p, (int)blockIdx.x, (int)gridDim.x, lds, 4096);
+    moe_rows_index_share<16>(p, (int)blockIdx.x, (int)gridDim.x, lds, 4096);
 }
 
 template <int OUT>
