@@ -7,7 +7,14 @@ The library is the only compute path: if it is missing or fails to load, ``lib()
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
+import struct
+
+try:
+    from . import _native  # operand checks and launches in native code (csrc/native.cpp)
+except ImportError as e:
+    _native, _native_error = None, e
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libpsgemm.so")
@@ -212,6 +219,8 @@ def lib() -> ctypes.CDLL:
     global _lib
     if _lib is not None:
         return _lib
+    if _native is None:
+        raise RuntimeError(f"flydsl_amd/_native.so cannot be loaded ({_native_error}); run `make -C {os.path.join(_HERE, 'csrc')}`")
     if not os.path.exists(LIB_PATH):
         raise RuntimeError(
             f"{LIB_PATH} is not built; run `make -C {os.path.join(_HERE, 'csrc')}` "
@@ -270,6 +279,22 @@ def lib() -> ctypes.CDLL:
         raise RuntimeError(f"{LIB_PATH} has ABI version {got}, this package needs {ABI_VERSION}")
     _lib = handle
     return _lib
+
+
+@functools.lru_cache(maxsize=None)
+def address(name: str) -> int:
+    """Address of an entry point of the library, for the launches of ``_native``."""
+    return ctypes.cast(getattr(lib(), name), ctypes.c_void_p).value
+
+
+TYPE_ANY, TYPE_INT32, TYPE_FP32, TYPE_BF16, TYPE_FP16 = range(5)
+OPTIONAL = 256  # added to a type: None may stand in the operand's place
+
+
+def operands(*ops) -> bytes:
+    """The operands of a launch the way ``_native.launch`` reads them: ``(field of the argument struct, bytes of an element or 0,
+    TYPE_*, least bytes[, index of the struct])`` each, ``field`` being a ctypes field descriptor."""
+    return b"".join(struct.pack("<iiiiq", op[4] if len(op) > 4 else 0, op[0].offset, op[1], op[2], op[3]) for op in ops)
 
 
 def check(rc: int, what: str) -> None:

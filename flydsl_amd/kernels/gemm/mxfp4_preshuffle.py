@@ -42,8 +42,9 @@ def _operand(t, name, need):
 def _plan(M, i32_n, N, K, tile_m, tile_n, tile_k, a_dtype, out_dtype, b_dtype, B, a_row_stride, a_batch_stride, sca_row_stride, sca_batch_stride,
           c_row_stride, c_batch_stride, xcd_swizzle, force_path, tile, wave_layout, splits, no_split):
     """What a call's sizes, formats and strides alone decide (a function of values, kept for the next call with the same ones): the argument
-    struct without its addresses, the bytes that c, a, b, scale_a and scale_b must hold, and the bytes of workspace.  Working it out
-    took 4 of the 7 us a call spent on the host, more than the kernel of a decode-sized problem runs."""
+    struct without its addresses, the bytes that c, a, b, scale_a and scale_b must hold, the bytes of workspace, and the struct and the
+    operands the way the native launch takes them.  Working it out took 4 of the 7 us a call spent on the host, more than the kernel of a
+    decode-sized problem runs."""
     if a_dtype not in _lib.MX_DTYPE:
         raise ValueError(f"a_dtype must be fp4/fp6/fp8, got {a_dtype!r}")
     if b_dtype not in ("fp4", "fp8"):
@@ -99,7 +100,12 @@ def _plan(M, i32_n, N, K, tile_m, tile_n, tile_k, a_dtype, out_dtype, b_dtype, B
         need = lib.psg_workspace_bytes(args.M, args.N, args.K, 5)
     else:
         need = 0
-    return bytes(args), needs, need
+    ops = [(getattr(_lib.MxArgs, name), 0, _lib.TYPE_ANY, n) for name, n in zip(("c", "a", "b", "scale_a", "scale_b"), needs)]
+    native = _lib.MxArgs.from_buffer_copy(args)
+    if need:
+        native.workspace_bytes = need
+        ops.append((_lib.MxArgs.workspace, 1, _lib.TYPE_ANY, need))
+    return bytes(args), needs, need, (bytes(native),), _lib.operands(*ops)
 
 
 def launch_gemm(
@@ -145,9 +151,18 @@ def launch_gemm(
     # (anything but plain numbers and texts is worked out anew: other types may hash by identity)
     plain = type(N) is type(K) is type(tile_m) is type(tile_n) is type(tile_k) is int and type(a_dtype) is type(b_dtype) is type(out_dtype) is str
     plan = _plan if plain else _plan.__wrapped__
-    proto, needs, need = plan(int(i32_m), int(i32_n), N, K, tile_m, tile_n, tile_k, a_dtype, out_dtype, b_dtype, int(batch), int(a_row_stride),
+    proto, needs, need, native, ops = plan(int(i32_m), int(i32_n), N, K, tile_m, tile_n, tile_k, a_dtype, out_dtype, b_dtype, int(batch), int(a_row_stride),
                               int(a_batch_stride), int(sca_row_stride), int(sca_batch_stride), int(c_row_stride), int(c_batch_stride), int(xcd_swizzle),
                               int(_force_path), None if _tile is None else (int(_tile[0]), int(_tile[1])), int(_wave_layout), int(_splits), bool(_no_split))
+    if _acc is None and stream is not None:
+        tensors = (arg_c, arg_a, arg_b, arg_scale_a, arg_scale_b)
+        if need and hasattr(arg_c, "device"):
+            tensors += (_lib.workspace(arg_c.device, need, _lib.stream_handle(stream), owner="mxfp4"),)
+        rc = _lib._native.launch(_lib.address("psg_gemm_mxfp4"), native, ops, stream, *tensors)
+        if rc != _lib._native.DECLINED:
+            if rc:
+                _lib.check(rc, "psg_gemm_mxfp4")
+            return
     # operands given as tensors are checked on the host (raw addresses cannot be): device, contiguity, extent
     args = _lib.MxArgs.from_buffer_copy(proto)
     args.c = None if _acc is not None else _operand(arg_c, "c", needs[0])

@@ -50,9 +50,49 @@ class MoeStage:
         self.no_pairing = False  # True: one workgroup per block of the sorted list even for blocks of 16 / 32 rows (tests)
         self.out_dtype, self.in_dtype = _OUT[str(out_dtype).strip().lower()], _lib.IN_DTYPE["int8" if in_dtype == "int8smooth" else in_dtype]
         self._lib = _lib.lib()
+        self._plans = {}  # what numbers alone decide about a call, by those numbers
+
+    def _plan(self, tokens, blocks, size):
+        """(argument struct without its addresses, operands) of a call as the native launch takes them, ``None`` twice when it needs scratch;
+        and the library's rule for that, which the plan holds for."""
+        rule = self._lib.psg_moe_rows_workspace_bytes
+        n_out, K = (self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)
+        rows_x = tokens if (self.stage == 1 and not self.slot_major) else tokens * self.topk
+        rows_w = self.experts * (2 * n_out if self.stage == 1 else n_out)
+        rows_out = tokens * self.topk if (self.stage == 1 or not self.accumulate) else tokens
+        osize = 4 if self.out_dtype == 2 else 2
+        if self.stage == 2 and self.accumulate and rule(tokens, self.topk, size, n_out, self.out_dtype, 2 if self.w4 else 0):
+            return None, None, rule
+        a = _lib.MoeArgs()
+        a.tokens, a.topk, a.experts = tokens, self.topk, self.experts
+        a.model_dim, a.inter_dim = self.model_dim, self.inter_dim
+        a.sorted_size, a.blocks, a.block_m = size, blocks, self.tile_m
+        a.in_dtype, a.out_dtype, a.stage = self.in_dtype, self.out_dtype, self.stage
+        a.doweight, a.accumulate = int(self.doweight), int(self.accumulate)
+        a.x_slot_major, a.no_pairing = int(self.slot_major), int(self.no_pairing)
+        f, any_ = _lib.MoeArgs, _lib.TYPE_ANY
+        ops = _lib.operands((f.out, osize, any_, rows_out * n_out * osize), (f.x, 1, any_, rows_x * K), (f.w, 1, any_, rows_w * K // (2 if self.w4 else 1)),
+                            (f.scale_x, 4, any_, 4 * rows_x), (f.scale_w, 4, any_, 4 * rows_w), (f.sorted_token_ids, 4, any_, 4 * size),
+                            (f.sorted_expert_ids, 4, any_, 4 * blocks), (f.sorted_weights, 4, any_, 4 * size if self.doweight else 0),
+                            (f.num_valid_ids, 4, any_, 4))
+        return (bytes(a),), ops, rule
 
     def __call__(self, out, x, w, scale_x, scale_w, sorted_token_ids, sorted_expert_ids, sorted_weights, num_valid_ids,
                  tokens, dim0, dim1, blocks, stream=None):
+        if stream is not None and type(tokens) is type(blocks) is int and (dim0, dim1) == ((self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)):
+            key = (tokens, blocks, sorted_token_ids.numel(), self.no_pairing)
+            plan = self._plans.get(key)
+            if plan is None or plan[2] is not self._lib.psg_moe_rows_workspace_bytes:
+                if len(self._plans) >= 256:
+                    self._plans.clear()
+                plan = self._plans[key] = self._plan(*key[:3])
+            if plan[0] is not None:
+                rc = _lib._native.launch(_lib.address("psg_moe_gemm"), plan[0], plan[1], stream, out, x, w, scale_x, scale_w, sorted_token_ids,
+                                         sorted_expert_ids, sorted_weights, num_valid_ids)
+                if rc != _lib._native.DECLINED:
+                    if rc:
+                        _lib.check(rc, "psg_moe_gemm")
+                    return
         tokens, blocks = int(tokens), int(blocks)
         n_out, K = (self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)
         if (int(dim0), int(dim1)) != (n_out, K):
@@ -130,6 +170,12 @@ class MoeReduction:
         self._lib = _lib.lib()
 
     def __call__(self, X, Y, expert_mask, topk_ids, i32_m_tokens, stream=None):
+        if not self.use_mask and stream is not None:
+            rc = _lib._native.moe_reduce(_lib.address("psg_moe_reduce"), X, Y, 4 if self.dtype == 2 else 2, i32_m_tokens, self.topk, self.model_dim, self.dtype, stream)
+            if rc != _lib._native.DECLINED:
+                if rc:
+                    _lib.check(rc, "psg_moe_reduce")
+                return
         tokens = int(i32_m_tokens)
         esz = (4 if self.dtype == 2 else 2,)
         dev = _lib.check_operand("Y", Y, min_elems=tokens * self.model_dim, elem_sizes=esz)

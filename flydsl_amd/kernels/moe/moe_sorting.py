@@ -9,6 +9,7 @@ a graph); host tensors are sorted with torch (one stable sort of the (token, slo
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -74,6 +75,35 @@ def _sort_args(tokens, topk, sorted_ids, sorted_weights, sorted_expert_ids, num_
     return args, workspace
 
 
+@functools.lru_cache(maxsize=1024)
+def _routing_plan(tokens, E, topk, B, dtype_str, renormalize, ids, blocks, buf_bytes, ws_bytes, has_ids, has_weights, no_workspace):
+    """What numbers alone decide about gating + sorting, as the native launch takes it: the two argument structs without their addresses, the
+    operands; ``None`` for the calls that need memory of the library's, or that the checks have to look at."""
+    from .topk_gating_softmax import _DTYPES
+
+    handle = _lib.lib()
+    fused = bool(handle.psg_moe_softmax_sorting_fused(tokens, topk, E))
+    want = int(handle.psg_moe_sorting_workspace_bytes(tokens, topk, E))
+    if dtype_str not in _DTYPES or (not fused and not (has_ids and has_weights)) or (want and no_workspace) or B < 1 or tokens < 1 or topk < 1 or E < 1:
+        return None
+    rows, _ = sorted_sizes(tokens, topk, E, B)
+    g, s, n = _lib.MoeGatingArgs(), _lib.MoeSortArgs(), tokens * topk
+    code = _DTYPES[dtype_str][0]
+    g.tokens, g.experts, g.topk, g.dtype, g.renormalize = tokens, E, topk, code, int(bool(renormalize))
+    s.tokens, s.topk, s.experts, s.block_m, s.sorted_size = tokens, topk, E, B, ids
+    s.blocks = min(blocks, (ids + B - 1) // B)
+    s.zero_bytes, s.workspace_bytes = buf_bytes, ws_bytes
+    f, h = _lib.MoeGatingArgs, _lib.MoeSortArgs
+    i32, f32, any_, opt = _lib.TYPE_INT32, _lib.TYPE_FP32, _lib.TYPE_ANY, _lib.OPTIONAL
+    ops = [(f.gating, 0, (f32, _lib.TYPE_BF16, _lib.TYPE_FP16)[code], tokens * E * (4 if code == 0 else 2)), (f.weights, 4, f32 + opt, 4 * n),
+           (f.indices, 4, (any_ if fused else i32) + opt, 4 * n), (h.sorted_ids, 4, i32, 4 * rows, 1), (h.sorted_weights, 4, f32, 4 * max(rows, ids), 1),
+           (h.sorted_expert_ids, 4, i32, 4 * ((rows + B - 1) // B), 1), (h.num_valid_ids, 4, i32, 8, 1), (h.zero_buf, 0, any_ + opt, buf_bytes, 1),
+           (h.workspace, 0, any_ + opt, ws_bytes, 1)]
+    if not fused:
+        ops += [(h.topk_ids, 4, i32, 4 * n, 1), (h.topk_weights, 4, f32, 4 * n, 1)]
+    return (bytes(g), bytes(s)), _lib.operands(*ops), fused
+
+
 def _local_tokens(num_local_tokens, rows):
     """The reference's ``num_local_tokens`` (moe_sorting_kernel.py:2100-2104): only the first so many rows are routed; a tensor is
     read with ``.item()`` (a host synchronisation, as in the reference), an int costs nothing."""
@@ -123,6 +153,20 @@ def moe_softmax_sort_flydsl(gating_logits, sorted_ids, sorted_weights, sorted_ex
 
     if gating_logits.dim() != 2 or gating_logits.shape[1] != int(num_experts):
         raise ValueError("gating_logits must be [tokens, num_experts]")
+    if stream is not None and num_local_tokens is None and expert_mask is None and type(num_experts) is type(topk) is type(unit_size) is int:
+        buf = moe_buf if moe_buf is not None and moe_buf.numel() else None
+        ws = None if workspace is None or workspace is False else workspace
+        plan = _routing_plan(gating_logits.shape[0], num_experts, topk, unit_size, dtype_str, bool(renormalize), sorted_ids.numel(), sorted_expert_ids.numel(),
+                             0 if buf is None else buf.numel() * buf.element_size(), 0 if ws is None else ws.numel() * ws.element_size(),
+                             topk_ids is not None, topk_weights is not None, workspace is None)
+        if plan is not None:
+            routing = () if plan[2] else (topk_ids, topk_weights)
+            rc = _lib._native.launch(_lib.address("psg_moe_softmax_sorting"), plan[0], plan[1], stream, gating_logits, topk_weights, topk_ids, sorted_ids,
+                                     sorted_weights, sorted_expert_ids, num_valid_ids, buf, ws, *routing)
+            if rc != _lib._native.DECLINED:
+                if rc:
+                    raise (ValueError if rc < 0 else RuntimeError)(_lib.lib().psg_last_error().decode())
+                return sorted_ids, sorted_weights, sorted_expert_ids, num_valid_ids, moe_buf
     tokens, topk = _local_tokens(num_local_tokens, int(gating_logits.shape[0])), int(topk)
     handle = _lib.lib()
     fused = bool(handle.psg_moe_softmax_sorting_fused(tokens, topk, int(num_experts)))

@@ -16,6 +16,7 @@ reference does for the variants it does not build (host.py:142-146, :203-204).
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -55,12 +56,60 @@ def _rows(t, row_bytes):
     return t.numel() * t.element_size() // row_bytes
 
 
+@functools.lru_cache(maxsize=1024)
+def _gemm1_plan(tokens, BM, NE, H, I, BN, BK, inline_quant, interleave, a_dtype, size, blocks):
+    """Argument struct without its addresses and operands of a stage 1, as the native launch takes them; ``None`` for what the checks refuse."""
+    if BN < 1 or BK < 1 or H % BK or (2 * I) % BN or interleave or a_dtype not in _A_DTYPE or H % 256 or I % 256:
+        return None
+    if (BM not in (32, 64, 128)) if not inline_quant else (BM != 16 or a_dtype != "fp4"):
+        return None
+    args = _lib.MoeMxArgs()
+    args.tokens, args.experts, args.model_dim, args.inter_dim = tokens, NE, H, I
+    args.sorted_size, args.blocks = size, min(blocks, size // BM)
+    args.block_m, args.a_dtype, args.stage = BM, 3 if inline_quant else _A_DTYPE[a_dtype], 1
+    f, i32, any_, r32 = _lib.MoeMxArgs, _lib.TYPE_INT32, _lib.TYPE_ANY, (size + 31) // 32 * 32
+    a = [(f.a, 2, _lib.TYPE_BF16, 2 * tokens * H)] if inline_quant else [(f.a, 1, any_, tokens * (H // 2 if a_dtype == "fp4" else H)), (f.a_scale, 1, any_, r32 * (H // 32))]
+    return (bytes(args),), _lib.operands((f.w, 1, any_, NE * 2 * I * (H // 2)), (f.w_scale, 1, any_, NE * 2 * I * (H // 32)), (f.sorted_expert_ids, 4, i32, 4 * blocks),
+                                         (f.num_valid_ids, 4, i32, 4), (f.sorted_token_ids, 4, i32, 4 * size), (f.out, 1, any_, size * (I // 2)),
+                                         (f.out_scale, 1, any_, r32 * (I // 32)), *a)
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm2_plan(tokens, max_sorted, BM, NE, H, I, topk, BN, BK, epilog, out_dtype, blocks):
+    """The same of a stage 2, ``None`` twice when it needs scratch; and the library's rule for that, which the plan holds for."""
+    rule = _lib.lib().psg_moe_rows_workspace_bytes
+    if BN < 1 or BK < 1 or I % BK or H % BN or H % 256 or I % 256 or epilog not in _G2_EPILOGS or BM not in (16, 32, 64, 128) or out_dtype not in (torch.bfloat16, torch.float16):
+        return None, None, rule
+    code, atomic = 0 if out_dtype == torch.bfloat16 else 1, epilog == "atomic"
+    if atomic and topk and rule(tokens, topk, max_sorted, H, code, 1):
+        return None, None, rule
+    args = _lib.MoeMxArgs()
+    args.tokens, args.experts, args.model_dim, args.inter_dim = tokens, NE, H, I
+    args.sorted_size, args.blocks, args.block_m = max_sorted, min(blocks, max_sorted // BM), BM
+    args.out_dtype, args.stage, args.atomic = code, 2, int(atomic)
+    f, i32, any_ = _lib.MoeMxArgs, _lib.TYPE_INT32, _lib.TYPE_ANY
+    return (bytes(args),), _lib.operands((f.a, 1, any_, max_sorted * (I // 2)), (f.a_scale, 1, any_, (max_sorted + 31) // 32 * 32 * (I // 32)),
+                                         (f.w, 1, any_, NE * H * (I // 2)), (f.w_scale, 1, any_, NE * H * (I // 32)), (f.sorted_expert_ids, 4, i32, 4 * blocks),
+                                         (f.num_valid_ids, 4, i32, 4), (f.sorted_token_ids, 4, i32, 4 * max_sorted), (f.sorted_weights, 4, _lib.TYPE_FP32, 4 * max_sorted),
+                                         (f.out, 2, (_lib.TYPE_BF16, _lib.TYPE_FP16)[code], 2 * (tokens if atomic else max_sorted) * H)), rule
+
+
 def flydsl_mxfp4_gemm1(*, a_quant, a_scale_sorted_shuffled, w1_u8, w1_scale_u8, sorted_expert_ids, cumsum_tensor, m_indices,
                        inter_sorted_quant, inter_sorted_shuffled_scale, hidden_states=None, n_tokens, BM, use_nt=False,
                        inline_quant=False, NE, D_HIDDEN, D_INTER, topk, BN=256, BK=256, interleave=False, xcd_swizzle=0,
                        a_dtype="fp4", stream=None):
     """Stage 1.  ``m_indices`` holds the token of every sorted row (entries >= ``n_tokens`` are padding; the packed
     ``(slot << 24) | token`` ids of the sorter are accepted as they are).  Returns the two output tensors."""
+    if stream is not None and type(n_tokens) is type(BM) is type(NE) is type(D_HIDDEN) is type(D_INTER) is type(BN) is type(BK) is int:
+        plan = _gemm1_plan(n_tokens, BM, NE, D_HIDDEN, D_INTER, BN, BK, bool(inline_quant), bool(interleave), a_dtype, m_indices.numel(), sorted_expert_ids.numel())
+        if plan is not None:
+            a = (hidden_states,) if inline_quant else (a_quant, a_scale_sorted_shuffled)
+            rc = _lib._native.launch(_lib.address("psg_moe_mx_gemm"), plan[0], plan[1], stream, w1_u8, w1_scale_u8, sorted_expert_ids, cumsum_tensor,
+                                     m_indices, inter_sorted_quant, inter_sorted_shuffled_scale, *a)
+            if rc != _lib._native.DECLINED:
+                if rc:
+                    _lib.check(rc, "psg_moe_mx_gemm (stage 1)")
+                return inter_sorted_quant, inter_sorted_shuffled_scale
     if D_HIDDEN % BK != 0:
         raise NotImplementedError(f"mxfp_moe gemm1 requires D_HIDDEN (K) % {BK} == 0, got H={D_HIDDEN}")
     if (2 * D_INTER) % BN != 0:
@@ -122,6 +171,18 @@ def flydsl_mxfp4_gemm2(*, inter_sorted_quant, inter_sorted_shuffled_scale, w2_u8
                        D_INTER, topk, flat_out_scale=None, D_INTER_REAL=None, BN=256, BK=256, xcd_swizzle=0, stream=None):
     """Stage 2.  ``flat_out`` is ``[M_logical, D_HIDDEN]`` (atomic; zeroed by the caller) or ``[max_sorted, D_HIDDEN]``
     (nonatomic), bf16 or fp16.  Returns ``flat_out``."""
+    if stream is not None and D_INTER_REAL is None and type(M_logical) is type(max_sorted) is type(BM) is type(NE) is type(D_HIDDEN) is type(D_INTER) is type(topk) is type(BN) is type(BK) is int:
+        numbers = (M_logical, max_sorted, BM, NE, D_HIDDEN, D_INTER, topk, BN, BK, epilog, flat_out.dtype, sorted_expert_ids.numel())
+        plan = _gemm2_plan(*numbers)
+        if plan[2] is not _lib.lib().psg_moe_rows_workspace_bytes:
+            plan = _gemm2_plan.__wrapped__(*numbers)
+        if plan[0] is not None:
+            rc = _lib._native.launch(_lib.address("psg_moe_mx_gemm"), plan[0], plan[1], stream, inter_sorted_quant, inter_sorted_shuffled_scale, w2_u8, w2_scale_u8,
+                                     sorted_expert_ids, cumsum_tensor, sorted_token_ids, sorted_weights, flat_out)
+            if rc != _lib._native.DECLINED:
+                if rc:
+                    _lib.check(rc, "psg_moe_mx_gemm (stage 2)")
+                return flat_out
     if D_INTER % BK != 0:
         raise NotImplementedError(f"mxfp_moe gemm2 contraction D_INTER (inter_dim) must be a multiple of {BK}, got D_INTER={D_INTER}")
     if D_HIDDEN % BN != 0:
@@ -183,6 +244,12 @@ def moe_mxfp4_sort(blockscale_e8m0, sorted_ids, num_valid_ids, token_num, block_
     given, which keeps the call allocation-free).  Rows of padding ids and rows past ``num_valid_ids[0]`` are zero."""
     if block_size % 32:
         raise AssertionError(f"block_size={block_size} must be a multiple of 32")
+    if out is not None and stream is not None:
+        rc = _lib._native.moe_scale_sort(_lib.address("psg_moe_mx_scale_sort"), blockscale_e8m0, sorted_ids, num_valid_ids, out, token_num, stream)
+        if rc != _lib._native.DECLINED:
+            if rc:
+                _lib.check(rc, "psg_moe_mx_scale_sort")
+            return out
     _need(blockscale_e8m0, "blockscale_e8m0", itemsize=1)
     _need(sorted_ids, "sorted_ids", dtype=torch.int32)
     _need(num_valid_ids, "num_valid_ids", dtype=torch.int32)

@@ -10,6 +10,7 @@ import torch
 from . import _lib
 from .quant import fp4x2, fp8_e8m0
 
+_OUT_CODE = {torch.int8: 0, torch.float8_e4m3fn: 1}
 _X_DTYPE = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
 
 
@@ -32,6 +33,13 @@ def pertoken_quant(x: torch.Tensor, quant_dtype=torch.int8, stream=None, out=Non
     """Per-row symmetric quantisation on the device.  Returns ``(y [M,K] quant_dtype, scale [M,1] fp32)``.
     ``out=(y, scale)`` reuses caller-owned outputs (1-byte ``[M,K]`` and fp32 ``[M]`` / ``[M,1]``): no allocation, so the
     call can be recorded into a HIP graph."""
+    if out is not None and stream is not None and quant_dtype in _OUT_CODE:
+        y, scale = out
+        rc = _lib._native.quant_pertoken(_lib.address("psg_quant_pertoken"), x, y, scale, _OUT_CODE[quant_dtype], stream)
+        if rc != _lib._native.DECLINED:
+            if rc:
+                _lib.check(rc, "psg_quant_pertoken")
+            return y if y.dtype == quant_dtype else y.view(quant_dtype), scale if scale.dim() == 2 and scale.shape[1] == 1 else scale.view(-1, 1)
     code = _x_code(x)
     if quant_dtype == torch.int8:
         out_code = 0
@@ -59,6 +67,13 @@ def per_1x32_f4_quant(x: torch.Tensor, shuffle: bool = True, stream=None, out=No
     ``ceil(M/32)*32`` rows x ``K/32``: in the GEMM's shuffled layout when ``shuffle`` (default), row-major otherwise.
     Finite inputs only: a NaN / Inf in a block does not give the reference's 0xFF scale byte (the block maximum drops
     NaN)."""
+    if out is not None and stream is not None:
+        packed, scales = out
+        rc = _lib._native.quant_mxfp4(_lib.address("psg_quant_mxfp4"), x, packed, scales, 1 if shuffle else 0, stream)
+        if rc != _lib._native.DECLINED:
+            if rc:
+                _lib.check(rc, "psg_quant_mxfp4")
+            return packed if packed.dtype == fp4x2 else packed.view(fp4x2), scales if scales.dtype == fp8_e8m0 else scales.view(fp8_e8m0)
     code = _x_code(x)
     m, k = x.shape
     r = (m + 31) // 32 * 32
