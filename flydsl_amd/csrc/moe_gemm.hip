@@ -57,9 +57,10 @@ __device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g));
 // of 16 or 32 rows: an expert with 17 to 32 routed rows would otherwise stream its weights once per block).  Blocks pair up
 // from the start of each run of equal expert ids: the workgroup of the second block of a pair ends at once, and the
 // first one treats the second half of its tile as padding when the run ends there.
+// DEEP: operands three steps ahead (the rule and its figures: takes_deep).
 // ROWS = MoeRowsParams: the down stage by rows, whose first `rows.wgs` rows of the grid make the lists of the tokens' rows.  A build of
 // its own: the decode layers, which add directly, lost 0.4 to 0.8 us of 55 to 140 to the longer arguments and the branch.
-template <int KIND, int MR, int NR, int STAGE, int CO, class... ROWS>
+template <int KIND, int MR, int NR, int STAGE, int CO, bool DEEP, class... ROWS>
 __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     using acc_t = typename MoeAcc<KIND>::type;
     constexpr int BM = 16 * MR, TN = 64 * NR;
@@ -126,24 +127,26 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
 
     uint32_t a_voff[A_LOADS];
     int a_ldsoff[A_LOADS];
-    v4i areg[A_LOADS];
-    auto load_a = [&](int kt) {
+    constexpr int NAS = DEEP ? 4 : 1;  // register sets of the A tile on its way to LDS
+    v4i areg[NAS][A_LOADS];
+    auto load_a = [&](int kt, int set) {
 #pragma unroll
         for (int j = 0; j < A_LOADS; j++) {
             const bool ok = kt < KT;
-            areg[j] = buf_load16(ra, ok ? a_voff[j] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 128u : 0u);
+            areg[set][j] = buf_load16(ra, ok ? a_voff[j] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 128u : 0u);
         }
     };
-    auto store_a = [&](int stage) {
+    auto store_a = [&](int stage, int set) {
 #pragma unroll
         for (int j = 0; j < A_LOADS; j++)
-            if (a_ldsoff[j] >= 0) *reinterpret_cast<v4i*>(&lds[stage][a_ldsoff[j]]) = areg[j];
+            if (a_ldsoff[j] >= 0) *reinterpret_cast<v4i*>(&lds[stage][a_ldsoff[j]]) = areg[set][j];
     };
     using wreg_t = typename std::conditional<W4, v2i, v4i>::type;  // a lane's piece of a W fragment as it is loaded
+    // DEEP: A and W are both asked for three steps ahead, in rings of four register sets (loads return in order, so A has to be as far ahead as W).
     // W register sets: the fragments of step kt live in set kt % NWS and are requested WPF steps ahead.  Stage-1 tiles of up
     // to 32 rows (decode) are bound by the bytes of W a workgroup keeps in flight (64 tokens x top-8 on 32 experts: 86 -> 80 us
     // with three steps ahead); stage 2 (34 -> 36 us) and packed int4 weights (36 -> 38) are not and stay one step ahead
-    constexpr int WPF = (MR <= 2 && STAGE == 1 && !W4) ? 3 : 1;
+    constexpr int WPF = DEEP || (MR <= 2 && STAGE == 1 && !W4) ? 3 : 1;
     constexpr int NWS = WPF + 1;
     wreg_t blo[NWS][NSET][NR], bhi[NWS][NSET][NR];
     auto load_b = [&](int kt, int set) {
@@ -183,7 +186,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     auto step = [&](int kt, auto SP, auto WP) __attribute__((always_inline)) {
         constexpr int S = decltype(SP)::value;    // LDS stage of this step's A tile
         constexpr int WS = decltype(WP)::value;   // register set of this step's W fragments
-        load_a(kt + 1);
+        load_a(kt + (DEEP ? 3 : 1), DEEP ? (WS + 3) % NAS : 0);
         load_b(kt + WPF, (WS + WPF) % NWS);
         // packed int4: this step's fragments unpacked once, in front of the row blocks that share them
         v4i ulo[W4 ? NSET : 1][W4 ? NR : 1], uhi[W4 ? NSET : 1][W4 ? NR : 1];
@@ -219,7 +222,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
                 });
             });
         });
-        store_a(S ^ 1);
+        store_a(S ^ 1, DEEP ? (WS + 1) % NAS : 0);
         __syncthreads();
     };
 
@@ -254,12 +257,16 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
         a_voff[j] = xr >= 0 ? (uint32_t)xr * (uint32_t)K + (uint32_t)kc * 16u : 0xFFFFFFF0u;
         a_ldsoff[j] = row < BM ? moe_lds_off(row, kc) : -1;
     }
-    load_a(0);
-    store_a(0);
+    static_for<DEEP ? 3 : 1>([&](auto I) { load_a(decltype(I)::value, decltype(I)::value); });
+    store_a(0, 0);
     __syncthreads();
     // unrolled over lcm(2 LDS stages, NWS register sets) steps so that both indices are compile-time
     constexpr int UN = NWS % 2 == 0 ? NWS : 2 * NWS;
-    for (int kt0 = 0; kt0 < KT; kt0 += UN) {
+    int kt0 = 0;
+    if constexpr (DEEP)  // whole rounds without a condition: the compiler's count of the loads on their way is then exact
+        for (; kt0 + UN <= KT; kt0 += UN)
+            static_for<UN>([&](auto I) { step(kt0 + decltype(I)::value, std::integral_constant<int, decltype(I)::value & 1>{}, std::integral_constant<int, decltype(I)::value % NWS>{}); });
+    for (; kt0 < KT; kt0 += UN) {
         static_for<UN>([&](auto I) {
             constexpr int i = decltype(I)::value;
             if (kt0 + i < KT) step(kt0 + i, std::integral_constant<int, i & 1>{}, std::integral_constant<int, i % NWS>{});
@@ -333,6 +340,23 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     });
 }
 
+// Whether a stage on 64- or 128-row tiles takes the build that asks for its operands three steps ahead.  With few workgroups on a CU nothing else
+// covers a load: up to two of them per CU that build is the faster one in either stage.  With more of them stage 2 is better off with the
+// registers of more workgroups (683 to 1,891 workgroups), stage 1 only where the rows are short.  Workgroups on average over routings.  Measured,
+// us one step ahead / three: stage 1, 1086 tokens x top-4 on 17 experts, 4096 x 256 (170 workgroups of 128 rows) fp8 41.4 / 26.8, int4 47.6 / 29.6; 813 x
+// top-4 on 32, 4096 x 512 (331) 49.8 / 34.3; 600 x top-1 on 8, 3072 x 768, 64 rows (160) 23.9 / 17.6; 1024 x top-8, 4096 x 1536 (1,920) fp8 170 / 156, int8
+// 190 / 164, int4 161 / 143; 400 x top-6, 4096 x 1536, 64 rows (1,284) 96.7 / 93.1; but 1052 x top-8, 1536 x 1024 (1,180) fp8 43.3 / 45.2, 1726 x top-2,
+// 2816 x 512, 64 rows (688) 39.3 / 40.9.  Stage 2: 339 x top-4 on 16, 1024 x 2048 (234) 19.9 / 15.7; 200 x top-2 on 8, 4096 x 2048 (328) 26.8 / 20.9; but
+// 1086 x top-4, 4096 x 256 (1,358) 24.0 / 29.6.
+template <int KIND, int STAGE>
+bool takes_deep(const MoeParams& p, int block_m, int blocks, int nx) {
+    const long pairs = (long)p.tokens * p.topk, likely = pairs / block_m + p.experts / 2;
+    const long wgs = (likely < blocks ? likely : blocks) * nx;
+    if (wgs <= 2L * psg_cu_count()) return true;
+    if (STAGE == 2) return false;
+    return p.K >= 4096 || (block_m == 128 && (p.K >= 2048 || KIND == KIND_INT8W4));
+}
+
 template <int KIND, int STAGE, int NR>
 hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int blocks, bool pair, hipStream_t stream) {
     const unsigned nx = (unsigned)((p.n_out + 64 * NR - 1) / (64 * NR));
@@ -348,19 +372,27 @@ hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int bl
             if (e != hipSuccess) return e;
         }
     }
+    const bool deep = takes_deep<KIND, STAGE>(p, block_m, blocks, (int)nx);
     const dim3 grid(nx, blocks + rows.wgs, 1);
 #define PSG_MOE(MR_, CO_)                                                                                \
     {                                                                                                    \
-        if constexpr (STAGE == 2)                                                                        \
+        constexpr bool kHas = MR_ >= 4 && !(STAGE == 1 && NR == 2);  /* the tiles with a deep build */   \
+        constexpr bool kOnly = MR_ == 4 && CO_ == 2;                 /* ... and with no other */         \
+        if constexpr (STAGE == 2) {                                                                      \
             if (lists) {                                                                                 \
-                hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
+                if (kHas && deep) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kHas, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
+                else hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, false, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
                 return hipGetLastError();                                                                \
             }                                                                                            \
-        hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_>), grid, dim3(256), 0, stream, p);     \
+        }                                                                                                \
+        if (kHas && (deep || kOnly)) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kHas>), grid, dim3(256), 0, stream, p); \
+        else hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kHas && kOnly>), grid, dim3(256), 0, stream, p); \
         return hipGetLastError();                                                                        \
     }
-    if (pair && block_m == 16) PSG_MOE(2, 2)
-    if (pair && block_m == 32) PSG_MOE(4, 2)
+    if constexpr (STAGE == 1) {
+        if (pair && block_m == 16) PSG_MOE(2, 2)
+        if (pair && block_m == 32) PSG_MOE(4, 2)
+    }
     if (block_m == 16) PSG_MOE(1, 1)
     if (block_m == 32) PSG_MOE(2, 1)
     if (block_m == 64) PSG_MOE(4, 1)

@@ -1,0 +1,56 @@
+"""The builds of the MoE stages that ask for their operands one and three steps ahead, on both sides of the rule that chooses them and on every remainder of
+the K steps by the four register sets.  Whole numbers as operands and powers of two as scales: the sums are exact, stage 2 is one rounding of them."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(64, 130, 2, 4, 64), (128, 300, 3, 4, 192), (128, 290, 1, 2, 128), (64, 700, 2, 4, 4096), (128, 900, 2, 4, 4160), (32, 130, 2, 4, 192)]
+
+
+@pytest.mark.parametrize("kind", ["fp8", "int8", "int4"])
+@pytest.mark.parametrize("block,tokens,topk,experts,n_out,steps", [s + (k,) for s in SHAPES for k in (1, 2, 3, 4, 5, 6, 7, 8, 11) if s[4] < 4000 or k <= 4])
+@pytest.mark.parametrize("stage", [1, 2])
+def test_depths(stage, block, tokens, topk, experts, n_out, kind, steps):
+    from flydsl_amd import layout
+    from flydsl_amd.kernels.moe.moe_gemm_2stage import compile_moe_gemm1, compile_moe_gemm2
+    from flydsl_amd.kernels.moe.moe_sorting import moe_sorting
+
+    K = 128 * steps
+    if stage == 1 and steps % 2:
+        K *= 2  # the builder wants an even number of steps there
+    g = torch.Generator(device="cuda").manual_seed(steps + block)
+    logits = torch.randn(tokens, experts, generator=g, device="cuda")
+    wts, ids = logits.softmax(-1).topk(topk, dim=-1)
+    wts = 2.0 ** torch.randint(-2, 2, wts.shape, generator=g, device="cuda").float()
+    sid, swt, se, nv = moe_sorting(ids.int(), wts, num_experts=experts, block_size=block)
+    rows_x, rows_w = (tokens, 2 * n_out) if stage == 1 else (tokens * topk, n_out)
+    x, w = (torch.randint(-4, 5, (r, K), generator=g, device="cuda") for r in (rows_x, experts * rows_w))
+    td = torch.float8_e4m3fn if kind == "fp8" else torch.int8
+    ws = layout.shuffle_weight(w.to(td).view(torch.int8))
+    ws = layout.pack_shuffled_int8_to_int4(ws) if kind == "int4" else ws.view(td)
+    sx, sw = (2.0 ** torch.randint(-9, -5, (r,), generator=g, device="cuda").float() for r in (rows_x, experts * rows_w))
+    kw = dict(experts=experts, topk=topk, tile_m=block, tile_n=64, tile_k=128, in_dtype=kind, out_dtype="bf16")
+    if stage == 1:
+        fn = compile_moe_gemm1(model_dim=K, inter_dim=n_out, doweight_stage1=False, **kw)
+    else:
+        fn = compile_moe_gemm2(model_dim=n_out, inter_dim=K, doweight_stage2=True, accumulate=False, **kw)
+    out = torch.full((tokens * topk, n_out), -8192.0, dtype=torch.bfloat16, device="cuda")
+    fn(out, x.to(td), ws.contiguous(), sx, sw, sid, se, swt, nv, tokens, n_out, K, se.numel(), torch.cuda.current_stream())
+    xs = (x.double() * sx.double()[:, None]).view(rows_x, K)
+    wsd = (w.double() * sw.double()[:, None]).view(experts, rows_w, K)
+    want = torch.empty(tokens, topk, n_out, dtype=torch.float64, device="cuda")
+    for e in range(experts):
+        t, s = (ids == e).nonzero(as_tuple=True)
+        y = (xs[t] if stage == 1 else xs[t * topk + s]) @ wsd[e].T
+        if stage == 1:
+            gate, up = y[:, :n_out], y[:, n_out:]
+            y = gate / (1 + torch.exp(-gate)) * up
+        want[t, s] = y
+    want = want.view(tokens * topk, n_out)
+    if stage == 2:
+        assert torch.equal(out, (want * wts.view(-1, 1).double()).float().bfloat16())
+    else:
+        # half a unit in the last place of bf16, and the fp32 exponential and division
+        assert ((out.double() - want).abs() <= (2.0 ** -8 + 2.0 ** -18) * want.abs() + 1e-30).all()
