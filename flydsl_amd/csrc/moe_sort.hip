@@ -11,15 +11,18 @@
 //   2. it walks the pairs again in order and compacts those of its expert with wavefront ballots and a prefix over the
 //      wavefronts of the workgroup;
 //   3. it fills its padding rows, its block ids and its share of the unused tails.
-// Large routings (prefill) with a caller workspace: THREE launches, because E workgroups that each count all pairs
+// Large routings (prefill) with a caller workspace: TWO launches, because E workgroups that each count all pairs
 // spend their time in LDS atomics (4096 tokens x top-8 on 32 experts: 109 us in one launch).
-//   1. the pairs are cut into slices; one workgroup per slice writes the slice's histogram to the workspace;
-//   2. one workgroup turns the histograms into per-(slice, expert) offsets, the start row and local number of every
-//      expert, the total, the block ids;
-//   3. one workgroup per slice moves the slice's pairs straight to their final rows (lanes with the same expert find each
-//      other with ballots and share a running base in LDS).
+//   1. the pairs are cut into slices; one workgroup per slice writes the slice's histogram to the workspace (with the gating in front of it,
+//      the workgroup that gates a slice's tokens does that too);
+//   2. one workgroup per slice turns the histograms into the rows its pairs start at (every workgroup for itself: slices x experts numbers
+//      out of L2) and moves the pairs straight there (lanes with the same expert find each other with ballots and share a running base in
+//      LDS).  Beyond 1024 experts a launch of one workgroup in between does the first part.
+// (Gating, histograms, offsets and moving as four launches: 4096 tokens x top-8 on 32 experts 30 us, 1052 x top-8 on 16 21.)
 // Either way extra workgroups of the first launch clear the caller's accumulate buffer at full memory bandwidth.
 #include "moe_gating.h"
+
+hipError_t psg_launch_moe_gating(MoeGatingParams p, int dtype, hipStream_t stream);
 
 namespace {
 
@@ -27,8 +30,10 @@ constexpr int SORT_THREADS = 256;
 constexpr int SORT_WAVES = SORT_THREADS / 64;
 constexpr int SORT_MAX_EXPERTS = 4096;
 constexpr int SORT_ONESHOT_PAIRS = 4096;   // routings up to this many pairs always take the single launch
-constexpr int SORT_SLICE = 1024;           // pairs per slice of the three-launch path (more when there would be > 64 slices)
-constexpr int SORT_MAX_SLICES = 64;
+constexpr int SORT_SLICE = 256;            // pairs per slice of the sliced path (more when there would be too many slices)
+constexpr int SORT_MAX_SLICES = 128;       // ... of them, and as many histogram entries as a workgroup of the last launch reads (or 32 slices)
+constexpr int SORT_COUNTS = 8192;
+constexpr int SORT_MERGE_EXPERTS = 1024;   // up to here every workgroup of the last launch works out the offsets itself
 constexpr int FUSE_MAX_TOKENS = 128;       // the gating + sorting launch: every sorting workgroup repeats the gating of all tokens
 constexpr int FUSE_MAX_PAIRS = 1024;
 
@@ -155,7 +160,71 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_sort(MoeSortParams p) {
         clear_share(p, e - p.experts, (int)gridDim.x - p.experts);
         return;
     }
-    sort_one_expert(p, p.topk_ids, p.topk_weights, e);
+    // the routing into LDS first, in batches of independent loads: read where it lies, each of the three passes over it pays a memory latency for
+    // every 256 pairs (339 tokens x top-4 on 16 experts 9.2 us, now 6.7)
+    __shared__ int s_ids[SORT_ONESHOT_PAIRS];
+    __shared__ float s_w[SORT_ONESHOT_PAIRS];
+    const int P = p.tokens * p.topk;
+    if (P > SORT_ONESHOT_PAIRS) {  // (a large routing without a workspace)
+        sort_one_expert(p, p.topk_ids, p.topk_weights, e);
+        return;
+    }
+    constexpr int B = 4;
+    for (int q0 = threadIdx.x; q0 < P; q0 += B * SORT_THREADS) {
+        int id[B];
+        float w[B];
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const int q = q0 + j * SORT_THREADS;
+            id[j] = p.topk_ids[q < P ? q : 0];
+            w[j] = p.topk_weights[q < P ? q : 0];
+        }
+#pragma unroll
+        for (int j = 0; j < B; j++) {
+            const int q = q0 + j * SORT_THREADS;
+            if (q < P) {
+                s_ids[q] = id[j];
+                s_w[q] = w[j];
+            }
+        }
+    }
+    __syncthreads();
+    sort_one_expert(p, s_ids, s_w, e);
+}
+
+// Gating of the tokens [first, last) by the whole workgroup: id(pair, expert) and weight(pair, w) for every routed pair; `store`: the routing goes to
+// g.indices / g.weights / g.tei too, where those are given
+template <typename T, int VPT, class I, class W>
+__device__ __forceinline__ void gate_tokens(const MoeGatingParams& g, int first, int last, I&& id, W&& weight, bool store) {
+    const int L = g.lanes, sh = __builtin_ctz(L), tpb = SORT_THREADS >> sh;
+    const int gl = threadIdx.x & (L - 1);
+    for (int t0 = first; t0 < last; t0 += tpb) {
+        const int t = t0 + (int)(threadIdx.x >> sh);
+        const bool live = t < last;
+        const T* row = static_cast<const T*>(g.gating) + (size_t)(live ? t : 0) * g.experts;
+        float keep[GATE_KEEP];
+        const float f = gate_row<T, VPT>(row, g.experts, g.topk, g.renorm != 0, L, gl, g.vec != 0, keep, [&](int k, int index) {
+            if (live && gl == 0) {
+                const int q = t * g.topk + k;
+                id(q, index);
+                if (store) {
+                    if (g.indices) g.indices[q] = index;
+                    if (g.tei) g.tei[q] = k * g.tokens + t;
+                }
+            }
+        });
+        if (live) {
+#pragma unroll
+            for (int j = 0; j < GATE_KEEP; j++) {
+                const int k = (j << sh) + gl;
+                if (k < g.topk) {
+                    const int q = t * g.topk + k;
+                    weight(q, keep[j] * f);
+                    if (store && g.weights) g.weights[q] = keep[j] * f;
+                }
+            }
+        }
+    }
 }
 
 // ---- gating + sorting in one launch (decode): every sorting workgroup first computes the routing of all tokens from the
@@ -170,42 +239,16 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_gate_sort(MoeSortParams p,
         clear_share(p, e - p.experts, (int)gridDim.x - p.experts);
         return;
     }
-    const int L = g.lanes, sh = __builtin_ctz(L), tpb = SORT_THREADS >> sh;
-    const int gl = threadIdx.x & (L - 1);
-    for (int t0 = 0; t0 < p.tokens; t0 += tpb) {
-        const int t = t0 + (int)(threadIdx.x >> sh);
-        const bool live = t < p.tokens;
-        const T* row = static_cast<const T*>(g.gating) + (size_t)(live ? t : 0) * p.experts;
-        float keep[GATE_KEEP];
-        const float f = gate_row<T, VPT>(row, p.experts, p.topk, g.renorm != 0, L, gl, g.vec != 0, keep, [&](int k, int index) {
-            if (live && gl == 0) {
-                const int q = t * p.topk + k;
-                s_ids[q] = index;
-                if (e == 0) {
-                    if (g.indices) g.indices[q] = index;
-                    if (g.tei) g.tei[q] = k * p.tokens + t;
-                }
-            }
-        });
-        if (live) {
-#pragma unroll
-            for (int j = 0; j < GATE_KEEP; j++) {
-                const int k = (j << sh) + gl;
-                if (k < p.topk) {
-                    const int q = t * p.topk + k;
-                    s_w[q] = keep[j] * f;
-                    if (e == 0 && g.weights) g.weights[q] = keep[j] * f;
-                }
-            }
-        }
-    }
+    gate_tokens<T, VPT>(g, 0, p.tokens, [&](int q, int index) { s_ids[q] = index; }, [&](int q, float w) { s_w[q] = w; }, e == 0);
     __syncthreads();
     sort_one_expert(p, s_ids, s_w, e);
 }
 
-// ---- three launches.  Workspace (ints): off[(slices + 1) * experts] | start[experts] | local[experts] | total ----
+// ---- slices.  Workspace (ints): off[(slices + 1) * experts] | start[experts] | local[experts] | total; the two-launch form has the slices'
+// histograms in the first slices * experts of them and leaves the rest alone ----
 struct SortPlan {
     int slices, slice_len;
+    int waves, passes;  // with the gating in front: wavefronts per slice (1, 2, 4), passes of the workgroup over its tokens (1 unless waves is 4)
 };
 
 // launch 1: histogram of one slice -> off[g][*]; clearing workgroups behind the slices
@@ -220,15 +263,39 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_sort_count(MoeSortParams p
     for (int i = tid; i < p.experts; i += SORT_THREADS) hist[i] = 0;
     __syncthreads();
     const int lo = g * plan.slice_len, hi = lo + plan.slice_len < P ? lo + plan.slice_len : P;
-    for (int q = lo + tid; q < hi; q += SORT_THREADS) {
-        const int id = p.topk_ids[q];
-        if ((unsigned)id < (unsigned)p.experts) atomicAdd(&hist[id], 1);
+    for (int q0 = lo + tid; q0 < hi; q0 += 4 * SORT_THREADS) {
+        int id[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) id[j] = q0 + j * SORT_THREADS < hi ? p.topk_ids[q0 + j * SORT_THREADS] : -1;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if ((unsigned)id[j] < (unsigned)p.experts) atomicAdd(&hist[id[j]], 1);
     }
     __syncthreads();
     for (int i = tid; i < p.experts; i += SORT_THREADS) ws[g * p.experts + i] = hist[i];
 }
 
-// launch 2 (one workgroup): counts per slice -> running offsets per expert; start row, local number, block ids, total
+// launch 1 with the gating in front: the workgroup gates the tokens of SORT_WAVES / plan.waves slices and counts their pairs on the way
+template <typename T, int VPT>
+__global__ void __launch_bounds__(SORT_THREADS) k_moe_gate_count(MoeSortParams p, MoeGatingParams gp, SortPlan plan, int* ws) {
+    __shared__ int hist[SORT_WAVES][GATE_MAX_EXPERTS];
+    const int per = SORT_WAVES / plan.waves, wgs = (plan.slices + per - 1) / per, g = (int)blockIdx.x;
+    if (g >= wgs) {
+        clear_share(p, g - wgs, (int)gridDim.x - wgs);
+        return;
+    }
+    for (int s = 0; s < per; s++)
+        for (int i = threadIdx.x; i < p.experts; i += SORT_THREADS) hist[s][i] = 0;
+    __syncthreads();
+    const int tokens = plan.slice_len / p.topk * per, first = g * tokens, last = first + tokens < p.tokens ? first + tokens : p.tokens;
+    int* mine = hist[(threadIdx.x >> 6) / plan.waves];
+    gate_tokens<T, VPT>(gp, first, last, [&](int, int index) { if ((unsigned)index < (unsigned)p.experts) atomicAdd(&mine[index], 1); }, [](int, float) {}, true);
+    __syncthreads();
+    for (int s = 0; s < per && g * per + s < plan.slices; s++)
+        for (int i = threadIdx.x; i < p.experts; i += SORT_THREADS) ws[(g * per + s) * p.experts + i] = hist[s][i];
+}
+
+// beyond SORT_MERGE_EXPERTS, one workgroup: counts per slice -> running offsets per expert; start row, local number, block ids, total
 __global__ void __launch_bounds__(1024) k_moe_sort_plan(MoeSortParams p, SortPlan plan, int* ws) {
     __shared__ int padded[SORT_MAX_EXPERTS];
     __shared__ int on[SORT_MAX_EXPERTS];
@@ -300,28 +367,120 @@ __global__ void __launch_bounds__(1024) k_moe_sort_plan(MoeSortParams p, SortPla
     }
 }
 
-// launch 3: one workgroup per slice moves the slice's pairs straight to their final rows (work proportional to the pairs,
+// The offsets of the last launch, worked out by each of its workgroups (experts <= SORT_MERGE_EXPERTS): from the slices' histograms the pairs of every
+// expert, those in slices before `g`, and by a scan over the experts the start rows and the numbers of the enabled ones.  -> padded rows in all
+struct SortOffsets {
+    int kept[SORT_MERGE_EXPERTS], before[SORT_MERGE_EXPERTS], start[SORT_MERGE_EXPERTS], local[SORT_MERGE_EXPERTS];
+    int wave[2][SORT_WAVES];
+};
+__device__ __forceinline__ int slice_offsets(const MoeSortParams& p, const SortPlan& plan, const int* counts, int g, SortOffsets& o) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, E = p.experts, B = p.block_m;
+    for (int i = tid; i < E; i += SORT_THREADS) o.kept[i] = o.before[i] = 0;
+    int sh = 0;  // log2 of the experts side by side over the threads
+    while ((1 << sh) < E && sh < 8) sh++;
+    __syncthreads();
+    for (int e = tid & ((1 << sh) - 1); e < E; e += SORT_THREADS) {  // (more than one round beyond 256 experts)
+        const int first = tid >> sh, step = SORT_THREADS >> sh;
+        int kept = 0, before = 0;
+        for (int g0 = first; g0 < plan.slices; g0 += 16 * step) {
+            int c[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) c[j] = g0 + j * step < plan.slices ? counts[(g0 + j * step) * E + e] : 0;
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                kept += c[j];
+                before += g0 + j * step < g ? c[j] : 0;
+            }
+        }
+        if (kept) atomicAdd(&o.kept[e], kept);
+        if (before) atomicAdd(&o.before[e], before);
+    }
+    __syncthreads();
+    constexpr int IPT = SORT_MERGE_EXPERTS / SORT_THREADS;  // experts per thread of the scan, neighbours
+    int rows = 0, on = 0, r[IPT], n[IPT];
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+        const int e = tid * IPT + i;
+        r[i] = rows;
+        n[i] = on;
+        if (e < E) {
+            const bool enabled = !p.expert_mask || p.expert_mask[e] != 0;
+            if (!enabled) o.kept[e] = 0;
+            rows += (o.kept[e] + B - 1) / B * B;
+            on += enabled;
+        }
+    }
+    int rows_in = rows, on_in = on;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int a = __shfl_up(rows_in, d), b = __shfl_up(on_in, d);
+        if (lane >= d) {
+            rows_in += a;
+            on_in += b;
+        }
+    }
+    if (lane == 63) {
+        o.wave[0][wave] = rows_in;
+        o.wave[1][wave] = on_in;
+    }
+    __syncthreads();
+    int total = 0, rows0 = rows_in - rows, on0 = on_in - on;
+#pragma unroll
+    for (int w = 0; w < SORT_WAVES; w++) {
+        if (w < wave) {
+            rows0 += o.wave[0][w];
+            on0 += o.wave[1][w];
+        }
+        total += o.wave[0][w];
+    }
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+        const int e = tid * IPT + i;
+        if (e < E) {
+            o.start[e] = rows0 + r[i];
+            o.local[e] = on0 + n[i];
+        }
+    }
+    __syncthreads();
+    return total;
+}
+
+// last launch: one workgroup per slice moves the slice's pairs straight to their final rows (work proportional to the pairs,
 // whatever the expert count); one more workgroup fills the tails.  Every wavefront owns a contiguous quarter of the slice:
 //   pass 1  histogram of the quarter in a row of LDS counters of its own;
-//   then    the counters become running bases: rows of the expert taken by earlier slices (launch 2) + by earlier wavefronts;
+//   then    the counters become running bases: rows of the expert taken by earlier slices + by earlier wavefronts;
 //   pass 2  64 pairs at a time, in order: the lanes with the same expert find each other with one ballot per bit of the
 //           expert id, rank themselves by lane, read the running base, and the first of them advances it.
 // Stable by construction (slices, wavefronts, chunks and lanes all in pair order) and free of global atomics.
+template <bool MERGED>
 __global__ void __launch_bounds__(SORT_THREADS) k_moe_sort_scatter(MoeSortParams p, SortPlan plan, const int* ws) {
-    __shared__ int base[SORT_WAVES][SORT_MAX_EXPERTS];
+    __shared__ int base[SORT_WAVES][MERGED ? SORT_MERGE_EXPERTS : SORT_MAX_EXPERTS];
+    __shared__ SortOffsets offsets[1];
     const int g = (int)blockIdx.x, E = p.experts, B = p.block_m;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int* off = ws;
     const int* start = ws + (plan.slices + 1) * E;
+    int total = 0;
+    if constexpr (MERGED) total = slice_offsets(p, plan, ws, g, offsets[0]);
     if (g == plan.slices) {
-        fill_tails(p, start[2 * E], 0, 1);
+        if constexpr (MERGED) {
+            for (int e = tid; e < E; e += SORT_THREADS) {
+                const int blk = offsets[0].start[e] / B, n = (offsets[0].kept[e] + B - 1) / B;
+                for (int b = 0; b < n; b++) p.sorted_expert_ids[blk + b] = offsets[0].local[e];
+            }
+            if (tid == 0) {
+                p.num_valid[0] = total;
+                p.num_valid[1] = p.tokens;
+            }
+        }
+        fill_tails(p, MERGED ? total : start[2 * E], 0, 1);
         return;
     }
-    // padding rows: one thread per expert (independent loads; an expert has fewer than block_m padding rows)
+    // padding rows: one wavefront per expert (which has fewer than block_m of them)
     const int sentinel = pack_id(p.topk, p.tokens);
-    for (int e = g * SORT_THREADS + tid; e < E; e += plan.slices * SORT_THREADS) {
-        const int kept = off[plan.slices * E + e], padded = (kept + B - 1) / B * B, st = start[e];
-        for (int i = kept; i < padded; i++) {
+    for (int e = g * SORT_WAVES + wave; e < E; e += plan.slices * SORT_WAVES) {
+        const int kept = MERGED ? offsets[0].kept[e] : off[plan.slices * E + e], padded = (kept + B - 1) / B * B, st = MERGED ? offsets[0].start[e] : start[e];
+        for (int i = kept + lane; i < padded; i += 64) {
             p.sorted_ids[st + i] = sentinel;
             p.sorted_weights[st + i] = 0.f;
         }
@@ -346,7 +505,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_sort_scatter(MoeSortParams
     }
     __syncthreads();
     for (int e = tid; e < E; e += SORT_THREADS) {
-        int run = start[e] + off[g * E + e];
+        int run = MERGED ? offsets[0].start[e] + offsets[0].before[e] : start[e] + off[g * E + e];
 #pragma unroll
         for (int w = 0; w < SORT_WAVES; w++) {
             const int c = base[w][e];
@@ -397,10 +556,11 @@ int clear_wgs(const MoeSortParams& p) {
     return (int)(want < 1 ? 1 : (want > 1024 ? 1024 : want));
 }
 
-SortPlan make_plan(int64_t pairs) {
-    SortPlan plan;
-    int64_t slices = (pairs + SORT_SLICE - 1) / SORT_SLICE;
-    if (slices > SORT_MAX_SLICES) slices = SORT_MAX_SLICES;
+SortPlan make_plan(int64_t pairs, int experts) {
+    SortPlan plan{};
+    int64_t slices = (pairs + SORT_SLICE - 1) / SORT_SLICE, most = SORT_COUNTS / experts;
+    most = most < 32 ? 32 : most > SORT_MAX_SLICES ? SORT_MAX_SLICES : most;
+    if (slices > most) slices = most;
     plan.slices = (int)slices;
     plan.slice_len = (int)(((pairs + slices - 1) / slices + 63) / 64 * 64);
     return plan;
@@ -452,10 +612,10 @@ hipError_t psg_launch_moe_gate_sort(const MoeSortParams& p, MoeGatingParams g, i
     return hipErrorInvalidValue;
 }
 
-// bytes of workspace the three-launch path wants for this routing (0: the single launch is used anyway)
+// bytes of workspace the sliced path wants for this routing (0: the single launch is used anyway)
 uint64_t psg_moe_sort_workspace(int64_t pairs, int experts) {
     if (pairs <= SORT_ONESHOT_PAIRS) return 0;
-    const SortPlan plan = make_plan(pairs);
+    const SortPlan plan = make_plan(pairs, experts);
     return ((uint64_t)(plan.slices + 1) * experts + 2ull * experts + 4) * sizeof(int);
 }
 
@@ -467,10 +627,64 @@ hipError_t psg_launch_moe_sort(const MoeSortParams& p, void* workspace, uint64_t
         hipLaunchKernelGGL(k_moe_sort, dim3(p.experts + zwgs), dim3(SORT_THREADS), 0, stream, p);
         return hipGetLastError();
     }
-    const SortPlan plan = make_plan(pairs);
+    const SortPlan plan = make_plan(pairs, p.experts);
     int* ws = static_cast<int*>(workspace);
     hipLaunchKernelGGL(k_moe_sort_count, dim3(plan.slices + zwgs), dim3(SORT_THREADS), 0, stream, p, plan, ws);
+    if (p.experts <= SORT_MERGE_EXPERTS) {
+        hipLaunchKernelGGL(k_moe_sort_scatter<true>, dim3(plan.slices + 1), dim3(SORT_THREADS), 0, stream, p, plan, (const int*)ws);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_moe_sort_plan, dim3(1), dim3(1024), 0, stream, p, plan, ws);
-    hipLaunchKernelGGL(k_moe_sort_scatter, dim3(plan.slices + 1), dim3(SORT_THREADS), 0, stream, p, plan, (const int*)ws);
+    hipLaunchKernelGGL(k_moe_sort_scatter<false>, dim3(plan.slices + 1), dim3(SORT_THREADS), 0, stream, p, plan, (const int*)ws);
+    return hipGetLastError();
+}
+
+namespace {
+template <typename T>
+void launch_gate_count_t(const MoeSortParams& p, const MoeGatingParams& g, const SortPlan& plan, int* ws, int vpt, int grid, hipStream_t stream) {
+    switch (vpt) {
+        case 1: hipLaunchKernelGGL((k_moe_gate_count<T, 1>), dim3(grid), dim3(SORT_THREADS), 0, stream, p, g, plan, ws); break;
+        case 2: hipLaunchKernelGGL((k_moe_gate_count<T, 2>), dim3(grid), dim3(SORT_THREADS), 0, stream, p, g, plan, ws); break;
+        case 4: hipLaunchKernelGGL((k_moe_gate_count<T, 4>), dim3(grid), dim3(SORT_THREADS), 0, stream, p, g, plan, ws); break;
+        case 8: hipLaunchKernelGGL((k_moe_gate_count<T, 8>), dim3(grid), dim3(SORT_THREADS), 0, stream, p, g, plan, ws); break;
+        default: hipLaunchKernelGGL((k_moe_gate_count<T, 16>), dim3(grid), dim3(SORT_THREADS), 0, stream, p, g, plan, ws); break;
+    }
+}
+}  // namespace
+
+// Gating and sorting of a routing beyond psg_moe_gate_sort_fuses: with the sliced path's workspace as two launches, the gating in the first;
+// else the gating as a launch in front of the sorter's.  p.topk_ids / p.topk_weights are what the gating writes.
+hipError_t psg_launch_moe_gate_then_sort(const MoeSortParams& p, MoeGatingParams g, int dtype, void* workspace, uint64_t workspace_bytes, hipStream_t stream) {
+    const int64_t pairs = (int64_t)p.tokens * p.topk;
+    const uint64_t want = psg_moe_sort_workspace(pairs, p.experts);
+    if (want == 0 || !workspace || workspace_bytes < want || p.experts > SORT_MERGE_EXPERTS) {
+        const hipError_t e = psg_launch_moe_gating(g, dtype, stream);
+        return e == hipSuccess ? psg_launch_moe_sort(p, workspace, workspace_bytes, stream) : e;
+    }
+    int vpt;
+    gate_layout(p.experts, &vpt, &g.lanes);
+    const int esz = dtype == 0 ? 4 : 2, chunk = vpt * esz, need = chunk < 16 ? chunk : 16;
+    g.vec = p.experts % vpt == 0 && reinterpret_cast<uintptr_t>(g.gating) % need == 0 && ((size_t)p.experts * esz) % need == 0;
+    // a slice = the tokens of one, two or four wavefronts, or two passes of all four: the smallest that makes no more slices than the workspace is for.
+    // (More passes would be a chain of gatings, 3 us each: the gating is then better off as a launch over all CUs.)
+    SortPlan plan{};
+    const int64_t most = make_plan(pairs, p.experts).slices, group = 64 / g.lanes;
+    plan.passes = 1;
+    for (plan.waves = 1; plan.waves < SORT_WAVES && (p.tokens + group * plan.waves - 1) / (group * plan.waves) > most;) plan.waves *= 2;
+    if ((p.tokens + group * SORT_WAVES - 1) / (group * SORT_WAVES) > most) plan.passes = 2;
+    const int64_t tokens = group * plan.waves * plan.passes, slices = (p.tokens + tokens - 1) / tokens;
+    if (slices > most) {
+        const hipError_t e = psg_launch_moe_gating(g, dtype, stream);
+        return e == hipSuccess ? psg_launch_moe_sort(p, workspace, workspace_bytes, stream) : e;
+    }
+    plan.slices = (int)slices;
+    plan.slice_len = (int)tokens * p.topk;
+    int* ws = static_cast<int*>(workspace);
+    const int grid = (plan.slices + SORT_WAVES / plan.waves - 1) / (SORT_WAVES / plan.waves) + clear_wgs(p);
+    if (dtype == 0) launch_gate_count_t<float>(p, g, plan, ws, vpt, grid, stream);
+    else if (dtype == 1) launch_gate_count_t<uint16_t>(p, g, plan, ws, vpt, grid, stream);
+    else if (dtype == 2) launch_gate_count_t<_Float16>(p, g, plan, ws, vpt, grid, stream);
+    else return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_moe_sort_scatter<true>, dim3(plan.slices + 1), dim3(SORT_THREADS), 0, stream, p, plan, (const int*)ws);
     return hipGetLastError();
 }

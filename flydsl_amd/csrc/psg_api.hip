@@ -23,6 +23,7 @@ uint64_t psg_moe_sort_workspace(int64_t pairs, int experts);
 int psg_moe_sort_max_experts();
 hipError_t psg_launch_moe_gating(MoeGatingParams p, int dtype, hipStream_t stream);
 hipError_t psg_launch_moe_gate_sort(const MoeSortParams& p, MoeGatingParams g, int dtype, hipStream_t stream);
+hipError_t psg_launch_moe_gate_then_sort(const MoeSortParams& p, MoeGatingParams g, int dtype, void* workspace, uint64_t workspace_bytes, hipStream_t stream);
 bool psg_moe_gate_sort_fuses(int tokens, int topk, int experts);
 hipError_t psg_launch_moe_reduce(const void* x, void* y, int tokens, int topk, int dim, int out_dtype, const int32_t* mask,
                                  const int32_t* ids, int experts, hipStream_t stream);
@@ -1017,8 +1018,7 @@ int psg_moe_softmax_sorting(const psg_moe_gating_args* ga, const psg_moe_sort_ar
         // two steps: the sorter reads what the gating kernel wrote
         if ((const void*)sa->topk_ids != (const void*)ga->indices || (const void*)sa->topk_weights != (const void*)ga->weights)
             return fail(PSG_E_NULL, "beyond the fused range the sorter's topk_ids / topk_weights must be the gating's indices / weights");
-        e = psg_launch_moe_gating(g, ga->dtype, static_cast<hipStream_t>(stream));
-        if (e == hipSuccess) e = psg_launch_moe_sort(p, sa->workspace, sa->workspace ? sa->workspace_bytes : 0, static_cast<hipStream_t>(stream));
+        e = psg_launch_moe_gate_then_sort(p, g, ga->dtype, sa->workspace, sa->workspace ? sa->workspace_bytes : 0, static_cast<hipStream_t>(stream));
     }
     if (e != hipSuccess) return hip_fail(e, "psg_moe_softmax_sorting launch");
     g_err[0] = 0;

@@ -121,8 +121,8 @@ def moe_sorting_flydsl(topk_ids, topk_weights, sorted_ids, sorted_weights, sorte
     """The reference's call shape (moe_sorting_kernel.py:2070-2083): every output is pre-allocated by the caller and
     ``moe_buf`` (the buffer stage 2 accumulates into; may be ``None`` here) is cleared by the same launch.  ``topk_ids``
     int32 ``[tokens, topk]``, ``topk_weights`` fp32, ``expert_mask`` int32 ``[num_experts]`` or ``None``.  ``workspace``:
-    a device tensor of ``moe_sorting_get_workspace_size(...)`` bytes lets routings of more than 4096 pairs sort in three
-    short launches; ``None`` allocates one when it is needed (pass your own under graph capture or in serving loops),
+    a device tensor of ``moe_sorting_get_workspace_size(...)`` bytes lets routings of more than 4096 pairs sort in two
+    short launches (three beyond 1024 experts); ``None`` allocates one when it is needed (pass your own under graph capture or in serving loops),
     ``False`` forces the single launch.  ``num_local_tokens`` (int, or a tensor read with ``.item()``): sort only the first so
     many tokens; the padding value and ``num_valid_ids[1]`` then carry that count."""
     if topk_ids.dim() != 2 or topk_ids.shape != topk_weights.shape:

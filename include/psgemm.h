@@ -378,8 +378,8 @@ int psg_moe_reduce_masked(const void *x, void *y, const int32_t *expert_mask, co
  *   zero_buf NULL or a 16-byte aligned buffer of zero_bytes (a multiple of 16) that is cleared in the same launch (the
  *   reference clears moe_buf, the accumulate target of stage 2, in its sorter).
  *   workspace NULL or psg_moe_sorting_workspace_bytes(tokens, topk, experts) bytes of device memory (4-byte aligned;
- *   nothing in it has to be initialised): routings of more than 4096 pairs are then sorted by three launches
- *   (histograms per slice of the pairs, offsets, scatter) instead of one; without it they still sort correctly in one
+ *   nothing in it has to be initialised): routings of more than 4096 pairs are then sorted by two launches (three beyond 1024 experts)
+ *   (histograms per slice of the pairs, then offsets and scatter) instead of one; without it they still sort correctly in one
  *   launch, several times slower.  The reference's sorter takes a workspace in the same place (moe_sorting_kernel.py:2030).
  * No atomics on global memory and a stable order: the output does not depend on timing.  experts <= 4096, topk <= experts
  * (PSG_E_SHAPE otherwise: the padded total can reach tokens*topk + experts*(block_m - 1), which the bound on sorted_size above
