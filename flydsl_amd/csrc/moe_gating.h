@@ -34,15 +34,47 @@ __device__ __forceinline__ int gate_xchg(int v) {
 template <int S>
 __device__ __forceinline__ float gate_xchg(float v) { return __builtin_bit_cast(float, gate_xchg<S>(__builtin_bit_cast(int, v))); }
 
-constexpr int GATE_KEEP = 16;  // winners a lane may have to keep: topk <= experts <= 16 * lanes
+constexpr int GATE_KEEP = 16;  // winners per lane at most: topk <= experts <= 16 * lanes
+
+// f(0), f(1), ... f(n - 1) for a uniform n <= 6: one branch out of the chain instead of one around every step
+template <int S = 0, class F>
+__device__ __forceinline__ void gate_steps(int n, F&& f) {
+    if constexpr (S < 6) {
+        if (S < n) {
+            f(std::integral_constant<int, S>{});
+            gate_steps<S + 1>(n, f);
+        }
+    }
+}
+
+// Arg-max of x[LO .. LO + N) (column c0 + i) as a tree: short dependency chains; the higher column of a pair wins only when strictly
+// greater, so the lowest column of equal values stays.  By values on purpose: with the columns in an array the compiler may turn the selects
+// into indexed reads, ten times the instructions.
+struct GateBest {
+    float v;
+    int i;
+};
+template <int LO, int N, int VPT>
+__device__ __forceinline__ GateBest gate_best(const float (&x)[VPT], int c0) {
+    if constexpr (N == 1) {
+        return {x[LO], c0 + LO};
+    } else {
+        const GateBest a = gate_best<LO, N / 2>(x, c0), b = gate_best<LO + N / 2, N / 2>(x, c0);
+        const bool hi = b.v > a.v;
+        return {hi ? b.v : a.v, hi ? b.i : a.i};
+    }
+}
 
 // Lane gl of the group owns the columns [gl * VPT, gl * VPT + VPT) of `row`; columns >= E count as -inf.  `vec`: every
 // lane's columns can be fetched as one aligned vector (E % VPT == 0, base and row pitch aligned).  All L lanes of the
-// group must call this together.  Winner k (k = 0 .. K-1, descending weight) is reported through found(k, index) on every
-// lane, and its weight stays with lane k % L in keep[k / L]; the return value is the factor to apply to the weights
-// (1 without renormalisation), the same on every lane.
+// group must call this together.  Winner k (k = 0 .. K-1, descending weight) is reported through found(k, index, weight) on every
+// lane; the return value is the factor to apply to the weights (1 without renormalisation), the same on every lane.
+// One wavefront's chain of dependent instructions bounds a round, so what counts is its length: the winners go to LDS through found() (16 registers
+// predicated by the round made 60 of a round's 300 instructions, now 130), the exchanges have no branches of their own, and the rounds are a loop
+// (unrolled eight times over they took 1.7 us each, all of it instruction fetch).  Gating and sorting of 64 tokens x top-8 on 32 experts in one
+// launch 9.35 -> 7.0 us, a round 0.6 -> 0.34.
 template <typename T, int VPT, class F>
-__device__ __forceinline__ float gate_row(const T* row, int E, int K, bool renorm, int L, int gl, bool vec, float (&keep)[GATE_KEEP], F&& found) {
+__device__ __forceinline__ float gate_row(const T* row, int E, int K, bool renorm, int L, int gl, bool vec, F&& found) {
     struct alignas(sizeof(T) * VPT) Vec {
         T v[VPT];
     };
@@ -65,60 +97,33 @@ __device__ __forceinline__ float gate_row(const T* row, int E, int K, bool renor
     float mx = -INFINITY;
 #pragma unroll
     for (int v = 0; v < VPT; v++) mx = fmaxf(mx, x[v]);
-    static_for<6>([&](auto S) {
-        if (decltype(S)::value < sh) mx = fmaxf(mx, gate_xchg<decltype(S)::value>(mx));
-    });
+    gate_steps(sh, [&](auto S) { mx = fmaxf(mx, gate_xchg<decltype(S)::value>(mx)); });
     float sum = 0.f;
 #pragma unroll
     for (int v = 0; v < VPT; v++) {
         x[v] = __builtin_amdgcn_exp2f((x[v] - mx) * 1.4426950408889634f);  // the hardware exp2 (the reference's is fast-math too); exp2(-inf) = 0
         sum += x[v];
     }
-    static_for<6>([&](auto S) {
-        if (decltype(S)::value < sh) sum += gate_xchg<decltype(S)::value>(sum);
-    });
+    gate_steps(sh, [&](auto S) { sum += gate_xchg<decltype(S)::value>(sum); });
     const float inv = __builtin_amdgcn_rcpf(sum);  // sum >= 1 (the maximum contributes exp2(0))
 #pragma unroll
     for (int v = 0; v < VPT; v++) x[v] = c0 + v < E ? x[v] * inv : -INFINITY;
     float picked = 0.f;
     for (int k = 0; k < K; k++) {
-        // arg-max of the lane's values as a tree (short dependency chains: one wavefront per SIMD has nothing else to
-        // issue); the higher column of a pair wins only when strictly greater, so the lowest column of equal values stays
-        float tv[VPT];
-        int ti[VPT];
-#pragma unroll
-        for (int v = 0; v < VPT; v++) {
-            tv[v] = x[v];
-            ti[v] = c0 + v;
-        }
-#pragma unroll
-        for (int w = 1; w < VPT; w <<= 1)
-#pragma unroll
-            for (int v = 0; v + w < VPT; v += 2 * w) {
-                const bool hi = tv[v + w] > tv[v];
-                tv[v] = hi ? tv[v + w] : tv[v];
-                ti[v] = hi ? ti[v + w] : ti[v];
-            }
-        float bv = tv[0];
-        int bi = tv[0] == -INFINITY ? -1 : ti[0];
-        static_for<6>([&](auto S) {
-            if (decltype(S)::value < sh) {
-                const float pv = gate_xchg<decltype(S)::value>(bv);
-                const int pi = gate_xchg<decltype(S)::value>(bi);
-                const bool take = pv > bv || (pv == bv && pi < bi);
-                bv = take ? pv : bv;
-                bi = take ? pi : bi;
-            }
+        const GateBest best = gate_best<0, VPT>(x, c0);
+        float bv = best.v;
+        int bi = best.v == -INFINITY ? -1 : best.i;
+        gate_steps(sh, [&](auto S) {
+            const float pv = gate_xchg<decltype(S)::value>(bv);
+            const int pi = gate_xchg<decltype(S)::value>(bi);
+            const bool take = (pv > bv) | ((pv == bv) & (pi < bi));
+            bv = take ? pv : bv;
+            bi = take ? pi : bi;
         });
-        found(k, bi);
-        const int slot = k >> sh;
-        const bool mine = gl == (k & (L - 1));
-#pragma unroll
-        for (int j = 0; j < GATE_KEEP; j++)
-            if (j == slot) keep[j] = mine ? bv : keep[j];  // (slot is uniform: one predicated move per round)
         picked += bv;
 #pragma unroll
-        for (int v = 0; v < VPT; v++) x[v] = c0 + v == bi ? -INFINITY : x[v];
+        for (int v = 0; v < VPT; v++) x[v] = c0 + v == bi ? -INFINITY : x[v];  // (against constants it becomes an indexed write, a loop over the lanes)
+        found(k, bi, bv);
     }
     return renorm ? 1.0f / fmaxf(picked, 1e-20f) : 1.0f;
 }

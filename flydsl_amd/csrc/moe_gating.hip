@@ -1,6 +1,6 @@
 // Router gating in front of the MoE expert sorter: softmax over the experts, top-k, optional renormalisation.
-// One group of L lanes per token (L * VPT >= experts, VPT <= 16 values per lane), 256 / L tokens per workgroup, no LDS:
-// every reduction is a butterfly inside the group.  The launch reads tokens * experts logits and writes 12 bytes per
+// One group of L lanes per token (L * VPT >= experts, VPT <= 16 values per lane), 256 / L tokens per workgroup: every reduction is a
+// butterfly inside the group.  The launch reads tokens * experts logits and writes 12 bytes per
 // (token, slot), so it is bound by launch latency for decode and by HBM for prefill.
 #include "moe_gating.h"
 
@@ -13,21 +13,19 @@ __global__ void __launch_bounds__(256) k_topk_gating(MoeGatingParams p) {
     const int t = (int)blockIdx.x * (256 >> sh) + (int)(threadIdx.x >> sh);
     const bool live = t < p.tokens;
     const T* row = static_cast<const T*>(p.gating) + (size_t)(live ? t : 0) * p.experts;
-    float keep[GATE_KEEP];
-    const float f = gate_row<T, VPT>(row, p.experts, p.topk, p.renorm != 0, L, gl, p.vec != 0, keep, [&](int k, int index) {
-        if (live && gl == 0) {
+    __shared__ float won[256 * GATE_KEEP];  // weights of a token's winners before the factor
+    float* mine = won + (threadIdx.x >> sh) * p.topk;
+    const float f = gate_row<T, VPT>(row, p.experts, p.topk, p.renorm != 0, L, gl, p.vec != 0, [&](int k, int index, float w) {
+        if (gl != 0) return;
+        mine[k] = w;
+        if (live) {
             p.indices[(size_t)t * p.topk + k] = index;
             if (p.tei) p.tei[(size_t)t * p.topk + k] = k * p.tokens + t;
         }
     });
-    // lane k % L holds the weight of winner k
-    if (live) {
-#pragma unroll
-        for (int j = 0; j < GATE_KEEP; j++) {
-            const int k = (j << sh) + gl;
-            if (k < p.topk) p.weights[(size_t)t * p.topk + k] = keep[j] * f;
-        }
-    }
+    // (a token's lanes are neighbours in one wavefront, whose LDS accesses stay in order)
+    if (live)
+        for (int k = gl; k < p.topk; k += L) p.weights[(size_t)t * p.topk + k] = mine[k] * f;
 }
 
 template <typename T>

@@ -192,38 +192,34 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_sort(MoeSortParams p) {
     sort_one_expert(p, s_ids, s_w, e);
 }
 
-// Gating of the tokens [first, last) by the whole workgroup: id(pair, expert) and weight(pair, w) for every routed pair; `store`: the routing goes to
-// g.indices / g.weights / g.tei too, where those are given
-template <typename T, int VPT, class I, class W>
-__device__ __forceinline__ void gate_tokens(const MoeGatingParams& g, int first, int last, I&& id, W&& weight, bool store) {
+// Gating of the tokens [first, last) by the whole workgroup: id(pair, expert) for every routed pair; the weights to `won` in LDS, all of them (held; first
+// = 0) or those of one pass over the tokens; `store`: the routing goes to g.indices / g.weights / g.tei too, where those are given
+template <typename T, int VPT, bool held, class I>
+__device__ __forceinline__ void gate_tokens(const MoeGatingParams& g, int first, int last, float* won, I&& id, bool store) {
     const int L = g.lanes, sh = __builtin_ctz(L), tpb = SORT_THREADS >> sh;
     const int gl = threadIdx.x & (L - 1);
     for (int t0 = first; t0 < last; t0 += tpb) {
         const int t = t0 + (int)(threadIdx.x >> sh);
         const bool live = t < last;
         const T* row = static_cast<const T*>(g.gating) + (size_t)(live ? t : 0) * g.experts;
-        float keep[GATE_KEEP];
-        const float f = gate_row<T, VPT>(row, g.experts, g.topk, g.renorm != 0, L, gl, g.vec != 0, keep, [&](int k, int index) {
-            if (live && gl == 0) {
-                const int q = t * g.topk + k;
-                id(q, index);
-                if (store) {
-                    if (g.indices) g.indices[q] = index;
-                    if (g.tei) g.tei[q] = k * g.tokens + t;
-                }
+        float* mine = won + (size_t)(t - (held ? 0 : t0)) * g.topk;
+        const float f = gate_row<T, VPT>(row, g.experts, g.topk, g.renorm != 0, L, gl, g.vec != 0, [&](int k, int index, float w) {
+            if (!live || gl != 0) return;
+            mine[k] = w;
+            const int q = t * g.topk + k;
+            id(q, index);
+            if (store) {
+                if (g.indices) g.indices[q] = index;
+                if (g.tei) g.tei[q] = k * g.tokens + t;
             }
         });
-        if (live) {
-#pragma unroll
-            for (int j = 0; j < GATE_KEEP; j++) {
-                const int k = (j << sh) + gl;
-                if (k < g.topk) {
-                    const int q = t * g.topk + k;
-                    weight(q, keep[j] * f);
-                    if (store && g.weights) g.weights[q] = keep[j] * f;
-                }
+        // (a token's lanes are neighbours in one wavefront, whose LDS accesses stay in order)
+        if (live && (held || store))
+            for (int k = gl; k < g.topk; k += L) {
+                const float w = mine[k] * f;
+                if (held) mine[k] = w;
+                if (store && g.weights) g.weights[(size_t)t * g.topk + k] = w;
             }
-        }
     }
 }
 
@@ -239,7 +235,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_gate_sort(MoeSortParams p,
         clear_share(p, e - p.experts, (int)gridDim.x - p.experts);
         return;
     }
-    gate_tokens<T, VPT>(g, 0, p.tokens, [&](int q, int index) { s_ids[q] = index; }, [&](int q, float w) { s_w[q] = w; }, e == 0);
+    gate_tokens<T, VPT, true>(g, 0, p.tokens, s_w, [&](int q, int index) { s_ids[q] = index; }, e == 0);
     __syncthreads();
     sort_one_expert(p, s_ids, s_w, e);
 }
@@ -279,6 +275,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_sort_count(MoeSortParams p
 template <typename T, int VPT>
 __global__ void __launch_bounds__(SORT_THREADS) k_moe_gate_count(MoeSortParams p, MoeGatingParams gp, SortPlan plan, int* ws) {
     __shared__ int hist[SORT_WAVES][GATE_MAX_EXPERTS];
+    __shared__ float won[SORT_THREADS * GATE_KEEP];
     const int per = SORT_WAVES / plan.waves, wgs = (plan.slices + per - 1) / per, g = (int)blockIdx.x;
     if (g >= wgs) {
         clear_share(p, g - wgs, (int)gridDim.x - wgs);
@@ -289,7 +286,7 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_gate_count(MoeSortParams p
     __syncthreads();
     const int tokens = plan.slice_len / p.topk * per, first = g * tokens, last = first + tokens < p.tokens ? first + tokens : p.tokens;
     int* mine = hist[(threadIdx.x >> 6) / plan.waves];
-    gate_tokens<T, VPT>(gp, first, last, [&](int, int index) { if ((unsigned)index < (unsigned)p.experts) atomicAdd(&mine[index], 1); }, [](int, float) {}, true);
+    gate_tokens<T, VPT, false>(gp, first, last, won, [&](int, int index) { if ((unsigned)index < (unsigned)p.experts) atomicAdd(&mine[index], 1); }, true);
     __syncthreads();
     for (int s = 0; s < per && g * per + s < plan.slices; s++)
         for (int i = threadIdx.x; i < p.experts; i += SORT_THREADS) ws[(g * per + s) * p.experts + i] = hist[s][i];
