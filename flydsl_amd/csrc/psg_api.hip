@@ -2,6 +2,7 @@
 // Nothing here allocates, synchronises or touches any stream but the caller's.
 #include "../../include/psgemm.h"
 
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -179,6 +180,49 @@ Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
     return t;
 }
 
+// Tile of an fp4 x fp4 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 3 % below that of the
+// score's tile.  A tile's estimate is a start, one `round` per set of tiles that the CUs hold together and, per K step of 128 bytes, what a CU takes for
+// the 1 .. per_cu tiles it works on at once, so it knows what the score doesn't: a second tile on a CU costs little while a step is bound by its
+// loads, short rows are bound by the rounds' ends, and a last round with few tiles is shorter.  The constants are a least-squares fit to 722
+// problems (65 to 8192 rows, 1024 to 16384 columns, K 1024 to 14336), every tile timed on each; the estimates are 4 to 7 % off (r.m.s.), which is
+// why the score's tile stays where they are close: without that eight of the 722 got more than 3 % slower, with it one does (282x9216x1280 9.4 us
+// against 9.9).  199 take another tile, 10 % faster on average (us score / estimate: 4887x4256x1024 31.3 / 22.7, 2127x14560x2304 63 / 56, 1285x14048x3072
+// 56 / 44, 788x5280x4608 22.0 / 20.5, 5678x3584x4608 70.6 / 60.0, 48x4096x1024 6.5 / 4.3).
+Tile pick_mxfp4_tile(int M, int N, int kbytes) {
+    struct Cost {
+        int m, n, waves, per_cu;
+        double start, round, step[5];  // us; step[r]: r tiles on a CU
+    };
+    static const Cost costs[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
+                                 {64, 256, 4, 2, 3.5, 2.8, {0, 0.58, 1.12}},      {32, 256, 4, 3, 3.6, 1.4, {0, 0.50, 0.95, 1.28}},
+                                 {64, 128, 4, 3, 3.8, 1.2, {0, 0.37, 0.67, 0.95}}, {32, 128, 4, 4, 3.0, 1.2, {0, 0.31, 0.50, 0.77, 0.90}}};
+    const double cus = psg_cu_count(), steps = (kbytes + 127) / 128;
+    const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;  // us of the memory bus; near that bound a launch takes longer than either estimate
+    const Tile scored = pick_tile(M, N, true, 0, 0);
+    double best = 0, kept = 0;
+    Tile t = scored;
+    for (const Cost& c : costs) {
+        const double tiles = (double)((M + c.m - 1) / c.m) * (double)((N + c.n - 1) / c.n), slots = cus * c.per_cu;
+        const double full = std::floor(tiles / slots), rest = (tiles - full * slots) / cus;
+        double us = full * (c.round + steps * c.step[c.per_cu]);
+        if (rest > 0) {
+            // the last round: CUs with one tile more than others finish last, but those with fewer are done sooner and leave them the bus
+            const double r = rest > 1 ? 0.25 * rest + 0.75 * std::ceil(rest) : 1;
+            const int lo = (int)r;
+            double step = c.step[lo] + (lo < c.per_cu ? (r - lo) * (c.step[lo + 1] - c.step[lo]) : 0);
+            if (full == 0 && tiles < cus) step *= std::sqrt(std::sqrt(std::sqrt(std::sqrt(tiles / cus))));  // fewer CUs at work clock higher
+            us += c.round + steps * step;
+        }
+        us = c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
+        if (c.m == scored.m && c.n == scored.n) kept = us;
+        if (best == 0 || us < best) {
+            best = us;
+            t = {c.m, c.n, c.waves};
+        }
+    }
+    return best < 0.97 * kept ? t : scored;
+}
+
 // Split-K for the regime between the streaming kernel (takes_stream) and problems with enough tiles to fill the GPU:
 // with few tiles every workgroup walks all of K behind a one-step prefetch and the launch is latency-bound.
 // Splitting K over `splits` workgroups per tile multiplies the loads in flight; the price is one fp32 slice of
@@ -281,7 +325,9 @@ Plan plan_tiled(int M, int N, int kbytes, bool mx) {
     // (fp8, weights not cache-resident: M=128, N=K=4096 14.0 us against 19.4 with 128x128 tiles and two K splits; M=256,
     // N=8192 22.0 against 23.7; M=384, N=8192, 768 tiles: 28.0 against 26.5, so the larger tile is kept there)
     if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4};
-    return {t, pick_splits(M, N, kbytes, t)};
+    const int splits = pick_splits(M, N, kbytes, t);
+    if (mx && splits == 1) t = pick_mxfp4_tile(M, N, kbytes);
+    return {t, splits};
 }
 
 uint64_t splitk_bytes(int M, int N, int splits) { return splits > 1 ? (uint64_t)splits * M * N * 4ull : 0; }
@@ -599,7 +645,8 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
                            c_bs % 16 == 0 && sa_bs % 4 == 0;
     if (fp8_tiled || per_batch) {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
-        const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : pick_tile(a->M, a->N, true, 0, 0);
+        const bool fp4 = a->a_dtype == PSG_MX_FP4;
+        const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : fp4 ? pick_mxfp4_tile(a->M, a->N, a->K / 2) : pick_tile(a->M, a->N, true, 0, 0);
         A8W8Params q{};
         q.c = out;
         q.a = static_cast<const uint8_t*>(a->a);
@@ -615,7 +662,6 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         q.splits = 1;
         q.epi = EPI_NONE;
         q.out = a->out_dtype;
-        const bool fp4 = a->a_dtype == PSG_MX_FP4;
         if (fp4) q.wave_layout = t.waves == 8 ? 8 : 1;
         for (int z = 0; z < batch; z++) {
             const hipError_t te = w4 ? psg_launch_tiled_mxw4(q, a->a_dtype == PSG_MX_FP6, static_cast<hipStream_t>(stream))
