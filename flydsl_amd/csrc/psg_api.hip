@@ -85,32 +85,43 @@ bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p
 constexpr int kSmallM = 32;      // rows the split-K path covers
 constexpr int kStreamMaxM = 64;  // rows the small-M kernels can hold (four 16-row blocks)
 
-// Which regime an fp4 x fp4 problem takes: the small-M kernel up to 32 rows; up to 64 rows while the weight is at most 40 MB
-// and K at least 2048 (measured, us small-M / tiled plan: M=33 7168x2048 4.9 / 6.5, 8192x8192 10.9 / 14.6, 1024x2048 4.3 / 5.3,
-// 4096x1024 4.8 / 4.1, 28672x4096 16.5 / 17.0; M=64 5.9 / 6.7, 13.2 / 15.8, 5.4 / 5.3, 5.8 / 4.2, 22.0 / 17.8).
-bool mx_takes_small(int M, int N, int K) {
-    if (M <= kSmallM) return true;
-    return M <= kStreamMaxM && K >= 2048 && (long)N * (K / 2) <= (40L << 20);
-}
+// Which regime an fp4 x fp4 problem takes: the small-M kernel up to 32 rows; up to 64 rows while the weight is at most 40 MB, K at least
+// 2048 and its workgroups of 32 columns come one to a CU (measured, us small-M / tiled plan: M=33 7168x2048 4.9 / 6.5, 8192x8192 10.9 / 14.6,
+// 1024x2048 4.3 / 5.3, 4096x1024 4.8 / 4.1; M=64 5.9 / 6.7, 13.2 / 15.8, 5.4 / 5.3, 5.8 / 4.2).  With more columns a few CUs work a second round
+// while the others wait, and 32x128 tiles, two or three to a CU, take over at once: M=33 8960x8704 16.7 / 13.5, 12288x4096 9.4 / 8.0,
+// 16384x2048 6.5 / 5.8, 24576x2048 8.2 / 7.8; M=64 8224x2048 7.1 / 5.2, 16384x2048 8.3 / 6.2, 20480x4096 17.2 / 10.7.  Up to 32 rows the two are
+// too close to draw a line by (32x10240x4096 8.7 / 8.0, 17x8224x4096 7.0 / 7.8, 32x16384x14336 25.8 / 33.1).
+bool mx_small_holds(int M, int N, int K) { return M > kSmallM && M <= kStreamMaxM && K >= 2048 && (long)N * (K / 2) <= (40L << 20); }
+bool mx_takes_small(int M, int N, int K) { return M <= kSmallM || (mx_small_holds(M, N, K) && N <= 32 * psg_cu_count()); }
 
 // Which regime an 8- / 16-bit problem takes when the caller does not force one.  Up to 32 rows always the streaming
 // kernel.  Above that every workgroup of the streaming kernel still reads all of A (M x K bytes through its texture
 // path), so it only wins while the weight is small enough that the split-K pair of the tiled kernel is bound by its
 // two launches and its partial sums rather than by bandwidth (measured, fp8, us streaming / tiled+split-K: M=33 1024x2048
-// 4.3 / 8.0, 6144x4096 9.2 / 14.1, 8192x8192 15.3 / 19.6, 28672x4096 31.7 / 32.3, 2048x16384 15.5 / 16.0; M=48 9.7 / 14.4,
-// 16.5 / 20.4, 33.0 / 31.3, 17.3 / 16.3; M=64 1024x2048 5.5 / 8.2, 6144x4096 11.3 / 15.0, 8192x8192 18.3 / 22.2,
-// 5120x8192 15.8 / 19.0, 28672x4096 37.5 / 32.7, 2048x16384 20.0 / 15.6).
+// 4.3 / 8.0, 6144x4096 9.2 / 14.1, 8192x8192 15.3 / 19.6, 2048x16384 15.5 / 16.0; M=48 9.7 / 14.4, 16.5 / 20.4, 17.3 / 16.3; M=64
+// 1024x2048 5.5 / 8.2, 6144x4096 11.3 / 15.0, 8192x8192 18.3 / 22.2, 5120x8192 15.8 / 19.0, 2048x16384 20.0 / 15.6), and while 32
+// columns for each CU are all there are.  With more columns the CUs go round again, and 64x64 tiles, several to a CU and without a split,
+// are better from the first column on (us streaming / 64x64 tiles: fp8 33x8208x1024 8.6 / 5.0, 33x9216x8064 23.2 / 20.5, 64x8208x4096
+// 16.0 / 11.7, 48x10240x6144 20.6 / 16.5, 33x16384x4096 17.3 / 13.7, 64x28672x2048 23.8 / 12.6, 33x65536x1024 35.6 / 13.7; fp16
+// 33x16384x2048 17.4 / 14.4, 40x12288x3328 23.4 / 18.5; just below the line 60x8192x4096 10.7 / 14).
 // Beyond 64 rows a workgroup takes 64 of them, and the kernel is the better one while 32 columns a workgroup make one round of the CUs (N
 // times the 64-row groups up to 8192) on rows of 2 to 4 KB (us streaming / tiled plan: fp8 80x1024x4096 6.6 / 9.5, 256x1024x4096 7.2 /
 // 10.1, 128x2048x2048 4.8 / 7.3, 128x4096x4096 9.9 / 11.9, 192x2048x2048 7.2 / 7.4; bf16 256x1024x1024 4.8 / 6.8, 128x2048x2048 7.4 /
-// 10.4; but fp8 128x4096x1024 6.2 / 5.5, 192x4096x4096, one and a half rounds, 19.2 / 11.9).  On rows of 4 to 8 KB it is the better one
-// in the same range of columns too (fp8 128x2048x6144 9.8 / 15.7, 128x2048x8192 11.7 / 18.8, 192x2048x8192 16.6 / 19.1, 128x4096x5120 12.1 /
-// 14.0; bf16 128x2048x4096 11.5 / 19.6): the line at 4 KB is a cautious one, which leaves those calls their split-K plan.
+// 10.4; but fp8 128x4096x1024 6.2 / 5.5, 192x4096x4096, one and a half rounds, 19.2 / 11.9).  On rows of 4 to 8 KB it is while they fill half of
+// the CUs (fp8 65x1024x4224 7.1 / 9.1, 80x2048x8128 11.4 / 13.7, 128x2048x6144 9.2 / 12.9, 256x1024x8128 12.2 / 15.7; int8 256x1024x4224 7.9 /
+// 11.0; bf16 66x2048x2112 7.0 / 9.8; fp16 128x2048x4032 11.2 / 14.1); between a half and one round it depends on the columns (256x2048x5120 11.0 /
+// 12.7, but 192x2048x4160 11.8 / 11.4, 128x4096x7168 14.2 / 13.6, 192x2720x6144 15.1 / 13.9) and the tiles stay.
+bool stream_holds(int M, int N, int kbytes) {
+    const long w = (long)N * kbytes, a = (long)M * kbytes;
+    return M > kSmallM && M <= kStreamMaxM && a <= (512L << 10) && w <= (80L << 20);
+}
 bool takes_stream(int M, int N, int kbytes) {
     if (M <= kSmallM) return true;
-    if (M > kStreamMaxM) return M <= 256 && kbytes >= 2048 && kbytes <= 4096 && (long)N * ((M + 63) / 64) <= 8192;
-    const long w = (long)N * kbytes, a = (long)M * kbytes;
-    return a <= (512L << 10) && w <= (80L << 20);
+    if (M > kStreamMaxM) {
+        const long columns = (long)N * ((M + 63) / 64);
+        return M <= 256 && (kbytes >= 2048 && kbytes <= 4096 ? columns <= 8192 : kbytes > 4096 && kbytes < 8192 && N >= 1024 && columns <= 4096);
+    }
+    return stream_holds(M, N, kbytes) && N <= 32 * psg_cu_count();
 }
 constexpr int kTargetWaves = 1536;  // wavefronts wanted in flight for the streaming path (6 per CU)
 
@@ -311,6 +322,8 @@ struct Plan {
     int splits;
 };
 Plan plan_tiled(int M, int N, int kbytes, bool mx) {
+    // more columns than the streaming kernel takes in one round: 64x64 tiles, unsplit (these problems have no workspace)
+    if (!mx && stream_holds(M, N, kbytes) && N > 32 * psg_cu_count()) return {Tile{64, 64, 4}, 1};
     Tile t = pick_tile(M, N, mx, 0, 0);
     const long tiles_big = (long)((M + 127) / 128) * (long)((N + 255) / 256);
     const int steps = (kbytes + 127) / 128;
@@ -325,7 +338,7 @@ Plan plan_tiled(int M, int N, int kbytes, bool mx) {
     // (fp8, weights not cache-resident: M=128, N=K=4096 14.0 us against 19.4 with 128x128 tiles and two K splits; M=256,
     // N=8192 22.0 against 23.7; M=384, N=8192, 768 tiles: 28.0 against 26.5, so the larger tile is kept there)
     if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4};
-    const int splits = pick_splits(M, N, kbytes, t);
+    const int splits = mx && mx_small_holds(M, N, kbytes * 2) ? 1 : pick_splits(M, N, kbytes, t);
     if (mx && splits == 1) t = pick_mxfp4_tile(M, N, kbytes);
     return {t, splits};
 }
