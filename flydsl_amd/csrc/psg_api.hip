@@ -191,28 +191,32 @@ Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
     return t;
 }
 
-// Tile of an fp4 x fp4 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 3 % below that of the
-// score's tile.  A tile's estimate is a start, one `round` per set of tiles that the CUs hold together and, per K step of 128 bytes, what a CU takes for
-// the 1 .. per_cu tiles it works on at once, so it knows what the score doesn't: a second tile on a CU costs little while a step is bound by its
-// loads, short rows are bound by the rounds' ends, and a last round with few tiles is shorter.  The constants are a least-squares fit to 722
-// problems (65 to 8192 rows, 1024 to 16384 columns, K 1024 to 14336), every tile timed on each; the estimates are 4 to 7 % off (r.m.s.), which is
-// why the score's tile stays where they are close: without that eight of the 722 got more than 3 % slower, with it one does (282x9216x1280 9.4 us
-// against 9.9).  199 take another tile, 10 % faster on average (us score / estimate: 4887x4256x1024 31.3 / 22.7, 2127x14560x2304 63 / 56, 1285x14048x3072
-// 56 / 44, 788x5280x4608 22.0 / 20.5, 5678x3584x4608 70.6 / 60.0, 48x4096x1024 6.5 / 4.3).
-Tile pick_mxfp4_tile(int M, int N, int kbytes) {
+// Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 3 % below that of
+// the score's tile.  A tile's estimate is a start, one `round` per set of tiles that the CUs hold together and, per K step of 128 bytes, what a CU
+// takes for the 1 .. per_cu tiles it works on at once, so it knows what the score doesn't: a second tile on a CU costs little while a step is bound by
+// its loads, short rows are bound by the rounds' ends, and a last round with few tiles is shorter.  The constants are a least-squares fit to 722
+// fp4 and 208 fp8 problems (65 to 8192 rows, 1024 to 16384 columns, K 1024 to 14336), every tile timed on each; the estimates are 4 to 7 % off
+// (r.m.s.; fp8 3 to 5), which is why the score's tile stays where they are close: without that eight of the 722 got more than 3 % slower, with it one
+// does (282x9216x1280 9.4 us against 9.9).  199 take another tile, 10 % faster on average (us score / estimate: 4887x4256x1024 31.3 / 22.7,
+// 2127x14560x2304 63 / 56, 1285x14048x3072 56 / 44, 788x5280x4608 22.0 / 20.5, 5678x3584x4608 70.6 / 60.0, 48x4096x1024 6.5 / 4.3).
+Tile pick_mx_tile(int M, int N, int kbytes, bool fp8) {
     struct Cost {
         int m, n, waves, per_cu;
         double start, round, step[5];  // us; step[r]: r tiles on a CU
     };
-    static const Cost costs[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
-                                 {64, 256, 4, 2, 3.5, 2.8, {0, 0.58, 1.12}},      {32, 256, 4, 3, 3.6, 1.4, {0, 0.50, 0.95, 1.28}},
-                                 {64, 128, 4, 3, 3.8, 1.2, {0, 0.37, 0.67, 0.95}}, {32, 128, 4, 4, 3.0, 1.2, {0, 0.31, 0.50, 0.77, 0.90}}};
+    static const Cost costs4[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
+                                  {64, 256, 4, 2, 3.5, 2.8, {0, 0.58, 1.12}},      {32, 256, 4, 3, 3.6, 1.4, {0, 0.50, 0.95, 1.28}},
+                                  {64, 128, 4, 3, 3.8, 1.2, {0, 0.37, 0.67, 0.95}}, {32, 128, 4, 4, 3.0, 1.2, {0, 0.31, 0.50, 0.77, 0.90}}};
+    // (the fp8 launcher runs its 256x256 tile on four wavefronts whatever `waves` says)
+    static const Cost costs8[] = {{256, 256, 8, 1, 2.3, 9.5, {0, 1.45}},           {128, 256, 4, 1, 2.3, 5.7, {0, 0.85}},
+                                  {64, 256, 4, 2, 3.9, 1.9, {0, 0.58, 1.02}},      {32, 256, 4, 3, 4.6, 0.0, {0, 0.50, 0.90, 1.21}},
+                                  {64, 128, 4, 3, 4.1, 0.5, {0, 0.37, 0.60, 0.88}}, {32, 128, 4, 4, 3.6, 0.2, {0, 0.31, 0.48, 0.73, 0.87}}};
     const double cus = psg_cu_count(), steps = (kbytes + 127) / 128;
     const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;  // us of the memory bus; near that bound a launch takes longer than either estimate
     const Tile scored = pick_tile(M, N, true, 0, 0);
     double best = 0, kept = 0;
     Tile t = scored;
-    for (const Cost& c : costs) {
+    for (const Cost& c : fp8 ? costs8 : costs4) {
         const double tiles = (double)((M + c.m - 1) / c.m) * (double)((N + c.n - 1) / c.n), slots = cus * c.per_cu;
         const double full = std::floor(tiles / slots), rest = (tiles - full * slots) / cus;
         double us = full * (c.round + steps * c.step[c.per_cu]);
@@ -315,6 +319,21 @@ int mx_general_splits(int M, int N, int K) {
     return s;
 }
 
+// Whether dense, unbatched fp8 x fp8 runs on the tiles of the dense kernels: beyond 32 rows everywhere except where the small-M kernel's
+// workgroups make one round of the CUs (N / 32 times the 64-row groups), and where the general kernel splits K (`room`: the caller brought the
+// workspace) and the splits make one round.  Over 208 problems of 65 to 8192 rows the tiles were 16 % faster on average than
+// what ran there (us tiles / small-M or general kernel: 383x12384x6912 49.8 / 90.5, 365x10336x2304 15.9 / 27.0, 1164x2880x4096 23.2 / 37.1, 524x9440x5376
+// 42.4 / 69.8, 128x512x4096 12.6 / 17.7, 4096x1024x512 8.1 / 10.1; small-M, two rounds, 389x1984x4352 14.5 / 21.0, 186x5184x2048 8.8 / 12.3, 64x8224x2048
+// 8.9 / 9.7, 33x16384x4096 15.0 / 18.7; one round 228x1056x9216 25.7 / 18.6, 64x8192x4096 13.8 / 10.5; splits 33x992x14336 37.0 / 19.3, 87x8160x12032
+// 33.4 / 29.6, more than one round of them 67x9568x8960 26.3 / 36.7).  Up to 32 rows the small-M kernel is the better one (32x12288x4096 14.2 / 13.6).
+bool mxfp8_takes_tiles(int M, int N, int K, bool room) {
+    if (M <= kSmallM) return false;
+    const long cus = psg_cu_count(), groups = (M + 63) / 64;
+    if ((long)(N / 32) * groups <= cus && mx_general_small(M, N, K, false, true, 1)) return false;
+    const int splits = mx_general_splits(M, N, K);
+    return !(room && splits > 1 && groups * ((N + 127) / 128) * splits <= cus);
+}
+
 // Tile + split plan of the tiled path.  With few tiles and a long K (the regime between the streaming kernel and
 // GPU-filling problems) small square-ish tiles with split-K measured best: 64x64 up to M=64, 128x128 above.
 struct Plan {
@@ -339,7 +358,7 @@ Plan plan_tiled(int M, int N, int kbytes, bool mx) {
     // N=8192 22.0 against 23.7; M=384, N=8192, 768 tiles: 28.0 against 26.5, so the larger tile is kept there)
     if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4};
     const int splits = mx && mx_small_holds(M, N, kbytes * 2) ? 1 : pick_splits(M, N, kbytes, t);
-    if (mx && splits == 1) t = pick_mxfp4_tile(M, N, kbytes);
+    if (mx && splits == 1) t = pick_mx_tile(M, N, kbytes, false);
     return {t, splits};
 }
 
@@ -639,11 +658,10 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
     if (a->force_path < 0 || a->force_path > 3) return fail(PSG_E_SHAPE, "force_path=%d unknown", a->force_path);
     const bool dense = a_rs == a_row && c_rs == (uint64_t)a->N && sa_cs == chunk;
     const bool fp4_fast = a->a_dtype == PSG_MX_FP4 && a->b_dtype == PSG_MX_FP4 && batch == 1 && dense;
-    // fp8 x fp8 (MXFP8) also runs on the tiled mainloop when the problem has enough 128x256 tiles to fill the GPU (that
-    // kernel has no split-K for this format; decode-like shapes go to the general kernel and its split-K plan)
     const bool fp8_pair = a->a_dtype == PSG_MX_FP8 && a->b_dtype == PSG_MX_FP8 && batch == 1 && dense;
-    const bool fp8_tiled = fp8_pair && a->force_path != 3 &&
-                           (a->force_path == 1 || (a->M > kSmallM && (long)((a->M + 127) / 128) * (long)((a->N + 255) / 256) >= 192));
+    // what the general kernel's split-K plan needs is there
+    const bool room = store == STORE_C && a->workspace && aligned(a->workspace, 16) && a->workspace_bytes >= splitk_bytes(a->M, a->N, mx_general_splits(a->M, a->N, a->K));
+    const bool fp8_tiled = fp8_pair && (a->force_path == 1 || (a->force_path == 0 && mxfp8_takes_tiles(a->M, a->N, a->K, room)));
     if (a->force_path == 2 && !fp4_fast) return fail(PSG_E_SHAPE, "force_path=2 is for dense, unbatched fp4 x fp4 only");
     if (a->force_path == 1 && !fp4_fast && !fp8_pair)
         return fail(PSG_E_SHAPE, "force_path=1 is for dense, unbatched fp4 x fp4 or fp8 x fp8 only");
@@ -659,7 +677,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
     if (fp8_tiled || per_batch) {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
         const bool fp4 = a->a_dtype == PSG_MX_FP4;
-        const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : fp4 ? pick_mxfp4_tile(a->M, a->N, a->K / 2) : pick_tile(a->M, a->N, true, 0, 0);
+        const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : w4 ? Tile{256, 256, 8} : pick_mx_tile(a->M, a->N, fp4 ? a->K / 2 : a->K, !fp4);
         A8W8Params q{};
         q.c = out;
         q.a = static_cast<const uint8_t*>(a->a);
