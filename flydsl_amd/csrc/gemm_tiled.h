@@ -116,8 +116,9 @@ __device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, in
 // (the MFMAs of a step hide one memory latency).  3 for the few-tile / split-K regime, where a workgroup's MFMAs take no time
 // and the launch is bound by the bytes of W in flight: one 128x128 tile per CU with one step ahead keeps 16 KB per CU on
 // its way, far from what HBM needs (fp8 M=128, N=K=8192: 27 us for a 67 MB weight).
+constexpr bool is_mx_kind(int kind) { return kind == KIND_MXFP4 || kind == KIND_MXFP8 || kind == KIND_MXA8W4 || kind == KIND_MXA6W4; }
 template <int KIND, int MR, int NR, int WM, int STORE, int WAVES = 4, int OCC = 0, int PFW = 1>
-__global__ void __launch_bounds__(WAVES * 64, (OCC > 0 ? OCC : (WAVES == 4 && MR * NR <= 32 && !((KIND == KIND_MXFP4 || KIND == KIND_MXFP8) && MR * NR == 32) ? 2 : 1)))
+__global__ void __launch_bounds__(WAVES * 64, (OCC > 0 ? OCC : (WAVES == 4 && MR * NR <= 32 && !(is_mx_kind(KIND) && MR * NR == 32) ? 2 : 1)))
 k_a8w8_tiled(A8W8Params p) {
     using acc_t = typename Acc<KIND>::type;
     constexpr int WN = WAVES / WM;
@@ -145,7 +146,8 @@ k_a8w8_tiled(A8W8Params p) {
     // K counts BYTES of one operand row from here on (two fp4 elements per byte)
     constexpr bool IS16 = KIND == KIND_FP16 || KIND == KIND_BF16;
     constexpr bool SCALED = KIND == KIND_INT8 || KIND == KIND_FP8;  // per-token x per-channel fp32 scales in the epilogue
-    constexpr bool MX = KIND == KIND_MXFP4 || KIND == KIND_MXFP8;   // e8m0 scales applied by the MFMA
+    constexpr bool MX = is_mx_kind(KIND);                           // e8m0 scales applied by the MFMA
+    constexpr bool W4 = KIND == KIND_MXA8W4 || KIND == KIND_MXA6W4; // fp4 W against a wider A: half a row's bytes
     const int K = KIND == KIND_MXFP4 ? (p.K >> 1) : (IS16 ? (p.K << 1) : p.K);
     const int KT = (K + TK - 1) / TK;
     // split-K: workgroup blockIdx.y of p.splits covers K steps [kt_begin, kt_end) and (STORE_ACC only) writes its
@@ -154,13 +156,14 @@ k_a8w8_tiled(A8W8Params p) {
     const int kt_begin = (int)blockIdx.y * kt_per;
     const int kt_end = (kt_begin + kt_per) < KT ? (kt_begin + kt_per) : KT;
 
+    const int KW = W4 ? K >> 1 : K;  // bytes of one W row
     // A: this tile's rows; rows >= M read as zero through the descriptor bound
     const uint64_t a_rows = (uint64_t)(p.M - m0);
     __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a + (uint64_t)m0 * K, a_rows * (uint64_t)K);
     // B: this wave's NR n-blocks; blocks >= N/16 read as zero
     const int nb0 = (n0 >> 4) + wn * NR;
-    const uint64_t b_off = (uint64_t)nb0 * 16ull * (uint64_t)K;
-    const uint64_t b_total = (uint64_t)p.N * (uint64_t)K;
+    const uint64_t b_off = (uint64_t)nb0 * 16ull * (uint64_t)KW;
+    const uint64_t b_total = (uint64_t)p.N * (uint64_t)KW;
     __amdgpu_buffer_rsrc_t rb = make_rsrc(p.b + (b_off < b_total ? b_off : b_total), b_off < b_total ? b_total - b_off : 0);
 
     // MXFP4 scales: 256 bytes per (32-row chunk, 256-K chunk); this tile's / this wave's chunks; chunks past the
@@ -170,7 +173,7 @@ k_a8w8_tiled(A8W8Params p) {
     uint32_t chunk_bytes = 0;
     if constexpr (MX) {
         static_assert(!MX || (MR % 2 == 0 && NR % 2 == 0), "scale chunks cover 32 rows");
-        // one 256-byte block of scale dwords per 256 K elements: every K step for mxfp4, every second one for mxfp8
+        // one 256-byte block of scale dwords per 256 K elements: every K step for mxfp4, every second one for the others
         chunk_bytes = KIND == KIND_MXFP4 ? (uint32_t)KT * 256u : (uint32_t)(p.K >> 8) * 256u;
         const uint64_t sa_chunks = (uint64_t)((p.M + 31) >> 5), sa_first = (uint64_t)((m0 >> 5) + wm * MP);
         rsa = make_rsrc(p.mx_sa + (sa_first < sa_chunks ? sa_first : sa_chunks) * chunk_bytes,
@@ -195,6 +198,7 @@ k_a8w8_tiled(A8W8Params p) {
     // Register sets: areg holds the A tile of the next K step on its way to LDS (each register is written to
     // LDS and immediately reloaded for the step after); blo/bhi[q] hold the W fragments of the steps with kt % NB == q.
     constexpr int NB = PFW + 1;
+    constexpr int N_W = W4 ? NR : 2 * NR;  // W fragment loads per wavefront per step
     static_assert(NB == 2 || (NB == 4 && !MX), "W register sets: 2, or 4 for the kinds without MX scale dwords");
     // With four W sets the A tile is fetched just as far ahead (loads return in order: a wait for A of the next step would
     // otherwise also wait for every W fragment requested before it): four A register sets, A(j) in set j % 4, loaded five
@@ -221,7 +225,7 @@ k_a8w8_tiled(A8W8Params p) {
     // MXFP4: load number 2*NR + q fetches scale dword q of the step (A-side chunks first, then W-side)
     auto load_sc1 = [&](int kt, int q, int* sa_dst, int* sb_dst) {
         const bool has = kt < kt_end;
-        const uint32_t soff = has ? (uint32_t)(KIND == KIND_MXFP8 ? (kt >> 1) : kt) * 256u : 0u;
+        const uint32_t soff = has ? (uint32_t)(KIND == KIND_MXFP4 ? kt : (kt >> 1)) * 256u : 0u;
         if (q < MP) {
             sa_dst[q] = buf_load4(rsa, has ? (uint32_t)q * chunk_bytes + (uint32_t)lane * 4u : 0xFFFFFFF0u, soff);
         } else {
@@ -233,18 +237,18 @@ k_a8w8_tiled(A8W8Params p) {
     // (row li, 16-byte K group lg) reads row li of the n-block at K offset 16*lg; 16 segments of 64 bytes per load
     // instead of one contiguous KB.  Either way an n-block of 16 rows is 16*K bytes, so the descriptor is the same.
     const uint32_t b_lane_off = p.b_rowmajor ? (uint32_t)li * (uint32_t)K + (uint32_t)lg * 16u : (uint32_t)lane * 16u;
-    const uint32_t b_step = p.b_rowmajor ? 128u : 2048u, b_half = p.b_rowmajor ? 64u : 1024u;
+    const uint32_t b_step = p.b_rowmajor ? 128u : W4 ? 1024u : 2048u, b_half = p.b_rowmajor ? 64u : 1024u;
     auto load_b1 = [&](int kt, int idx, v4i* lo, v4i* hi) {
-        const int ni = idx >> 1;
-        const bool has = kt < kt_end && (kt * TK + (idx & 1) * 64) < K;
-        const uint32_t voff = b_lane_off + (uint32_t)ni * 16u * (uint32_t)K;
-        const v4i v = buf_load16(rb, has ? voff : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)(idx & 1) * b_half : 0u);
-        if (idx & 1) hi[ni] = v; else lo[ni] = v;
+        const int ni = W4 ? idx : idx >> 1, half = W4 ? 0 : idx & 1;
+        const bool has = kt < kt_end && (kt * TK + half * 64) < K;
+        const uint32_t voff = b_lane_off + (uint32_t)ni * 16u * (uint32_t)KW;
+        const v4i v = buf_load16(rb, has ? voff : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
+        if (half) hi[ni] = v; else lo[ni] = v;
     };
     auto read_frag = [&](int stage, int mi, v4i& flo, v4i& fhi) {
         const int row = (wm * MR + mi) * 16 + li;
-        flo = *reinterpret_cast<const v4i*>(&lds[stage][lds_off(row, lg)]);
-        fhi = *reinterpret_cast<const v4i*>(&lds[stage][lds_off(row, 4 + lg)]);
+        flo = *reinterpret_cast<const v4i*>(&lds[stage][lds_off(row, KIND == KIND_MXA6W4 ? 2 * lg : lg)]);
+        fhi = *reinterpret_cast<const v4i*>(&lds[stage][lds_off(row, KIND == KIND_MXA6W4 ? 2 * lg + 1 : 4 + lg)]);
     };
 
     // One K step (tile kt, parity S): MFMAs on LDS stage S and W set S, with the memory work of the next
@@ -259,7 +263,7 @@ k_a8w8_tiled(A8W8Params p) {
         constexpr int S = SB & 1;                // LDS stage (and MX scale set) of this step
         constexpr int SN = (SB + PFW) % NB;      // W register set the loads of this step fill
         constexpr int HALF = MR / 2;
-        constexpr int N_LOADS = 2 * NR + (MX ? MP + NP : 0);  // W fragments (+ scale dwords)
+        constexpr int N_LOADS = N_W + (MX ? MP + NP : 0);  // W fragments (+ scale dwords)
         constexpr int B_PER = (N_LOADS + HALF - 1) / HALF;
         // A fragments are read FRAG_AHEAD m-blocks ahead of the MFMAs that use them (register ring buffer)
         // (one block ahead for the int8 128x256 tile held to two workgroups per CU: with two the build spilled 48 bytes per
@@ -278,8 +282,8 @@ k_a8w8_tiled(A8W8Params p) {
             if constexpr (mi < HALF) {
                 static_for<B_PER>([&](auto Q) {
                     constexpr int idx = mi * B_PER + decltype(Q)::value;
-                    if constexpr (idx < 2 * NR) load_b1(kt + PFW, idx, blo[SN], bhi[SN]);
-                    else if constexpr (idx < N_LOADS) load_sc1(kt + 1, idx - 2 * NR, sav[S ^ 1], sbv[S ^ 1]);
+                    if constexpr (idx < N_W) load_b1(kt + PFW, idx, blo[SN], bhi[SN]);
+                    else if constexpr (idx < N_LOADS) load_sc1(kt + 1, idx - N_W, sav[S ^ 1], sbv[S ^ 1]);
                 });
             } else {
                 constexpr int A_PER = (A_LOADS + (MR - HALF) - 1) / (MR - HALF);
@@ -328,6 +332,17 @@ k_a8w8_tiled(A8W8Params p) {
                                     bhi[SB][ni][0], bhi[SB][ni][1], bhi[SB][ni][2], bhi[SB][ni][3]};
                     mfma_mx8<S, ni & 1, mi & 1>(acc[mi][ni], bf, af, sbv[S][ni / 2], sav[S][mi / 2]);
                 });
+            } else if constexpr (W4) {
+                static_for<NR>([&](auto NI) {
+                    constexpr int ni = decltype(NI)::value;
+                    if constexpr (KIND == KIND_MXA8W4) {
+                        const v8i af = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1], ahi[2], ahi[3]};
+                        mfma_mx4w<S, ni & 1, mi & 1>(acc[mi][ni], blo[SB][ni], af, sbv[S][ni / 2], sav[S][mi / 2]);
+                    } else {
+                        const v6i af = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1]};
+                        mfma_mx4w<S, ni & 1, mi & 1>(acc[mi][ni], blo[SB][ni], af, sbv[S][ni / 2], sav[S][mi / 2]);
+                    }
+                });
             } else {
                 const v8i af = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1], ahi[2], ahi[3]};
 #pragma unroll
@@ -355,7 +370,7 @@ k_a8w8_tiled(A8W8Params p) {
     static_for<PFW>([&](auto I) {
         constexpr int i = decltype(I)::value;
 #pragma unroll
-        for (int idx = 0; idx < 2 * NR; idx++) load_b1(kt_begin + i, idx, blo[i], bhi[i]);
+        for (int idx = 0; idx < N_W; idx++) load_b1(kt_begin + i, idx, blo[i], bhi[i]);
         if constexpr (NA == 4) {
 #pragma unroll
             for (int j = 0; j < A_LOADS; j++) load_a1(kt_begin + 1 + i, j, areg[1 + i][j]);

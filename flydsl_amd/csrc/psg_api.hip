@@ -29,7 +29,7 @@ bool psg_moe_gate_sort_fuses(int tokens, int topk, int experts);
 hipError_t psg_launch_moe_reduce(const void* x, void* y, int tokens, int topk, int dim, int out_dtype, const int32_t* mask,
                                  const int32_t* ids, int experts, hipStream_t stream);
 hipError_t psg_launch_mx_generic(const MxGenParams& p, int af, int bf, int store, int batch, hipStream_t stream);
-hipError_t psg_launch_tiled_mxw4(const A8W8Params& p, bool fp6, hipStream_t stream);
+hipError_t psg_launch_tiled_mxw4(const A8W8Params& p, bool fp6, int tile_m, int tile_n, hipStream_t stream);
 hipError_t psg_launch_mx_smallm(const MxGenParams& p, int af, int bf, int batch, hipStream_t stream);
 hipError_t psg_launch_mxfp4_smallm(const MxParams& p, int store, int nw, hipStream_t stream);
 hipError_t psg_launch_splitk_finalize(const A8W8Params& p, const void* partial, int is_int, int scaled, hipStream_t stream);
@@ -192,14 +192,15 @@ Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
 }
 
 // Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 3 % below that of
-// the score's tile.  A tile's estimate is a start, one `round` per set of tiles that the CUs hold together and, per K step of 128 bytes, what a CU
+// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  A tile's estimate is a start, one `round` per set of tiles that the CUs hold together and, per K step of 128 bytes, what a CU
 // takes for the 1 .. per_cu tiles it works on at once, so it knows what the score doesn't: a second tile on a CU costs little while a step is bound by
 // its loads, short rows are bound by the rounds' ends, and a last round with few tiles is shorter.  The constants are a least-squares fit to 722
-// fp4 and 208 fp8 problems (65 to 8192 rows, 1024 to 16384 columns, K 1024 to 14336), every tile timed on each; the estimates are 4 to 7 % off
+// fp4 x fp4, 208 fp8 x fp8 and 312 fp8 / fp6 x fp4 problems (65 to 8192 rows, 1024 to 16384 columns, K 1024 to 14336), every tile timed on each; the estimates are 4 to 7 % off
 // (r.m.s.; fp8 3 to 5), which is why the score's tile stays where they are close: without that eight of the 722 got more than 3 % slower, with it one
 // does (282x9216x1280 9.4 us against 9.9).  199 take another tile, 10 % faster on average (us score / estimate: 4887x4256x1024 31.3 / 22.7,
 // 2127x14560x2304 63 / 56, 1285x14048x3072 56 / 44, 788x5280x4608 22.0 / 20.5, 5678x3584x4608 70.6 / 60.0, 48x4096x1024 6.5 / 4.3).
-Tile pick_mx_tile(int M, int N, int kbytes, bool fp8) {
+enum { MX_FP4, MX_FP8, MX_W4 };
+Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
     struct Cost {
         int m, n, waves, per_cu;
         double start, round, step[5];  // us; step[r]: r tiles on a CU
@@ -211,12 +212,15 @@ Tile pick_mx_tile(int M, int N, int kbytes, bool fp8) {
     static const Cost costs8[] = {{256, 256, 8, 1, 2.3, 9.5, {0, 1.45}},           {128, 256, 4, 1, 2.3, 5.7, {0, 0.85}},
                                   {64, 256, 4, 2, 3.9, 1.9, {0, 0.58, 1.02}},      {32, 256, 4, 3, 4.6, 0.0, {0, 0.50, 0.90, 1.21}},
                                   {64, 128, 4, 3, 4.1, 0.5, {0, 0.37, 0.60, 0.88}}, {32, 128, 4, 4, 3.6, 0.2, {0, 0.31, 0.48, 0.73, 0.87}}};
+    static const Cost costs48[] = {{256, 256, 8, 1, 0.0, 7.1, {0, 1.14}},               {128, 256, 4, 2, 4.0, 3.5, {0, 0.77, 1.36}},
+                                   {64, 256, 4, 3, 3.4, 2.2, {0, 0.48, 0.77, 1.13}},    {32, 256, 4, 3, 3.6, 0.8, {0, 0.37, 0.58, 0.76}},
+                                   {64, 128, 4, 3, 3.4, 1.0, {0, 0.34, 0.49, 0.68}},    {32, 128, 4, 4, 3.1, 0.5, {0, 0.28, 0.35, 0.49, 0.60}}};
     const double cus = psg_cu_count(), steps = (kbytes + 127) / 128;
-    const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;  // us of the memory bus; near that bound a launch takes longer than either estimate
+    const double mem = ((double)M * kbytes + (double)N * (formats == MX_W4 ? kbytes / 2 : kbytes) + 2.0 * M * N) / 4.3e6;  // us of the memory bus; near that bound a launch takes longer than either estimate
     const Tile scored = pick_tile(M, N, true, 0, 0);
-    double best = 0, kept = 0;
+    double best = 0, kept = 1e30;
     Tile t = scored;
-    for (const Cost& c : fp8 ? costs8 : costs4) {
+    for (const Cost& c : formats == MX_FP4 ? costs4 : formats == MX_FP8 ? costs8 : costs48) {
         const double tiles = (double)((M + c.m - 1) / c.m) * (double)((N + c.n - 1) / c.n), slots = cus * c.per_cu;
         const double full = std::floor(tiles / slots), rest = (tiles - full * slots) / cus;
         double us = full * (c.round + steps * c.step[c.per_cu]);
@@ -229,7 +233,7 @@ Tile pick_mx_tile(int M, int N, int kbytes, bool fp8) {
             us += c.round + steps * step;
         }
         us = c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
-        if (c.m == scored.m && c.n == scored.n) kept = us;
+        if (formats != MX_W4 && c.m == scored.m && c.n == scored.n) kept = us;
         if (best == 0 || us < best) {
             best = us;
             t = {c.m, c.n, c.waves};
@@ -269,15 +273,11 @@ int pick_splits(int M, int N, int kbytes, Tile t) {
     return s;
 }
 
-// Whether fp8 / fp6 x fp4, and one batch of several of the fp4 and fp8 pairs too, runs on the tiles of the dense kernels: where 128x256
-// tiles would give every CU one.  There the general kernel works on 128x256 tiles, and one of those takes as long as a 256x256
-// tile does here (fp8 x fp4, us 256x256 / general: 500x16384x4096 42.9 / 48.7, 1000x8192x4096 42.6 / 47.3, 1024x16384x2048 30.4 /
-// 51.7, 1280x8192x4096 41.3 / 87.2, 4096x4096x8192 92.2 / 169.5, 8192x1024x14336 124 / 146); with fewer its 64x128 tiles and its K
-// splits are the better way (768x8192x4096 39.4 / 34.7, 1000x4096x14336 115 / 63).  Batches, one launch each against the general kernel's one
-// over all: fp8 x fp8 2 x 1024x8192x4096 78 / 104, 8 324 / 497, 12 473 / 744, 4 x 1280x8192x2048 139 / 139; fp4 x fp4 2 x 512x16384x2048
-// 34.8 / 45.7, 8 x 2048x4096x4096 194 / 277; fp8 x fp4 2 x 2048x4096x4096 88 / 93, 8 327 / 371; fp6 x fp4 2 x 512x16384x2048 53.6 / 52.6, 8
-// 205 / 216; with half as many tiles fp8 x fp4 8 x 512x8192x2048 183 / 104.  More batches gain as much; the limit of eight (mx_common) is
-// what one call may queue as launches of its own.
+// Whether a batch of several dense MX products runs on the tiles of the dense kernels, a launch each: where 128x256 tiles of one product would
+// give every CU one, since the general kernel takes all batches in one launch (us tiles / general: fp8 x fp8 2 x 1024x8192x4096 78 / 104, 8 324 /
+// 497, 12 473 / 744, 4 x 1280x8192x2048 139 / 139; fp4 x fp4 2 x 512x16384x2048 34.8 / 45.7, 8 x 2048x4096x4096 194 / 277; fp8 x fp4 2 x 2048x4096x4096
+// 88 / 93, 8 327 / 371; fp6 x fp4 2 x 512x16384x2048 53.6 / 52.6, 8 205 / 216; with half as many tiles fp8 x fp4 8 x 512x8192x2048 183 / 104).
+// More batches gain as much; the limit of eight (mx_common) is what one call may queue as launches of its own.
 bool mx_fills_tiles(int M, int N) {
     return M > kStreamMaxM && (long)((M + 127) / 128) * (long)((N + 255) / 256) >= psg_cu_count();
 }
@@ -319,17 +319,19 @@ int mx_general_splits(int M, int N, int K) {
     return s;
 }
 
-// Whether dense, unbatched fp8 x fp8 runs on the tiles of the dense kernels: beyond 32 rows everywhere except where the small-M kernel's
-// workgroups make one round of the CUs (N / 32 times the 64-row groups), and where the general kernel splits K (`room`: the caller brought the
-// workspace) and the splits make one round.  Over 208 problems of 65 to 8192 rows the tiles were 16 % faster on average than
-// what ran there (us tiles / small-M or general kernel: 383x12384x6912 49.8 / 90.5, 365x10336x2304 15.9 / 27.0, 1164x2880x4096 23.2 / 37.1, 524x9440x5376
-// 42.4 / 69.8, 128x512x4096 12.6 / 17.7, 4096x1024x512 8.1 / 10.1; small-M, two rounds, 389x1984x4352 14.5 / 21.0, 186x5184x2048 8.8 / 12.3, 64x8224x2048
-// 8.9 / 9.7, 33x16384x4096 15.0 / 18.7; one round 228x1056x9216 25.7 / 18.6, 64x8192x4096 13.8 / 10.5; splits 33x992x14336 37.0 / 19.3, 87x8160x12032
-// 33.4 / 29.6, more than one round of them 67x9568x8960 26.3 / 36.7).  Up to 32 rows the small-M kernel is the better one (32x12288x4096 14.2 / 13.6).
-bool mxfp8_takes_tiles(int M, int N, int K, bool room) {
+// Whether dense, unbatched fp8 x fp8 and fp8 / fp6 x fp4 run on the tiles of the dense kernels: beyond 32 rows everywhere except where the small-M
+// kernel's workgroups make one round of the CUs (N / 32 times the 64-row groups; an eighth more on short rows, whose second round is soon
+// over), and where the general kernel splits K (`room`: the caller brought the workspace) and the splits make one round.  Against what ran there
+// (small-M or general kernel), over 208 and 250 problems of 33 to 8192 rows, fp8 x fp8 is 16 % faster on average, fp8 / fp6 x fp4 20 % (us tiles /
+// before: fp8 x fp8 383x12384x6912 49.8 / 90.5, 365x10336x2304 15.9 / 27.0, 1164x2880x4096 23.2 / 37.1, 128x512x4096 12.6 / 17.7, 4096x1024x512 8.1 /
+// 10.1; small-M, two rounds, 389x1984x4352 14.5 / 21.0, 64x8224x2048 8.9 / 9.7, 33x16384x4096 15.0 / 18.7; one round 228x1056x9216 25.7 / 18.6,
+// 64x8192x4096 13.8 / 10.5; splits 33x992x14336 37.0 / 19.3, 87x8160x12032 33.4 / 29.6, more than one round of them 67x9568x8960 26.3 / 36.7;
+// fp8 x fp4 591x8032x5632 33.4 / 51.5, 812x8000x3584 27.3 / 42.0; fp6 x fp4 293x14656x1280 12.1 / 19.0, 6322x1024x4608 30.3 / 48.0, 1040x13696x6144
+// 66 / 113).  Up to 32 rows the small-M kernel is the better one (fp8 x fp8 32x12288x4096 13.6 / 14.2 on tiles).
+bool mx_takes_tiles(int M, int N, int K, bool fp8_weights, bool room) {
     if (M <= kSmallM) return false;
-    const long cus = psg_cu_count(), groups = (M + 63) / 64;
-    if ((long)(N / 32) * groups <= cus && mx_general_small(M, N, K, false, true, 1)) return false;
+    const long cus = psg_cu_count(), groups = (M + 63) / 64, wgs = (long)(N / 32) * groups;
+    if ((K < 1536 ? wgs * 8 <= cus * 9 : wgs <= cus) && mx_general_small(M, N, K, false, fp8_weights, 1)) return false;
     const int splits = mx_general_splits(M, N, K);
     return !(room && splits > 1 && groups * ((N + 127) / 128) * splits <= cus);
 }
@@ -358,7 +360,7 @@ Plan plan_tiled(int M, int N, int kbytes, bool mx) {
     // N=8192 22.0 against 23.7; M=384, N=8192, 768 tiles: 28.0 against 26.5, so the larger tile is kept there)
     if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4};
     const int splits = mx && mx_small_holds(M, N, kbytes * 2) ? 1 : pick_splits(M, N, kbytes, t);
-    if (mx && splits == 1) t = pick_mx_tile(M, N, kbytes, false);
+    if (mx && splits == 1) t = pick_mx_tile(M, N, kbytes, MX_FP4);
     return {t, splits};
 }
 
@@ -661,7 +663,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
     const bool fp8_pair = a->a_dtype == PSG_MX_FP8 && a->b_dtype == PSG_MX_FP8 && batch == 1 && dense;
     // what the general kernel's split-K plan needs is there
     const bool room = store == STORE_C && a->workspace && aligned(a->workspace, 16) && a->workspace_bytes >= splitk_bytes(a->M, a->N, mx_general_splits(a->M, a->N, a->K));
-    const bool fp8_tiled = fp8_pair && (a->force_path == 1 || (a->force_path == 0 && mxfp8_takes_tiles(a->M, a->N, a->K, room)));
+    const bool fp8_tiled = fp8_pair && (a->force_path == 1 || (a->force_path == 0 && mx_takes_tiles(a->M, a->N, a->K, true, room)));
     if (a->force_path == 2 && !fp4_fast) return fail(PSG_E_SHAPE, "force_path=2 is for dense, unbatched fp4 x fp4 only");
     if (a->force_path == 1 && !fp4_fast && !fp8_pair)
         return fail(PSG_E_SHAPE, "force_path=1 is for dense, unbatched fp4 x fp4 or fp8 x fp8 only");
@@ -672,12 +674,13 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
     const int64_t sa_bs = a->scale_a_batch_stride ? a->scale_a_batch_stride : (int64_t)((uint64_t)((a->M + 31) / 32) * sa_cs);
     const bool w4 = a->b_dtype == PSG_MX_FP4 && a->a_dtype != PSG_MX_FP4;
     const bool same = a->b_dtype == a->a_dtype && batch > 1;
-    const bool per_batch = (w4 || same) && dense && store == STORE_C && a->force_path == 0 && batch <= 8 && mx_fills_tiles(a->M, a->N) && a_bs % 16 == 0 &&
+    const bool per_batch = (w4 || same) && dense && store == STORE_C && a->force_path == 0 && batch <= 8 &&
+                           (batch == 1 ? mx_takes_tiles(a->M, a->N, a->K, false, room) : mx_fills_tiles(a->M, a->N)) && a_bs % 16 == 0 &&
                            c_bs % 16 == 0 && sa_bs % 4 == 0;
     if (fp8_tiled || per_batch) {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
         const bool fp4 = a->a_dtype == PSG_MX_FP4;
-        const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : w4 ? Tile{256, 256, 8} : pick_mx_tile(a->M, a->N, fp4 ? a->K / 2 : a->K, !fp4);
+        const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : pick_mx_tile(a->M, a->N, fp4 ? a->K / 2 : a->K, fp4 ? MX_FP4 : w4 ? MX_W4 : MX_FP8);
         A8W8Params q{};
         q.c = out;
         q.a = static_cast<const uint8_t*>(a->a);
@@ -695,7 +698,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         q.out = a->out_dtype;
         if (fp4) q.wave_layout = t.waves == 8 ? 8 : 1;
         for (int z = 0; z < batch; z++) {
-            const hipError_t te = w4 ? psg_launch_tiled_mxw4(q, a->a_dtype == PSG_MX_FP6, static_cast<hipStream_t>(stream))
+            const hipError_t te = w4 ? psg_launch_tiled_mxw4(q, a->a_dtype == PSG_MX_FP6, t.m, t.n, static_cast<hipStream_t>(stream))
                                      : psg_launch_a8w8_tiled(q, fp4 ? KIND_MXFP4 : KIND_MXFP8, store, t.m, t.n, static_cast<hipStream_t>(stream));
             if (te != hipSuccess) return hip_fail(te, "psg_gemm_mxfp4 launch");
             q.c = static_cast<uint8_t*>(q.c) + c_bs;

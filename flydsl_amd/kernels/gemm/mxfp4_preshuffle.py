@@ -146,8 +146,8 @@ def launch_gemm(
     constraints are kept: ``tile_k in {128, 256}``, ``tile_n % 128 == 0``, ``K % tile_k == 0``
     (mxfp4_preshuffle.py:122,316).  Dense unbatched fp4 x fp4 runs on the tuned fp4 kernels (``tile_*`` are hints the
     planner may override).  Every other combination is planned from its sizes alone, whatever ``tile_*`` say: few rows run on the small-M
-    MX kernel, dense fp8 x fp8 from 33 rows on and fp8 / fp6 x fp4 problems that fill the GPU on the dense tiles (batches that fill it, those of
-    fp4 x fp4 too, one launch each), the rest on the general MX kernel."""
+    MX kernel, dense fp8 x fp8 and fp8 / fp6 x fp4 from 33 rows on mostly on the dense tiles (batches that fill the GPU, those of fp4 x fp4 too,
+    one launch each), the rest on the general MX kernel."""
     # (anything but plain numbers and texts is worked out anew: other types may hash by identity)
     plain = type(N) is type(K) is type(tile_m) is type(tile_n) is type(tile_k) is int and type(a_dtype) is type(b_dtype) is type(out_dtype) is str
     plan = _plan if plain else _plan.__wrapped__

@@ -135,8 +135,8 @@ enum psg_mx_dtype { PSG_MX_FP4 = 0, PSG_MX_FP6 = 1, PSG_MX_FP8 = 2,
  * ceil(M/32) chunks for scale_a).  W and scale_b are always batch-dense (mxfp4_preshuffle.py:177-193).  Batch z reads
  * a + z*a_batch_stride etc. (bytes) and all batches run in ONE launch (grid.z = batch).
  * Which kernel runs: fp4 x fp4 with batch 1 and dense strides takes the tuned fp4 kernels (tiled mainloop, small-M
- * split-K; workspace / tile_* / force_path 1, 2 apply to them only); everything else is planned from its sizes (dense fp8 x fp8 of
- * more than 32 rows mostly on the same tiles, few rows on the small-M MX kernel); the rest, or force_path 3, takes the general kernel, which ignores the tile arguments and uses workspace (psg_workspace_bytes(M, N, K, 5) bytes) for
+ * split-K; workspace / tile_* / force_path 1, 2 apply to them only); everything else is planned from its sizes (dense fp8 x fp8 and
+ * fp8 / fp6 x fp4 of more than 32 rows mostly on such tiles, few rows on the small-M MX kernel); the rest, or force_path 3, takes the general kernel, which ignores the tile arguments and uses workspace (psg_workspace_bytes(M, N, K, 5) bytes) for
  * split-K when batch is 1 and C is dense.
  */
 typedef struct psg_mxfp4_args {

@@ -1,4 +1,4 @@
-"""The kernel and tile that an fp4 x fp4 or fp8 x fp8 problem takes by itself: sizes on whose tile the estimate decides against the score, either side of
+"""The kernel and tile that an fp4 x fp4, fp8 x fp8 or fp8 / fp6 x fp4 problem takes by itself: sizes on whose tile the estimate decides against the score, either side of
 the lines between the small-M kernel, the general kernel's K splits and the tiles, ragged rows and columns, one tile and several rounds of them,
 against the general MX kernel on the same operands.
 
@@ -19,6 +19,9 @@ pytestmark = pytest.mark.gpu
 ]] + [("fp8",) + s for s in [
     (32, 8224, 512, 1), (33, 992, 512, 1), (33, 992, 14336, 1), (64, 8192, 1024, 1), (64, 8224, 1024, 1), (65, 32, 256, 1), (65, 4096, 512, 1), (128, 4128, 512, 1),
     (87, 8160, 4096, 1), (67, 9568, 8960, 1), (300, 992, 4096, 1), (383, 12384, 768, 1), (1164, 2880, 1024, 1), (4096, 1024, 512, 1), (2127, 4384, 1536, 2),
+]] + [(f,) + s for f in ("fp8-fp4", "fp6-fp4") for s in [
+    (32, 8224, 512, 1), (33, 992, 512, 1), (33, 992, 14336, 1), (64, 8192, 1024, 1), (64, 8224, 2304, 1), (64, 9248, 1024, 1), (65, 32, 256, 1), (128, 4128, 1536, 1),
+    (300, 992, 4096, 1), (383, 12384, 768, 1), (1164, 2880, 1024, 1), (293, 14656, 1280, 1), (2311, 4544, 768, 1), (5000, 1024, 512, 1), (2127, 4384, 1536, 2),
 ]])
 def test_planned_tile(fmt, M, N, K, batch):
     g = torch.Generator(device="cuda")
@@ -28,27 +31,28 @@ def test_planned_tile(fmt, M, N, K, batch):
     def data(lo, hi, *shape):
         return torch.randint(lo, hi, shape, generator=g, device="cuda", dtype=torch.uint8)
 
+    fa, fb = (fmt, fmt) if "-" not in fmt else fmt.split("-")
     if fmt == "fp4":
         a, b = data(0, 256, batch, M, K // 2), data(0, 256, batch, N, K // 2)
     else:  # every finite positive and small negative code (0x7f and 0xff are NaN)
-        a, b = data(0, 127, batch, M, K), data(0, 127, batch, N, K)
+        a, b = data(0, 127, batch, M, K), data(0, 127, batch, N, K) if fb == "fp8" else data(0, 256, batch, N, K // 2)
         a[..., ::3] |= 128
     sa, sb = data(120, 130, batch, chunks * K), data(120, 130, batch, N // 32 * K)
 
     def run(path):
         c = torch.full((batch * M + 64, N), -8192.0, dtype=torch.bfloat16, device="cuda")
-        launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, fmt, "bf16", fmt, batch, -1, -1, -1, -1, -1, -1, 0, 0,
+        launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, fa, "bf16", fb, batch, -1, -1, -1, -1, -1, -1, 0, 0,
                     _force_path=path)
         acc = torch.empty(batch, M, N, dtype=torch.float32, device="cuda")
         if batch == 1:
-            launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, fmt, "bf16", fmt, 1, -1, -1, -1, -1, -1, -1, 0, 0,
+            launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, fa, "bf16", fb, 1, -1, -1, -1, -1, -1, -1, 0, 0,
                         _force_path=path, _acc=acc)
         torch.cuda.synchronize()
         assert (c[batch * M:] == -8192.0).all()
         return c[:batch * M].view(batch, M, N), acc
 
     (c, acc), (ref_c, ref) = run(0), run(3)
-    if batch == 1:
+    if batch == 1 and fa == fb:  # (the others' tiles store no fp32)
         assert (acc - ref).abs().max() <= 1e-5 * ref.abs().max()
         if fmt == "fp4":
             assert torch.equal(c[0], acc[0].bfloat16())
