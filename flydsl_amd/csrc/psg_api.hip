@@ -191,50 +191,76 @@ Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
     return t;
 }
 
+// A tile's estimated time on a problem whose K isn't split: a start, one `round` per set of tiles that the CUs hold together and, per K step of 128
+// bytes, what a CU takes for the 1 .. per_cu tiles it works on at once.  It knows what the score above doesn't: a second tile on a CU costs little
+// while a step is bound by its loads, short rows are bound by the rounds' ends, and a last round with few tiles is shorter.  The constants are
+// least-squares fits to timed problems of 65 to 8192 rows, 1024 to 16384 columns (8 and 16 bits: 28672) and K 1024 to 14336, every tile timed on each.
+struct TileCost {
+    int m, n, waves, per_cu;
+    double start, round, step[5];  // us; step[r]: r tiles on a CU
+};
+
+// mem: us of the memory bus; near that bound a launch takes longer than either estimate
+double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
+    const double cus = psg_cu_count(), tiles = (double)((M + c.m - 1) / c.m) * (double)((N + c.n - 1) / c.n), slots = cus * c.per_cu;
+    const double full = std::floor(tiles / slots), rest = (tiles - full * slots) / cus;
+    double us = full * (c.round + steps * c.step[c.per_cu]);
+    if (rest > 0) {
+        // the last round: CUs with one tile more than others finish last, but those with fewer are done sooner and leave them the bus
+        const double r = rest > 1 ? 0.25 * rest + 0.75 * std::ceil(rest) : 1;
+        const int lo = (int)r;
+        double step = c.step[lo] + (lo < c.per_cu ? (r - lo) * (c.step[lo + 1] - c.step[lo]) : 0);
+        if (full == 0 && tiles < cus) step *= std::sqrt(std::sqrt(std::sqrt(std::sqrt(tiles / cus))));  // fewer CUs at work clock higher
+        us += c.round + steps * step;
+    }
+    return c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
+}
+
+// Of the three large tiles of the 8- and 16-bit kinds the one with the smallest estimate, where that is 7 % below the planned one's.  Fitted to 835 fp8 and bf16
+// problems (5 to 8 % off, r.m.s.): 51 of them take another tile, 15 % faster on average and none slower (us planned / estimate: fp8 1614x4896x6656
+// 75.4 / 50.9, 4329x1840x1856 31.5 / 23.0, 411x16720x2944 40.0 / 30.5, 3683x2288x8448 93.9 / 74.1; at 5 % two would lose 10 %).  The estimates of
+// smaller tiles are too coarse to add them (64x64 with them: 433x8560x8768 57 / 66).
+Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
+    static const TileCost costs[] = {{256, 256, 8, 1, 0.0, 7.0, {0, 1.17}}, {128, 256, 4, 2, 2.3, 7.1, {0, 0.77, 1.52}}, {128, 128, 4, 2, 5.0, 1.4, {0, 0.40, 0.91}}};
+    const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;
+    double best = 1e30, kept = 0;
+    Tile t = planned;
+    for (const TileCost& c : costs) {
+        const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
+        if (c.m == planned.m && c.n == planned.n) kept = us;
+        if (us < best) {
+            best = us;
+            t = {c.m, c.n, c.waves};
+        }
+    }
+    return best < 0.93 * kept ? t : planned;
+}
+
 // Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 3 % below that of
-// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  A tile's estimate is a start, one `round` per set of tiles that the CUs hold together and, per K step of 128 bytes, what a CU
-// takes for the 1 .. per_cu tiles it works on at once, so it knows what the score doesn't: a second tile on a CU costs little while a step is bound by
-// its loads, short rows are bound by the rounds' ends, and a last round with few tiles is shorter.  The constants are a least-squares fit to 722
-// fp4 x fp4, 208 fp8 x fp8 and 312 fp8 / fp6 x fp4 problems (65 to 8192 rows, 1024 to 16384 columns, K 1024 to 14336), every tile timed on each; the estimates are 4 to 7 % off
-// (r.m.s.; fp8 3 to 5), which is why the score's tile stays where they are close: without that eight of the 722 got more than 3 % slower, with it one
-// does (282x9216x1280 9.4 us against 9.9).  199 take another tile, 10 % faster on average (us score / estimate: 4887x4256x1024 31.3 / 22.7,
+// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  The constants are fits to 722 fp4 x
+// fp4, 208 fp8 x fp8 and 312 fp8 / fp6 x fp4 problems; the estimates are 4 to 7 % off (r.m.s.; fp8 3 to 5), which is why the score's tile stays where
+// they are close: without that eight of the 722 got more than 3 % slower, with it one does (282x9216x1280 9.4 us against 9.9).  199 take another tile, 10 % faster on average (us score / estimate: 4887x4256x1024 31.3 / 22.7,
 // 2127x14560x2304 63 / 56, 1285x14048x3072 56 / 44, 788x5280x4608 22.0 / 20.5, 5678x3584x4608 70.6 / 60.0, 48x4096x1024 6.5 / 4.3).
 enum { MX_FP4, MX_FP8, MX_W4 };
 Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
-    struct Cost {
-        int m, n, waves, per_cu;
-        double start, round, step[5];  // us; step[r]: r tiles on a CU
-    };
-    static const Cost costs4[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
-                                  {64, 256, 4, 2, 3.5, 2.8, {0, 0.58, 1.12}},      {32, 256, 4, 3, 3.6, 1.4, {0, 0.50, 0.95, 1.28}},
-                                  {64, 128, 4, 3, 3.8, 1.2, {0, 0.37, 0.67, 0.95}}, {32, 128, 4, 4, 3.0, 1.2, {0, 0.31, 0.50, 0.77, 0.90}}};
+    static const TileCost costs4[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
+                                      {64, 256, 4, 2, 3.5, 2.8, {0, 0.58, 1.12}},      {32, 256, 4, 3, 3.6, 1.4, {0, 0.50, 0.95, 1.28}},
+                                      {64, 128, 4, 3, 3.8, 1.2, {0, 0.37, 0.67, 0.95}}, {32, 128, 4, 4, 3.0, 1.2, {0, 0.31, 0.50, 0.77, 0.90}}};
     // (the fp8 launcher runs its 256x256 tile on four wavefronts whatever `waves` says)
-    static const Cost costs8[] = {{256, 256, 8, 1, 2.3, 9.5, {0, 1.45}},           {128, 256, 4, 1, 2.3, 5.7, {0, 0.85}},
-                                  {64, 256, 4, 2, 3.9, 1.9, {0, 0.58, 1.02}},      {32, 256, 4, 3, 4.6, 0.0, {0, 0.50, 0.90, 1.21}},
-                                  {64, 128, 4, 3, 4.1, 0.5, {0, 0.37, 0.60, 0.88}}, {32, 128, 4, 4, 3.6, 0.2, {0, 0.31, 0.48, 0.73, 0.87}}};
-    static const Cost costs48[] = {{256, 256, 8, 1, 0.0, 7.1, {0, 1.14}},               {128, 256, 4, 2, 4.0, 3.5, {0, 0.77, 1.36}},
-                                   {64, 256, 4, 3, 3.4, 2.2, {0, 0.48, 0.77, 1.13}},    {32, 256, 4, 3, 3.6, 0.8, {0, 0.37, 0.58, 0.76}},
-                                   {64, 128, 4, 3, 3.4, 1.0, {0, 0.34, 0.49, 0.68}},    {32, 128, 4, 4, 3.1, 0.5, {0, 0.28, 0.35, 0.49, 0.60}}};
-    const double cus = psg_cu_count(), steps = (kbytes + 127) / 128;
-    const double mem = ((double)M * kbytes + (double)N * (formats == MX_W4 ? kbytes / 2 : kbytes) + 2.0 * M * N) / 4.3e6;  // us of the memory bus; near that bound a launch takes longer than either estimate
+    static const TileCost costs8[] = {{256, 256, 8, 1, 2.3, 9.5, {0, 1.45}},           {128, 256, 4, 1, 2.3, 5.7, {0, 0.85}},
+                                      {64, 256, 4, 2, 3.9, 1.9, {0, 0.58, 1.02}},      {32, 256, 4, 3, 4.6, 0.0, {0, 0.50, 0.90, 1.21}},
+                                      {64, 128, 4, 3, 4.1, 0.5, {0, 0.37, 0.60, 0.88}}, {32, 128, 4, 4, 3.6, 0.2, {0, 0.31, 0.48, 0.73, 0.87}}};
+    static const TileCost costs48[] = {{256, 256, 8, 1, 0.0, 7.1, {0, 1.14}},               {128, 256, 4, 2, 4.0, 3.5, {0, 0.77, 1.36}},
+                                       {64, 256, 4, 3, 3.4, 2.2, {0, 0.48, 0.77, 1.13}},    {32, 256, 4, 3, 3.6, 0.8, {0, 0.37, 0.58, 0.76}},
+                                       {64, 128, 4, 3, 3.4, 1.0, {0, 0.34, 0.49, 0.68}},    {32, 128, 4, 4, 3.1, 0.5, {0, 0.28, 0.35, 0.49, 0.60}}};
+    const double mem = ((double)M * kbytes + (double)N * (formats == MX_W4 ? kbytes / 2 : kbytes) + 2.0 * M * N) / 4.3e6;
     const Tile scored = pick_tile(M, N, true, 0, 0);
-    double best = 0, kept = 1e30;
+    double best = 1e30, kept = 1e30;
     Tile t = scored;
-    for (const Cost& c : formats == MX_FP4 ? costs4 : formats == MX_FP8 ? costs8 : costs48) {
-        const double tiles = (double)((M + c.m - 1) / c.m) * (double)((N + c.n - 1) / c.n), slots = cus * c.per_cu;
-        const double full = std::floor(tiles / slots), rest = (tiles - full * slots) / cus;
-        double us = full * (c.round + steps * c.step[c.per_cu]);
-        if (rest > 0) {
-            // the last round: CUs with one tile more than others finish last, but those with fewer are done sooner and leave them the bus
-            const double r = rest > 1 ? 0.25 * rest + 0.75 * std::ceil(rest) : 1;
-            const int lo = (int)r;
-            double step = c.step[lo] + (lo < c.per_cu ? (r - lo) * (c.step[lo + 1] - c.step[lo]) : 0);
-            if (full == 0 && tiles < cus) step *= std::sqrt(std::sqrt(std::sqrt(std::sqrt(tiles / cus))));  // fewer CUs at work clock higher
-            us += c.round + steps * step;
-        }
-        us = c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
+    for (const TileCost& c : formats == MX_FP4 ? costs4 : formats == MX_FP8 ? costs8 : costs48) {
+        const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
         if (formats != MX_W4 && c.m == scored.m && c.n == scored.n) kept = us;
-        if (best == 0 || us < best) {
+        if (us < best) {
             best = us;
             t = {c.m, c.n, c.waves};
         }
@@ -360,7 +386,7 @@ Plan plan_tiled(int M, int N, int kbytes, bool mx) {
     // N=8192 22.0 against 23.7; M=384, N=8192, 768 tiles: 28.0 against 26.5, so the larger tile is kept there)
     if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4};
     const int splits = mx && mx_small_holds(M, N, kbytes * 2) ? 1 : pick_splits(M, N, kbytes, t);
-    if (mx && splits == 1) t = pick_mx_tile(M, N, kbytes, MX_FP4);
+    if (splits == 1) t = mx ? pick_mx_tile(M, N, kbytes, MX_FP4) : pick_large_tile(t, M, N, kbytes);
     return {t, splits};
 }
 

@@ -1,5 +1,5 @@
 """Either side of the lines at which a problem of few rows leaves the kernel that streams W for the tiles: the columns that make one round of the
-CUs (33 to 64 rows), rows of 4 to 8 KB (65 to 256 rows).  The automatic plan against the general tiled path of the same problem.
+CUs (33 to 64 rows), rows of 4 to 8 KB (65 to 256 rows); and sizes whose large tile the estimated time decides.  The automatic plan against the general tiled path of the same problem.
 
 int8 sums are whole numbers, so those results are the same bits; of the other kinds the two fp32 sums differ by their order alone, and a result by one
 rounding to 16 bits at most."""
@@ -18,6 +18,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("M,N,KB", [
     (33, 8192, 512), (33, 8208, 512), (64, 8224, 64), (64, 8224, 1088), (40, 9216, 6144), (33, 16400, 2048), (64, 66048, 128),
     (65, 1024, 4224), (129, 1040, 8128), (256, 1024, 4160), (65, 1008, 4224), (192, 1360, 4992),
+    # (the large tiles, by their estimated times)
+    (4329, 1840, 1856), (1614, 4896, 1664), (411, 16720, 2944), (3683, 2288, 1088), (617, 11008, 1536),
 ])
 def test_lines(dtype, M, N, KB):
     K = KB // 2 if dtype in ("bf16", "fp16") else KB
