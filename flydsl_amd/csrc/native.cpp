@@ -82,13 +82,15 @@ PyObject* guarded(F&& f) {
     return PyLong_FromLong(rc);
 }
 
+// f() without the interpreter's lock: the queue may be full.  f is the call into the library and nothing else, its arguments read before: asking a
+// tensor for anything may throw or change it, and another thread may resize it meanwhile.
 template <class F>
 int released(F&& f) {
-    int rc;
-    Py_BEGIN_ALLOW_THREADS  // the queue may be full
-    rc = f();
-    Py_END_ALLOW_THREADS
-    return rc;
+    struct Unlocked {
+        PyThreadState* const state = PyEval_SaveThread();
+        ~Unlocked() { PyEval_RestoreThread(state); }
+    } unlocked;
+    return f();
 }
 
 // launch(function address, (struct, ...), operands, stream, tensor or None, ...) -> return code of the library, or DECLINED.
@@ -150,9 +152,10 @@ PyObject* quant_pertoken(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!s || x->dim() != 2 || x_code(*x) < 0 || y->element_size() != 1 || y->numel() != x->numel() || s->scalar_type() != at::kFloat || s->numel() != x->size(0) ||
             x->size(0) > INT32_MAX || x->size(1) > INT32_MAX || !stream_of(a[5], &stream))
             return DECLINED;
-        const int code = (int)PyLong_AsLong(a[4]);
+        const int code = (int)PyLong_AsLong(a[4]), from = x_code(*x), rows = (int)x->size(0), cols = (int)x->size(1);
+        void *xp = x->data_ptr(), *yp = y->data_ptr(), *sp = s->data_ptr();
         auto fn = reinterpret_cast<int (*)(const void*, int32_t, void*, void*, int32_t, int32_t, int32_t, void*)>(PyLong_AsVoidPtr(a[0]));
-        return released([&] { return fn(x->data_ptr(), x_code(*x), y->data_ptr(), s->data_ptr(), (int32_t)x->size(0), (int32_t)x->size(1), code, stream); });
+        return released([&] { return fn(xp, from, yp, sp, rows, cols, code, stream); });
     });
 }
 
@@ -166,9 +169,10 @@ PyObject* quant_mxfp4(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!s || x->dim() != 2 || x_code(*x) < 0 || y->element_size() != 1 || s->element_size() != 1 || x->size(0) > INT32_MAX || x->size(1) > INT32_MAX ||
             y->numel() != x->size(0) * (x->size(1) / 2) || s->numel() != (x->size(0) + 31) / 32 * 32 * (x->size(1) / 32) || !stream_of(a[5], &stream))
             return DECLINED;
-        const int shuffle = (int)PyLong_AsLong(a[4]);
+        const int shuffle = (int)PyLong_AsLong(a[4]), from = x_code(*x), rows = (int)x->size(0), cols = (int)x->size(1);
+        void *xp = x->data_ptr(), *yp = y->data_ptr(), *sp = s->data_ptr();
         auto fn = reinterpret_cast<int (*)(const void*, int32_t, void*, void*, int32_t, int32_t, int32_t, void*)>(PyLong_AsVoidPtr(a[0]));
-        return released([&] { return fn(x->data_ptr(), x_code(*x), y->data_ptr(), s->data_ptr(), (int32_t)x->size(0), (int32_t)x->size(1), shuffle, stream); });
+        return released([&] { return fn(xp, from, yp, sp, rows, cols, shuffle, stream); });
     });
 }
 
@@ -191,7 +195,8 @@ PyObject* moe_reduce(PyObject*, PyObject* const* a, Py_ssize_t n) {
             return DECLINED;
         }
         auto fn = reinterpret_cast<int (*)(const void*, void*, int32_t, int32_t, int32_t, int32_t, void*)>(PyLong_AsVoidPtr(a[0]));
-        return released([&] { return fn(x->data_ptr(), y->data_ptr(), (int32_t)tokens, (int32_t)topk, (int32_t)dim, (int32_t)v[4], stream); });
+        void *xp = x->data_ptr(), *yp = y->data_ptr();
+        return released([&] { return fn(xp, yp, (int32_t)tokens, (int32_t)topk, (int32_t)dim, (int32_t)v[4], stream); });
     });
 }
 
@@ -211,7 +216,9 @@ PyObject* moe_scale_sort(PyObject*, PyObject* const* a, Py_ssize_t n) {
             return DECLINED;
         }
         auto fn = reinterpret_cast<int (*)(const void*, const void*, const void*, void*, int32_t, int32_t, int32_t, int32_t, void*)>(PyLong_AsVoidPtr(a[0]));
-        return released([&] { return fn(s->data_ptr(), ids->data_ptr(), nv->data_ptr(), out->data_ptr(), (int32_t)tokens, 1, (int32_t)s->size(1), (int32_t)ids->numel(), stream); });
+        const int cols = (int)s->size(1), size = (int)ids->numel();
+        void *sp = s->data_ptr(), *ip = ids->data_ptr(), *np = nv->data_ptr(), *op = out->data_ptr();
+        return released([&] { return fn(sp, ip, np, op, (int32_t)tokens, 1, cols, size, stream); });
     });
 }
 

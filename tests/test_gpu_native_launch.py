@@ -193,3 +193,25 @@ def test_fused_mx_pair(rcs):
         first(s, interleave=True)
     with pytest.raises(NotImplementedError):
         second(s, BM=48)
+
+
+def test_tensors_without_an_address_are_refused_with_an_error(rcs):
+    """Under vmap a tensor looks like a plain device tensor and has no storage: asking for its address throws in native code."""
+    from flydsl_amd import quant_device as Q
+    from flydsl_amd.kernels.moe.moe_gemm_2stage import compile_moe_reduction
+    from flydsl_amd.kernels.moe.mxfp_moe import moe_mxfp4_sort
+
+    s, declined = torch.cuda.current_stream(), _lib._native.DECLINED
+    dev = dict(device="cuda")
+    x = torch.randn(2, 32, 256, dtype=torch.bfloat16, **dev)
+    y, sc = torch.empty(32, 256, dtype=torch.int8, **dev), torch.empty(32, **dev)
+    p, e = torch.empty(32, 128, dtype=torch.uint8, **dev), torch.empty(32, 8, dtype=torch.uint8, **dev)
+    red, r = compile_moe_reduction(topk=2, model_dim=64, dtype_str="bf16"), torch.empty(64, 64, dtype=torch.bfloat16, **dev)
+    ids, nv = torch.zeros(32, dtype=torch.int32, **dev), torch.tensor([32, 32], dtype=torch.int32, **dev)
+    scales = torch.ones(2, 32, 8, dtype=torch.uint8, **dev)
+    for call, arg in ((lambda t: Q.pertoken_quant(t, torch.int8, stream=s, out=(y, sc)), x), (lambda t: Q.per_1x32_f4_quant(t, stream=s, out=(p, e)), x),
+                      (lambda t: red(t, r, None, None, 64, s), x), (lambda t: moe_mxfp4_sort(t, ids, nv, 32, block_size=32, out=e, stream=s), scales)):
+        n = len(rcs)
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(call)(arg)
+        assert rcs[n:] == [declined]
