@@ -215,3 +215,16 @@ def test_tensors_without_an_address_are_refused_with_an_error(rcs):
         with pytest.raises(RuntimeError):
             torch.func.vmap(call)(arg)
         assert rcs[n:] == [declined]
+
+
+def test_without_the_extension_the_results_are_the_same(monkeypatch):
+    from flydsl_amd import quant_device as Q
+
+    s, d = torch.cuda.current_stream(), _mx()
+    x, y, sc = torch.randn(33, 512, device="cuda"), torch.empty(33, 512, dtype=torch.int8, device="cuda"), torch.empty(33, device="cuda")
+    go = lambda: [t.clone() for t in (_launch(d, s), *Q.pertoken_quant(x, torch.int8, stream=s, out=(y, sc)))]
+    want = go()
+    for t in (d["c"], y, sc):
+        t.zero_()
+    monkeypatch.setattr(_lib, "_native", _lib._Declines)
+    assert all(torch.equal(a, b) for a, b in zip(go(), want))

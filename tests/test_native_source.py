@@ -34,3 +34,34 @@ def test_no_tensor_is_touched_without_the_lock():
 def test_the_lock_comes_back_when_something_throws():
     # the macros restore the thread state only where the block is left at its end
     assert "Py_BEGIN_ALLOW_THREADS" not in _without_comments()
+
+
+def test_without_the_extension_the_python_checks_do_it():
+    """The extension spares a launch its host time and nothing else: where it does not load, a warning names the cause and the calls go on."""
+    import subprocess
+    import sys
+
+    code = """
+import sys, warnings
+sys.modules["flydsl_amd._native"] = None  # what an extension that is not built, or built against another torch, looks like
+import pytest, torch
+from flydsl_amd import _lib, quant_device
+from flydsl_amd.kernels.gemm.mxfp4_preshuffle import launch_gemm
+from flydsl_amd.kernels.moe.moe_gemm_2stage import compile_moe_reduction
+from flydsl_amd.kernels.moe.mxfp_moe import moe_mxfp4_sort
+z = lambda *s, dt=torch.uint8: torch.zeros(*s, dtype=dt)
+x = z(32, 256, dt=torch.bfloat16)
+with pytest.raises(ValueError, match="device tensor"), pytest.warns(RuntimeWarning, match="_native.so"):
+    quant_device.pertoken_quant(x, torch.int8, stream=7, out=(z(32, 256), z(32, dt=torch.float32)))
+warnings.simplefilter("error")  # once is enough
+with pytest.raises(ValueError, match="device tensor"):
+    quant_device.per_1x32_f4_quant(x, stream=7, out=(z(32, 128), z(32, 8)))
+with pytest.raises(ValueError, match="device tensor"):
+    launch_gemm(z(32, 64), z(32, 128), z(64, 128), z(32, 8), z(64, 8), 32, 64, 7, 64, 256, 64, 128, 256, "fp4", "bf16", "fp4", 1, -1, -1, -1, -1, -1, -1, 0, 0)
+with pytest.raises(ValueError, match="device"):
+    compile_moe_reduction(topk=2, model_dim=64, dtype_str="bf16")(x, x, None, None, 64, 7)
+with pytest.raises(TypeError, match="device tensor"):
+    moe_mxfp4_sort(z(32, 8), z(32), z(2), 32, out=z(32, 8), stream=7)
+"""
+    done = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(flydsl_amd.__file__)), capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
