@@ -100,7 +100,8 @@ def flydsl_mxfp4_gemm1(*, a_quant, a_scale_sorted_shuffled, w1_u8, w1_scale_u8, 
                        a_dtype="fp4", stream=None):
     """Stage 1.  ``m_indices`` holds the token of every sorted row (entries >= ``n_tokens`` are padding; the packed
     ``(slot << 24) | token`` ids of the sorter are accepted as they are).  Returns the two output tensors."""
-    if stream is not None and type(n_tokens) is type(BM) is type(NE) is type(D_HIDDEN) is type(D_INTER) is type(BN) is type(BK) is int:
+    if (stream is not None and type(n_tokens) is type(BM) is type(NE) is type(D_HIDDEN) is type(D_INTER) is type(BN) is type(BK) is int and
+            isinstance(m_indices, torch.Tensor) and isinstance(sorted_expert_ids, torch.Tensor)):
         plan = _gemm1_plan(n_tokens, BM, NE, D_HIDDEN, D_INTER, BN, BK, bool(inline_quant), bool(interleave), a_dtype, m_indices.numel(), sorted_expert_ids.numel())
         if plan is not None:
             a = (hidden_states,) if inline_quant else (a_quant, a_scale_sorted_shuffled)
@@ -171,7 +172,8 @@ def flydsl_mxfp4_gemm2(*, inter_sorted_quant, inter_sorted_shuffled_scale, w2_u8
                        D_INTER, topk, flat_out_scale=None, D_INTER_REAL=None, BN=256, BK=256, xcd_swizzle=0, stream=None):
     """Stage 2.  ``flat_out`` is ``[M_logical, D_HIDDEN]`` (atomic; zeroed by the caller) or ``[max_sorted, D_HIDDEN]``
     (nonatomic), bf16 or fp16.  Returns ``flat_out``."""
-    if stream is not None and D_INTER_REAL is None and type(M_logical) is type(max_sorted) is type(BM) is type(NE) is type(D_HIDDEN) is type(D_INTER) is type(topk) is type(BN) is type(BK) is int:
+    if (stream is not None and D_INTER_REAL is None and type(M_logical) is type(max_sorted) is type(BM) is type(NE) is type(D_HIDDEN) is type(D_INTER) is type(topk) is
+            type(BN) is type(BK) is int and type(epilog) is str and isinstance(flat_out, torch.Tensor) and isinstance(sorted_expert_ids, torch.Tensor)):
         numbers = (M_logical, max_sorted, BM, NE, D_HIDDEN, D_INTER, topk, BN, BK, epilog, flat_out.dtype, sorted_expert_ids.numel())
         plan = _gemm2_plan(*numbers)
         if plan[2] is not _lib.lib().psg_moe_rows_workspace_bytes:

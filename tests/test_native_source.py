@@ -65,3 +65,31 @@ with pytest.raises(TypeError, match="device tensor"):
 """
     done = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.dirname(flydsl_amd.__file__)), capture_output=True, text=True)
     assert done.returncode == 0, done.stderr
+
+
+def test_operands_that_are_no_tensors_get_the_errors_of_the_checks():
+    import pytest
+    import torch
+
+    from flydsl_amd.kernels.moe.moe_gemm_2stage import compile_moe_gemm1
+    from flydsl_amd.kernels.moe.moe_sorting import moe_softmax_sort_flydsl
+    from flydsl_amd.kernels.moe.mxfp_moe import flydsl_mxfp4_gemm1, flydsl_mxfp4_gemm2
+
+    t = torch.zeros(64, dtype=torch.int32)
+    stage = compile_moe_gemm1(model_dim=256, inter_dim=128, experts=2, topk=1, tile_m=16, tile_n=64, tile_k=128, doweight_stage1=False, in_dtype="int8")
+    for ids in (None, [0, 1], 4096):
+        with pytest.raises(ValueError, match="device"):
+            stage(t, t, t, t, t, ids, t, t, t, 3, 128, 256, 2, 7)
+        with pytest.raises(ValueError, match="device tensor"):
+            moe_softmax_sort_flydsl(torch.zeros(4, 8), ids, t, t, t, None, 8, 2, "f32", stream=7)
+        kw = dict(cumsum_tensor=t, BM=32, NE=2, D_HIDDEN=256, D_INTER=256, topk=1, stream=7)
+        u8 = t.view(torch.uint8)
+        with pytest.raises(TypeError, match="m_indices"):
+            flydsl_mxfp4_gemm1(a_quant=u8, a_scale_sorted_shuffled=u8, w1_u8=u8, w1_scale_u8=u8, sorted_expert_ids=t, m_indices=ids, inter_sorted_quant=u8,
+                               inter_sorted_shuffled_scale=u8, n_tokens=3, **kw)
+        with pytest.raises(TypeError, match="device tensor"):
+            flydsl_mxfp4_gemm2(inter_sorted_quant=u8, inter_sorted_shuffled_scale=u8, w2_u8=u8, w2_scale_u8=u8, sorted_expert_ids=ids, sorted_token_ids=t, sorted_weights=t,
+                               flat_out=t.bfloat16(), M_logical=3, max_sorted=64, epilog="atomic", **kw)
+    with pytest.raises(NotImplementedError):
+        flydsl_mxfp4_gemm2(inter_sorted_quant=u8, inter_sorted_shuffled_scale=u8, w2_u8=u8, w2_scale_u8=u8, sorted_expert_ids=t, sorted_token_ids=t, sorted_weights=t,
+                           flat_out=t.bfloat16(), M_logical=3, max_sorted=64, epilog=["atomic"], **kw)
