@@ -156,7 +156,7 @@ def launch_gemm(
                               int(_force_path), None if _tile is None else (int(_tile[0]), int(_tile[1])), int(_wave_layout), int(_splits), bool(_no_split))
     if _acc is None and stream is not None:
         tensors = (arg_c, arg_a, arg_b, arg_scale_a, arg_scale_b)
-        if need and hasattr(arg_c, "device"):
+        if need and getattr(arg_c, "is_cuda", False):  # (anything else the checks refuse, before scratch is asked for)
             tensors += (_lib.workspace(arg_c.device, need, _lib.stream_handle(stream), owner="mxfp4"),)
         rc = _lib._native.launch(_lib.address("psg_gemm_mxfp4"), native, ops, stream, *tensors)
         if rc != _lib._native.DECLINED:

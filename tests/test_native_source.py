@@ -93,3 +93,16 @@ def test_operands_that_are_no_tensors_get_the_errors_of_the_checks():
     with pytest.raises(NotImplementedError):
         flydsl_mxfp4_gemm2(inter_sorted_quant=u8, inter_sorted_shuffled_scale=u8, w2_u8=u8, w2_scale_u8=u8, sorted_expert_ids=t, sorted_token_ids=t, sorted_weights=t,
                            flat_out=t.bfloat16(), M_logical=3, max_sorted=64, epilog=["atomic"], **kw)
+
+
+def test_scratch_is_not_asked_for_before_the_output_is_looked_at():
+    import numpy as np
+    import pytest
+    import torch
+
+    from flydsl_amd.kernels.gemm.mxfp4_preshuffle import launch_gemm
+
+    u8 = torch.zeros(64, dtype=torch.uint8)
+    for c, error in ((u8, ValueError), (np.zeros(64), TypeError)):  # 33 x 992 x 14336 splits K and needs scratch
+        with pytest.raises(error):
+            launch_gemm(c, u8, u8, u8, u8, 33, 992, 7, 992, 14336, 64, 128, 256, "fp8", "bf16", "fp4", 1, -1, -1, -1, -1, -1, -1, 0, 0)
