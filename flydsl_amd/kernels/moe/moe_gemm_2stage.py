@@ -81,7 +81,7 @@ class MoeStage:
 
     def __call__(self, out, x, w, scale_x, scale_w, sorted_token_ids, sorted_expert_ids, sorted_weights, num_valid_ids,
                  tokens, dim0, dim1, blocks, stream=None):
-        if stream is not None and type(tokens) is type(blocks) is int and isinstance(sorted_token_ids, torch.Tensor) and (dim0, dim1) == ((self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)):
+        if stream is not None and type(tokens) is type(blocks) is type(dim0) is type(dim1) is int and isinstance(sorted_token_ids, torch.Tensor) and (dim0, dim1) == ((self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)):
             key = (tokens, blocks, sorted_token_ids.numel(), self.no_pairing)
             plan = self._plans.get(key)
             if plan is None or plan[2] is not self._lib.psg_moe_rows_workspace_bytes:

@@ -154,7 +154,8 @@ def moe_softmax_sort_flydsl(gating_logits, sorted_ids, sorted_weights, sorted_ex
     if gating_logits.dim() != 2 or gating_logits.shape[1] != int(num_experts):
         raise ValueError("gating_logits must be [tokens, num_experts]")
     if (stream is not None and num_local_tokens is None and expert_mask is None and type(num_experts) is type(topk) is type(unit_size) is int and
-            isinstance(sorted_ids, torch.Tensor) and isinstance(sorted_expert_ids, torch.Tensor)):
+            type(renormalize) in (bool, int) and isinstance(sorted_ids, torch.Tensor) and isinstance(sorted_expert_ids, torch.Tensor) and
+            (moe_buf is None or isinstance(moe_buf, torch.Tensor)) and (workspace is None or workspace is False or isinstance(workspace, torch.Tensor))):
         buf = moe_buf if moe_buf is not None and moe_buf.numel() else None
         ws = None if workspace is None or workspace is False else workspace
         plan = _routing_plan(gating_logits.shape[0], num_experts, topk, unit_size, dtype_str, bool(renormalize), sorted_ids.numel(), sorted_expert_ids.numel(),

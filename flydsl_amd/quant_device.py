@@ -33,7 +33,7 @@ def pertoken_quant(x: torch.Tensor, quant_dtype=torch.int8, stream=None, out=Non
     """Per-row symmetric quantisation on the device.  Returns ``(y [M,K] quant_dtype, scale [M,1] fp32)``.
     ``out=(y, scale)`` reuses caller-owned outputs (1-byte ``[M,K]`` and fp32 ``[M]`` / ``[M,1]``): no allocation, so the
     call can be recorded into a HIP graph."""
-    if out is not None and stream is not None and quant_dtype in _OUT_CODE:
+    if type(out) in (tuple, list) and len(out) == 2 and stream is not None and isinstance(quant_dtype, torch.dtype) and quant_dtype in _OUT_CODE:
         y, scale = out
         rc = _lib._native.quant_pertoken(_lib.address("psg_quant_pertoken"), x, y, scale, _OUT_CODE[quant_dtype], stream)
         if rc != _lib._native.DECLINED:
@@ -67,7 +67,7 @@ def per_1x32_f4_quant(x: torch.Tensor, shuffle: bool = True, stream=None, out=No
     ``ceil(M/32)*32`` rows x ``K/32``: in the GEMM's shuffled layout when ``shuffle`` (default), row-major otherwise.
     Finite inputs only: a NaN / Inf in a block does not give the reference's 0xFF scale byte (the block maximum drops
     NaN)."""
-    if out is not None and stream is not None:
+    if type(out) in (tuple, list) and len(out) == 2 and stream is not None and type(shuffle) in (bool, int):
         packed, scales = out
         rc = _lib._native.quant_mxfp4(_lib.address("psg_quant_mxfp4"), x, packed, scales, 1 if shuffle else 0, stream)
         if rc != _lib._native.DECLINED:

@@ -74,6 +74,7 @@ def test_operands_that_are_no_tensors_get_the_errors_of_the_checks():
     from flydsl_amd.kernels.moe.moe_gemm_2stage import compile_moe_gemm1
     from flydsl_amd.kernels.moe.moe_sorting import moe_softmax_sort_flydsl
     from flydsl_amd.kernels.moe.mxfp_moe import flydsl_mxfp4_gemm1, flydsl_mxfp4_gemm2
+    from flydsl_amd.quant_device import per_1x32_f4_quant, pertoken_quant
 
     t = torch.zeros(64, dtype=torch.int32)
     stage = compile_moe_gemm1(model_dim=256, inter_dim=128, experts=2, topk=1, tile_m=16, tile_n=64, tile_k=128, doweight_stage1=False, in_dtype="int8")
@@ -90,6 +91,22 @@ def test_operands_that_are_no_tensors_get_the_errors_of_the_checks():
         with pytest.raises(TypeError, match="device tensor"):
             flydsl_mxfp4_gemm2(inter_sorted_quant=u8, inter_sorted_shuffled_scale=u8, w2_u8=u8, w2_scale_u8=u8, sorted_expert_ids=ids, sorted_token_ids=t, sorted_weights=t,
                                flat_out=t.bfloat16(), M_logical=3, max_sorted=64, epilog="atomic", **kw)
+        with pytest.raises(ValueError, match="device tensor"):  # the clear buffer, the workspace; numbers that are no plain ones
+            moe_softmax_sort_flydsl(torch.zeros(4, 8), t, t, t, t, ids, 8, 2, "f32", workspace=False if ids is None else ids, stream=7)
+    with pytest.raises(ValueError, match="device tensor"):
+        moe_softmax_sort_flydsl(torch.zeros(4, 8), t, t, t, t, None, 8, 2, "f32", renormalize=t, stream=7)
+    with pytest.raises(ValueError, match="one element"):
+        stage(t, t, t, t, t, t, t, t, t, 3, t, 256, 2, 7)
+    x = torch.zeros(4, 64)
+    for out in (7, "y", t, {}):
+        with pytest.raises(ValueError, match="device tensor"):
+            pertoken_quant(x, torch.int8, stream=7, out=out)
+        with pytest.raises(ValueError, match="device tensor"):
+            per_1x32_f4_quant(x, stream=7, out=out)
+    with pytest.raises(ValueError, match="device tensor"):
+        pertoken_quant(x, [torch.int8], stream=7, out=(t, t))
+    with pytest.raises(ValueError, match="device tensor"):
+        per_1x32_f4_quant(x, shuffle=t, stream=7, out=(t, t))
     with pytest.raises(NotImplementedError):
         flydsl_mxfp4_gemm2(inter_sorted_quant=u8, inter_sorted_shuffled_scale=u8, w2_u8=u8, w2_scale_u8=u8, sorted_expert_ids=t, sorted_token_ids=t, sorted_weights=t,
                            flat_out=t.bfloat16(), M_logical=3, max_sorted=64, epilog=["atomic"], **kw)
