@@ -51,13 +51,14 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
-// 1 / (1 + exp2(t)).  The reciprocal instruction with one Newton step in place of the compiler's division: 1 + exp2(t) is at least 1, so
-// none of the division's scaling is needed.  Where exp2 overflows the reciprocal is 0 and has to stay 0: the step's factor is
-// bounded so that it is not infinity times zero.
-__device__ __forceinline__ float sigmoid_neg_log2(float t) {
-    const float d = 1.0f + __builtin_amdgcn_exp2f(t);
+// v / (1 + exp2(t)).  The reciprocal instruction with one Newton step in place of the compiler's division, on a quarter of the divisor: 1 +
+// exp2(t) reaches 2^128, whose reciprocal is below the normal range, where the instruction returns 0; its quarter ends at 2^126, whose
+// reciprocal is normal.  (Both quarters are exact but for |v| < 2^-124.)  Where exp2 overflows the reciprocal is 0 and has to stay 0:
+// the step's factor is bounded so that it is not infinity times zero.
+__device__ __forceinline__ float times_sigmoid_neg_log2(float v, float t) {
+    const float d = __builtin_fmaf(0.25f, __builtin_amdgcn_exp2f(t), 0.25f);
     const float r = __builtin_amdgcn_rcpf(d);
-    return __builtin_fmaf(__builtin_fmaf(-fminf(d, 0x1p126f), r, 1.0f), r, r);
+    return 0.25f * v * __builtin_fmaf(__builtin_fmaf(-fminf(d, 0x1p126f), r, 1.0f), r, r);
 }
 
 // bias / activation of the fused epilogue, fp32 in, fp32 out.  silu(v) = v * sigmoid(v); the tanh form of gelu is v * sigmoid(2 y)
@@ -68,10 +69,10 @@ __device__ __forceinline__ float epi_act(float v, float bias) {
     constexpr float kLog2e = 1.4426950408889634f;
     if constexpr (EPI != EPI_NONE) v = v + bias;
     if constexpr (EPI == EPI_BIAS_RELU) v = fmaxf(v, 0.0f);
-    if constexpr (EPI == EPI_BIAS_SILU) v = v * sigmoid_neg_log2(-kLog2e * v);
+    if constexpr (EPI == EPI_BIAS_SILU) v = times_sigmoid_neg_log2(v, -kLog2e * v);
     if constexpr (EPI == EPI_BIAS_GELU) {
         constexpr float c1 = -2.0f * 0.7978845608f * kLog2e, c3 = c1 * 0.044715f;
-        v = v * sigmoid_neg_log2(v * __builtin_fmaf(c3, v * v, c1));
+        v = times_sigmoid_neg_log2(v, v * __builtin_fmaf(c3, v * v, c1));
     }
     return v;
 }

@@ -56,3 +56,32 @@ def test_every_tile(kind, epilogue, out, half):
             assert ((c[:M].double() - v).abs() <= (half + 2.0 ** -16) * v.abs() + 2.0 ** -24 + 1e-6).all(), tile
         else:
             assert torch.equal(c[:M], v.to(tout)), tile
+
+
+@pytest.mark.parametrize("epilogue", ["bias_silu", "bias_gelu"])
+def test_far_negative_tail(epilogue):
+    """Divisors up to 2^128, whose reciprocals are below the normal range of fp32 while the product with v is not: silu(-88.5) = -3.3e-37."""
+    from flydsl_amd import layout
+    from kernels.gemm.preshuffle_gemm import compile_preshuffle_gemm
+
+    M, N, K = 277, 272, 128
+    bias = torch.zeros(N)
+    bias[:40] = torch.arange(-88.5, -68.5, 0.5)
+    bias[40:200] = torch.arange(-10.0, 0.0, 0.0625)
+    bias[200:206] = torch.tensor([-1e30, 1e30, 1e38, -0.0, 1e-37, -1e-37])
+    bias = bias.bfloat16().cuda()
+    v = bias.double().expand(M, N)
+    if epilogue == "bias_silu":
+        want, exponent = torch.where(v < -88.7, 0.0, v * torch.sigmoid(v)), v.abs()
+    else:
+        y = 0.7978845608 * (v + 0.044715 * v ** 3)
+        want, exponent = v * torch.sigmoid(2 * y), 2 * y.abs()
+        want = torch.where(exponent > 88.7, torch.where(v > 0, v, 0.0), want)  # the divisor is past 2^128
+    # half a unit of bf16, and 2^-23 times what goes into exp2 (two roundings), which is at most 128 where the result is not 0 or v
+    rel = 2.0 ** -8 + 2.0 ** -22 * (1 + exponent.clamp(max=128))
+    a, w = torch.zeros(M, K, device="cuda").to(torch.float8_e4m3fn), layout.shuffle_weight(torch.zeros(N, K, dtype=torch.int8, device="cuda")).view(torch.float8_e4m3fn)
+    fn = compile_preshuffle_gemm(N=N, K=K, tile_m=64, tile_n=128, tile_k=64, in_dtype="fp8", out_dtype="bf16", epilogue=epilogue)
+    for m, kw in [(M, dict(force_path=1, tile=tile, wave_layout=layout_)) for tile, layout_ in TILES] + [(16, dict(force_path=2)), (64, dict(force_path=2))]:
+        c = torch.empty(m, N, dtype=torch.bfloat16, device="cuda")
+        fn.launch_forced(c, a[:m], w, torch.ones(m, device="cuda"), torch.ones(N, device="cuda"), bias, m, N, torch.cuda.current_stream(), **kw)
+        assert ((c.double() - want[:m]).abs() <= rel[:m] * want[:m].abs()).all(), kw
