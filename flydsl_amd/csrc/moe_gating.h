@@ -34,6 +34,14 @@ __device__ __forceinline__ int gate_xchg(int v) {
 template <int S>
 __device__ __forceinline__ float gate_xchg(float v) { return __builtin_bit_cast(float, gate_xchg<S>(__builtin_bit_cast(int, v))); }
 
+// Between an access to LDS by one lane and one to the same place by another lane of its wavefront.  The hardware completes a wavefront's LDS
+// accesses in order, so it costs no instruction; the compiler, which orders a lane's own accesses only, has to be told.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 constexpr int GATE_KEEP = 16;  // winners per lane at most: topk <= experts <= 16 * lanes
 
 // f(0), f(1), ... f(n - 1) for a uniform n <= 6: one branch out of the chain instead of one around every step

@@ -23,7 +23,7 @@ __global__ void __launch_bounds__(256) k_topk_gating(MoeGatingParams p) {
             if (p.tei) p.tei[(size_t)t * p.topk + k] = k * p.tokens + t;
         }
     });
-    // (a token's lanes are neighbours in one wavefront, whose LDS accesses stay in order)
+    wave_lds_order();  // (a token's lanes are neighbours in one wavefront)
     if (live)
         for (int k = gl; k < p.topk; k += L) p.weights[(size_t)t * p.topk + k] = mine[k] * f;
 }

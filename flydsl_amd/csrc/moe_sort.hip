@@ -213,13 +213,14 @@ __device__ __forceinline__ void gate_tokens(const MoeGatingParams& g, int first,
                 if (g.tei) g.tei[q] = k * g.tokens + t;
             }
         });
-        // (a token's lanes are neighbours in one wavefront, whose LDS accesses stay in order)
+        wave_lds_order();  // (a token's lanes are neighbours in one wavefront)
         if (live && (held || store))
             for (int k = gl; k < g.topk; k += L) {
                 const float w = mine[k] * f;
                 if (held) mine[k] = w;
                 if (store && g.weights) g.weights[(size_t)t * g.topk + k] = w;
             }
+        if (!held) wave_lds_order();  // (the next pass stores its winners there)
     }
 }
 
@@ -541,8 +542,10 @@ __global__ void __launch_bounds__(SORT_THREADS) k_moe_sort_scatter(MoeSortParams
                 p.sorted_ids[row] = pack_id(slot, token);
                 p.sorted_weights[row] = wt[c];
             }
-            // every lane has read its base: now the first lane of each expert advances it (LDS operations of a wavefront complete in order)
+            // every lane has read its base: now the first lane of each expert advances it
+            wave_lds_order();
             if (ok[c] && below == 0) base[wave][id[c]] += __popcll(peers);
+            wave_lds_order();
         }
     }
 }
