@@ -57,7 +57,7 @@ __device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g));
 // of 16 or 32 rows: an expert with 17 to 32 routed rows would otherwise stream its weights once per block).  Blocks pair up
 // from the start of each run of equal expert ids: the workgroup of the second block of a pair ends at once, and the
 // first one treats the second half of its tile as padding when the run ends there.
-// DEEP: operands three steps ahead (the rule and its figures: takes_deep).
+// DEEP: operands three steps ahead (the rule and its figures: takes_deep; a stage by rows never, having more workgroups than that).
 // ROWS = MoeRowsParams: the down stage by rows, whose first `rows.wgs` rows of the grid make the lists of the tokens' rows.  A build of
 // its own: the decode layers, which add directly, lost 0.4 to 0.8 us of 55 to 140 to the longer arguments and the branch.
 template <int KIND, int MR, int NR, int STAGE, int CO, bool DEEP, class... ROWS>
@@ -380,8 +380,7 @@ hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int bl
         constexpr bool kOnly = MR_ == 4 && CO_ == 2;                 /* ... and with no other */         \
         if constexpr (STAGE == 2) {                                                                      \
             if (lists) {                                                                                 \
-                if (kHas && deep) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kHas, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
-                else hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, false, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
+                hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, false, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
                 return hipGetLastError();                                                                \
             }                                                                                            \
         }                                                                                                \

@@ -4,6 +4,8 @@ magnitude is exact in bf16 and fp16 and the results must be equal, whatever the 
 what the device has to find out by itself: tokens named more often than topk times, tokens without a row, padding ids in the
 middle of a block, blocks whose expert does not exist, and blocks past the rows in use."""
 
+import sys
+
 import pytest
 import torch
 
@@ -110,4 +112,25 @@ class _RealRule:
 
 @pytest.mark.parametrize("kind,tokens,topk,block,model,inter", [("mx", 410, 8, 64, 2048, 256), ("fp8", 515, 6, 128, 4096, 128), ("int8", 813, 4, 32, 4096, 128), ("int4", 410, 8, 64, 4096, 128)])
 def test_stage2_by_rows_where_the_library_takes_it(monkeypatch, kind, tokens, topk, block, model, inter):
+    test_stage2_by_rows_equals_the_exact_sum(_RealRule(monkeypatch), kind, tokens, topk, block, model, inter, torch.bfloat16)
+
+
+def _full_list(tokens, topk, experts, block, g):
+    """The list a sorter makes: every (token, slot) once, each expert's rows filled up to whole blocks."""
+    expert = torch.randint(0, experts, (tokens, topk), generator=g)
+    ids, eids = [], []
+    for e in range(experts):
+        rows = [(s << 24) | t for t, s in (expert == e).nonzero().tolist()]
+        rows += [tokens | (topk << 24)] * (-len(rows) % block)
+        ids += rows
+        eids += [e] * (len(rows) // block)
+    return ids, eids, len(ids)
+
+
+@pytest.mark.parametrize("kind,tokens,topk,block,model,inter", [
+    ("int4", 830, 8, 64, 2048, 256), ("int4", 830, 8, 128, 2048, 384), ("int8", 830, 8, 64, 2048, 384), ("fp8", 830, 8, 64, 2048, 256), ("fp8", 515, 6, 32, 4096, 128),
+    ("int8", 515, 6, 128, 4096, 128)])
+def test_stage2_by_rows_of_a_whole_layer(monkeypatch, kind, tokens, topk, block, model, inter):
+    """What an accumulating layer runs: all pairs in the list, more than two workgroups a CU on 128-column tiles."""
+    monkeypatch.setattr(sys.modules[__name__], "_sorted_list", _full_list)
     test_stage2_by_rows_equals_the_exact_sum(_RealRule(monkeypatch), kind, tokens, topk, block, model, inter, torch.bfloat16)

@@ -58,3 +58,30 @@ def test_planned_tile(fmt, M, N, K, batch):
             assert torch.equal(c[0], acc[0].bfloat16())
     # the two fp32 sums may round to neighbouring bf16 values
     assert ((c.float() - ref_c.float()).abs() <= 2.0 ** -7 * ref_c.float().abs() + 1e-5 * ref_c.float().abs().max()).all()
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [("fp8",) + s for s in [  # 32x128, 64x128, 64x256, 128x256, 256x256 tiles
+    (39, 32, 256), (101, 8416, 1024), (641, 9376, 512), (836, 8768, 1280), (1220, 9824, 1024)]] + [(f,) + s for f in ("fp8-fp4", "fp6-fp4") for s in [  # and 32x256
+        (59, 32, 256), (393, 10048, 256), (644, 8864, 512), (802, 8736, 512), (554, 22080, 512), (1185, 10080, 256)]])
+def test_planned_tile_in_fp16(fmt, M, N, K):
+    """Builds of their own.  The scales keep the sums finite in fp16: 1280 products of up to 448 x 448 x 2^-18, 512 of 448 x 6 x 2^-7."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(N)
+
+    def data(lo, hi, *shape):
+        return torch.randint(lo, hi, shape, generator=g, device="cuda", dtype=torch.uint8)
+
+    fa, fb = (fmt, fmt) if "-" not in fmt else fmt.split("-")
+    a, b = data(0, 127, M, K), data(0, 127, N, K) if fb == "fp8" else data(0, 256, N, K // 2)
+    a[..., ::3] |= 128
+    sa, sb = data(112, 119, (M + 31) // 32 * K), data(112, 119, N // 32 * K) if fb == "fp8" else data(124, 130, N // 32 * K)
+    out = []
+    for path in (0, 3):
+        c = torch.full((M + 64, N), -8192.0, dtype=torch.float16, device="cuda")
+        launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, fa, "fp16", fb, 1, -1, -1, -1, -1, -1, -1, 0, 0, _force_path=path)
+        assert (c[M:] == -8192.0).all()
+        out.append(c[:M].float())
+    c, ref = out
+    assert ref.isfinite().all() and ref.abs().max() > 0.05
+    # two fp32 sums of different order, each rounded to fp16 (subnormal from 2^-14 down)
+    assert ((c - ref).abs() <= 2.0 ** -10 * ref.abs() + 2.0 ** -24 + 1e-5 * ref.abs().max()).all()
