@@ -361,16 +361,14 @@ template <int KIND, int STAGE, int NR>
 hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int blocks, bool pair, hipStream_t stream) {
     const unsigned nx = (unsigned)((p.n_out + 64 * NR - 1) / (64 * NR));
     rows.wgs = 0;
-    bool lists = STAGE == 2 && p.by_position;
+    // rows of the grid for the lists, as far as it has any left (65535 of them)
+    const int list_rows = (int)((ROWS_INDEX_WGS + nx - 1) / nx);
+    const bool lists = STAGE == 2 && p.by_position && rows.sorted_size <= moe_rows_share_max(block_m) && blocks + list_rows <= 65535;
     if (lists) {
-        // rows of the grid for the lists, as far as it has any left (65535 of them)
-        rows.wgs = (int)((ROWS_INDEX_WGS + nx - 1) / nx);
-        if (blocks + rows.wgs > 65535) {
-            rows.wgs = 0;
-            lists = false;
-            const hipError_t e = psg_launch_moe_rows_index(rows, stream);
-            if (e != hipSuccess) return e;
-        }
+        rows.wgs = list_rows;
+    } else if (STAGE == 2 && p.by_position) {
+        const hipError_t e = psg_launch_moe_rows_index(rows, stream);
+        if (e != hipSuccess) return e;
     }
     const bool deep = takes_deep<KIND, STAGE>(p, block_m, blocks, (int)nx);
     const dim3 grid(nx, blocks + rows.wgs, 1);

@@ -29,10 +29,27 @@ struct MoeRowsParams {
 // 93; 4096 x top-8 602 / 596; fp8 on 256-row tiles, which the power limit bounds, 807 / 809.)  A multiple of 8 leaves every tile on its XCD.
 constexpr int ROWS_INDEX_WGS = 32;
 
+// Every one of those workgroups looks through the whole list, so their work grows with its square; longer lists are made by two launches over
+// all CUs.  Beside the tiles of k_moe_gemm that is better from about 50,000 sorted rows on with blocks of 16 and 32 rows, 120,000 with 64 and 128 (us
+// beside the tiles / two launches, top-8 on 32 experts, 2048 x 512, fp8: blocks of 16 6000 tokens 249 / 247, 8192 356 / 350, 30000 1329 / 1293; of 32 8192 283 /
+// 282, 16384 582 / 574; of 64 8192 250 / 251, 12000 372 / 371, 16384 515 / 508, 30000 935 / 917; int4, 1024 x 256, 14000 tokens, blocks of 16, 64 and 128 268 / 263, 177 /
+// 179, 184 / 189); beside the MX pair's, with their 16 ids a thread, it never is (16384 tokens 394 / 402, 65536 1490 / 1492).  As a launch of their own, of 1024
+// threads a workgroup, the shares are the faster way up to about 40,000 rows (4096 tokens 8 / 9.5; stage 2 in blocks of 128 16384 tokens 570 / 563).
+inline int moe_rows_share_max(int block_m) { return block_m <= 32 ? 50000 : 120000; }
+constexpr int ROWS_LAUNCH_MAX = 40000;
+
 uint64_t psg_moe_rows_bytes(int64_t tokens, int64_t topk, int64_t sorted_size, int64_t dim);
 void psg_moe_rows_carve(MoeRowsParams& p, void* workspace);
 hipError_t psg_launch_moe_rows_index(const MoeRowsParams& p, hipStream_t stream);
 hipError_t psg_launch_moe_rows_add(const MoeRowsParams& p, hipStream_t stream);
+
+// the rows the stage computes: whole tiles up to num_valid, in blocks that are in the list
+__device__ __forceinline__ int moe_rows_limit(const MoeRowsParams& p) {
+    const int nv = p.num_valid[0];
+    int limit = nv >= p.sorted_size ? p.sorted_size : nv <= 0 ? 0 : (nv + p.granule - 1) / p.granule * p.granule;
+    if (limit > p.sorted_size) limit = p.sorted_size;
+    return (int64_t)p.blocks * p.block_m < limit ? p.blocks * p.block_m : limit;
+}
 
 // Share `wg` of `wgs` of the lists: a range of tokens, for which it looks through the whole sorted list (16 to 600 KB out of L2).  The counts stay in
 // LDS (`lds`, two ints a token, `lds_ints` in all), so nothing has to be cleared before.
@@ -45,11 +62,7 @@ __device__ __forceinline__ void moe_rows_index_share(const MoeRowsParams& p, int
     const int cap = lds_ints / 2;
     int* cnt = lds;
     int* head = lds + cap;
-    // the rows the stage computes: whole tiles up to num_valid, in blocks that are in the list
-    const int nv = p.num_valid[0];
-    int limit = nv >= p.sorted_size ? p.sorted_size : nv <= 0 ? 0 : (nv + p.granule - 1) / p.granule * p.granule;
-    if (limit > p.sorted_size) limit = p.sorted_size;
-    if ((int64_t)p.blocks * p.block_m < limit) limit = p.blocks * p.block_m;
+    const int limit = moe_rows_limit(p);
     const int sh = __builtin_ctz(p.block_m);
     for (int t0 = first; t0 < last; t0 += cap) {
         const int n = last - t0 < cap ? last - t0 : cap;

@@ -5,7 +5,7 @@
 // model 4096, i.e. 268 MB of additions: fp8 stage 2 434 us, MX-FP4 436), a store and a read of the same rows at 5.  So `topk`
 // additions per output element become one; that one stays atomic, because launches on other streams may be adding into `out` too.
 //
-// Which sorted rows belong to a token is found on the device, by workgroups beside the stage's tiles (moe_rows_index_share), so any sorted
+// Which sorted rows belong to a token is found on the device, by workgroups beside the stage's tiles (moe_rows_index_share) or in launches in front, so any sorted
 // list the atomic epilogue accepts works here: rows are entered into a list of `topk` places per token, and rows that do not fit (a
 // list that names a token more often than topk times) are chained behind its last entry.
 #include "psg_common.h"
@@ -26,6 +26,25 @@ __device__ __forceinline__ void add_packed(uint32_t* o, int bits, int out_dtype)
 __global__ void __launch_bounds__(1024) k_moe_rows_index(MoeRowsParams p) {
     __shared__ int lds[4096];
     moe_rows_index_share<16>(p, (int)blockIdx.x, (int)gridDim.x, lds, 4096);
+}
+
+// The same lists by all CUs, from counts and heads in memory (a list's last place is the head of its chain).
+__global__ void __launch_bounds__(256) k_moe_rows_clear(MoeRowsParams p) {
+    const int t = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (t >= p.tokens) return;
+    p.count[t] = 0;
+    p.list[(size_t)t * p.topk + p.topk - 1] = -1;
+}
+__global__ void __launch_bounds__(256) k_moe_rows_enter(MoeRowsParams p) {
+    const int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (i >= moe_rows_limit(p) || (unsigned)p.expert_ids[i / p.block_m] >= (unsigned)p.experts) return;
+    const uint32_t id = (uint32_t)p.sorted_ids[i];
+    const int t = (int)(id & 0xFFFFFFu);
+    if (t >= p.tokens || (int)(id >> 24) >= p.slots) return;
+    const int k = atomicAdd(&p.count[t], 1);
+    int* list = p.list + (size_t)t * p.topk;
+    if (k < p.topk - 1) list[k] = i;
+    else p.next[i] = atomicExch(&list[p.topk - 1], i);
 }
 
 template <int OUT>
@@ -91,9 +110,14 @@ void psg_moe_rows_carve(MoeRowsParams& p, void* workspace) {
     p.next = reinterpret_cast<int*>(w);
 }
 
-// the lists in a launch of their own, for the stages that do not make them beside their tiles
+// the lists in launches of their own, for the stages that do not make them beside their tiles
 hipError_t psg_launch_moe_rows_index(const MoeRowsParams& p, hipStream_t stream) {
-    hipLaunchKernelGGL(k_moe_rows_index, dim3(ROWS_INDEX_WGS), dim3(1024), 0, stream, p);
+    if (p.sorted_size <= ROWS_LAUNCH_MAX) {
+        hipLaunchKernelGGL(k_moe_rows_index, dim3(ROWS_INDEX_WGS), dim3(1024), 0, stream, p);
+    } else {
+        hipLaunchKernelGGL(k_moe_rows_clear, dim3((p.tokens + 255) / 256), dim3(256), 0, stream, p);
+        hipLaunchKernelGGL(k_moe_rows_enter, dim3((p.sorted_size + 255) / 256), dim3(256), 0, stream, p);
+    }
     return hipGetLastError();
 }
 

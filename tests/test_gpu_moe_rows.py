@@ -6,6 +6,7 @@ middle of a block, blocks whose expert does not exist, and blocks past the rows 
 
 import sys
 
+import numpy as np
 import pytest
 import torch
 
@@ -134,3 +135,29 @@ def test_stage2_by_rows_of_a_whole_layer(monkeypatch, kind, tokens, topk, block,
     """What an accumulating layer runs: all pairs in the list, more than two workgroups a CU on 128-column tiles."""
     monkeypatch.setattr(sys.modules[__name__], "_sorted_list", _full_list)
     test_stage2_by_rows_equals_the_exact_sum(_RealRule(monkeypatch), kind, tokens, topk, block, model, inter, torch.bfloat16)
+
+
+@pytest.mark.parametrize("kind,tokens,topk,block,model,inter,rows", [
+    ("int8", 9001, 3, 16, 64, 128, 50000), ("int4", 12347, 5, 32, 192, 128, 50000), ("fp8", 30011, 2, 64, 64, 128, 120000), ("fp8", 9001, 6, 128, 256, 256, 56000), ("mx", 9001, 3, 64, 256, 256, 130000)])
+def test_long_lists(monkeypatch, kind, tokens, topk, block, model, inter, rows):
+    """Lists that are made in launches of their own, by all CUs, and the longest the MX pair makes beside its tiles: more rows of some tokens than topk, tokens without one."""
+
+    def long_list(tokens, topk, experts, block, g):
+        ids, eids = [], []
+        for e in range(experts):
+            n = rows // experts + int(torch.randint(1, 2 * block, (1,), generator=g))
+            t = torch.randint(0, tokens - 1, (n,), generator=g)
+            t[:97 * 12:97] = t[0]  # (a dozen times from each of three experts: at most 36 rows of one token, whose sum stays below 256)
+            t[::101] = tokens  # padding
+            if e != 1:
+                t[5::7] = t[5]
+                t[5::7][2:] = tokens
+            s = torch.randint(0, topk, (n,), generator=g)
+            blk = torch.where(t == tokens, t, (s << 24) | t).tolist()
+            blk += [tokens | (topk << 24)] * (-len(blk) % block)
+            ids += blk
+            eids += [e if e != 1 else experts + 5] * (len(blk) // block)
+        return np.array(ids + [0] * block), eids + [0], len(ids)  # (an array: the comparison makes a tensor of it for every block)
+
+    monkeypatch.setattr(sys.modules[__name__], "_sorted_list", long_list)
+    test_stage2_by_rows_equals_the_exact_sum(monkeypatch, kind, tokens, topk, block, model, inter, torch.bfloat16)
