@@ -345,21 +345,36 @@ int mx_general_splits(int M, int N, int K) {
     return s;
 }
 
-// Whether dense, unbatched fp8 x fp8 and fp8 / fp6 x fp4 run on the tiles of the dense kernels: beyond 32 rows everywhere except where the small-M
-// kernel's workgroups make one round of the CUs (N / 32 times the 64-row groups; an eighth more on short rows, whose second round is soon
-// over), and where the general kernel splits K (`room`: the caller brought the workspace) and the splits make one round.  Against what ran there
-// (small-M or general kernel), over 208 and 250 problems of 33 to 8192 rows, fp8 x fp8 is 16 % faster on average, fp8 / fp6 x fp4 20 % (us tiles /
-// before: fp8 x fp8 383x12384x6912 49.8 / 90.5, 365x10336x2304 15.9 / 27.0, 1164x2880x4096 23.2 / 37.1, 128x512x4096 12.6 / 17.7, 4096x1024x512 8.1 /
-// 10.1; small-M, two rounds, 389x1984x4352 14.5 / 21.0, 64x8224x2048 8.9 / 9.7, 33x16384x4096 15.0 / 18.7; one round 228x1056x9216 25.7 / 18.6,
-// 64x8192x4096 13.8 / 10.5; splits 33x992x14336 37.0 / 19.3, 87x8160x12032 33.4 / 29.6, more than one round of them 67x9568x8960 26.3 / 36.7;
-// fp8 x fp4 591x8032x5632 33.4 / 51.5, 812x8000x3584 27.3 / 42.0; fp6 x fp4 293x14656x1280 12.1 / 19.0, 6322x1024x4608 30.3 / 48.0, 1040x13696x6144
-// 66 / 113).  Up to 32 rows the small-M kernel is the better one (fp8 x fp8 32x12288x4096 13.6 / 14.2 on tiles).
-bool mx_takes_tiles(int M, int N, int K, bool fp8_weights, bool room) {
-    if (M <= kSmallM) return false;
+// Where a dense, unbatched fp8 x fp8 or fp8 / fp6 x fp4 problem runs: on the small-M kernel, on the general kernel with its K splits (`room`: the caller
+// brought their workspace), or on the tiles of the dense kernels.  Up to 32 rows on the first two (fp8 x fp8 32x12288x4096 13.6 / 14.2 on tiles).
+// Beyond that the small-M kernel, whose N / 32 workgroups for every 64 rows stream W best, while they make one round of the CUs; the tiles read W
+// from the last-level cache faster than that, but from memory slower, so in the second round it depends.  The lines are from 900 problems of 33 to 400 rows,
+// 200 to 1100 such workgroups and K 1024 to 14336, each with W in memory and with W in that cache (us small-M / splits / tiles, memory; cache):
+//   short rows, fp4 weights: two rounds of the small-M kernel (68x5120x1280 5.4 / 8.3 / 6.8; 5.2 / 8.1 / 5.5, 106x6432x1792 7.3 / 10.1 / 8.5; 6.7 / 9.9 / 7.0);
+//     fp8 weights an eighth of a round more than one
+//   splits, up to 64 rows while they make at most two workgroups a CU, beyond at most one: fp8 x fp8 42x8544x10240 33.0 / 30.5 / 40.0;
+//     31.5 / 24.5 / 29.1, 48x10400x13312 43.3 / 40.6 / 52.6; 40.8 / 32.1 / 36.2, 75x5216x10752 33.7 / 30.5 / 40.0; 32.3 / 26.3 / 29.2; fp8 x fp4 38x10112x9984
+//     24.7 / 21.2 / 33.2; 23.7 / 18.6 / 24.2; but more of them fp8 x fp8 67x9568x8960 - / 36.6 / 36.3; - / 36.0 / 25.7.
+//     With fp4 weights and at most one workgroup a CU, or without the workspace, the small-M kernel is as good or better: 38x12992x6912 19.4 / 20.6 / 24.5;
+//     18.6 / 18.6 / 18.3, 47x11456x8448 23.0 / 24.1 / 29.3; 22.2 / 21.0 / 21.4
+//   long rows of fp4 weights in the second round: 94x6400x7424 20.5 / 30.4 / 25.3; 17.1 / 26.7 / 18.4, 149x3040x6912 17.6 / 27.4 / 23.6; 17.3 / 26.1 / 17.0, 140x4480x7680
+//     23.2 / 31.4 / 25.9; 21.1 / 27.5 / 18.5
+//   everything else on tiles (33x9184x3072 10.7 / 13.9 / 12.3; 9.7 / 13.3 / 9.4, 40x15456x3840 18.7 / 23.2 / 21.4; 16.7 / 17.4 / 13.7, 65x13664x12032 56 / 38 /
+//     43.6; 55 / 36 / 31.5; three rounds or more always, where against the general kernel 1164x2880x4096 takes 23.2 / 37.1, 591x8032x5632 33.4 / 51.5)
+enum MxRoute { MX_SMALL, MX_GENERAL, MX_TILES };
+MxRoute mx_route(int M, int N, int K, bool fp8_weights, bool room) {
+    const bool holds = mx_general_small(M, N, K, false, fp8_weights, 1);
+    if (M <= kSmallM) return holds ? MX_SMALL : MX_GENERAL;
     const long cus = psg_cu_count(), groups = (M + 63) / 64, wgs = (long)(N / 32) * groups;
-    if ((K < 1536 ? wgs * 8 <= cus * 9 : wgs <= cus) && mx_general_small(M, N, K, false, fp8_weights, 1)) return false;
+    const bool small = holds && wgs <= 2 * cus;
+    if (small && (K >= 2048 ? wgs <= cus : fp8_weights ? wgs * 8 <= cus * 9 : true)) return MX_SMALL;
     const int splits = mx_general_splits(M, N, K);
-    return !(room && splits > 1 && groups * ((N + 127) / 128) * splits <= cus);
+    const long split_wgs = groups * ((N + 127) / 128) * splits;
+    if (splits > 1 && split_wgs <= (M <= kStreamMaxM ? 2 : 1) * cus) {
+        if (small && (!room || (!fp8_weights && split_wgs <= cus))) return MX_SMALL;
+        return room ? MX_GENERAL : MX_TILES;
+    }
+    return small && !fp8_weights && K >= 6144 ? MX_SMALL : MX_TILES;
 }
 
 // Tile + split plan of the tiled path.  With few tiles and a long K (the regime between the streaming kernel and
@@ -582,6 +597,14 @@ const char* psg_last_error(void) { return g_err; }
 uint64_t psg_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t in_dtype) {
     // Only the split-K variant of the tiled path (few tiles, long K) uses global scratch: one fp32 / int32 slice of
     // [M,N] per split.  Without it (NULL or too small) the library runs the same problem unsplit.
+    if (in_dtype >= 16) {  // psg_gemm_mxfp4, whichever kernel takes the pair of formats
+        const int fa = (in_dtype - 16) >> 2, fb = (in_dtype - 16) & 3;
+        if (M < 1 || N < 32 || K < 256 || fa > PSG_MX_FP8 || (fb != PSG_MX_FP4 && fb != PSG_MX_FP8)) return 0;
+        if (fa == PSG_MX_FP4 && fb == PSG_MX_FP4) return psg_workspace_bytes(M, N, K, 4);
+        const bool planned = fb == PSG_MX_FP4 || fa == PSG_MX_FP8;
+        if (planned ? mx_route(M, N, K, fb == PSG_MX_FP8, true) != MX_GENERAL : mx_general_small(M, N, K, fa == PSG_MX_FP4, fb == PSG_MX_FP8, 1)) return 0;
+        return splitk_bytes(M, N, mx_general_splits(M, N, K));
+    }
     if (in_dtype == 5) return M >= 1 && N >= 32 && K >= 256 ? splitk_bytes(M, N, mx_general_splits(M, N, K)) : 0;  // general MX kernel
     if (M <= kSmallM || M < 1 || N < 16 || K < 64) return 0;
     const bool mx = in_dtype == 4;  // MXFP4 (psg_gemm_mxfp4)
@@ -687,23 +710,22 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
     const bool dense = a_rs == a_row && c_rs == (uint64_t)a->N && sa_cs == chunk;
     const bool fp4_fast = a->a_dtype == PSG_MX_FP4 && a->b_dtype == PSG_MX_FP4 && batch == 1 && dense;
     const bool fp8_pair = a->a_dtype == PSG_MX_FP8 && a->b_dtype == PSG_MX_FP8 && batch == 1 && dense;
+    const bool w4 = a->b_dtype == PSG_MX_FP4 && a->a_dtype != PSG_MX_FP4;
     // what the general kernel's split-K plan needs is there
     const bool room = store == STORE_C && a->workspace && aligned(a->workspace, 16) && a->workspace_bytes >= splitk_bytes(a->M, a->N, mx_general_splits(a->M, a->N, a->K));
-    const bool fp8_tiled = fp8_pair && (a->force_path == 1 || (a->force_path == 0 && mx_takes_tiles(a->M, a->N, a->K, true, room)));
+    const bool routed = a->force_path == 0 && (fp8_pair || (w4 && batch == 1 && dense && store == STORE_C));
+    const MxRoute route = routed ? mx_route(a->M, a->N, a->K, fp8_pair, room) : MX_GENERAL;
     if (a->force_path == 2 && !fp4_fast) return fail(PSG_E_SHAPE, "force_path=2 is for dense, unbatched fp4 x fp4 only");
     if (a->force_path == 1 && !fp4_fast && !fp8_pair)
         return fail(PSG_E_SHAPE, "force_path=1 is for dense, unbatched fp4 x fp4 or fp8 x fp8 only");
     if (a->force_path == 2 && a->M > kStreamMaxM) return fail(PSG_E_SHAPE, "small-M path needs M <= %d, got %d", kStreamMaxM, a->M);
-    // fp8 / fp6 x fp4, and batches of these and of the fp4 and fp8 pairs: a launch of the dense tiles per batch
+    // batches of the fp4 and fp8 pairs and of fp8 / fp6 x fp4: a launch of the dense tiles per batch
     const int64_t a_bs = a->a_batch_stride ? a->a_batch_stride : (int64_t)((uint64_t)a->M * a_rs);
     const int64_t c_bs = a->c_batch_stride ? a->c_batch_stride : (int64_t)((uint64_t)a->M * c_rs * 2);
     const int64_t sa_bs = a->scale_a_batch_stride ? a->scale_a_batch_stride : (int64_t)((uint64_t)((a->M + 31) / 32) * sa_cs);
-    const bool w4 = a->b_dtype == PSG_MX_FP4 && a->a_dtype != PSG_MX_FP4;
-    const bool same = a->b_dtype == a->a_dtype && batch > 1;
-    const bool per_batch = (w4 || same) && dense && store == STORE_C && a->force_path == 0 && batch <= 8 &&
-                           (batch == 1 ? mx_takes_tiles(a->M, a->N, a->K, false, room) : mx_fills_tiles(a->M, a->N)) && a_bs % 16 == 0 &&
-                           c_bs % 16 == 0 && sa_bs % 4 == 0;
-    if (fp8_tiled || per_batch) {
+    const bool per_batch = (w4 || a->b_dtype == a->a_dtype) && batch > 1 && dense && store == STORE_C && a->force_path == 0 && batch <= 8 && mx_fills_tiles(a->M, a->N) &&
+                           a_bs % 16 == 0 && c_bs % 16 == 0 && sa_bs % 4 == 0;
+    if (route == MX_TILES || per_batch || (fp8_pair && a->force_path == 1)) {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
         const bool fp4 = a->a_dtype == PSG_MX_FP4;
         const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : pick_mx_tile(a->M, a->N, fp4 ? a->K / 2 : a->K, fp4 ? MX_FP4 : w4 ? MX_W4 : MX_FP8);
@@ -757,7 +779,8 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         g.sa_batch = sa_bs;
         g.sb_batch = (int64_t)((uint64_t)(a->N / 32) * chunk);
         hipError_t ge;
-        const bool small = store == STORE_C && a->force_path == 0 && mx_general_small(a->M, a->N, a->K, a->a_dtype == PSG_MX_FP4, a->b_dtype == PSG_MX_FP8, batch);
+        const bool small = store == STORE_C && a->force_path == 0 &&
+                           (routed ? route == MX_SMALL : mx_general_small(a->M, a->N, a->K, a->a_dtype == PSG_MX_FP4, a->b_dtype == PSG_MX_FP8, batch));
         const int splits = !small && batch == 1 && c_rs == (uint64_t)a->N && store == STORE_C ? mx_general_splits(a->M, a->N, a->K) : 1;
         if (small) {
             ge = psg_launch_mx_smallm(g, a->a_dtype, a->b_dtype, batch, static_cast<hipStream_t>(stream));

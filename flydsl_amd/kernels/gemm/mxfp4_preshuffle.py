@@ -97,7 +97,7 @@ def _plan(M, i32_n, N, K, tile_m, tile_n, tile_k, a_dtype, out_dtype, b_dtype, B
         else:
             need = lib.psg_workspace_bytes(args.M, args.N, args.K, 4)
     elif B == 1 and c_rs == Nn and not no_split:
-        need = lib.psg_workspace_bytes(args.M, args.N, args.K, 5)
+        need = lib.psg_workspace_bytes(args.M, args.N, args.K, 5 if force_path else 16 + 4 * args.a_dtype + args.b_dtype)
     else:
         need = 0
     ops = [(getattr(_lib.MxArgs, name), 0, _lib.TYPE_ANY, n) for name, n in zip(("c", "a", "b", "scale_a", "scale_b"), needs)]

@@ -135,9 +135,10 @@ enum psg_mx_dtype { PSG_MX_FP4 = 0, PSG_MX_FP6 = 1, PSG_MX_FP8 = 2,
  * ceil(M/32) chunks for scale_a).  W and scale_b are always batch-dense (mxfp4_preshuffle.py:177-193).  Batch z reads
  * a + z*a_batch_stride etc. (bytes) and all batches run in ONE launch (grid.z = batch).
  * Which kernel runs: fp4 x fp4 with batch 1 and dense strides takes the tuned fp4 kernels (tiled mainloop, small-M
- * split-K; workspace / tile_* / force_path 1, 2 apply to them only); everything else is planned from its sizes (dense fp8 x fp8 and
- * fp8 / fp6 x fp4 of more than 32 rows mostly on such tiles, few rows on the small-M MX kernel); the rest, or force_path 3, takes the general kernel, which ignores the tile arguments and uses workspace (psg_workspace_bytes(M, N, K, 5) bytes) for
- * split-K when batch is 1 and C is dense.
+ * split-K; tile_* / force_path 1, 2 apply to them only); everything else is planned from its sizes (dense fp8 x fp8 and
+ * fp8 / fp6 x fp4 of more than 32 rows mostly on such tiles, few rows on the small-M MX kernel); the rest, or force_path 3, takes the general
+ * kernel, which ignores the tile arguments and uses workspace for split-K when batch is 1 and C is dense (psg_workspace_bytes says how much, and
+ * that it is 0 where another kernel takes the problem; without it nothing is split).
  */
 typedef struct psg_mxfp4_args {
     void *c;
@@ -172,8 +173,9 @@ int psg_abi_version(void);
 const char *psg_last_error(void);
 
 /* Bytes of workspace the split-K plan would use for this problem (0 when the chosen plan needs none).
- * in_dtype: enum psg_in_dtype, 4 for psg_gemm_mxfp4 on its fp4 x fp4 kernels, 5 for psg_gemm_mxfp4 on the general MX
- * kernel (any other format pair, or force_path 3; batch 1 and dense C only, otherwise it runs unsplit). */
+ * in_dtype: enum psg_in_dtype; 16 + 4 * a_dtype + b_dtype (enum psg_mx_dtype) for psg_gemm_mxfp4 on dense operands, batch 1 and
+ * force_path 0; 4 for its fp4 x fp4 kernels, 5 for the general MX kernel (force_path 3; more than one batch or a C that is not dense run
+ * unsplit). */
 uint64_t psg_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t in_dtype);
 
 /* C = epilogue((acc * scale_a[m]) * scale_b[n]) on `stream` (a hipStream_t passed as void*). */

@@ -85,3 +85,28 @@ def test_planned_tile_in_fp16(fmt, M, N, K):
     assert ref.isfinite().all() and ref.abs().max() > 0.05
     # two fp32 sums of different order, each rounded to fp16 (subnormal from 2^-14 down)
     assert ((c - ref).abs() <= 2.0 ** -10 * ref.abs() + 2.0 ** -24 + 1e-5 * ref.abs().max()).all()
+
+
+@pytest.mark.parametrize("fmt,M,N,K", [
+    ("fp8-fp4", 33, 9248, 4352), ("fp6-fp4", 64, 8224, 8192), ("fp8-fp4", 38, 10112, 9984), ("fp6-fp4", 67, 9568, 8960), ("fp8-fp4", 94, 6400, 7424), ("fp6-fp4", 65, 8160, 1280),
+    ("fp8-fp4", 33, 16416, 1792), ("fp8", 33, 8224, 4352), ("fp8", 51, 9440, 7680), ("fp8", 35, 9216, 1792), ("fp8", 65, 4096, 8448), ("fp8", 70, 8032, 9216)])
+def test_with_and_without_a_workspace(fmt, M, N, K):
+    """Either side of the lines between one and two rounds of the small-M kernel, the K splits and the tiles, ragged in rows and columns."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N)
+    fa, fb = (fmt, fmt) if "-" not in fmt else fmt.split("-")
+
+    def data(lo, hi, *shape):
+        return torch.randint(lo, hi, shape, generator=g, device="cuda", dtype=torch.uint8)
+
+    a, b = data(0, 127, M, K), data(0, 127, N, K) if fb == "fp8" else data(0, 256, N, K // 2)
+    a[..., ::3] |= 128
+    sa, sb = data(120, 130, (M + 31) // 32 * K), data(120, 130, N // 32 * K)
+    out = []
+    for kw in (dict(), dict(_no_split=True), dict(_force_path=3, _no_split=True)):
+        c = torch.full((M + 64, N), -8192.0, dtype=torch.bfloat16, device="cuda")
+        launch_gemm(c, a, b, sa, sb, M, N, torch.cuda.current_stream(), N, K, 64, 128, 256, fa, "bf16", fb, 1, -1, -1, -1, -1, -1, -1, 0, 0, **kw)
+        assert (c[M:] == -8192.0).all()
+        out.append(c[:M].float())
+    for c in out[:2]:  # fp32 sums of different order, which may round to neighbouring bf16 values
+        assert ((c - out[2]).abs() <= 2.0 ** -7 * out[2].abs() + 1e-5 * out[2].abs().max()).all()
