@@ -194,7 +194,8 @@ Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
 // A tile's estimated time on a problem whose K isn't split: a start, one `round` per set of tiles that the CUs hold together and, per K step of 128
 // bytes, what a CU takes for the 1 .. per_cu tiles it works on at once.  It knows what the score above doesn't: a second tile on a CU costs little
 // while a step is bound by its loads, short rows are bound by the rounds' ends, and a last round with few tiles is shorter.  The constants are
-// least-squares fits to timed problems of 65 to 8192 rows, 1024 to 16384 columns (8 and 16 bits: 28672) and K 1024 to 14336, every tile timed on each.
+// least-squares fits to problems of 65 to 8192 rows, 1024 to 16384 columns (8 and 16 bits: 28672) and K 1024 to 14336, every tile timed on each, most weights in the
+// last-level cache.
 struct TileCost {
     int m, n, waves, per_cu;
     double start, round, step[5];  // us; step[r]: r tiles on a CU
@@ -216,9 +217,9 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
     return c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
 }
 
-// Of the three large tiles of the 8- and 16-bit kinds the one with the smallest estimate, where that is 7 % below the planned one's.  Fitted to 835 fp8 and bf16
-// problems (5 to 8 % off, r.m.s.): 51 of them take another tile, 15 % faster on average and none slower (us planned / estimate: fp8 1614x4896x6656
-// 75.4 / 50.9, 4329x1840x1856 31.5 / 23.0, 411x16720x2944 40.0 / 30.5, 3683x2288x8448 93.9 / 74.1; at 5 % two would lose 10 %).  The estimates of
+// Of the three large tiles of the 8- and 16-bit kinds the one with the smallest estimate, where that is 7 % below the planned one's.  On 151 drawn
+// problems, most weights in memory (profiles/tile_choice.md), the estimates are 12 % off (r.m.s.); 17 take another tile, 14 % faster on average and none slower (us
+// planned / estimate: fp8 1614x4896x6656 87.6 / 61.2, 4329x1840x1856 31.9 / 23.0, 411x16720x2944 41.7 / 34.1, 3683x2288x8448 91.6 / 81.9).  The estimates of
 // smaller tiles are too coarse to add them (64x64 with them: 433x8560x8768 57 / 66).
 Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
     static const TileCost costs[] = {{256, 256, 8, 1, 0.0, 7.0, {0, 1.17}}, {128, 256, 4, 2, 2.3, 7.1, {0, 0.77, 1.52}}, {128, 128, 4, 2, 5.0, 1.4, {0, 0.40, 0.91}}};
@@ -236,11 +237,12 @@ Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
     return best < 0.93 * kept ? t : planned;
 }
 
-// Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 3 % below that of
-// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  The constants are fits to 722 fp4 x
-// fp4, 208 fp8 x fp8 and 312 fp8 / fp6 x fp4 problems; the estimates are 4 to 7 % off (r.m.s.; fp8 3 to 5), which is why the score's tile stays where
-// they are close: without that eight of the 722 got more than 3 % slower, with it one does (282x9216x1280 9.4 us against 9.9).  199 take another tile, 10 % faster on average (us score / estimate: 4887x4256x1024 31.3 / 22.7,
-// 2127x14560x2304 63 / 56, 1285x14048x3072 56 / 44, 788x5280x4608 22.0 / 20.5, 5678x3584x4608 70.6 / 60.0, 48x4096x1024 6.5 / 4.3).
+// Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 6 % below that of
+// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  The estimates are 10 to 13 % off (r.m.s.) with most
+// weights in memory, which is why the score's tile stays where they are close: at 3 % fp4 510x10432x9728 got 46.8 us instead of 42.6, 400x4832x11776 34.4
+// instead of 32.9, fp8 724x5792x11520 98.5 instead of 88.  On drawn problems (profiles/tile_choice.md) 33 of 164 fp4 x fp4 take another tile, 11 % faster on
+// average and none more than 2 % slower, of 115 fp8 x fp8 34, 9 % and three 5 to 7 % slower (us score / estimate: fp4 4887x4256x1024 32.6 / 25.1, 1285x14048x3072 53.8 / 47.2,
+// 788x5280x4608 22.8 / 20.6, 5678x3584x4608 70.7 / 62.6; but 282x9216x1280 9.6 / 9.7, fp8 600x7680x3840 35.8 / 38.2).
 enum { MX_FP4, MX_FP8, MX_W4 };
 Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
     static const TileCost costs4[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
@@ -265,7 +267,7 @@ Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
             t = {c.m, c.n, c.waves};
         }
     }
-    return best < 0.97 * kept ? t : scored;
+    return best < 0.94 * kept ? t : scored;
 }
 
 // Split-K for the regime between the streaming kernel (takes_stream) and problems with enough tiles to fill the GPU:
