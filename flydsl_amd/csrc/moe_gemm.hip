@@ -347,7 +347,9 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
 // top-4 on 32, 4096 x 512 (331) 49.8 / 34.3; 600 x top-1 on 8, 3072 x 768, 64 rows (160) 23.9 / 17.6; 1024 x top-8, 4096 x 1536 (1,920) fp8 170 / 156, int8
 // 190 / 164, int4 161 / 143; 400 x top-6, 4096 x 1536, 64 rows (1,284) 96.7 / 93.1; but 1052 x top-8, 1536 x 1024 (1,180) fp8 43.3 / 45.2, 1726 x top-2,
 // 2816 x 512, 64 rows (688) 39.3 / 40.9.  Stage 2: 339 x top-4 on 16, 1024 x 2048 (234) 19.9 / 15.7; 200 x top-2 on 8, 4096 x 2048 (328) 26.8 / 20.9; but
-// 1086 x top-4, 4096 x 256 (1,358) 24.0 / 29.6.
+// 1086 x top-4, 4096 x 256 (1,358) 24.0 / 29.6.  Two blocks of 32 rows in one tile (stage 1) have that build alone: of 54 layers of 8 to 128 experts, 72 to 3,108 such workgroups,
+// 50 are faster with it, weights in memory or in the last-level cache (int8 45 x top-6 on 8, 3072 x 768 28.7 / 17.8, fp8 100 x top-2 on 8, 4096 x 2048 36.9 / 30.7, 564 x
+// top-6 on 128, 1280 x 768 58.9 / 55.3), and four 1 to 6 % slower (150 x top-4 on 16, 4096 x 2048 59.4 / 60.6; from the cache 49.8 / 52.8).
 template <int KIND, int STAGE>
 bool takes_deep(const MoeParams& p, int block_m, int blocks, int nx) {
     const long pairs = (long)p.tokens * p.topk, likely = pairs / block_m + p.experts / 2;

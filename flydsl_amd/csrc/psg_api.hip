@@ -89,7 +89,9 @@ constexpr int kStreamMaxM = 64;  // rows the small-M kernels can hold (four 16-r
 // 2048 and its workgroups of 32 columns come one to a CU (measured, us small-M / tiled plan: M=33 7168x2048 4.9 / 6.5, 8192x8192 10.9 / 14.6,
 // 1024x2048 4.3 / 5.3, 4096x1024 4.8 / 4.1; M=64 5.9 / 6.7, 13.2 / 15.8, 5.4 / 5.3, 5.8 / 4.2).  With more columns a few CUs work a second round
 // while the others wait, and 32x128 tiles, two or three to a CU, take over at once: M=33 8960x8704 16.7 / 13.5, 12288x4096 9.4 / 8.0,
-// 16384x2048 6.5 / 5.8, 24576x2048 8.2 / 7.8; M=64 8224x2048 7.1 / 5.2, 16384x2048 8.3 / 6.2, 20480x4096 17.2 / 10.7.  Up to 32 rows the two are
+// 16384x2048 6.5 / 5.8, 24576x2048 8.2 / 7.8; M=64 8224x2048 7.1 / 5.2, 16384x2048 8.3 / 6.2, 20480x4096 17.2 / 10.7, with the weights in the last-level cache.  From
+// memory the tiles are 9 % faster from 49 rows on, level from 40, and 8 to 16 % slower below that, where from the cache they are as much faster (34x15552x3840
+// 10.5 / 12.7; 10.0 / 8.8, 44 to 48 rows 1.0 to 1.05; 0.80 to 0.82, 62x9920x4608 13.9 / 12.0; 13.9 / 9.0).  Up to 32 rows the two are
 // too close to draw a line by (32x10240x4096 8.7 / 8.0, 17x8224x4096 7.0 / 7.8, 32x16384x14336 25.8 / 33.1).
 bool mx_small_holds(int M, int N, int K) { return M > kSmallM && M <= kStreamMaxM && K >= 2048 && (long)N * (K / 2) <= (40L << 20); }
 bool mx_takes_small(int M, int N, int K) { return M <= kSmallM || (mx_small_holds(M, N, K) && N <= 32 * psg_cu_count()); }
@@ -101,16 +103,21 @@ bool mx_takes_small(int M, int N, int K) { return M <= kSmallM || (mx_small_hold
 // 4.3 / 8.0, 6144x4096 9.2 / 14.1, 8192x8192 15.3 / 19.6, 2048x16384 15.5 / 16.0; M=48 9.7 / 14.4, 16.5 / 20.4, 17.3 / 16.3; M=64
 // 1024x2048 5.5 / 8.2, 6144x4096 11.3 / 15.0, 8192x8192 18.3 / 22.2, 5120x8192 15.8 / 19.0, 2048x16384 20.0 / 15.6), and while 32
 // columns for each CU are all there are.  With more columns the CUs go round again, and 64x64 tiles, several to a CU and without a split,
-// are better from the first column on (us streaming / 64x64 tiles: fp8 33x8208x1024 8.6 / 5.0, 33x9216x8064 23.2 / 20.5, 64x8208x4096
+// are better from the first column on (us streaming / 64x64 tiles, weights in the last-level cache: fp8 33x8208x1024 8.6 / 5.0, 33x9216x8064 23.2 / 20.5, 64x8208x4096
 // 16.0 / 11.7, 48x10240x6144 20.6 / 16.5, 33x16384x4096 17.3 / 13.7, 64x28672x2048 23.8 / 12.6, 33x65536x1024 35.6 / 13.7; fp16
-// 33x16384x2048 17.4 / 14.4, 40x12288x3328 23.4 / 18.5; just below the line 60x8192x4096 10.7 / 14).
+// 33x16384x2048 17.4 / 14.4, 40x12288x3328 23.4 / 18.5; just below the line 60x8192x4096 10.7 / 14).  With the weights in memory too, at 102 of 120 drawn
+// problems by more than 5 % (fp8 44x40512x1024 24.1 / 12.1, 51x13744x4032 20.4 / 20.1); at ten, rows of 5 KB and more just past the line, the streaming
+// kernel is up to 15 % faster there and as much slower from the cache (int8 36x9472x6080 21.5 / 24.4; 20.7 / 18.4, fp8 42x8512x5888 20.0 / 22.8; 18.8 / 17.2).
 // Beyond 64 rows a workgroup takes 64 of them, and the kernel is the better one while 32 columns a workgroup make one round of the CUs (N
 // times the 64-row groups up to 8192) on rows of 2 to 4 KB (us streaming / tiled plan: fp8 80x1024x4096 6.6 / 9.5, 256x1024x4096 7.2 /
 // 10.1, 128x2048x2048 4.8 / 7.3, 128x4096x4096 9.9 / 11.9, 192x2048x2048 7.2 / 7.4; bf16 256x1024x1024 4.8 / 6.8, 128x2048x2048 7.4 /
 // 10.4; but fp8 128x4096x1024 6.2 / 5.5, 192x4096x4096, one and a half rounds, 19.2 / 11.9).  On rows of 4 to 8 KB it is while they fill half of
 // the CUs (fp8 65x1024x4224 7.1 / 9.1, 80x2048x8128 11.4 / 13.7, 128x2048x6144 9.2 / 12.9, 256x1024x8128 12.2 / 15.7; int8 256x1024x4224 7.9 /
 // 11.0; bf16 66x2048x2112 7.0 / 9.8; fp16 128x2048x4032 11.2 / 14.1); between a half and one round it depends on the columns (256x2048x5120 11.0 /
-// 12.7, but 192x2048x4160 11.8 / 11.4, 128x4096x7168 14.2 / 13.6, 192x2720x6144 15.1 / 13.9) and the tiles stay.
+// 12.7, but 192x2048x4160 11.8 / 11.4, 128x4096x7168 14.2 / 13.6, 192x2720x6144 15.1 / 13.9) and the tiles stay.  On rows of 8 KB and more they are the better
+// ones from the first (165x1056x8576 15.0 / 15.2, 65x1968x10880 17.2 / 14.9, 163x2128x9216 19.8 / 16.6, 89x320x10752 14.7 / 11.9).  With fewer than 1024 columns, 32
+// workgroups of the streaming kernel, rows of 4 to 8 KB go either way too (fp8 202x368x5440 10.4 / 11.5, int8 221x336x4864 9.7 / 11.0, but fp8 93x368x8128 12.7 /
+// 10.7, bf16 109x880x3456 11.9 / 11.3), and the tiles stay; on 2 to 4 KB it is better with any number of columns (86x288x2688 6.4 / 10.8).
 bool stream_holds(int M, int N, int kbytes) {
     const long w = (long)N * kbytes, a = (long)M * kbytes;
     return M > kSmallM && M <= kStreamMaxM && a <= (512L << 10) && w <= (80L << 20);
@@ -119,7 +126,8 @@ bool takes_stream(int M, int N, int kbytes) {
     if (M <= kSmallM) return true;
     if (M > kStreamMaxM) {
         const long columns = (long)N * ((M + 63) / 64);
-        return M <= 256 && (kbytes >= 2048 && kbytes <= 4096 ? columns <= 8192 : kbytes > 4096 && kbytes < 8192 && N >= 1024 && columns <= 4096);
+        const long round = 32L * psg_cu_count();
+        return M <= 256 && (kbytes >= 2048 && kbytes <= 4096 ? columns <= round : kbytes > 4096 && kbytes < 8192 && N >= 1024 && columns <= round / 2);
     }
     return stream_holds(M, N, kbytes) && N <= 32 * psg_cu_count();
 }
