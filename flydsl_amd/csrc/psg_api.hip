@@ -226,7 +226,7 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
 }
 
 // Of the three large tiles of the 8- and 16-bit kinds the one with the smallest estimate, where that is 7 % below the planned one's.  On 151 drawn
-// problems, most weights in memory (profiles/tile_choice.md), the estimates are 12 % off (r.m.s.); 17 take another tile, 14 % faster on average and none slower (us
+// problems, most weights in memory, the estimates are 12 % off (r.m.s.); 17 take another tile, 14 % faster on average and none slower (us
 // planned / estimate: fp8 1614x4896x6656 87.6 / 61.2, 4329x1840x1856 31.9 / 23.0, 411x16720x2944 41.7 / 34.1, 3683x2288x8448 91.6 / 81.9).  The estimates of
 // smaller tiles are too coarse to add them (64x64 with them: 433x8560x8768 57 / 66).
 Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
@@ -248,7 +248,7 @@ Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
 // Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 6 % below that of
 // the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  The estimates are 10 to 13 % off (r.m.s.) with most
 // weights in memory, which is why the score's tile stays where they are close: at 3 % fp4 510x10432x9728 got 46.8 us instead of 42.6, 400x4832x11776 34.4
-// instead of 32.9, fp8 724x5792x11520 98.5 instead of 88.  On drawn problems (profiles/tile_choice.md) 33 of 164 fp4 x fp4 take another tile, 11 % faster on
+// instead of 32.9, fp8 724x5792x11520 98.5 instead of 88.  On drawn problems 33 of 164 fp4 x fp4 take another tile, 11 % faster on
 // average and none more than 2 % slower, of 115 fp8 x fp8 34, 9 % and three 5 to 7 % slower (us score / estimate: fp4 4887x4256x1024 32.6 / 25.1, 1285x14048x3072 53.8 / 47.2,
 // 788x5280x4608 22.8 / 20.6, 5678x3584x4608 70.7 / 62.6; but 282x9216x1280 9.6 / 9.7, fp8 600x7680x3840 35.8 / 38.2).
 enum { MX_FP4, MX_FP8, MX_W4 };

@@ -55,16 +55,14 @@ class MoeStage:
         self._plans = {}  # what numbers alone decide about a call, by those numbers
 
     def _plan(self, tokens, blocks, size):
-        """(argument struct without its addresses, operands) of a call as the native launch takes them, ``None`` twice when it needs scratch;
-        and the library's rule for that, which the plan holds for."""
-        rule = self._lib.psg_moe_rows_workspace_bytes
+        """(argument struct without its addresses, operands) of a call as the native launch takes them, ``None`` when it needs scratch."""
         n_out, K = (self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)
         rows_x = tokens if (self.stage == 1 and not self.slot_major) else tokens * self.topk
         rows_w = self.experts * (2 * n_out if self.stage == 1 else n_out)
         rows_out = tokens * self.topk if (self.stage == 1 or not self.accumulate) else tokens
         osize = 4 if self.out_dtype == 2 else 2
-        if self.stage == 2 and self.accumulate and rule(tokens, self.topk, size, n_out, self.out_dtype, 2 if self.w4 else 0):
-            return None, None, rule
+        if self.stage == 2 and self.accumulate and self._lib.psg_moe_rows_workspace_bytes(tokens, self.topk, size, n_out, self.out_dtype, 2 if self.w4 else 0):
+            return None
         a = _lib.MoeArgs()
         a.tokens, a.topk, a.experts = tokens, self.topk, self.experts
         a.model_dim, a.inter_dim = self.model_dim, self.inter_dim
@@ -77,18 +75,18 @@ class MoeStage:
                             (f.scale_x, 4, any_, 4 * rows_x), (f.scale_w, 4, any_, 4 * rows_w), (f.sorted_token_ids, 4, any_, 4 * size),
                             (f.sorted_expert_ids, 4, any_, 4 * blocks), (f.sorted_weights, 4, any_, 4 * size if self.doweight else 0),
                             (f.num_valid_ids, 4, any_, 4))
-        return (bytes(a),), ops, rule
+        return (bytes(a),), ops
 
     def __call__(self, out, x, w, scale_x, scale_w, sorted_token_ids, sorted_expert_ids, sorted_weights, num_valid_ids,
                  tokens, dim0, dim1, blocks, stream=None):
         if stream is not None and type(tokens) is type(blocks) is type(dim0) is type(dim1) is int and isinstance(sorted_token_ids, torch.Tensor) and (dim0, dim1) == ((self.inter_dim, self.model_dim) if self.stage == 1 else (self.model_dim, self.inter_dim)):
             key = (tokens, blocks, sorted_token_ids.numel(), self.no_pairing)
-            plan = self._plans.get(key)
-            if plan is None or plan[2] is not self._lib.psg_moe_rows_workspace_bytes:
+            if key not in self._plans:
                 if len(self._plans) >= 256:
                     self._plans.clear()
-                plan = self._plans[key] = self._plan(*key[:3])
-            if plan[0] is not None:
+                self._plans[key] = self._plan(*key[:3])
+            plan = self._plans.get(key)
+            if plan is not None:
                 rc = _lib._native.launch(_lib.address("psg_moe_gemm"), plan[0], plan[1], stream, out, x, w, scale_x, scale_w, sorted_token_ids,
                                          sorted_expert_ids, sorted_weights, num_valid_ids)
                 if rc != _lib._native.DECLINED:

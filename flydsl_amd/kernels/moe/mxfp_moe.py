@@ -76,13 +76,12 @@ def _gemm1_plan(tokens, BM, NE, H, I, BN, BK, inline_quant, interleave, a_dtype,
 
 @functools.lru_cache(maxsize=1024)
 def _gemm2_plan(tokens, max_sorted, BM, NE, H, I, topk, BN, BK, epilog, out_dtype, blocks):
-    """The same of a stage 2, ``None`` twice when it needs scratch; and the library's rule for that, which the plan holds for."""
-    rule = _lib.lib().psg_moe_rows_workspace_bytes
+    """The same of a stage 2, ``None`` also when it needs scratch."""
     if BN < 1 or BK < 1 or I % BK or H % BN or H % 256 or I % 256 or epilog not in _G2_EPILOGS or BM not in (16, 32, 64, 128) or out_dtype not in (torch.bfloat16, torch.float16):
-        return None, None, rule
+        return None
     code, atomic = 0 if out_dtype == torch.bfloat16 else 1, epilog == "atomic"
-    if atomic and topk and rule(tokens, topk, max_sorted, H, code, 1):
-        return None, None, rule
+    if atomic and topk and _lib.lib().psg_moe_rows_workspace_bytes(tokens, topk, max_sorted, H, code, 1):
+        return None
     args = _lib.MoeMxArgs()
     args.tokens, args.experts, args.model_dim, args.inter_dim = tokens, NE, H, I
     args.sorted_size, args.blocks, args.block_m = max_sorted, min(blocks, max_sorted // BM), BM
@@ -91,7 +90,7 @@ def _gemm2_plan(tokens, max_sorted, BM, NE, H, I, topk, BN, BK, epilog, out_dtyp
     return (bytes(args),), _lib.operands((f.a, 1, any_, max_sorted * (I // 2)), (f.a_scale, 1, any_, (max_sorted + 31) // 32 * 32 * (I // 32)),
                                          (f.w, 1, any_, NE * H * (I // 2)), (f.w_scale, 1, any_, NE * H * (I // 32)), (f.sorted_expert_ids, 4, i32, 4 * blocks),
                                          (f.num_valid_ids, 4, i32, 4), (f.sorted_token_ids, 4, i32, 4 * max_sorted), (f.sorted_weights, 4, _lib.TYPE_FP32, 4 * max_sorted),
-                                         (f.out, 2, (_lib.TYPE_BF16, _lib.TYPE_FP16)[code], 2 * (tokens if atomic else max_sorted) * H)), rule
+                                         (f.out, 2, (_lib.TYPE_BF16, _lib.TYPE_FP16)[code], 2 * (tokens if atomic else max_sorted) * H))
 
 
 def flydsl_mxfp4_gemm1(*, a_quant, a_scale_sorted_shuffled, w1_u8, w1_scale_u8, sorted_expert_ids, cumsum_tensor, m_indices,
@@ -174,11 +173,8 @@ def flydsl_mxfp4_gemm2(*, inter_sorted_quant, inter_sorted_shuffled_scale, w2_u8
     (nonatomic), bf16 or fp16.  Returns ``flat_out``."""
     if (stream is not None and D_INTER_REAL is None and type(M_logical) is type(max_sorted) is type(BM) is type(NE) is type(D_HIDDEN) is type(D_INTER) is type(topk) is
             type(BN) is type(BK) is int and type(epilog) is str and isinstance(flat_out, torch.Tensor) and isinstance(sorted_expert_ids, torch.Tensor)):
-        numbers = (M_logical, max_sorted, BM, NE, D_HIDDEN, D_INTER, topk, BN, BK, epilog, flat_out.dtype, sorted_expert_ids.numel())
-        plan = _gemm2_plan(*numbers)
-        if plan[2] is not _lib.lib().psg_moe_rows_workspace_bytes:
-            plan = _gemm2_plan.__wrapped__(*numbers)
-        if plan[0] is not None:
+        plan = _gemm2_plan(M_logical, max_sorted, BM, NE, D_HIDDEN, D_INTER, topk, BN, BK, epilog, flat_out.dtype, sorted_expert_ids.numel())
+        if plan is not None:
             rc = _lib._native.launch(_lib.address("psg_moe_mx_gemm"), plan[0], plan[1], stream, inter_sorted_quant, inter_sorted_shuffled_scale, w2_u8, w2_scale_u8,
                                      sorted_expert_ids, cumsum_tensor, sorted_token_ids, sorted_weights, flat_out)
             if rc != _lib._native.DECLINED:
