@@ -309,8 +309,10 @@ OPTIONAL = 256  # added to a type: None may stand in the operand's place
 
 def operands(*ops) -> bytes:
     """The operands of a launch the way ``_native.launch`` reads them: ``(field of the argument struct, bytes of an element or 0,
-    TYPE_*, least bytes[, index of the struct])`` each, ``field`` being a ctypes field descriptor."""
-    return b"".join(struct.pack("<iiiiq", op[4] if len(op) > 4 else 0, op[0].offset, op[1], op[2], op[3]) for op in ops)
+    TYPE_*, least bytes[, index of the struct])`` each, ``field`` being a ctypes field descriptor.  A number of bytes that no tensor has leaves
+    the call to the Python checks."""
+    most = (1 << 63) - 1
+    return b"".join(struct.pack("<iiiiq", op[4] if len(op) > 4 else 0, op[0].offset, op[1], op[2], op[3] if 0 <= op[3] < most else most) for op in ops)
 
 
 def check(rc: int, what: str) -> None:

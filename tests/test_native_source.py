@@ -4,6 +4,8 @@ is not made to happen): nothing but the call into the library, and the lock is t
 import os
 import re
 
+import pytest
+
 import flydsl_amd
 
 SOURCE = os.path.join(os.path.dirname(flydsl_amd.__file__), "csrc", "native.cpp")
@@ -123,3 +125,28 @@ def test_scratch_is_not_asked_for_before_the_output_is_looked_at():
     for c, error in ((u8, ValueError), (np.zeros(64), TypeError)):  # 33 x 992 x 14336 splits K and needs scratch
         with pytest.raises(error):
             launch_gemm(c, u8, u8, u8, u8, 33, 992, 7, 992, 14336, 64, 128, 256, "fp8", "bf16", "fp4", 1, -1, -1, -1, -1, -1, -1, 0, 0)
+
+
+@pytest.mark.parametrize("big", [2**40, 2**60, 2**70, -2**62, -2**70])
+def test_numbers_beyond_any_size_get_the_errors_of_the_checks(big):
+    import torch
+
+    from flydsl_amd.kernels.gemm.mxfp4_preshuffle import launch_gemm
+    from flydsl_amd.kernels.moe.moe_gemm_2stage import compile_moe_gemm1
+    from flydsl_amd.kernels.moe.mxfp_moe import flydsl_mxfp4_gemm1, flydsl_mxfp4_gemm2
+
+    t = torch.zeros(64, dtype=torch.int32)
+    u8 = t.view(torch.uint8)
+    stage = compile_moe_gemm1(model_dim=256, inter_dim=128, experts=2, topk=1, tile_m=16, tile_n=64, tile_k=128, doweight_stage1=False, in_dtype="int8")
+    for tokens, blocks in ((big, 2), (3, big)):
+        with pytest.raises(ValueError, match="device"):
+            stage(t, t, t, t, t, t, t, t, t, tokens, 128, 256, blocks, 7)
+    kw = dict(cumsum_tensor=t, BM=32, NE=2, D_HIDDEN=256, D_INTER=256, topk=1, stream=7)
+    with pytest.raises(TypeError, match="device tensor"):
+        flydsl_mxfp4_gemm1(a_quant=u8, a_scale_sorted_shuffled=u8, w1_u8=u8, w1_scale_u8=u8, sorted_expert_ids=t, m_indices=t, inter_sorted_quant=u8,
+                           inter_sorted_shuffled_scale=u8, n_tokens=big, **kw)
+    with pytest.raises(TypeError, match="device tensor"):
+        flydsl_mxfp4_gemm2(inter_sorted_quant=u8, inter_sorted_shuffled_scale=u8, w2_u8=u8, w2_scale_u8=u8, sorted_expert_ids=t, sorted_token_ids=t, sorted_weights=t.float(),
+                           flat_out=t.bfloat16(), M_logical=big, max_sorted=64, epilog="atomic", **kw)
+    with pytest.raises(ValueError, match="device tensor"):
+        launch_gemm(u8, u8, u8, u8, u8, big, 64, 7, 64, 256, 64, 128, 256, "fp4", "bf16", "fp4", 1, -1, -1, -1, -1, -1, -1, 0, 0)
