@@ -245,11 +245,11 @@ Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
     return best < 0.93 * kept ? t : planned;
 }
 
-// Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 6 % below that of
+// Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 6 % (fp4) or 3 % below that of
 // the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  The estimates are 10 to 13 % off (r.m.s.) with most
 // weights in memory, which is why the score's tile stays where they are close: at 3 % fp4 510x10432x9728 got 46.8 us instead of 42.6, 400x4832x11776 34.4
-// instead of 32.9, fp8 724x5792x11520 98.5 instead of 88.  On drawn problems 33 of 164 fp4 x fp4 take another tile, 11 % faster on
-// average and none more than 2 % slower, of 115 fp8 x fp8 34, 9 % and three 5 to 7 % slower (us score / estimate: fp4 4887x4256x1024 32.6 / 25.1, 1285x14048x3072 53.8 / 47.2,
+// instead of 32.9; fp8, which gains as much between the two lines as it loses, 724x5792x11520 98.5 instead of 88, 172x11264x4096 24.6 instead of 28.7.  On drawn problems 33
+// of 164 fp4 x fp4 take another tile, 11 % faster on average and none more than 2 % slower, with 6 % 34 of 115 fp8 x fp8, 9 % and three 5 to 7 % slower (us score / estimate: fp4 4887x4256x1024 32.6 / 25.1, 1285x14048x3072 53.8 / 47.2,
 // 788x5280x4608 22.8 / 20.6, 5678x3584x4608 70.7 / 62.6; but 282x9216x1280 9.6 / 9.7, fp8 600x7680x3840 35.8 / 38.2).
 enum { MX_FP4, MX_FP8, MX_W4 };
 Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
@@ -275,7 +275,7 @@ Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
             t = {c.m, c.n, c.waves};
         }
     }
-    return best < 0.94 * kept ? t : scored;
+    return best < (formats == MX_FP4 ? 0.94 : 0.97) * kept ? t : scored;
 }
 
 // Split-K for the regime between the streaming kernel (takes_stream) and problems with enough tiles to fill the GPU:
@@ -360,15 +360,15 @@ int mx_general_splits(int M, int N, int K) {
 // Beyond that the small-M kernel, whose N / 32 workgroups for every 64 rows stream W best, while they make one round of the CUs; the tiles read W
 // from the last-level cache faster than that, but from memory slower, so in the second round it depends.  The lines are from 900 problems of 33 to 400 rows,
 // 200 to 1100 such workgroups and K 1024 to 14336, each with W in memory and with W in that cache (us small-M / splits / tiles, memory; cache):
-//   short rows, fp4 weights: two rounds of the small-M kernel (68x5120x1280 5.4 / 8.3 / 6.8; 5.2 / 8.1 / 5.5, 106x6432x1792 7.3 / 10.1 / 8.5; 6.7 / 9.9 / 7.0);
-//     fp8 weights an eighth of a round more than one
+//   rows below 1536 elements: an eighth of a round more than one; below 2048 and with fp4 weights two rounds, up to 320 rows (68x5120x1280 5.4 / 8.3 / 6.8; 5.2 /
+//     8.1 / 5.5, 106x6432x1792 7.3 / 10.1 / 8.5; 6.7 / 9.9 / 7.0; but 389x1248x1536 8.4 / 10.0 / 7.3)
 //   splits, up to 64 rows while they make at most two workgroups a CU, beyond at most one: fp8 x fp8 42x8544x10240 33.0 / 30.5 / 40.0;
 //     31.5 / 24.5 / 29.1, 48x10400x13312 43.3 / 40.6 / 52.6; 40.8 / 32.1 / 36.2, 75x5216x10752 33.7 / 30.5 / 40.0; 32.3 / 26.3 / 29.2; fp8 x fp4 38x10112x9984
 //     24.7 / 21.2 / 33.2; 23.7 / 18.6 / 24.2; but more of them fp8 x fp8 67x9568x8960 - / 36.6 / 36.3; - / 36.0 / 25.7.
 //     With fp4 weights and at most one workgroup a CU, or without the workspace, the small-M kernel is as good or better: 38x12992x6912 19.4 / 20.6 / 24.5;
 //     18.6 / 18.6 / 18.3, 47x11456x8448 23.0 / 24.1 / 29.3; 22.2 / 21.0 / 21.4
-//   long rows of fp4 weights in the second round: 94x6400x7424 20.5 / 30.4 / 25.3; 17.1 / 26.7 / 18.4, 149x3040x6912 17.6 / 27.4 / 23.6; 17.3 / 26.1 / 17.0, 140x4480x7680
-//     23.2 / 31.4 / 25.9; 21.1 / 27.5 / 18.5
+//   long rows of fp4 weights in the second round up to 192 rows: 94x6400x7424 20.5 / 30.4 / 25.3; 17.1 / 26.7 / 18.4, 149x3040x6912 17.6 / 27.4 / 23.6; 17.3 / 26.1 / 17.0, 140x4480x7680
+//     23.2 / 31.4 / 25.9; 21.1 / 27.5 / 18.5; beyond, 345x1472x6144 17.9 / 26.6 / 20.6; 16.1 / 22.8 / 15.0, the cache loses as much as the memory gains
 //   everything else on tiles (33x9184x3072 10.7 / 13.9 / 12.3; 9.7 / 13.3 / 9.4, 40x15456x3840 18.7 / 23.2 / 21.4; 16.7 / 17.4 / 13.7, 65x13664x12032 56 / 38 /
 //     43.6; 55 / 36 / 31.5; three rounds or more always, where against the general kernel 1164x2880x4096 takes 23.2 / 37.1, 591x8032x5632 33.4 / 51.5)
 enum MxRoute { MX_SMALL, MX_GENERAL, MX_TILES };
@@ -377,14 +377,14 @@ MxRoute mx_route(int M, int N, int K, bool fp8_weights, bool room) {
     if (M <= kSmallM) return holds ? MX_SMALL : MX_GENERAL;
     const long cus = psg_cu_count(), groups = (M + 63) / 64, wgs = (long)(N / 32) * groups;
     const bool small = holds && wgs <= 2 * cus;
-    if (small && (K >= 2048 ? wgs <= cus : fp8_weights ? wgs * 8 <= cus * 9 : true)) return MX_SMALL;
+    if (small && (wgs <= cus || (K < 1536 && wgs * 8 <= cus * 9) || (K < 2048 && !fp8_weights && M <= 320))) return MX_SMALL;
     const int splits = mx_general_splits(M, N, K);
     const long split_wgs = groups * ((N + 127) / 128) * splits;
     if (splits > 1 && split_wgs <= (M <= kStreamMaxM ? 2 : 1) * cus) {
         if (small && (!room || (!fp8_weights && split_wgs <= cus))) return MX_SMALL;
         return room ? MX_GENERAL : MX_TILES;
     }
-    return small && !fp8_weights && K >= 6144 ? MX_SMALL : MX_TILES;
+    return small && !fp8_weights && K >= 6144 && M <= 192 ? MX_SMALL : MX_TILES;
 }
 
 // Tile + split plan of the tiled path.  With few tiles and a long K (the regime between the streaming kernel and
