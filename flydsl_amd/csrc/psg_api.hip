@@ -246,12 +246,12 @@ Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
 }
 
 // Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 6 % below that of
-// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  The estimates are 10 to 13 % off (r.m.s.) with most
-// weights in memory, which is why the score's tile stays where they are close: at 3 % fp4 510x10432x9728 got 46.8 us instead of 42.6, 400x4832x11776 34.4
-// instead of 32.9, fp8 724x5792x11520 98.5 instead of 88, and twelve drawn fp8
-// problems between the two lines 2 % more on average.  On drawn problems 33
-// of 164 fp4 x fp4 take another tile, 11 % faster on average and none more than 2 % slower, of 115 fp8 x fp8 34, 9 % and three 5 to 7 % slower (us score / estimate: fp4 4887x4256x1024 32.6 / 25.1, 1285x14048x3072 53.8 / 47.2,
-// 788x5280x4608 22.8 / 20.6, 5678x3584x4608 70.7 / 62.6; but 282x9216x1280 9.6 / 9.7, fp8 600x7680x3840 35.8 / 38.2).
+// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  With most weights in memory the estimates
+// are 10 to 13 % off (r.m.s.), which is why the score's tile stays where they are close: at 3 % fp4 510x10432x9728 got 46.8 us instead of 42.6, 400x4832x11776
+// 34.4 instead of 32.9, and twelve of 115 drawn fp8 problems, those between the two lines, 2 % more on average (590x14048x10496 154 instead of 126).  Of 164 drawn fp4
+// problems 33 take another tile, 11 % faster on average and none more than 2 % slower, of the 115 fp8 ones 34, 10 % faster and three 5 to 7 % slower (us score
+// / estimate: fp4 4887x4256x1024 32.6 / 25.1, 1285x14048x3072 53.8 / 47.2, 788x5280x4608 22.8 / 20.6, 5678x3584x4608 70.7 / 62.6, 282x9216x1280 9.6 / 9.7; fp8
+// 600x7680x3840 35.8 / 38.2).
 enum { MX_FP4, MX_FP8, MX_W4 };
 Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
     static const TileCost costs4[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
