@@ -371,7 +371,7 @@ int mx_general_splits(int M, int N, int K) {
 //   long rows of fp4 weights in the second round up to 192 rows: 94x6400x7424 20.5 / 30.4 / 25.3; 17.1 / 26.7 / 18.4, 149x3040x6912 17.6 / 27.4 / 23.6; 17.3 / 26.1 / 17.0, 140x4480x7680
 //     23.2 / 31.4 / 25.9; 21.1 / 27.5 / 18.5; beyond, 345x1472x6144 17.9 / 26.6 / 20.6; 16.1 / 22.8 / 15.0, the cache loses as much as the memory gains
 //   everything else on tiles (33x9184x3072 10.7 / 13.9 / 12.3; 9.7 / 13.3 / 9.4, 40x15456x3840 18.7 / 23.2 / 21.4; 16.7 / 17.4 / 13.7, 65x13664x12032 56 / 38 /
-//     43.6; 55 / 36 / 31.5; three rounds or more always, where against the general kernel 1164x2880x4096 takes 23.2 / 37.1, 591x8032x5632 33.4 / 51.5)
+//     43.6; 55 / 36 / 31.5; three rounds or more always, where against the general kernel, from memory, fp8 x fp8 1164x2880x4096 takes 24.6 / 36.8, fp8 x fp4 591x8032x5632 37 / 55)
 enum MxRoute { MX_SMALL, MX_GENERAL, MX_TILES };
 MxRoute mx_route(int M, int N, int K, bool fp8_weights, bool room) {
     const bool holds = mx_general_small(M, N, K, false, fp8_weights, 1);
