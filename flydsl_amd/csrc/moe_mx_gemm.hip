@@ -15,7 +15,7 @@
 // by side along N; each covers 64 W rows: in stage 1 32 gate rows and the 32 up rows of the same columns, so a wavefront
 // owns whole 32-column quantisation groups.
 #include "moe_rows.h"
-#include "psg_common.h"
+#include "mx_pair_loop.h"
 
 namespace {
 
@@ -352,7 +352,131 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     }
 }
 
-// Blocks of 128 sorted rows run as two workgroups of 64 rows each: a 128-row tile needs every register of the wavefront for its
+// Blocks of 128 sorted rows, fp4 activations: a 128 x 256 tile each (stage 1: the gate and the up rows of 128 columns), two workgroups a CU, on
+// the mainloop of mx_pair_loop.h.  Stage 2 stores rows (p.atomic != 1).
+// Bound: MFMA at the clock the power limit leaves, stage 2 besides by its rows (268 MB, 51 us at the rate of a copy).  The 64-row tiles of k_moe_mx are
+// bound by their operands, 20 KB for every 64 MFMAs of a wavefront against 24 KB for 128 here.  Measured, 4096 tokens x top-8 on 32 experts, 4096 x 1536
+// (rocprofv3, 64-row workgroups / these): stage 1 290 / 198 us, stage 2 228 / 174; the layer 584 / 464.  The bits are those of k_moe_mx.
+// How many blocks there are is only known on the device: every workgroup takes its tile in the XCD-aware order of the GEMM tiles over the real count
+// (groups of 8 blocks: 4 to 16 are the same but for the ends, 479 / 474 / 474 / 477 / 478 us a layer with 4 / 6 / 8 / 12 / 16).
+template <int STAGE>
+__global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsParams rows) {
+    constexpr int MR = MxPair::MR, NR = MxPair::NR, TM = MxPair::TM;
+    constexpr int TN = STAGE == 1 ? 128 : 256;  // output columns
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[MxPair::LDS_BYTES];
+    __shared__ float s_w[STAGE == 2 ? TM : 1];
+
+    if constexpr (STAGE == 2) {
+        if ((int)blockIdx.x < rows.wgs) {
+            moe_rows_index_share<16>(rows, (int)blockIdx.x, rows.wgs, reinterpret_cast<int*>(lds), MxPair::LDS_BYTES / 4);
+            return;
+        }
+    }
+    const int wg = (int)blockIdx.x - (STAGE == 2 ? rows.wgs : 0);
+    const int used = p.num_valid[0];
+    int units = used > 0 ? (used - 1) / TM + 1 : 0;
+    units = units < p.blocks ? units : p.blocks;
+    if (wg >= units * p.n_tiles) return;
+    int blk, n_tile;
+    tile_coords(wg, units, p.n_tiles, 8, blk, n_tile);
+    const int e = __builtin_amdgcn_readfirstlane(p.expert_ids[blk]);
+    if ((unsigned)e >= (unsigned)p.experts) return;
+    const int tid = threadIdx.x;
+    const int wave = wave_id();
+    const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
+    const int n0 = n_tile * TN;
+    const uint32_t row_bytes = (uint32_t)p.K >> 1;
+    const uint32_t chunk_bytes = (uint32_t)(p.K >> 8) * 256u;  // one 32-row chunk of shuffled scales
+    const int w_rows = STAGE == 1 ? 2 * p.n_out : p.n_out;     // rows of one expert's matrix
+
+    // A: stage 1 gathers token rows, stage 2 reads the block's sorted rows; rows without a token read as zero
+    const int a_rows = STAGE == 1 ? p.tokens : p.sorted_size;
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc_uniform(p.a, (uint64_t)a_rows * row_bytes);
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc_uniform(p.w + (uint64_t)e * (uint64_t)w_rows * row_bytes, (uint64_t)w_rows * row_bytes);
+    uint32_t a_voff[4], b_voff[NR];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int row = (wave * 4 + j) * 8 + (lane >> 3);
+        const int src = STAGE == 1 ? (p.sorted_ids[blk * TM + row] & 0xFFFFFF) : blk * TM + row;
+        a_voff[j] = src < a_rows ? (uint32_t)src * row_bytes + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16) : 0xFFFFFFF0u;
+    }
+    // W: the wavefront's four 16-row blocks; in stage 1 two of gate and two of up rows, so it owns whole 32-column quantisation groups
+#pragma unroll
+    for (int ni = 0; ni < NR; ni++) {
+        const int nb = STAGE == 1 ? (ni >> 1) * (p.n_out >> 4) + (n0 >> 4) + wave * 2 + (ni & 1) : (n0 >> 4) + wave * 4 + ni;
+        b_voff[ni] = (uint32_t)nb * 16u * row_bytes + (uint32_t)lane * 16u;
+    }
+    // scales: four chunks a wavefront, in stage 1 wavefront 1 brings those of the gate rows and wavefront 2 of the up rows
+    const bool a_side = wave == 0 || wave == 3;
+    const uint8_t* s_base = a_side ? p.a_scale + (uint64_t)((blk * TM) >> 5) * chunk_bytes : p.w_scale + (uint64_t)e * (uint64_t)(w_rows >> 5) * chunk_bytes;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc_uniform(s_base, (uint64_t)(a_side ? 4 : w_rows >> 5) * chunk_bytes);
+    const int ch = (lane >> 4) + (a_side ? 0 : STAGE == 1 ? (wave - 1) * (p.n_out >> 5) + (n0 >> 5) : (n0 >> 5) + (wave - 1) * 4);
+    const uint32_t s_voff = (uint32_t)ch * chunk_bytes + (uint32_t)(lane & 15) * 16u;
+    if constexpr (STAGE == 2) {
+        if (tid < TM) s_w[tid] = p.atomic ? p.sorted_w[blk * TM + tid] : 1.0f;
+    }
+
+    v4f acc[MR][NR];
+    mx_pair_loop(acc, lds, ra, a_voff, rb, b_voff, rs, s_voff, STAGE == 1 ? wave : wave * 2, STAGE == 1 ? wave + 4 : wave * 2 + 1, p.K >> 8, wave, lane);
+
+    // rows past the last 64 in use are not written
+    const int end = (used + 63) / 64 * 64 - blk * TM, live = end < TM ? end : TM;
+    if constexpr (STAGE == 1) {
+        const uint32_t out_row_bytes = (uint32_t)p.n_out >> 1;
+        const uint32_t sc_chunk = (uint32_t)(p.n_out >> 8) * 256u;
+        const int c32 = (n0 >> 5) + wave;  // scale column
+        uint8_t* codes = static_cast<uint8_t*>(p.out);
+        static_for<MR>([&](auto MI) {
+            constexpr int mi = decltype(MI)::value;
+            uint32_t bexp;
+            const int word = quant_silu_mul(acc[mi][0], acc[mi][1], acc[mi][2], acc[mi][3], bexp);
+            const int r = mi * 16 + li;
+            const size_t sr = (size_t)blk * TM + r;
+            uint8_t* dst = lds + r * 64 + wave * 16 + lg * 2;
+            *reinterpret_cast<uint16_t*>(dst) = (uint16_t)(word & 0xFFFF);
+            *reinterpret_cast<uint16_t*>(dst + 8) = (uint16_t)((uint32_t)word >> 16);
+            if (lg == 0 && r < live) {
+                const size_t off = ((sr >> 5) * (size_t)sc_chunk) + (size_t)(c32 >> 3) * 256u + (size_t)((c32 & 3) * 16 + li) * 4u + (size_t)(((c32 >> 2) & 1) * 2 + ((sr >> 4) & 1));
+                p.out_scale[off] = (uint8_t)bexp;
+            }
+        });
+        __syncthreads();
+        for (int q = tid; q < live * 4; q += 256) {
+            const int r = q >> 2, c = q & 3;
+            *reinterpret_cast<v4i*>(codes + ((size_t)blk * TM + r) * out_row_bytes + (uint32_t)((n0 >> 1) + c * 16)) = *reinterpret_cast<const v4i*>(lds + r * 64 + c * 16);
+        }
+    } else {
+        // as 16-bit rows through LDS (512 bytes, 16-byte granules XORed with the row), in halves: the stores of one are under way while the other
+        // is converted
+        const size_t N = (size_t)p.n_out;
+        uint16_t* out = static_cast<uint16_t*>(p.out);
+        static_for<2>([&](auto HALF) {
+            constexpr int half = decltype(HALF)::value;
+            static_for<MR / 2>([&](auto MI) {
+                constexpr int mi = half * (MR / 2) + decltype(MI)::value;
+                const int r = mi * 16 + li;
+                const float wgt = s_w[r];
+                static_for<NR>([&](auto NI) {
+                    constexpr int ni = decltype(NI)::value;
+                    const int cb = ((wave * NR + ni) * 16 + lg * 4) * 2;
+                    const v4f v = acc[mi][ni] * wgt;
+                    const v2i pk = p.out_dtype == OUT_BF16 ? pack4_out16<OUT_BF16>(v[0], v[1], v[2], v[3]) : pack4_out16<OUT_FP16>(v[0], v[1], v[2], v[3]);
+                    *reinterpret_cast<v2i*>(lds + r * 512 + ((((cb >> 4) ^ r) & 31) << 4) + (cb & 15)) = pk;
+                });
+            });
+            __syncthreads();
+            if (half * 64 < live) {  // `live` is a multiple of 64
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int q = half * 64 * 32 + i * 256 + tid, r = q >> 5, g = q & 31;
+                    *reinterpret_cast<v4i*>(out + ((size_t)blk * TM + r) * N + n0 + g * 8) = *reinterpret_cast<const v4i*>(lds + r * 512 + (((g ^ r) & 31) << 4));
+                }
+            }
+        });
+    }
+}
+
+// Blocks of 128 sorted rows that k_moe_mx_pair does not take run as two workgroups of 64 rows each: a 128-row tile needs every register of the wavefront for its
 // accumulators, so one workgroup per CU would run with nothing to overlap its loads and its epilogue with (measured, 4096
 // tokens x top-8 on 32 experts, 4096 x 1536, operands three steps ahead in both: stage 1 364 us with 128-row tiles against 292 with
 // 64-row tiles, stage 2 with the atomic epilogue 655 against 393, one row per sorted position 271 against 225).
@@ -362,6 +486,17 @@ hipError_t launch_rows(MoeMxParams p, MoeRowsParams rows, int block_m, int block
     rows.wgs = p.atomic == 2 ? ROWS_INDEX_WGS : 0;
     p.blocks = blocks;
     p.n_tiles = p.n_out / (STAGE == 1 ? 128 : 256);
+    if constexpr (AF == MXF_FP4) {
+        // The 128x256 tiles, where there are enough of them (us 64-row workgroups / these, tiles the list has room for; in use: stage 1 62; 52 11.6 / 12.6, 120; 96
+        // 8.3 / 9.7, 128; 128 11.0 / 12.3, 136; 128 18.2 / 17.0, 142; 138 10.4 / 10.1, 180; 144 26.6 / 17.4, 240; 192 15.8 / 11.4, 240; 128 9.6 / 10.1, 672; 384
+        // 67.7 / 47.9; stage 2 by rows 279; 234 20.5 / 21.5, 284; 276 25.2 / 24.1, 368; 304 30.9 / 28.0, 896; 512 45.5 / 39.6).  Adding directly, which is left to
+        // stages with little to add, takes longer from a few large tiles (92; 84 17.8 / 31.6, 240; 192 27.4 / 36.6).  Scales are fetched 16 bytes a lane.
+        const bool wide = (reinterpret_cast<uintptr_t>(p.a_scale) | reinterpret_cast<uintptr_t>(p.w_scale)) % 16 == 0;
+        if (block_m == 128 && p.atomic != 1 && wide && (long)blocks * p.n_tiles * 8 >= 5L * psg_cu_count()) {
+            hipLaunchKernelGGL((k_moe_mx_pair<STAGE>), dim3((unsigned)(blocks * p.n_tiles + rows.wgs)), dim3(256), 0, stream, p, rows);
+            return hipGetLastError();
+        }
+    }
     p.n_groups = (p.n_tiles + 7) / 8;
     // Keyed by expert while an expert has few rows (then sharing an L2 is what saves re-reads: 256 tokens x top-8 on 32 experts,
     // blocks of 32, stage 1 66 -> 49 us; blocks of 16: 84 -> 71); from about 200 sorted rows per expert on the other orders measured

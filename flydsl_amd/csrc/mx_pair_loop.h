@@ -1,0 +1,141 @@
+// Mainloop of the 128x256 tile for fp4 operands with e8m0 scales on both sides, two workgroups per CU (gfx950): both
+// stages of the MX MoE pair on blocks of 128 sorted rows (moe_mx_gemm.hip).
+//
+// Four wavefronts side by side along N, each 128 rows x 64 weight rows (128 accumulator registers a lane), 256 elements of K a step:
+//   * A goes global -> LDS by DMA into four stages of 16 KB (rows of 128 bytes, 16-byte pieces XORed with row / 2), requested three steps
+//     ahead; a lane's source address is its row's, so rows may be gathered.
+//   * W never touches LDS: a wavefront's fragments are its own.  They are fetched three half steps (64 bytes of K) ahead into a ring of four
+//     half-step register sets; two whole-step sets need the same 64 registers and are ahead by half as much.
+//   * The scale dwords of a step, 4 chunks of 256 bytes on the A side and 8 on the W side, are one 16-byte DMA of three of the wavefronts: a DMA
+//     takes 64 lanes anywhere, so 16 lanes bring a chunk and one instruction four of them.
+//   * At most one memory instruction stands behind an MFMA: what is issued between two of them in a row, the matrix cores wait for (one
+//     workgroup alone on a CU, zero operands: 1,580 core cycles a step with the instructions in front of each block of four MFMAs, 1,450 like
+//     this; 1,088 is what 64 MFMAs take).
+// Two workgroups on a CU take 2,600 to 3,000 cycles for a step of both, the 256x256 tile of eight wavefronts (gemm_tiled8.h) 2,850 to 3,100 for as much
+// work; but they are not in step with each other, so that the start and the end of one, 7 of the 18 us of a tile with K = 2048, stand beside
+// MFMAs of the other.
+#pragma once
+#include "gemm_tiled.h"
+#include "lds_dma.h"
+
+namespace {
+
+struct MxPair {
+    static constexpr int MR = 8, NR = 4, NS = 4;  // 16-row blocks of A, of W a wavefront; LDS stages
+    static constexpr int TM = 128, TN = 256;
+    static constexpr int STAGE = TM * TK;         // bytes of one A stage
+    static constexpr int SC_SLOT = 12 * 256;      // scale dwords of a step
+    static constexpr int LDS_BYTES = NS * (STAGE + SC_SLOT);
+    static_assert(2 * LDS_BYTES + 2048 <= 160 * 1024, "two workgroups a CU, with 1 KB each for what a kernel adds");
+};
+
+// acc[mi][ni] = A (rows 16 mi ..) x W (the wavefront's 16-row block ni) over KT steps; 0 without any.
+//   lds      LDS_BYTES, 1 KB aligned: the A stages, behind them the scale slots; free again at the end
+//   a_voff   this lane's offsets into `ra` of the four 1 KB blocks (8 rows) that its wavefront fetches of a stage: of row (4 wave + j) 8 + lane / 8,
+//            16-byte piece (lane % 8) ^ (row / 2 % 8); out of the descriptor's bounds for a row that reads as zero
+//   b_voff   this lane's offsets into `rb` of the wavefront's four 16-row blocks
+//   s_voff   this lane's offset into `rs`, the scales of wavefront 0 and 3: A side, 1 and 2: W side chunks 0..3 and 4..7 of the tile: chunk
+//            lane / 16, 16-byte piece lane % 16
+//   chunk0/1 which of the eight W-side chunks belong to the wavefront's blocks 0, 1 and 2, 3
+__device__ __forceinline__ void mx_pair_loop(v4f (&acc)[MxPair::MR][MxPair::NR], uint8_t* lds, const __amdgpu_buffer_rsrc_t ra, const uint32_t (&a_voff)[4],
+                                             const __amdgpu_buffer_rsrc_t rb, const uint32_t (&b_voff)[MxPair::NR], const __amdgpu_buffer_rsrc_t rs,
+                                             const uint32_t s_voff, const int chunk0, const int chunk1, const int KT, const int wave, const int lane) {
+    constexpr int MR = MxPair::MR, NR = MxPair::NR, NS = MxPair::NS, STAGE = MxPair::STAGE, SC_SLOT = MxPair::SC_SLOT;
+    const int li = lane & 15, lg = lane >> 4;
+    const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
+    uint8_t* const lds_x = lds + NS * STAGE;
+    // (wavefront 3 brings the bytes of wavefront 0 once more: all of them count the same number of DMAs)
+    const uint32_t sc_dst = lds_base + (uint32_t)(NS * STAGE) + (uint32_t)(wave == 3 ? 0 : wave) * 1024u;
+
+    // DMA j of step kt: 0..3 A, 4 scales.  Without CHK the step is known to be before the end
+    constexpr int N_DMA = 5;
+    auto dma = [&](int kt, int stage, int j, auto CHK) __attribute__((always_inline)) {
+        const bool has = !decltype(CHK)::value || kt < KT;
+        if (j < 4) dma16(ra, lds_base + (uint32_t)(stage * STAGE + (wave * 4 + j) * 1024), has ? a_voff[j < 4 ? j : 0] : 0xFFFFFFF0u, has ? (uint32_t)kt * TK : 0u);
+        else dma16(rs, sc_dst + (uint32_t)(stage * SC_SLOT), has ? s_voff : 0xFFFFFFF0u, has ? (uint32_t)kt * 256u : 0u);
+    };
+    v4i bw[4][NR];
+    auto load_w = [&](int kt, int half, int ni, v4i* dst, auto CHK) __attribute__((always_inline)) {
+        const bool has = !decltype(CHK)::value || kt < KT;
+        dst[ni] = buf_load16(rb, has ? b_voff[ni] : 0xFFFFFFF0u, has ? (uint32_t)kt * 2048u + (uint32_t)half * 1024u : 0u);
+    };
+    const int f_base[2] = {li * TK + ((lg ^ ((li >> 1) & 7)) << 4), li * TK + (((4 + lg) ^ ((li >> 1) & 7)) << 4)};
+    constexpr int AHEAD = 2;  // blocks of four MFMAs that an A fragment is read ahead
+    v4i fr[4];
+    auto read_frag = [&](int stage, int half, int mi, v4i& dst) __attribute__((always_inline)) {
+        dst = *reinterpret_cast<const v4i*>(&lds[stage * STAGE + mi * 16 * TK + f_base[half]]);
+    };
+    int sav[2][4], sbv[2][2];
+    auto read_sc = [&](int slot, int q, int set) __attribute__((always_inline)) {
+        if (q < 4) sav[set][q < 4 ? q : 0] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + q * 256 + lane * 4);
+        else sbv[set][q < 4 ? 0 : q - 4] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + 1024 + (q == 4 ? chunk0 : chunk1) * 256 + lane * 4);
+    };
+
+    // Step kt (kt % 4 = S): sixteen blocks of four MFMAs, eight m-blocks of the lower half of K and eight of the upper.  A's stage and scales of the step
+    // have landed for everybody a step ago, so its first fragments and scales were read before the barrier in front of it.
+    auto step = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
+        constexpr int S = decltype(SP)::value, SS = S & 1;
+        static_for<16>([&](auto BI) {
+            constexpr int b = decltype(BI)::value, half = b >> 3, mi = b & 7, nb = b + AHEAD;
+            static_for<NR>([&](auto NI) {
+                constexpr int ni = decltype(NI)::value;
+                mfma_mx<half, ni & 1, mi & 1>(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3], sbv[SS][ni / 2], sav[SS][mi / 2]);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (ni == 0) {
+                    if constexpr (nb < 16) read_frag(S, nb >> 3, nb & 7, fr[nb & 3]);
+                    else read_frag((S + 1) % NS, 0, nb - 16, fr[nb & 3]);
+                }
+                if constexpr (ni == 1 && b >= 10) read_sc((S + 1) % NS, b - 10, SS ^ 1);
+                // The DMAs of step kt + 3 and the W fragments three half steps ahead.  The compiler counts only the loads it knows, W's, so its waits
+                // for W let as many instructions be on their way as there are W loads behind the awaited one, DMAs among them: in each half the DMAs
+                // go first, and both halves have some.
+                if constexpr (ni == 2) {
+                    if constexpr (b >= 1 && b < 4) dma(kt + 3, (S + 3) % NS, b - 1, CHK);
+                    if constexpr (b >= 4 && b < 8) load_w(kt + 1, 1, b - 4, bw[(2 * S + 3) % 4], CHK);
+                    if constexpr (b >= 9 && b < 11) dma(kt + 3, (S + 3) % NS, b - 6, CHK);
+                    if constexpr (b >= 11 && b < 15) load_w(kt + 2, 0, b - 11, bw[(2 * S + 4) % 4], CHK);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+        // the DMAs this wavefront issued a step ago (of step kt + 2) have landed before the barrier: behind the last of them it has issued four W
+        // loads of that step and everything of this one
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NR + N_DMA + 2 * NR) : "memory");
+    };
+
+    // prologue: A and scales of steps 0 and 1, W of the first half step, A and scales of step 2, W of the two half steps behind
+#pragma unroll
+    for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int j = 0; j < N_DMA; j++) dma(s, s, j, std::true_type{});
+#pragma unroll
+    for (int ni = 0; ni < NR; ni++) load_w(0, 0, ni, bw[0], std::true_type{});
+#pragma unroll
+    for (int j = 0; j < N_DMA; j++) dma(2, 2, j, std::true_type{});
+#pragma unroll
+    for (int ni = 0; ni < NR; ni++) load_w(0, 1, ni, bw[1], std::true_type{});
+#pragma unroll
+    for (int ni = 0; ni < NR; ni++) load_w(1, 0, ni, bw[2], std::true_type{});
+#pragma unroll
+    for (int mi = 0; mi < MR; mi++)
+#pragma unroll
+        for (int ni = 0; ni < NR; ni++) acc[mi][ni] = (v4f){0.f, 0.f, 0.f, 0.f};
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * NR + N_DMA) : "memory");
+    static_for<AHEAD>([&](auto I) { read_frag(0, 0, decltype(I)::value, fr[decltype(I)::value]); });
+#pragma unroll
+    for (int q = 0; q < 6; q++) read_sc(0, q, 0);
+
+    // four steps an iteration (stages and register sets are compile-time); the first loop while every load of it is before the end, then with
+    // checks, then what is left
+    int kt = 0;
+    for (; kt + 7 <= KT; kt += NS) static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::false_type{}); });
+    for (; kt + NS <= KT; kt += NS) static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::true_type{}); });
+    static_for<NS - 1>([&](auto I) {
+        if (kt + decltype(I)::value < KT) step(kt + decltype(I)::value, I, std::true_type{});
+    });
+    // wait states between the last MFMA and the first ordinary read of an accumulator (the compiler does not know that the asm statements are
+    // MFMAs); every DMA still on its way (redirected past the bounds) is done before the stages are reused
+    asm volatile("s_nop 15\n\ts_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+}  // namespace

@@ -349,3 +349,48 @@ def test_unbuilt_variants_raise_like_the_reference():
         flydsl_mxfp4_gemm1(BM=32, **ok1)  # 64 bytes of weights
     with pytest.raises(TypeError):
         flydsl_mxfp4_gemm2(epilog="atomic", **{**g2, "sorted_expert_ids": i32, "cumsum_tensor": i32, "sorted_token_ids": i32, "sorted_weights": i32})
+
+
+# ---- blocks of 128 rows on the 128x256 tiles: from 160 tiles on (five eighths of 256 CUs), with scales on 16 bytes.  The 64-row workgroups, which calls with scales off 16
+# bytes keep, accumulate in the same K order: the same bits everywhere, at one to nine K steps, with cut last blocks, blocks of masked
+# experts, blocks past num_valid and a num_valid that ends inside a block (in the middle of one 64 rows are not written).
+@pytest.mark.parametrize("tokens,model_dim,inter,experts,topk,cut,mask", [
+    (700, 256, 2304, 3, 2, 0, False), (650, 2304, 512, 7, 4, 0, True), (333, 1280, 1024, 9, 5, 64, False), (1030, 1024, 256, 4, 3, 128, True),
+    (2600, 256, 256, 5, 4, 64, False), (300, 512, 1536, 20, 2, 0, True)])
+def test_blocks_of_128_on_large_tiles_equal_the_small_ones(tokens, model_dim, inter, experts, topk, cut, mask):
+    bm, dev = 128, torch.device("cuda")
+    g = torch.Generator(device=dev).manual_seed(tokens)
+    u8 = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
+    sc = lambda n: torch.randint(118, 130, (n + 16,), generator=g, device=dev, dtype=torch.uint8)
+    rng = np.random.default_rng(tokens)
+    ids = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int32)
+    sid, sw, se, npp = O.moe_sorting(ids, rng.uniform(0.1, 1.0, size=(tokens, topk)).astype(np.float32), experts, bm)
+    rows, nv = sid.size // bm * bm, int(npp[0]) - cut
+    se = se.copy()
+    if mask:
+        se[se == int(se[1])] = -1
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    sid, sw, se, nvt = t(sid[:rows]), t(sw[:rows]), t(se), torch.tensor([nv], dtype=torch.int32, device=dev)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for tiles in (rows // bm * (inter // 128), rows // bm * (model_dim // 256)):
+        assert tiles * 8 >= 5 * cus or tiles * 8 < 4 * cus  # on either side of the line, and not by a hair
+    a, w1, w2 = u8(tokens, model_dim // 2), u8(experts * 2 * inter, model_dim // 2), u8(experts * model_dim, inter // 2)
+    sa, s1, s2 = sc(rows * (model_dim // 32)), sc(experts * 2 * inter * (model_dim // 32)), sc(experts * model_dim * (inter // 32))
+
+    def run(off, dt):
+        at = lambda s: torch.cat((torch.zeros(off, dtype=torch.uint8, device=dev), s))[off:]  # the same bytes, `off` past an aligned address
+        codes = torch.full((rows, inter // 2), 0x77, dtype=torch.uint8, device=dev)
+        hs = torch.full((off + rows * (inter // 32) + 256,), 0x77, dtype=torch.uint8, device=dev)[off:]
+        kw = dict(sorted_expert_ids=se, cumsum_tensor=nvt, BM=bm, NE=experts, D_HIDDEN=model_dim, D_INTER=inter, topk=topk)
+        flydsl_mxfp4_gemm1(a_quant=a, a_scale_sorted_shuffled=at(sa), w1_u8=w1, w1_scale_u8=at(s1), m_indices=sid, inter_sorted_quant=codes,
+                           inter_sorted_shuffled_scale=hs, n_tokens=tokens, **kw)
+        flat = torch.full((rows, model_dim), 7.0, dtype=dt, device=dev)
+        flydsl_mxfp4_gemm2(inter_sorted_quant=codes, inter_sorted_shuffled_scale=hs, w2_u8=w2, w2_scale_u8=at(s2), sorted_token_ids=sid, sorted_weights=sw,
+                           flat_out=flat, M_logical=tokens, max_sorted=rows, epilog="nonatomic", **kw)
+        torch.cuda.synchronize()
+        return codes, hs, flat.view(torch.int16)
+
+    for dt in (torch.bfloat16, torch.float16):
+        for got, want, name in zip(run(0, dt), run(4, dt), ("codes", "scales", "rows")):
+            assert torch.equal(got, want), (name, dt)
+        assert (got[(nv + 63) // 64 * 64:] == torch.tensor(7.0, dtype=dt).view(torch.int16).item()).all()
