@@ -279,6 +279,51 @@ Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
     return best < 0.94 * kept ? t : scored;
 }
 
+// Where the eight XCDs' ranges of an order in groups of `g` M-tiles start: the longest stretch of column tiles without a start, as a share of all
+double widest_gap(int tiles_m, int tiles_n, int g) {
+    const int num = tiles_m * tiles_n, q = num >> 3, r = num & 7;
+    int at[8];
+    for (int x = 0; x < 8; x++) {
+        const int wg = x * q + (x < r ? x : r), grp = wg / (g * tiles_n), rows = tiles_m - grp * g < g ? tiles_m - grp * g : g;
+        const int tn = (wg - grp * g * tiles_n) / rows;
+        int i = x;
+        for (; i > 0 && at[i - 1] > tn; i--) at[i] = at[i - 1];
+        at[i] = tn;
+    }
+    int gap = at[0] + tiles_n - at[7];
+    for (int x = 1; x < 8; x++) gap = at[x] - at[x - 1] > gap ? at[x] - at[x - 1] : gap;
+    return (double)gap / tiles_n;
+}
+
+// M-tiles per group of the XCD-aware tile order.  Eight make the set of tiles that an XCD works on at a time roughly square in bytes, which
+// is the least for its L2 to fetch.  But where its range starts, every XCD asks for one panel of W and stores to one range of columns, and with eight many
+// problems have all of them start at the same column tile or at two (whenever num / 8 is a multiple of half a group): they then walk
+// the columns side by side, and the rows of C, a power of two apart, meet in a few memory channels.  So the group of about that size is taken
+// whose starts lie apart (us in groups of 8 / as chosen here: // fp8 8192x4096x4096 111.2 / 107.8, 8192x8192x1024 87.2 / 79.0, 4096x7168x2048 58.8 / 56.0, 4096x6144x4096 93.9 / 89.9; int8 8192x8192x1024 92.1 / 82.7; bf16
+// 8192x4096x2048 111.5 / 108.6; fp4 8192x8192x1024 65.4 / 58.1, 4221x7744x1536 49.9 / 45.7; over 40 drawn sizes, few of which are aligned like that,
+// 0.98 to 1.10 and 1.004 on average).
+// Only where A, W and C fit the last-level cache together: beyond, XCDs that walk side by side read a panel of W from memory once (int8
+// 4096x28672x8192 714 in groups of 8 or 6, four or three starts, 728 to 732 with 7, 9 or 11, eight).  A last group of one M-tile
+// reads all of W for it (fp8 4096x8192x2048, 16 M-tiles, 64 / 71 in groups of 8 / 5).  Up to a tile a CU all of them are at work at once in any order (fp8
+// 4096x4096x7168, 256 tiles, 87 / 89).
+int tile_group(int hint, int M, int N, Tile t, double bytes) {
+    if (hint > 0) return hint;
+    const int tiles_m = (M + t.m - 1) / t.m, tiles_n = (N + t.n - 1) / t.n;
+    if ((long)tiles_m * tiles_n <= psg_cu_count() || bytes > 200e6) return 8;
+    int best = 8;
+    double gap = 2;
+    for (const int g : {8, 7, 9, 6, 10, 11, 5}) {
+        if (tiles_m > g && tiles_m % g == 1) continue;
+        const double d = widest_gap(tiles_m, tiles_n, g);
+        if (d < gap - 0.02) {
+            gap = d;
+            best = g;
+        }
+        if (gap <= 0.16) break;
+    }
+    return best;
+}
+
 // Split-K for the regime between the streaming kernel (takes_stream) and problems with enough tiles to fill the GPU:
 // with few tiles every workgroup walks all of K behind a one-step prefetch and the launch is latency-bound.
 // Splitting K over `splits` workgroups per tile multiplies the loads in flight; the price is one fp32 slice of
@@ -555,9 +600,6 @@ int run_a8w8(const psg_a8w8_args* a, void* out, int store, void* stream) {
     p.epi = a->epilogue;
     p.out = a->out_dtype;
     p.b_rowmajor = a->b_layout;
-    // M-tiles per group of the XCD-aware tile order: 8 makes the set of tiles one XCD works on at a time roughly
-    // square in bytes (A rows vs W rows), which minimises what its L2 has to fetch
-    p.group_m = a->xcd_swizzle > 0 ? a->xcd_swizzle : 8;
     const int kinds[4] = {KIND_INT8, KIND_FP8, KIND_FP16, KIND_BF16};
     const int kind = kinds[a->in_dtype];
     const int kbytes = (kind == KIND_FP16 || kind == KIND_BF16) ? a->K * 2 : a->K;
@@ -576,6 +618,7 @@ int run_a8w8(const psg_a8w8_args* a, void* out, int store, void* stream) {
         int splits = forced ? (a->tile_k >= 1 && a->tile_k <= 16 ? a->tile_k : 1) : plan.splits;
         if (store != STORE_C || !a->workspace || a->workspace_bytes < splitk_bytes(a->M, a->N, splits)) splits = 1;
         p.splits = splits;
+        p.group_m = tile_group(a->xcd_swizzle, a->M, a->N, t, splits > 1 ? 1e30 : (double)(a->M + (double)a->N) * kbytes + 2.0 * a->M * a->N);
         // at most two workgroups per CU: the launch is bound by the bytes of W in flight, so the builds that fetch W three
         // steps ahead run (ksplit doubles as that mark for the tiled kernel); reserved = 7 keeps the one-step builds (tests)
         const long wgs = (long)((a->M + t.m - 1) / t.m) * (long)((a->N + t.n - 1) / t.n) * splits;
@@ -749,7 +792,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         q.M = a->M;
         q.N = a->N;
         q.K = a->K;
-        q.group_m = a->xcd_swizzle > 0 ? a->xcd_swizzle : 8;
+        q.group_m = tile_group(a->xcd_swizzle, a->M, a->N, t, (double)a->M * a_row + (double)a->N * b_row + 2.0 * a->M * a->N);
         q.ksplit = 1;
         q.wave_layout = a->reserved >= 2 ? a->reserved : 1;  // four wavefronts: 8192x4096x4096 117 us against 130 with eight
         q.splits = 1;
@@ -826,7 +869,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
     p.N = a->N;
     p.K = a->K;
     p.out = a->out_dtype;
-    p.group_m = a->xcd_swizzle > 0 ? a->xcd_swizzle : 8;
+    p.group_m = 8;
     const bool small = a->force_path == 2 || (a->force_path == 0 && mx_takes_small(a->M, a->N, a->K));
     hipError_t e;
     if (small) {
@@ -852,7 +895,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         q.M = p.M;
         q.N = p.N;
         q.K = p.K;
-        q.group_m = p.group_m;
+        q.group_m = tile_group(a->xcd_swizzle, a->M, a->N, t, splits > 1 ? 1e30 : (double)(a->M + (double)a->N) * (a->K / 2) + 2.0 * a->M * a->N);
         q.ksplit = 1;
         q.wave_layout = a->reserved >= 2 ? a->reserved : (!forced && t.waves == 8 ? 8 : 1);
         q.splits = splits;

@@ -84,7 +84,7 @@ enum psg_error {
  *   tile_m/tile_n/tile_k, xcd_swizzle: the reference's tuning keywords; accepted as hints
  *            (0 = library's choice).  The library picks its own tiling per regime.  xcd_swizzle > 0 is the number
  *            of M-tiles per group of the tile order (psg_tile_coords); 0, which switches the remap off in the
- *            reference, here means the library's default group of 8 (results do not depend on the tile order).
+ *            reference, here means the library's choice, 5 to 11 (results do not depend on the tile order).
  */
 typedef struct psg_a8w8_args {
     void *c;
