@@ -543,7 +543,7 @@ hipError_t launch_shape(const A8W8Params& p, int tile_m, int tile_n, hipStream_t
     if (p.wave_layout == 8) {  // eight wavefronts side by side along N: 256x256 tile, every W fragment loaded once
         if (tile_m == 256 && tile_n == 256) return launch_tiled8<KIND, STORE>(p, stream);
     }
-    if constexpr (KIND != KIND_MXFP4 && KIND != KIND_MXFP8) {
+    if constexpr (KIND != KIND_MXFP8) {
         // few tiles (p.ksplit = 3: the planner's mark for launches of at most two workgroups per CU): W fetched three steps ahead
         if (p.ksplit == 3) {
             // 128x128 with a deep ring of stages (gemm_tiled8.h); wave_layout 4 keeps the older build with W three steps ahead
@@ -558,7 +558,7 @@ hipError_t launch_shape(const A8W8Params& p, int tile_m, int tile_n, hipStream_t
     }
     PSG_CASE(16, 4, 1)
     PSG_CASE(8, 8, 1)
-    if constexpr (KIND != KIND_MXFP4 && KIND != KIND_MXFP8) {
+    if constexpr (KIND != KIND_MXFP8) {
         // 128x256 with at most one tile per CU: the build that is not held to two workgroups per CU
         if (tile_m == 128 && tile_n == 256) {
             const long tiles = (long)((p.M + 127) / 128) * (long)((p.N + 255) / 256) * (STORE == STORE_ACC && p.splits > 1 ? p.splits : 1);
@@ -568,7 +568,7 @@ hipError_t launch_shape(const A8W8Params& p, int tile_m, int tile_n, hipStream_t
     PSG_CASE(8, 4, 1)
     PSG_CASE(4, 4, 1)
     PSG_CASE(2, 4, 1)
-    if constexpr (KIND == KIND_MXFP4 || KIND == KIND_MXFP8) {
+    if constexpr (KIND == KIND_MXFP8) {
         PSG_CASE(4, 2, 1)
         PSG_CASE(2, 2, 1)
     } else {

@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     constexpr bool IS16 = KIND == KIND_FP16 || KIND == KIND_BF16;
     constexpr bool SCALED = KIND == KIND_INT8 || KIND == KIND_FP8;
     constexpr bool W4 = KIND == KIND_MXA8W4 || KIND == KIND_MXA6W4;  // fp4 W against a wider A: half a row's bytes
-    constexpr bool MX = KIND == KIND_MXFP4 || KIND == KIND_MXFP8 || W4;
+    constexpr bool MX = KIND == KIND_MXFP8 || W4;
     static_assert(!MX || (MR == 16 && NS == 4), "MX scale slots are laid out for the 256-row tile");
 
     // LDS: the A stages; behind them NS slots of MX scale dwords (per slot 8 A-side chunks + 8 W-side chunks of 256 bytes)
@@ -98,7 +98,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     tile_coords((int)blockIdx.x, tiles_m, tiles_n, p.group_m, tm, tn);
     const int m0 = tm * TM;
     const int n0 = tn * TN;
-    const int K = KIND == KIND_MXFP4 ? (p.K >> 1) : (IS16 ? (p.K << 1) : p.K);  // BYTES of one operand row
+    const int K = IS16 ? (p.K << 1) : p.K;  // BYTES of one operand row
     const int KT = (K + TK - 1) / TK;
     const int kt_per = (KT + p.splits - 1) / p.splits;
     const int kt_begin = (int)blockIdx.y * kt_per;
@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     constexpr int MP = MR / 2, NP = 1;
     __amdgpu_buffer_rsrc_t rsa = ra, rsb = ra;
     if constexpr (MX) {
-        const uint32_t chunk_bytes = KIND == KIND_MXFP4 ? (uint32_t)KT * 256u : (uint32_t)(p.K >> 8) * 256u;
+        const uint32_t chunk_bytes = (uint32_t)(p.K >> 8) * 256u;
         const uint64_t sa_chunks = (uint64_t)((p.M + 31) >> 5), sa_mine = (uint64_t)((m0 >> 5) + wave);
         rsa = make_rsrc_uniform(p.mx_sa + (sa_mine < sa_chunks ? sa_mine : sa_chunks) * chunk_bytes, sa_mine < sa_chunks ? chunk_bytes : 0);
         const uint64_t sb_chunks = (uint64_t)(p.N >> 5), sb_mine = (uint64_t)((n0 >> 5) + wave);
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     auto dma_sc = [&](int kt, int slot, int which) __attribute__((always_inline)) {
         const bool has = kt < kt_end;
         const uint32_t dst = lds_base + (uint32_t)(NS * STAGE + slot * SC_SLOT + which * 2048 + wave * 256);
-        dma4(which ? rsb : rsa, dst, has ? (uint32_t)lane * 4u : 0xFFFFFFF0u, has ? (uint32_t)(KIND == KIND_MXFP4 ? kt : (kt >> 1)) * 256u : 0u);
+        dma4(which ? rsb : rsa, dst, has ? (uint32_t)lane * 4u : 0xFFFFFFF0u, has ? (uint32_t)(kt >> 1) * 256u : 0u);
     };
     auto read_sc = [&](int slot, int q, int* sa_dst, int* sb_dst) __attribute__((always_inline)) {
         if (q < MP) sa_dst[q] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + q * 256 + lane * 4);
@@ -241,15 +241,6 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
                 for (int ni = 0; ni < NR; ni++) {
                     if constexpr (KIND == KIND_BF16) mfma_bf16(acc[mi][ni], bhi[SB][ni], ahi); else mfma_f16(acc[mi][ni], bhi[SB][ni], ahi);
                 }
-            } else if constexpr (KIND == KIND_MXFP4) {
-                static_for<NR>([&](auto NI) {
-                    constexpr int ni = decltype(NI)::value;
-                    mfma_mx<0, ni & 1, mi & 1>(acc[mi][ni], blo[SB][ni], alo, sbv[SS][ni / 2], sav[SS][mi / 2]);
-                });
-                static_for<NR>([&](auto NI) {
-                    constexpr int ni = decltype(NI)::value;
-                    mfma_mx<1, ni & 1, mi & 1>(acc[mi][ni], bhi[SB][ni], ahi, sbv[SS][ni / 2], sav[SS][mi / 2]);
-                });
             } else if constexpr (W4) {
                 static_for<NR>([&](auto NI) {
                     constexpr int ni = decltype(NI)::value;

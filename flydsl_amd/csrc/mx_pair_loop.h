@@ -1,5 +1,5 @@
-// Mainloop of the 128x256 tile for fp4 operands with e8m0 scales on both sides, two workgroups per CU (gfx950): both
-// stages of the MX MoE pair on blocks of 128 sorted rows (moe_mx_gemm.hip).
+// Mainloop of the 128x256 tile for fp4 operands with e8m0 scales on both sides, two workgroups per CU (gfx950): the dense
+// MXFP4 GEMM (gemm_mx_pair.hip) and both stages of the MX MoE pair on blocks of 128 sorted rows (moe_mx_gemm.hip).
 //
 // Four wavefronts side by side along N, each 128 rows x 64 weight rows (128 accumulator registers a lane), 256 elements of K a step:
 //   * A goes global -> LDS by DMA into four stages of 16 KB (rows of 128 bytes, 16-byte pieces XORed with row / 2), requested three steps

@@ -147,11 +147,8 @@ struct Tile {
 // Tile choice for the MFMA mainloop.  Each shape has a measured relative efficiency at full occupancy.  The 256x256
 // tile of eight wavefronts side by side along N loads every W fragment once per CU and moves the least data per flop:
 // on real data the chip is power-limited, so that is what decides (fp8 8192x4096x4096: 117 us against 134 us for
-// the 128x256 tile that runs two workgroups per CU; int8 4096x28672x8192: 775 against 940).  MXFP4 4096x7168x2048:
-// 46 us with eight wavefronts against 52 with four, 58 for the 128x256 tile (one workgroup per CU: with two it spilled) and
-// 48 for 64x256; MXFP4 1024x8192x8192, where 256x256 gives only 128 tiles: 40 us with 128x256 against 59.  The MX efficiencies of the 64x128
-// and 32x128 tiles come from timing every forced tile next to the automatic plan (M 96-5120 on five N x K pairs: 256x8192x8192 21.3 us
-// with 64x128 tiles against 25.0 with 32x256; 96x7168x2048 5.7 with 32x128 against 6.7 with 64x128).  The score multiplies the efficiency by
+// the 128x256 tile that runs two workgroups per CU; int8 4096x28672x8192: 775 against 940).  The MX table is for fp8 x fp8; an fp4 x fp4 problem takes from it
+// only whether and how its K is split (over 18 such problems 1 % from the best of that and the unsplit tiles).  The score multiplies the efficiency by
 // how evenly the tiles fill the CUs' workgroup slots and by the fraction of each tile that is not padding.
 Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
     struct Shape {
@@ -245,18 +242,18 @@ Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
     return best < 0.93 * kept ? t : planned;
 }
 
-// Tile of an fp4 x fp4 or fp8 x fp8 problem whose K isn't split: the score's, or the one whose estimated time is the smallest and 6 % below that of
-// the score's tile; of an fp8 / fp6 x fp4 problem the one with the smallest estimate (kbytes: of a row of A).  With most weights in memory the estimates
-// are 10 to 13 % off (r.m.s.), which is why the score's tile stays where they are close: at 3 % fp4 510x10432x9728 got 46.8 us instead of 42.6, 400x4832x11776
-// 34.4 instead of 32.9, and twelve of 115 drawn fp8 problems, those between the two lines, 2 % more on average (590x14048x10496 154 instead of 126).  Of 164 drawn fp4
-// problems 33 take another tile, 11 % faster on average and none more than 2 % slower, of the 115 fp8 ones 34, 10 % faster and three 5 to 7 % slower (us score
-// / estimate: fp4 4887x4256x1024 32.6 / 25.1, 1285x14048x3072 53.8 / 47.2, 788x5280x4608 22.8 / 20.6, 5678x3584x4608 70.7 / 62.6, 282x9216x1280 9.6 / 9.7; fp8
-// 600x7680x3840 35.8 / 38.2).
+// Tile of an MX problem whose K isn't split (kbytes: of a row of A): of an fp4 x fp4 or fp8 / fp6 x fp4 problem the one with the smallest estimated time; of
+// fp8 x fp8 the score's unless an estimate is 6 % below that of the score's tile.
+// fp4: on 410 timed problems, weights in memory and in the last-level cache, the estimates are 6 to 10 % off (r.m.s.) and the tile they choose takes 0.2 % longer
+// than the best of the five, at worst 7 %.
+// fp8: with most weights in memory the estimates are 10 to 13 % off, so the score's tile stays where they are close: at 3 % twelve of 115 drawn
+// problems, those between the two lines, took 2 % longer on average (590x14048x10496 154 instead of 126); of the 115 34 take another tile, 10 % faster and three
+// 4 to 7 % slower (us score / estimate 600x7680x3840 35.8 / 38.2).
 enum { MX_FP4, MX_FP8, MX_W4 };
 Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
-    static const TileCost costs4[] = {{256, 256, 8, 1, 0.0, 7.3, {0, 1.41}},           {128, 256, 4, 1, 2.2, 5.9, {0, 0.93}},
-                                      {64, 256, 4, 2, 3.5, 2.8, {0, 0.58, 1.12}},      {32, 256, 4, 3, 3.6, 1.4, {0, 0.50, 0.95, 1.28}},
-                                      {64, 128, 4, 3, 3.8, 1.2, {0, 0.37, 0.67, 0.95}}, {32, 128, 4, 4, 3.0, 1.2, {0, 0.31, 0.50, 0.77, 0.90}}};
+    static const TileCost costs4[] = {{128, 256, 4, 2, 1.3, 4.3, {0, 0.65, 1.66}},
+                                      {64, 256, 4, 2, 1.8, 3.6, {0, 0.61, 1.17}},      {32, 256, 4, 3, 2.3, 1.9, {0, 0.51, 0.96, 1.35}},
+                                      {64, 128, 4, 3, 2.7, 1.5, {0, 0.39, 0.68, 0.98}}, {32, 128, 4, 4, 2.4, 1.0, {0, 0.32, 0.52, 0.77, 0.96}}};
     // (the fp8 launcher runs its 256x256 tile on four wavefronts whatever `waves` says)
     static const TileCost costs8[] = {{256, 256, 8, 1, 2.3, 9.5, {0, 1.45}},           {128, 256, 4, 1, 2.3, 5.7, {0, 0.85}},
                                       {64, 256, 4, 2, 3.9, 1.9, {0, 0.58, 1.02}},      {32, 256, 4, 3, 4.6, 0.0, {0, 0.50, 0.90, 1.21}},
@@ -265,17 +262,22 @@ Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
                                        {64, 256, 4, 3, 3.4, 2.2, {0, 0.48, 0.77, 1.13}},    {32, 256, 4, 3, 3.6, 0.8, {0, 0.37, 0.58, 0.76}},
                                        {64, 128, 4, 3, 3.4, 1.0, {0, 0.34, 0.49, 0.68}},    {32, 128, 4, 4, 3.1, 0.5, {0, 0.28, 0.35, 0.49, 0.60}}};
     const double mem = ((double)M * kbytes + (double)N * (formats == MX_W4 ? kbytes / 2 : kbytes) + 2.0 * M * N) / 4.3e6;
-    const Tile scored = pick_tile(M, N, true, 0, 0);
+    const Tile scored = formats == MX_FP8 ? pick_tile(M, N, true, 0, 0) : Tile{};
     double best = 1e30, kept = 1e30;
     Tile t = scored;
-    for (const TileCost& c : formats == MX_FP4 ? costs4 : formats == MX_FP8 ? costs8 : costs48) {
-        const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
-        if (formats != MX_W4 && c.m == scored.m && c.n == scored.n) kept = us;
-        if (us < best) {
-            best = us;
-            t = {c.m, c.n, c.waves};
+    auto consider = [&](const auto& costs) {
+        for (const TileCost& c : costs) {
+            const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
+            if (formats == MX_FP8 && c.m == scored.m && c.n == scored.n) kept = us;
+            if (us < best) {
+                best = us;
+                t = {c.m, c.n, c.waves};
+            }
         }
-    }
+    };
+    if (formats == MX_FP4) consider(costs4);
+    else if (formats == MX_FP8) consider(costs8);
+    else consider(costs48);
     return best < 0.94 * kept ? t : scored;
 }
 

@@ -146,3 +146,31 @@ def test_mxfp4_strided_batched_default_strides():
     for b, d in enumerate(ds):
         ref = O.run_torch_w4(d["a_q"].numpy(), d["b_q"].numpy(), d["sa"].numpy(), d["sb"].numpy())
         _check(c[b].float().cpu().numpy(), ref)
+
+
+# ---- the 128x256 tile (two workgroups a CU): the same accumulator bits as the 64x256 tile, which has the same K order, at one to nine K steps, either side of a
+# tile's rows and columns, 32 columns, over K splits of uneven length (one of them empty), in both output types; with scales off 16 bytes
+# the call runs on 64x256 tiles
+@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (127, 256, 512), (128, 288, 768), (129, 544, 1024), (255, 224, 1280), (385, 1056, 1792), (64, 480, 2048), (300, 512, 2304)])
+def test_large_tile_equals_the_64_row_tile(M, N, K):
+    from kernels.gemm.mxfp4_preshuffle import launch_gemm
+
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    u8 = lambda lo, hi, *shape: torch.randint(lo, hi, shape, generator=g, device="cuda", dtype=torch.uint8)
+    a, b = u8(0, 256, M, K // 2), u8(0, 256, N, K // 2)
+    sa, sb = u8(100, 150, 4 + (M + 31) // 32 * K), u8(100, 150, 4 + N // 32 * K)
+
+    def run(tile, off=0, splits=0, dt="bf16", acc=False):
+        s = [torch.cat((t[:off], t[:-4]))[off:] for t in (sa, sb)]  # the same bytes, `off` past an aligned address
+        c = torch.full((M + 5, N), SENTINEL, dtype=torch.bfloat16 if dt == "bf16" else torch.float16, device="cuda")
+        x = torch.full((M, N), -7.0, device="cuda") if acc else None
+        launch_gemm(0 if acc else c, a, b, *s, M, N, None, N, K, 64, 128, 256, "fp4", dt, "fp4", 1, -1, -1, -1, -1, -1, -1, 0, 0, _force_path=1, _tile=tile, _splits=splits,
+                    _acc=x)
+        torch.cuda.synchronize()
+        assert acc or (c[M:] == SENTINEL).all()
+        return x.view(torch.int32) if acc else c.view(torch.int16)
+
+    for kw in (dict(acc=True), dict(), dict(dt="fp16"), dict(splits=2), dict(splits=3), dict(splits=8)):
+        want = run((64, 256), **kw)
+        assert torch.equal(run((128, 256), **kw), want), kw
+        assert torch.equal(run((256, 256), off=4, **kw), want), kw
