@@ -1,9 +1,9 @@
-// Dense MXFP4 x MXFP4 GEMM on 128x256 tiles, two workgroups per CU (mainloop: mx_pair_loop.h).
+// Dense MXFP4 x MXFP4 GEMM on 128x256 tiles, two workgroups per CU (mainloop: pair_loop.h).
 //
 // Bound: MFMA at the clock the power limit leaves, and for short K the start and the end of a tile.  us, 256x256 tiles of eight wavefronts / these, weights in
 // memory: 4096x7168x2048 42.9 / 39.4, 4096x4096x4096 38.8 / 36.9, 8192x8192x1024 59.6 / 50.9, 6000x3584x4608 68 / 54, 8192x4096x8192 128.6 / 123.1, each in
 // its best tile order; 128x256 tiles of one workgroup a CU / these: 1000x7168x2048 15.4 / 13.1.
-#include "mx_pair_loop.h"
+#include "pair_loop.h"
 
 namespace {
 
@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256, 2) k_mx_pair(A8W8Params p) {
     const uint32_t s_voff = (uint32_t)((a_side ? 0 : (wave - 1) * 4) + (lane >> 4)) * chunk_bytes + (uint32_t)(lane & 15) * 16u;
 
     v4f acc[MR][NR];
-    mx_pair_loop(acc, lds, ra, a_voff, rb, b_voff, rs, s_voff, wave * 2, wave * 2 + 1, KT, wave, lane);
+    pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, KT, wave, lane, rs, s_voff, wave * 2, wave * 2 + 1);
 
     if constexpr (STORE == STORE_ACC) {
         static_for<MR>([&](auto MI) {

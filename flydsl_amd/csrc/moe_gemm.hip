@@ -420,29 +420,23 @@ hipError_t launch_kind(const MoeParams& p, const MoeRowsParams& rows, int block_
 
 }  // namespace
 
-hipError_t psg_launch_moe_tiled(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int blocks, hipStream_t stream);
+hipError_t psg_launch_moe_pair(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int blocks, hipStream_t stream);
 
-// Whether the 256-row tiles (moe_gemm_tiled.hip) are the better way for blocks of 128 rows: enough rows per expert that most
-// blocks find a partner, and a tile count (on average over routings: pairs / 256, and half a tile more per expert) that fills its
-// rounds of one tile per CU to 80 %.  Measured, fp8, us k_moe_gemm / 256-row tiles: stage 1 4096 tokens x top-8 on 32 experts, 4096 x
-// 1536 (1728 tiles) 473 / 391; 4096 x top-6 on 64, 1024 x 256 (256 tiles) 34.7 / 27.4; but 1024 x top-8 (576 tiles) 168 / 179, 4096 x
-// top-2 on 8, 2048 x 1024 (288) 52.8 / 61.1.  Stage 2 without atomics: 4096 x top-8 (2304 tiles) 360 / 273, 1024 x top-8 (768) 119 /
-// 105; but 512 x top-8 (512 tiles, 128 rows per expert) 70.2 / 72.7, 4096 x top-1 on 8, 4096 x 1024 (320) 68.7 / 74.9.
-// Where stage 2 adds directly (no scratch, fewer than four slots, under capture) the rule holds as well, though one workgroup a CU leaves
-// nothing to run beside the additions: 4096 x top-8 405 / 388, 2048 x top-8 220 / 203, 2048 tokens x top-3 on 8 experts, 4096 x 1024, 83 /
-// 75, x 2048 110 / 98; on two or three slots and short rows it is a few per cent the other way (4096 x top-3 on 16, 4096 x 768 127 / 131, x 256
-// 102 / 111; but 2048 x 512 70 / 64), which no size of the call tells apart.
-bool takes_tiled(const MoeParams& p, int stage) {
+// Whether the 128x256 tiles (moe_gemm_pair.hip) are the better way for blocks of 128 rows: where there are about as many of them as CUs, blocks counted as
+// a routing needs them on average (the pairs' and half a block for every expert), and in stage 1, whose weights are the larger ones, more than a block an expert.
+// Measured, us k_moe_gemm / 128x256 tiles (fp8; int8 the same or a few per cent better), tiles by that count: stage 1 120 16.7 / 19.9, 136 15.7 / 16.3, 144 40.0 /
+// 39.9, 192 16.5 / 17.4, 198 19.5 / 17.7, 240 43.5 / 40.3, 984 75.6 / 55.6; but 128 rows an expert, 576 tiles, 107.5 / 111.3.  Stage 2 97 19.3 / 20.5, 128 21.1 / 23.4,
+// 160 18.6 / 18.3, 165 22.9 / 19.7, 192 26.6 / 24.5, 428 38.5 / 27.4, 656 76.1 / 61.1.  The same where stage 2 adds directly (no scratch, few slots, under capture: 4096 x
+// top-8 379 / 326, 2048 x top-3 75.5 / 67.5, 4096 x top-1 56.1 / 55.2).
+bool takes_pair(const MoeParams& p, int stage, int blocks) {
     const long pairs = (long)p.tokens * p.topk, cus = psg_cu_count(), tn = stage == 1 ? 128 : 256;
-    if (pairs < 192L * p.experts) return false;
-    const long tiles = (pairs / 256 + p.experts / 2) * ((p.n_out + tn - 1) / tn);
-    const long rounds = (tiles + cus - 1) / cus;
-    return tiles * 10 >= rounds * cus * 8;
+    const long expected = pairs / 128 + p.experts / 2, tiles = (expected < blocks ? expected : blocks) * ((p.n_out + tn - 1) / tn);
+    return stage == 1 ? tiles * 4 > cus * 3 && pairs >= 144L * p.experts : tiles * 8 >= cus * 5;
 }
 
 // kind: KIND_INT8 / KIND_FP8 / KIND_INT8W4; stage 1 or 2; rows: where p.by_position is set; block_m in {16, 32, 64, 128}; blocks = entries of expert_ids
 hipError_t psg_launch_moe_gemm(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int block_m, int blocks, hipStream_t stream) {
-    if (block_m == 128 && kind != KIND_INT8W4 && p.out_dtype != OUT_F32 && p.pair_blocks && takes_tiled(p, stage)) return psg_launch_moe_tiled(p, rows, kind, stage, blocks, stream);
+    if (block_m == 128 && kind != KIND_INT8W4 && p.out_dtype != OUT_F32 && p.pair_blocks && takes_pair(p, stage, blocks)) return psg_launch_moe_pair(p, rows, kind, stage, blocks, stream);
     if (kind == KIND_INT8) return stage == 1 ? launch_kind<KIND_INT8, 1>(p, rows, block_m, blocks, stream) : launch_kind<KIND_INT8, 2>(p, rows, block_m, blocks, stream);
     if (kind == KIND_INT8W4) return stage == 1 ? launch_kind<KIND_INT8W4, 1>(p, rows, block_m, blocks, stream) : launch_kind<KIND_INT8W4, 2>(p, rows, block_m, blocks, stream);
     return stage == 1 ? launch_kind<KIND_FP8, 1>(p, rows, block_m, blocks, stream) : launch_kind<KIND_FP8, 2>(p, rows, block_m, blocks, stream);

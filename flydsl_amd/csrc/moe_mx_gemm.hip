@@ -15,7 +15,7 @@
 // by side along N; each covers 64 W rows: in stage 1 32 gate rows and the 32 up rows of the same columns, so a wavefront
 // owns whole 32-column quantisation groups.
 #include "moe_rows.h"
-#include "mx_pair_loop.h"
+#include "pair_loop.h"
 
 namespace {
 
@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
 }
 
 // Blocks of 128 sorted rows, fp4 activations: a 128 x 256 tile each (stage 1: the gate and the up rows of 128 columns), two workgroups a CU, on
-// the mainloop of mx_pair_loop.h.  Stage 2 stores rows (p.atomic != 1).
+// the mainloop of pair_loop.h.  Stage 2 stores rows (p.atomic != 1).
 // Bound: MFMA at the clock the power limit leaves, stage 2 besides by its rows (268 MB, 51 us at the rate of a copy).  The 64-row tiles of k_moe_mx are
 // bound by their operands, 20 KB for every 64 MFMAs of a wavefront against 24 KB for 128 here.  Measured, 4096 tokens x top-8 on 32 experts, 4096 x 1536
 // (rocprofv3, 64-row workgroups / these): stage 1 290 / 198 us, stage 2 228 / 174; the layer 584 / 464.  The bits are those of k_moe_mx.
@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
     }
 
     v4f acc[MR][NR];
-    mx_pair_loop(acc, lds, ra, a_voff, rb, b_voff, rs, s_voff, STAGE == 1 ? wave : wave * 2, STAGE == 1 ? wave + 4 : wave * 2 + 1, p.K >> 8, wave, lane);
+    pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, p.K >> 8, wave, lane, rs, s_voff, STAGE == 1 ? wave : wave * 2, STAGE == 1 ? wave + 4 : wave * 2 + 1);
 
     // rows past the last 64 in use are not written
     const int end = (used + 63) / 64 * 64 - blk * TM, live = end < TM ? end : TM;

@@ -20,23 +20,19 @@ struct MoeRowsParams {
     int wgs;                    // workgroups (k_moe_gemm: rows of the grid) in front of a stage's tiles that make the lists; 0 = none
 };
 
-// Workgroups that make the lists above.  The stages of k_moe_gemm and k_moe_mx have them in front of their own tiles, where they work beside
+// Workgroups that make the lists above.  The stages have them in front of their own tiles, where they work beside
 // these and cost no time of their own (behind the tiles their own 15 us are the end of the launch: MX stage 2, 4096 tokens x top-8, 242 us against
-// 231); the 256-row tiles (one workgroup a CU, not a register to spare: with the lists in the same kernel it spilled 28 instead of 18 of
-// them and lost 20 us) have them in a launch in front.  (One launch that cleared the counts and
-// another that entered the rows took 9.5 us, 1024 or 4096 tokens x top-8; as one launch it is 8.  Whole layers, us before / now: int4 1052 tokens x
-// top-8, 1536 x 1024, 128 / 124; int8 813 x top-4, 4096 x 512, 140 / 135; MX 410 x top-8, 4096 x 1536, 140.6 / 134.6; 1500 x top-6, 2048 x 768, 99 /
-// 93; 4096 x top-8 602 / 596; fp8 on 256-row tiles, which the power limit bounds, 807 / 809.)  A multiple of 8 leaves every tile on its XCD.
+// 231).  (One launch that cleared the counts and another that entered the rows took 9.5 us, 1024 or 4096 tokens x top-8.  Whole layers, us before / now: int4 1052
+// tokens x top-8, 1536 x 1024, 128 / 124; int8 813 x top-4, 4096 x 512, 140 / 135; MX 410 x top-8, 4096 x 1536, 140.6 / 134.6; 1500 x top-6, 2048 x 768, 99 /
+// 93; 4096 x top-8 602 / 596.)  A multiple of 8 leaves every tile on its XCD.
 constexpr int ROWS_INDEX_WGS = 32;
 
 // Every one of those workgroups looks through the whole list, so their work grows with its square; longer lists are made by two launches over
 // all CUs.  Beside the tiles of k_moe_gemm that is better from about 50,000 sorted rows on with blocks of 16 and 32 rows, 120,000 with 64 and 128 (us
 // beside the tiles / two launches, top-8 on 32 experts, 2048 x 512, fp8: blocks of 16 6000 tokens 249 / 247, 8192 356 / 350, 30000 1329 / 1293; of 32 8192 283 /
 // 282, 16384 582 / 574; of 64 8192 250 / 251, 12000 372 / 371, 16384 515 / 508, 30000 935 / 917; int4, 1024 x 256, 14000 tokens, blocks of 16, 64 and 128 268 / 263, 177 /
-// 179, 184 / 189); beside the MX pair's, with their 16 ids a thread, it never is (16384 tokens 394 / 402, 65536 1490 / 1492).  As a launch of their own, of 1024
-// threads a workgroup, the shares are the faster way up to about 40,000 rows (4096 tokens 8 / 9.5; stage 2 in blocks of 128 16384 tokens 570 / 563).
+// 179, 184 / 189); beside the MX pair's and the 128x256 tiles, with their 16 ids a thread, it never is (MX 16384 tokens 394 / 402, 65536 1490 / 1492).
 inline int moe_rows_share_max(int block_m) { return block_m <= 32 ? 50000 : 120000; }
-constexpr int ROWS_LAUNCH_MAX = 40000;
 
 uint64_t psg_moe_rows_bytes(int64_t tokens, int64_t topk, int64_t sorted_size, int64_t dim);
 void psg_moe_rows_carve(MoeRowsParams& p, void* workspace);

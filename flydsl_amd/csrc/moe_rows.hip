@@ -23,11 +23,6 @@ __device__ __forceinline__ void add_packed(uint32_t* o, int bits, int out_dtype)
     else __builtin_amdgcn_global_atomic_fadd_v2f16((__attribute__((address_space(1))) v2h_t*)o, __builtin_bit_cast(v2h_t, bits));
 }
 
-__global__ void __launch_bounds__(1024) k_moe_rows_index(MoeRowsParams p) {
-    __shared__ int lds[4096];
-    moe_rows_index_share<16>(p, (int)blockIdx.x, (int)gridDim.x, lds, 4096);
-}
-
 // The same lists by all CUs, from counts and heads in memory (a list's last place is the head of its chain).
 __global__ void __launch_bounds__(256) k_moe_rows_clear(MoeRowsParams p) {
     const int t = (int)blockIdx.x * 256 + (int)threadIdx.x;
@@ -110,14 +105,10 @@ void psg_moe_rows_carve(MoeRowsParams& p, void* workspace) {
     p.next = reinterpret_cast<int*>(w);
 }
 
-// the lists in launches of their own, for the stages that do not make them beside their tiles
+// the lists in launches of their own, where the stage does not make them beside its tiles
 hipError_t psg_launch_moe_rows_index(const MoeRowsParams& p, hipStream_t stream) {
-    if (p.sorted_size <= ROWS_LAUNCH_MAX) {
-        hipLaunchKernelGGL(k_moe_rows_index, dim3(ROWS_INDEX_WGS), dim3(1024), 0, stream, p);
-    } else {
-        hipLaunchKernelGGL(k_moe_rows_clear, dim3((p.tokens + 255) / 256), dim3(256), 0, stream, p);
-        hipLaunchKernelGGL(k_moe_rows_enter, dim3((p.sorted_size + 255) / 256), dim3(256), 0, stream, p);
-    }
+    hipLaunchKernelGGL(k_moe_rows_clear, dim3((p.tokens + 255) / 256), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(k_moe_rows_enter, dim3((p.sorted_size + 255) / 256), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 

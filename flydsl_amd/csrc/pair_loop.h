@@ -1,11 +1,12 @@
-// Mainloop of the 128x256 tile for fp4 operands with e8m0 scales on both sides, two workgroups per CU (gfx950): the dense
-// MXFP4 GEMM (gemm_mx_pair.hip) and both stages of the MX MoE pair on blocks of 128 sorted rows (moe_mx_gemm.hip).
+// Mainloop of the 128x256 tile that runs two workgroups per CU (gfx950), for fp4 operands with e8m0 scales on both sides, fp8 and int8: the dense
+// MXFP4 GEMM (gemm_mx_pair.hip) and the stages of both MoE pairs on blocks of 128 sorted rows (moe_mx_gemm.hip, moe_gemm_pair.hip).
 //
-// Four wavefronts side by side along N, each 128 rows x 64 weight rows (128 accumulator registers a lane), 256 elements of K a step:
+// Four wavefronts side by side along N, each 128 rows x 64 weight rows (128 accumulator registers a lane), 128 bytes of K a step:
 //   * A goes global -> LDS by DMA into four stages of 16 KB (rows of 128 bytes, 16-byte pieces XORed with row / 2), requested three steps
 //     ahead; a lane's source address is its row's, so rows may be gathered.
 //   * W never touches LDS: a wavefront's fragments are its own.  They are fetched three half steps (64 bytes of K) ahead into a ring of four
-//     half-step register sets; two whole-step sets need the same 64 registers and are ahead by half as much.
+//     half-step register sets; two whole-step sets need the same 64 registers and are ahead by half as much.  (fp8, whose MFMA takes both
+//     halves, has those: a step ahead.)
 //   * The scale dwords of a step, 4 chunks of 256 bytes on the A side and 8 on the W side, are one 16-byte DMA of three of the wavefronts: a DMA
 //     takes 64 lanes anywhere, so 16 lanes bring a chunk and one instruction four of them.
 //   * At most one memory instruction stands behind an MFMA: what is issued between two of them in a row, the matrix cores wait for (one
@@ -20,27 +21,33 @@
 
 namespace {
 
-struct MxPair {
+template <int KIND>
+struct Pair {
     static constexpr int MR = 8, NR = 4, NS = 4;  // 16-row blocks of A, of W a wavefront; LDS stages
     static constexpr int TM = 128, TN = 256;
     static constexpr int STAGE = TM * TK;         // bytes of one A stage
-    static constexpr int SC_SLOT = 12 * 256;      // scale dwords of a step
+    static constexpr int SC_SLOT = KIND == KIND_MXFP4 ? 12 * 256 : 0;  // scale dwords of a step
     static constexpr int LDS_BYTES = NS * (STAGE + SC_SLOT);
     static_assert(2 * LDS_BYTES + 2048 <= 160 * 1024, "two workgroups a CU, with 1 KB each for what a kernel adds");
 };
+using MxPair = Pair<KIND_MXFP4>;
 
 // acc[mi][ni] = A (rows 16 mi ..) x W (the wavefront's 16-row block ni) over KT steps; 0 without any.
 //   lds      LDS_BYTES, 1 KB aligned: the A stages, behind them the scale slots; free again at the end
 //   a_voff   this lane's offsets into `ra` of the four 1 KB blocks (8 rows) that its wavefront fetches of a stage: of row (4 wave + j) 8 + lane / 8,
 //            16-byte piece (lane % 8) ^ (row / 2 % 8); out of the descriptor's bounds for a row that reads as zero
 //   b_voff   this lane's offsets into `rb` of the wavefront's four 16-row blocks
+// fp4 only (rs: any descriptor otherwise):
 //   s_voff   this lane's offset into `rs`, the scales of wavefront 0 and 3: A side, 1 and 2: W side chunks 0..3 and 4..7 of the tile: chunk
 //            lane / 16, 16-byte piece lane % 16
 //   chunk0/1 which of the eight W-side chunks belong to the wavefront's blocks 0, 1 and 2, 3
-__device__ __forceinline__ void mx_pair_loop(v4f (&acc)[MxPair::MR][MxPair::NR], uint8_t* lds, const __amdgpu_buffer_rsrc_t ra, const uint32_t (&a_voff)[4],
-                                             const __amdgpu_buffer_rsrc_t rb, const uint32_t (&b_voff)[MxPair::NR], const __amdgpu_buffer_rsrc_t rs,
-                                             const uint32_t s_voff, const int chunk0, const int chunk1, const int KT, const int wave, const int lane) {
-    constexpr int MR = MxPair::MR, NR = MxPair::NR, NS = MxPair::NS, STAGE = MxPair::STAGE, SC_SLOT = MxPair::SC_SLOT;
+template <int KIND, class ACC>
+__device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const __amdgpu_buffer_rsrc_t ra, const uint32_t (&a_voff)[4],
+                                          const __amdgpu_buffer_rsrc_t rb, const uint32_t (&b_voff)[4], const int KT, const int wave, const int lane,
+                                          const __amdgpu_buffer_rsrc_t rs, const uint32_t s_voff = 0, const int chunk0 = 0, const int chunk1 = 0) {
+    using P = Pair<KIND>;
+    constexpr int MR = P::MR, NR = P::NR, NS = P::NS, STAGE = P::STAGE, SC_SLOT = P::SC_SLOT;
+    constexpr bool MX = KIND == KIND_MXFP4, WHOLE = KIND == KIND_FP8;  // WHOLE: an MFMA takes both halves of a step
     const int li = lane & 15, lg = lane >> 4;
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
     uint8_t* const lds_x = lds + NS * STAGE;
@@ -48,7 +55,7 @@ __device__ __forceinline__ void mx_pair_loop(v4f (&acc)[MxPair::MR][MxPair::NR],
     const uint32_t sc_dst = lds_base + (uint32_t)(NS * STAGE) + (uint32_t)(wave == 3 ? 0 : wave) * 1024u;
 
     // DMA j of step kt: 0..3 A, 4 scales.  Without CHK the step is known to be before the end
-    constexpr int N_DMA = 5;
+    constexpr int N_DMA = MX ? 5 : 4;
     auto dma = [&](int kt, int stage, int j, auto CHK) __attribute__((always_inline)) {
         const bool has = !decltype(CHK)::value || kt < KT;
         if (j < 4) dma16(ra, lds_base + (uint32_t)(stage * STAGE + (wave * 4 + j) * 1024), has ? a_voff[j < 4 ? j : 0] : 0xFFFFFFF0u, has ? (uint32_t)kt * TK : 0u);
@@ -71,28 +78,53 @@ __device__ __forceinline__ void mx_pair_loop(v4f (&acc)[MxPair::MR][MxPair::NR],
         else sbv[set][q < 4 ? 0 : q - 4] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + 1024 + (q == 4 ? chunk0 : chunk1) * 256 + lane * 4);
     };
 
+    // fp8: eight m-blocks of four MFMAs of 32 cycles; the DMAs of step kt + 3, then the W fragments of the next step into the other set, early in
+    // the step, the A fragments an m-block ahead
+    auto whole_step = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
+        constexpr int S = decltype(SP)::value, B0 = 2 * (S & 1), B1 = 2 - B0;  // sets of W: halves B0, B0 + 1 and B1, B1 + 1
+        static_for<MR>([&](auto MI) {
+            constexpr int mi = decltype(MI)::value, f = 2 * (mi & 1), fn = 2 - f;
+            static_for<NR>([&](auto NI) {
+                constexpr int ni = decltype(NI)::value, slot = mi * NR + ni;
+                const v8i a = {fr[f][0], fr[f][1], fr[f][2], fr[f][3], fr[f + 1][0], fr[f + 1][1], fr[f + 1][2], fr[f + 1][3]};
+                const v8i b = {bw[B0][ni][0], bw[B0][ni][1], bw[B0][ni][2], bw[B0][ni][3], bw[B0 + 1][ni][0], bw[B0 + 1][ni][1], bw[B0 + 1][ni][2], bw[B0 + 1][ni][3]};
+                if constexpr (WHOLE) mfma_f8(acc[mi][ni], b, a);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (ni < 2) {
+                    if constexpr (mi + 1 < MR) read_frag(S, ni, mi + 1, fr[fn + ni]);
+                    else read_frag((S + 1) % NS, ni, 0, fr[fn + ni]);
+                }
+                if constexpr (slot >= 3 && slot < 7) dma(kt + 3, (S + 3) % NS, slot - 3, CHK);
+                if constexpr (slot >= 7 && slot < 15) load_w(kt + 1, slot & 1, (slot - 7) / 2, bw[B1 + (slot & 1)], CHK);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NR + N_DMA + 2 * NR) : "memory");
+    };
+
     // Step kt (kt % 4 = S): sixteen blocks of four MFMAs, eight m-blocks of the lower half of K and eight of the upper.  A's stage and scales of the step
     // have landed for everybody a step ago, so its first fragments and scales were read before the barrier in front of it.
-    auto step = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
+    auto half_steps = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
         constexpr int S = decltype(SP)::value, SS = S & 1;
         static_for<16>([&](auto BI) {
             constexpr int b = decltype(BI)::value, half = b >> 3, mi = b & 7, nb = b + AHEAD;
             static_for<NR>([&](auto NI) {
                 constexpr int ni = decltype(NI)::value;
-                mfma_mx<half, ni & 1, mi & 1>(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3], sbv[SS][ni / 2], sav[SS][mi / 2]);
+                if constexpr (MX) mfma_mx<half, ni & 1, mi & 1>(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3], sbv[SS][ni / 2], sav[SS][mi / 2]);
+                else if constexpr (!WHOLE) mfma_i8(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (ni == 0) {
                     if constexpr (nb < 16) read_frag(S, nb >> 3, nb & 7, fr[nb & 3]);
                     else read_frag((S + 1) % NS, 0, nb - 16, fr[nb & 3]);
                 }
-                if constexpr (ni == 1 && b >= 10) read_sc((S + 1) % NS, b - 10, SS ^ 1);
+                if constexpr (MX && ni == 1 && b >= 10) read_sc((S + 1) % NS, b - 10, SS ^ 1);
                 // The DMAs of step kt + 3 and the W fragments three half steps ahead.  The compiler counts only the loads it knows, W's, so its waits
                 // for W let as many instructions be on their way as there are W loads behind the awaited one, DMAs among them: in each half the DMAs
                 // go first, and both halves have some.
                 if constexpr (ni == 2) {
                     if constexpr (b >= 1 && b < 4) dma(kt + 3, (S + 3) % NS, b - 1, CHK);
                     if constexpr (b >= 4 && b < 8) load_w(kt + 1, 1, b - 4, bw[(2 * S + 3) % 4], CHK);
-                    if constexpr (b >= 9 && b < 11) dma(kt + 3, (S + 3) % NS, b - 6, CHK);
+                    if constexpr (b >= 9 && b < (MX ? 11 : 10)) dma(kt + 3, (S + 3) % NS, b - 6, CHK);
                     if constexpr (b >= 11 && b < 15) load_w(kt + 2, 0, b - 11, bw[(2 * S + 4) % 4], CHK);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -103,27 +135,48 @@ __device__ __forceinline__ void mx_pair_loop(v4f (&acc)[MxPair::MR][MxPair::NR],
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(NR + N_DMA + 2 * NR) : "memory");
     };
 
-    // prologue: A and scales of steps 0 and 1, W of the first half step, A and scales of step 2, W of the two half steps behind
+    auto step = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
+        if constexpr (WHOLE) whole_step(kt, SP, CHK);
+        else half_steps(kt, SP, CHK);
+    };
+
+    // prologue: A and scales of steps 0 and 1, W of the first half step, A and scales of step 2, W of the two half steps behind (fp8: A of steps 0
+    // to 2, W of step 0)
 #pragma unroll
     for (int s = 0; s < 2; s++)
 #pragma unroll
         for (int j = 0; j < N_DMA; j++) dma(s, s, j, std::true_type{});
+    if constexpr (!WHOLE) {
 #pragma unroll
-    for (int ni = 0; ni < NR; ni++) load_w(0, 0, ni, bw[0], std::true_type{});
+        for (int ni = 0; ni < NR; ni++) load_w(0, 0, ni, bw[0], std::true_type{});
+    }
 #pragma unroll
     for (int j = 0; j < N_DMA; j++) dma(2, 2, j, std::true_type{});
+    if constexpr (WHOLE) {
+#pragma unroll
+        for (int ni = 0; ni < NR; ni++) load_w(0, 0, ni, bw[0], std::true_type{});
+    }
 #pragma unroll
     for (int ni = 0; ni < NR; ni++) load_w(0, 1, ni, bw[1], std::true_type{});
+    if constexpr (!WHOLE) {
 #pragma unroll
-    for (int ni = 0; ni < NR; ni++) load_w(1, 0, ni, bw[2], std::true_type{});
+        for (int ni = 0; ni < NR; ni++) load_w(1, 0, ni, bw[2], std::true_type{});
+    }
 #pragma unroll
     for (int mi = 0; mi < MR; mi++)
 #pragma unroll
-        for (int ni = 0; ni < NR; ni++) acc[mi][ni] = (v4f){0.f, 0.f, 0.f, 0.f};
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(3 * NR + N_DMA) : "memory");
-    static_for<AHEAD>([&](auto I) { read_frag(0, 0, decltype(I)::value, fr[decltype(I)::value]); });
+        for (int ni = 0; ni < NR; ni++) acc[mi][ni] = (ACC){0, 0, 0, 0};
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((WHOLE ? 2 : 3) * NR + N_DMA) : "memory");
+    if constexpr (WHOLE) {
+        read_frag(0, 0, 0, fr[0]);
+        read_frag(0, 1, 0, fr[1]);
+    } else {
+        static_for<AHEAD>([&](auto I) { read_frag(0, 0, decltype(I)::value, fr[decltype(I)::value]); });
+    }
+    if constexpr (MX) {
 #pragma unroll
-    for (int q = 0; q < 6; q++) read_sc(0, q, 0);
+        for (int q = 0; q < 6; q++) read_sc(0, q, 0);
+    }
 
     // four steps an iteration (stages and register sets are compile-time); the first loop while every load of it is before the end, then with
     // checks, then what is left

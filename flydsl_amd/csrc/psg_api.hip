@@ -992,7 +992,7 @@ static int moe_gemm_common(const psg_moe_args* a, void* workspace, uint64_t work
     p.doweight = a->doweight ? 1 : 0;
     p.accumulate = a->stage == 2 && a->accumulate ? 1 : 0;
     p.by_position = 0;
-    p.blocks = p.group_m = 0;
+    p.blocks = 0;
     hipError_t e = hipSuccess;
     const bool rows = workspace && p.accumulate && a->out_dtype != PSG_OUT_F32 && workspace_bytes >= psg_moe_rows_bytes(a->tokens, a->topk, a->sorted_size, n_out);
     MoeRowsParams r{};

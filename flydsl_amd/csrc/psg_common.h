@@ -191,7 +191,7 @@ struct MoeParams {
     int doweight;               // multiply by the routing weight in this stage
     int accumulate;             // stage 2: atomic add into out[token] (else one row per (token, slot))
     int x_slot_major;           // stage 1: x / sx hold one row per (slot, token) at slot*tokens + token
-    int blocks, group_m;        // set by the launcher of the 256-row tiles: entries of expert_ids, tiles per group of the XCD order
+    int blocks;                 // set by the launcher of the 128x256 tiles: entries of expert_ids
     int by_position;            // stage 2 without accumulate: one row per sorted position instead of one per (token, slot)
     int pair_blocks;            // blocks of 16 / 32 rows: multiply two consecutive blocks of one expert in one workgroup
 };
