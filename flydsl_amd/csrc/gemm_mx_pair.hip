@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(256, 2) k_mx_pair(A8W8Params p) {
     const uint32_t s_voff = (uint32_t)((a_side ? 0 : (wave - 1) * 4) + (lane >> 4)) * chunk_bytes + (uint32_t)(lane & 15) * 16u;
 
     v4f acc[MR][NR];
-    pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, KT, wave, lane, rs, s_voff, wave * 2, wave * 2 + 1);
+    pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, KT * TK, wave, lane, 2048u, 1024u, rs, s_voff, wave * 2, wave * 2 + 1);
 
     if constexpr (STORE == STORE_ACC) {
         static_for<MR>([&](auto MI) {

@@ -32,6 +32,8 @@
 #include "psg_common.h"
 #include "tile_order.h"
 
+hipError_t psg_launch_pair(const A8W8Params& p, int kind, int store, hipStream_t stream);
+
 namespace {
 
 constexpr int TK = 128;  // bytes of K per mainloop step
@@ -108,10 +110,7 @@ __device__ __forceinline__ void tile_coords(int id, int tiles_m, int tiles_n, in
 // lane into the K loop when forced: MXFP4 4096x7168x2048 82 us).
 // STORE: STORE_ACC dumps raw accumulators; STORE_C writes bf16 with no bias/activation (the common case, kept
 // free of run-time epilogue switches); STORE_C_GENERIC handles fp16 output and the fused bias/activation variants.
-// OCC > 0 overrides that rule: the 128x256 tile of the 8- and 16-bit kinds spills 20-50 bytes per lane when held to two
-// workgroups per CU, which only pays when there are more tiles than CUs (fp8 8192x4096x4096: 127 us against 150 with one
-// workgroup per CU); with at most one tile per CU the unconstrained build is faster (int8 1024x8192x8192: 68 us against
-// 106, fp8 67 against 76), so the launcher picks per problem.
+// OCC > 0 overrides that rule (the 128x128 tile with four register sets).
 // PFW = K steps the W fragments are fetched ahead of their MFMAs (PFW + 1 register sets).  1 for problems that fill the GPU
 // (the MFMAs of a step hide one memory latency).  3 for the few-tile / split-K regime, where a workgroup's MFMAs take no time
 // and the launch is bound by the bytes of W in flight: one 128x128 tile per CU with one step ahead keeps 16 KB per CU on
@@ -558,17 +557,14 @@ hipError_t launch_shape(const A8W8Params& p, int tile_m, int tile_n, hipStream_t
     }
     PSG_CASE(16, 4, 1)
     PSG_CASE(8, 8, 1)
+    // the 128x256 tile of the 8- and 16-bit kinds has a kernel of its own too (gemm_pair.hip)
     if constexpr (KIND != KIND_MXFP8) {
-        // 128x256 with at most one tile per CU: the build that is not held to two workgroups per CU
-        if (tile_m == 128 && tile_n == 256) {
-            const long tiles = (long)((p.M + 127) / 128) * (long)((p.N + 255) / 256) * (STORE == STORE_ACC && p.splits > 1 ? p.splits : 1);
-            if (tiles <= 256) return launch_one<KIND, 8, 4, 1, STORE, 4, 1>(p, stream);
-        }
+        if (tile_m == 128 && tile_n == 256) return psg_launch_pair(p, KIND, STORE, stream);
     }
-    PSG_CASE(8, 4, 1)
     PSG_CASE(4, 4, 1)
     PSG_CASE(2, 4, 1)
     if constexpr (KIND == KIND_MXFP8) {
+        PSG_CASE(8, 4, 1)
         PSG_CASE(4, 2, 1)
         PSG_CASE(2, 2, 1)
     } else {

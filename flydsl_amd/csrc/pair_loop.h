@@ -32,23 +32,27 @@ struct Pair {
 };
 using MxPair = Pair<KIND_MXFP4>;
 
-// acc[mi][ni] = A (rows 16 mi ..) x W (the wavefront's 16-row block ni) over KT steps; 0 without any.
+// acc[mi][ni] = A (rows 16 mi ..) x W (the wavefront's 16-row block ni) over K bytes of a row (multiples of 64); 0 without any.
 //   lds      LDS_BYTES, 1 KB aligned: the A stages, behind them the scale slots; free again at the end
 //   a_voff   this lane's offsets into `ra` of the four 1 KB blocks (8 rows) that its wavefront fetches of a stage: of row (4 wave + j) 8 + lane / 8,
 //            16-byte piece (lane % 8) ^ (row / 2 % 8); out of the descriptor's bounds for a row that reads as zero
-//   b_voff   this lane's offsets into `rb` of the wavefront's four 16-row blocks
+//   b_voff   this lane's offsets into `rb` of the wavefront's four 16-row blocks, b_step and b_half from a step and a half step to the next (2048 and 1024 in the
+//            preshuffled order)
 // fp4 only (rs: any descriptor otherwise):
 //   s_voff   this lane's offset into `rs`, the scales of wavefront 0 and 3: A side, 1 and 2: W side chunks 0..3 and 4..7 of the tile: chunk
 //            lane / 16, 16-byte piece lane % 16
 //   chunk0/1 which of the eight W-side chunks belong to the wavefront's blocks 0, 1 and 2, 3
 template <int KIND, class ACC>
 __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const __amdgpu_buffer_rsrc_t ra, const uint32_t (&a_voff)[4],
-                                          const __amdgpu_buffer_rsrc_t rb, const uint32_t (&b_voff)[4], const int KT, const int wave, const int lane,
-                                          const __amdgpu_buffer_rsrc_t rs, const uint32_t s_voff = 0, const int chunk0 = 0, const int chunk1 = 0) {
+                                          const __amdgpu_buffer_rsrc_t rb, const uint32_t (&b_voff)[4], const int K, const int wave, const int lane,
+                                          const uint32_t b_step, const uint32_t b_half, const __amdgpu_buffer_rsrc_t rs, const uint32_t s_voff = 0, const int chunk0 = 0, const int chunk1 = 0) {
     using P = Pair<KIND>;
     constexpr int MR = P::MR, NR = P::NR, NS = P::NS, STAGE = P::STAGE, SC_SLOT = P::SC_SLOT;
     constexpr bool MX = KIND == KIND_MXFP4, WHOLE = KIND == KIND_FP8;  // WHOLE: an MFMA takes both halves of a step
     const int li = lane & 15, lg = lane >> 4;
+    const int KT = (K + TK - 1) / TK, KF = K / TK;  // steps, whole steps
+    // 16-byte piece of its row that this lane fetches, by the parity of the block (the rows of a block count from 8 j)
+    const int a_kc[2] = {(lane & 7) ^ (lane >> 4), (lane & 7) ^ (lane >> 4) ^ 4};
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
     uint8_t* const lds_x = lds + NS * STAGE;
     // (wavefront 3 brings the bytes of wavefront 0 once more: all of them count the same number of DMAs)
@@ -57,14 +61,14 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
     // DMA j of step kt: 0..3 A, 4 scales.  Without CHK the step is known to be before the end
     constexpr int N_DMA = MX ? 5 : 4;
     auto dma = [&](int kt, int stage, int j, auto CHK) __attribute__((always_inline)) {
-        const bool has = !decltype(CHK)::value || kt < KT;
-        if (j < 4) dma16(ra, lds_base + (uint32_t)(stage * STAGE + (wave * 4 + j) * 1024), has ? a_voff[j < 4 ? j : 0] : 0xFFFFFFF0u, has ? (uint32_t)kt * TK : 0u);
+        const bool has = !decltype(CHK)::value || kt < KT, in = !decltype(CHK)::value || kt * TK + a_kc[j & 1] * 16 < K;
+        if (j < 4) dma16(ra, lds_base + (uint32_t)(stage * STAGE + (wave * 4 + j) * 1024), in ? a_voff[j < 4 ? j : 0] : 0xFFFFFFF0u, has ? (uint32_t)kt * TK : 0u);
         else dma16(rs, sc_dst + (uint32_t)(stage * SC_SLOT), has ? s_voff : 0xFFFFFFF0u, has ? (uint32_t)kt * 256u : 0u);
     };
     v4i bw[4][NR];
     auto load_w = [&](int kt, int half, int ni, v4i* dst, auto CHK) __attribute__((always_inline)) {
-        const bool has = !decltype(CHK)::value || kt < KT;
-        dst[ni] = buf_load16(rb, has ? b_voff[ni] : 0xFFFFFFF0u, has ? (uint32_t)kt * 2048u + (uint32_t)half * 1024u : 0u);
+        const bool has = !decltype(CHK)::value || kt * TK + half * 64 < K;
+        dst[ni] = buf_load16(rb, has ? b_voff[ni] : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
     };
     const int f_base[2] = {li * TK + ((lg ^ ((li >> 1) & 7)) << 4), li * TK + (((4 + lg) ^ ((li >> 1) & 7)) << 4)};
     constexpr int AHEAD = 2;  // blocks of four MFMAs that an A fragment is read ahead
@@ -111,7 +115,9 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
             static_for<NR>([&](auto NI) {
                 constexpr int ni = decltype(NI)::value;
                 if constexpr (MX) mfma_mx<half, ni & 1, mi & 1>(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3], sbv[SS][ni / 2], sav[SS][mi / 2]);
-                else if constexpr (!WHOLE) mfma_i8(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
+                else if constexpr (KIND == KIND_INT8) mfma_i8(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
+                else if constexpr (KIND == KIND_BF16) mfma_bf16(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
+                else if constexpr (KIND == KIND_FP16) mfma_f16(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (ni == 0) {
                     if constexpr (nb < 16) read_frag(S, nb >> 3, nb & 7, fr[nb & 3]);
@@ -181,7 +187,7 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
     // four steps an iteration (stages and register sets are compile-time); the first loop while every load of it is before the end, then with
     // checks, then what is left
     int kt = 0;
-    for (; kt + 7 <= KT; kt += NS) static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::false_type{}); });
+    for (; kt + 7 <= KF; kt += NS) static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::false_type{}); });
     for (; kt + NS <= KT; kt += NS) static_for<NS>([&](auto I) { step(kt + decltype(I)::value, I, std::true_type{}); });
     static_for<NS - 1>([&](auto I) {
         if (kt + decltype(I)::value < KT) step(kt + decltype(I)::value, I, std::true_type{});

@@ -144,12 +144,9 @@ struct Tile {
     int waves;  // wavefronts per workgroup: 4 (side by side along N, or 2x2) or 8 (side by side along N)
 };
 
-// Tile choice for the MFMA mainloop.  Each shape has a measured relative efficiency at full occupancy.  The 256x256
-// tile of eight wavefronts side by side along N loads every W fragment once per CU and moves the least data per flop:
-// on real data the chip is power-limited, so that is what decides (fp8 8192x4096x4096: 117 us against 134 us for
-// the 128x256 tile that runs two workgroups per CU; int8 4096x28672x8192: 775 against 940).  The MX table is for fp8 x fp8; an fp4 x fp4 problem takes from it
-// only whether and how its K is split (over 18 such problems 1 % from the best of that and the unsplit tiles).  The score multiplies the efficiency by
-// how evenly the tiles fill the CUs' workgroup slots and by the fraction of each tile that is not padding.
+// Tile by score: what the split rules below start from, and the tile of an fp8 x fp8 problem unless an estimate is better (other problems whose K isn't split take
+// the smallest estimate).  Each shape has a measured relative efficiency at full occupancy; the score multiplies it by how evenly the tiles fill the CUs'
+// workgroup slots and by the fraction of each tile that is not padding.
 Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
     struct Shape {
         int m, n, waves, per_cu;
@@ -203,7 +200,7 @@ Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
 // last-level cache.
 struct TileCost {
     int m, n, waves, per_cu;
-    double start, round, step[5];  // us; step[r]: r tiles on a CU
+    double start, round, step[6];  // us; step[r]: r tiles on a CU
 };
 
 // mem: us of the memory bus; near that bound a launch takes longer than either estimate
@@ -222,24 +219,30 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
     return c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
 }
 
-// Of the three large tiles of the 8- and 16-bit kinds the one with the smallest estimate, where that is 7 % below the planned one's.  On 151 drawn
-// problems, most weights in memory, the estimates are 12 % off (r.m.s.); 17 take another tile, 14 % faster on average and none slower (us
-// planned / estimate: fp8 1614x4896x6656 87.6 / 61.2, 4329x1840x1856 31.9 / 23.0, 411x16720x2944 41.7 / 34.1, 3683x2288x8448 91.6 / 81.9).  The estimates of
-// smaller tiles are too coarse to add them (64x64 with them: 433x8560x8768 57 / 66).
-Tile pick_large_tile(Tile planned, int M, int N, int kbytes) {
-    static const TileCost costs[] = {{256, 256, 8, 1, 0.0, 7.0, {0, 1.17}}, {128, 256, 4, 2, 2.3, 7.1, {0, 0.77, 1.52}}, {128, 128, 4, 2, 5.0, 1.4, {0, 0.40, 0.91}}};
+// Tile of an 8- or 16-bit problem whose K isn't split: the one with the smallest estimate.  On 299 timed problems (33 to 8192 rows, weights in memory and in the
+// last-level cache) that are neither split nor streamed, the estimates are 7 to 11 % off (r.m.s.) and the chosen tile takes 0.7 % longer than the best of the five, at
+// worst 10 % (fp8 4197x1088x11904 79 on 128x256, 72 on 128x128).  us by the tiles' scores, with the 128x256 tile of that time / by estimate: int8 813x7600x3136
+// 30.1 / 22.4, 1416x3136x5568 41.8 / 31.2; fp8 137x16656x1152 13.5 / 10.8; bf16 3156x1536x2752 39.1 / 28.7, 643x9088x1344 25.0 / 18.4.
+// Two tiles are left out where they read W from memory more often than the estimate sees (us, W in memory): 64x256 up to 128 rows, where one row of 128x128 tiles does
+// (64x256 / 128x128: fp8 96x28672x4096 33.0 / 31.4, bf16 80x26624x1280 20.7 / 19.8, 128x28672x4096 59.5 / 54.1), and 64x64 on long rows (64x64 / 128x128: fp8
+// 302x5872x9920 43.4 / 38.6, bf16 302x5872x6208 50.6 / 45.7).
+Tile pick_plain_tile(int M, int N, int kbytes, bool wide, bool long_rows) {
+    static const TileCost costs8[] = {{256, 256, 8, 1, 0.0, 6.7, {0, 1.25}}, {128, 256, 4, 2, 4.8, 0.2, {0, 0.75, 1.60}}, {128, 128, 4, 2, 5.7, 0.0, {0, 0.47, 0.99}},
+                                      {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};
+    static const TileCost costs16[] = {{256, 256, 8, 1, 0.0, 5.1, {0, 1.26}}, {128, 256, 4, 2, 2.7, 0.0, {0, 0.71, 1.54}}, {128, 128, 4, 2, 4.8, 0.0, {0, 0.51, 0.94}},
+                                       {64, 64, 4, 5, 2.4, 0.0, {0, 0.33, 0.43, 0.64, 0.91, 0.99}}, {64, 256, 4, 2, 3.3, 0.0, {0, 0.60, 1.08}}};
     const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;
-    double best = 1e30, kept = 0;
-    Tile t = planned;
-    for (const TileCost& c : costs) {
+    double best = 1e30;
+    Tile t{};
+    for (const TileCost& c : wide ? costs16 : costs8) {
+        if ((c.m == 64 && c.n == 256 && M <= 128) || (c.n == 64 && long_rows)) continue;
         const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
-        if (c.m == planned.m && c.n == planned.n) kept = us;
         if (us < best) {
             best = us;
             t = {c.m, c.n, c.waves};
         }
     }
-    return best < 0.93 * kept ? t : planned;
+    return t;
 }
 
 // Tile of an MX problem whose K isn't split (kbytes: of a row of A): of an fp4 x fp4 or fp8 / fp6 x fp4 problem the one with the smallest estimated time; of
@@ -441,7 +444,8 @@ struct Plan {
     Tile t;
     int splits;
 };
-Plan plan_tiled(int M, int N, int kbytes, bool mx) {
+// wide: 16-bit operands
+Plan plan_tiled(int M, int N, int kbytes, bool mx, bool wide) {
     // more columns than the streaming kernel takes in one round: 64x64 tiles, unsplit (these problems have no workspace)
     if (!mx && stream_holds(M, N, kbytes) && N > 32 * psg_cu_count()) return {Tile{64, 64, 4}, 1};
     Tile t = pick_tile(M, N, mx, 0, 0);
@@ -452,14 +456,16 @@ Plan plan_tiled(int M, int N, int kbytes, bool mx) {
     // (tiles x steps, i.e. M N K / 2^19, up to 11,000: then twice as many workgroups count for more than the W fragments that are
     // loaded twice; fp8, us, 64x64 plan against 128x128 plan: 256x2112x7168 14.8 / 16.8; 320x2112x7168 15.6 / 18.4; 320x1664x10240
     // 18.3 / 20.2; 128x2048x16384 19.2 / 21.2; but 256x2304x14336 27.1 / 23.9; 320x2048x16384 30.0 / 26.3; 65x5120x13824 25.8 / 23.4)
-    if (!mx && tiles_big < psg_cu_count() * 3L / 4 && steps >= 48) t = M <= 64 || tiles64 * steps <= 11000 ? Tile{64, 64, 4} : Tile{128, 128, 4};
+    const bool long_rows = !mx && tiles_big < psg_cu_count() * 3L / 4 && steps >= 48;
+    bool fixed = long_rows && (M <= 64 || tiles64 * steps <= 11000);
+    if (long_rows) t = fixed ? Tile{64, 64, 4} : Tile{128, 128, 4};
     // Shorter rows (8..47 steps; K = 4096 one-byte elements is 32): while at most about 600 of them exist, 64x64 tiles beat
     // every larger shape, with or without split-K: many small workgroups keep more bytes of W in flight than a few large ones
     // (fp8, weights not cache-resident: M=128, N=K=4096 14.0 us against 19.4 with 128x128 tiles and two K splits; M=256,
     // N=8192 22.0 against 23.7; M=384, N=8192, 768 tiles: 28.0 against 26.5, so the larger tile is kept there)
-    if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4};
+    if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4}, fixed = true;
     const int splits = mx && mx_small_holds(M, N, kbytes * 2) ? 1 : pick_splits(M, N, kbytes, t);
-    if (splits == 1) t = mx ? pick_mx_tile(M, N, kbytes, MX_FP4) : pick_large_tile(t, M, N, kbytes);
+    if (splits == 1 && !fixed) t = mx ? pick_mx_tile(M, N, kbytes, MX_FP4) : pick_plain_tile(M, N, kbytes, wide, long_rows);
     return {t, splits};
 }
 
@@ -611,7 +617,7 @@ int run_a8w8(const psg_a8w8_args* a, void* out, int store, void* stream) {
         e = psg_launch_a8w8_stream(p, kind, store, static_cast<hipStream_t>(stream));
     } else {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
-        const Plan plan = plan_tiled(a->M, a->N, kbytes, false);
+        const Plan plan = plan_tiled(a->M, a->N, kbytes, false, kind == KIND_FP16 || kind == KIND_BF16);
         const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : plan.t;
         p.ksplit = 1;
         // wavefront layout of the 256x256 tile: the planner's choice, or forced (2 = 2x2, 8 = 1x8) by tests / tuning
@@ -666,7 +672,7 @@ uint64_t psg_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t in_dtype) 
     const bool mx = in_dtype == 4;  // MXFP4 (psg_gemm_mxfp4)
     const int kbytes = mx ? K / 2 : ((in_dtype == PSG_IN_FP16 || in_dtype == PSG_IN_BF16) ? K * 2 : K);
     if (mx ? mx_takes_small(M, N, K) : takes_stream(M, N, kbytes)) return 0;  // the small-M kernels reduce inside their workgroups
-    return splitk_bytes(M, N, plan_tiled(M, N, kbytes, mx).splits);
+    return splitk_bytes(M, N, plan_tiled(M, N, kbytes, mx, false).splits);
 }
 
 int psg_gemm_a8w8(const psg_a8w8_args* args, void* stream) {
@@ -884,7 +890,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         e = psg_launch_mxfp4_smallm(p, store, nw, static_cast<hipStream_t>(stream));
     } else {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
-        const Plan plan = plan_tiled(a->M, a->N, a->K / 2, true);
+        const Plan plan = plan_tiled(a->M, a->N, a->K / 2, true, false);
         const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : plan.t;
         int splits = forced ? (a->tile_k >= 1 && a->tile_k <= 16 ? a->tile_k : 1) : plan.splits;
         if (store != STORE_C || !a->workspace || !aligned(a->workspace, 16) || a->workspace_bytes < splitk_bytes(a->M, a->N, splits)) splits = 1;
