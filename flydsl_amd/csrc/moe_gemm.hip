@@ -57,10 +57,11 @@ __device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g));
 // of 16 or 32 rows: an expert with 17 to 32 routed rows would otherwise stream its weights once per block).  Blocks pair up
 // from the start of each run of equal expert ids: the workgroup of the second block of a pair ends at once, and the
 // first one treats the second half of its tile as padding when the run ends there.
-// DEEP: operands three steps ahead (the rule and its figures: takes_deep; a stage by rows never, having more workgroups than that).
+// AHEAD: 0 = operands a step ahead; 1 = three steps (the rule and its figures: takes_deep; a stage by rows never, having more workgroups than that); 2 = three steps,
+// and W past the caches (takes_nt).
 // ROWS = MoeRowsParams: the down stage by rows, whose first `rows.wgs` rows of the grid make the lists of the tokens' rows.  A build of
 // its own: the decode layers, which add directly, lost 0.4 to 0.8 us of 55 to 140 to the longer arguments and the branch.
-template <int KIND, int MR, int NR, int STAGE, int CO, bool DEEP, class... ROWS>
+template <int KIND, int MR, int NR, int STAGE, int CO, int AHEAD, class... ROWS>
 __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     using acc_t = typename MoeAcc<KIND>::type;
     constexpr int BM = 16 * MR, TN = 64 * NR;
@@ -69,6 +70,8 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     constexpr int A_LOADS = (BM * 8 + 255) / 256;      // 16-byte chunks of the A tile per thread
     constexpr bool W4 = KIND == KIND_INT8W4;           // packed int4 weights
     constexpr int WSH = W4 ? 1 : 0;                    // weight byte offsets are halved
+    constexpr bool DEEP = AHEAD != 0;
+    constexpr int W_CACHE = AHEAD == 2 ? 2 : 0;        // cache policy of a W load: nt or none
     __shared__ __attribute__((aligned(16))) uint8_t lds[2][BM * 128];
     __shared__ int ids[BM];
     __shared__ float s_sx[BM], s_rw[BM];  // per tile row: scale of its x row and routing weight, fetched before the K loop
@@ -142,13 +145,12 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
             if (a_ldsoff[j] >= 0) *reinterpret_cast<v4i*>(&lds[stage][a_ldsoff[j]]) = areg[set][j];
     };
     using wreg_t = typename std::conditional<W4, v2i, v4i>::type;  // a lane's piece of a W fragment as it is loaded
-    // DEEP: A and W are both asked for three steps ahead, in rings of four register sets (loads return in order, so A has to be as far ahead as W).
-    // W register sets: the fragments of step kt live in set kt % NWS and are requested WPF steps ahead.  Stage-1 tiles of up
-    // to 32 rows (decode) are bound by the bytes of W a workgroup keeps in flight (64 tokens x top-8 on 32 experts: 86 -> 80 us
-    // with three steps ahead); stage 2 (34 -> 36 us) and packed int4 weights (36 -> 38) are not and stay one step ahead
-    constexpr int WPF = DEEP || (MR <= 2 && STAGE == 1 && !W4) ? 3 : 1;
+    // W register sets: the fragments of step kt live in set kt % NWS and are requested WPF steps ahead; loads return in order, so A has to be as far ahead as W.
+    constexpr int WPF = DEEP ? 3 : 1;
     constexpr int NWS = WPF + 1;
     wreg_t blo[NWS][NSET][NR], bhi[NWS][NSET][NR];
+    auto w8 = [&](uint32_t voff, uint32_t soff) { return (v2i)__builtin_amdgcn_raw_buffer_load_b64(rb, (int)voff, (int)soff, W_CACHE); };
+    auto w16 = [&](uint32_t voff, uint32_t soff) { return (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)voff, (int)soff, W_CACHE); };
     auto load_b = [&](int kt, int set) {
 #pragma unroll
         for (int s = 0; s < NSET; s++)
@@ -156,11 +158,11 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
             for (int ni = 0; ni < NR; ni++) {
                 const bool ok = kt < KT;
                 if constexpr (W4) {
-                    blo[set][s][ni] = buf_load8(rb, ok ? b_voff[s][ni] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
-                    bhi[set][s][ni] = buf_load8(rb, ok ? b_voff[s][ni] + 512u : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
+                    blo[set][s][ni] = w8(ok ? b_voff[s][ni] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
+                    bhi[set][s][ni] = w8(ok ? b_voff[s][ni] + 512u : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
                 } else {
-                    blo[set][s][ni] = buf_load16(rb, ok ? b_voff[s][ni] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
-                    bhi[set][s][ni] = buf_load16(rb, ok ? b_voff[s][ni] + 1024u : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
+                    blo[set][s][ni] = w16(ok ? b_voff[s][ni] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
+                    bhi[set][s][ni] = w16(ok ? b_voff[s][ni] + 1024u : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
                 }
             }
     };
@@ -340,7 +342,11 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     });
 }
 
-// Whether a stage on 64- or 128-row tiles takes the build that asks for its operands three steps ahead.  With few workgroups on a CU nothing else
+// Whether a stage takes the build that asks for its operands three steps ahead (the builds that read W past the caches and those on two paired blocks always do).  Tiles of up to 32
+// rows are bound by the bytes of W on their way, and it gains (us, 32 experts, 4096 x 1536, one step ahead / three: 8 tokens x top-8 fp8 stage 1 66.6 / 64.9, there with W alone
+// ahead before, stage 2 36.1 / 33.3, int4 42.2 / 35.6 and 23.1 / 21.7; 4 x top-2 on 8, 4096 x 2048, fp8 30.5 / 21.8 and 16.9 / 13.4, int4 25.1 / 15.8 and 13.5 / 9.7) but in stage 2 with
+// more than 11 workgroups a CU (128 experts, 2048 x 768, 600 x top-8 in blocks of 32 51.6 / 56.6; 2048 x 512, 384 in blocks of 16 36.9 / 38.5) and with int4 weights in blocks of 16 with more
+// than four in stage 1, three in stage 2 (64 tokens 46.8 / 46.9 and 26.8 / 29.1, 200 x top-8 on 128, 2048 x 512 29.9 / 31.2 and 22.6 / 23.9).  On 64- and 128-row tiles: with few workgroups on a CU nothing else
 // covers a load: up to two of them per CU that build is the faster one in either stage.  With more of them stage 2 is better off with the
 // registers of more workgroups (683 to 1,891 workgroups), stage 1 only where the rows are short.  Workgroups on average over routings.  Measured,
 // us one step ahead / three: stage 1, 1086 tokens x top-4 on 17 experts, 4096 x 256 (170 workgroups of 128 rows) fp8 41.4 / 26.8, int4 47.6 / 29.6; 813 x
@@ -355,8 +361,35 @@ bool takes_deep(const MoeParams& p, int block_m, int blocks, int nx) {
     const long pairs = (long)p.tokens * p.topk, likely = pairs / block_m + p.experts / 2;
     const long wgs = (likely < blocks ? likely : blocks) * nx;
     if (wgs <= 2L * psg_cu_count()) return true;
+    if (block_m <= 32) return KIND == KIND_INT8W4 ? block_m == 32 || wgs <= (STAGE == 1 ? 4L : 3L) * psg_cu_count() : STAGE == 1 || wgs <= 11L * psg_cu_count();
     if (STAGE == 2) return false;
     return p.K >= 4096 || (block_m == 128 && (p.K >= 2048 || KIND == KIND_INT8W4));
+}
+
+// Whether a stage on tiles of up to 32 rows, or on two paired blocks of 32, reads W past the caches (non-temporal): where an expert's rows mostly make one tile, so that nothing
+// is read twice, and the weights are too many to stay in the last-level cache between two layers.  Streamed like this they come at 5.5 to 6.6 TB/s
+// instead of 5.0 to 6.0, us plain / non-temporal, weights in memory: stage 1, 32 experts, 4096 x 1536, fp8 8 tokens x top-8 64.9 / 59.2, 64 75.3 / 67.9, 96 75.8 /
+// 68.5; blocks of 32 110 80.7 / 73.0, 192 80.3 / 73.1; int4 8 tokens 35.6 / 32.7; 64 experts, 2048 x 768, 128 x top-4 39.1 / 35.9.  Stage 2 8 tokens 33.3 / 30.5, 128 x top-4 23.4 /
+// 21.3, but 96 x top-8 in blocks of 16 (one and a half tiles an expert) 45.6 / 50.9, 100 x top-6 on 16, 3072 x 512 11.6 / 12.3; and 33 MB of weights 10.9 / 11.2, from the
+// last-level cache, which keeps nothing that was read like this, 7.6 / 10.2.
+template <int KIND, int STAGE>
+bool takes_nt(const MoeParams& p, int tile_m) {
+    const int64_t rows_e = STAGE == 1 ? 2ll * p.n_out : p.n_out, bytes = (p.experts * rows_e * p.K) >> (KIND == KIND_INT8W4 ? 1 : 0);
+    return bytes >= 48000000 && 4ll * p.tokens * p.topk <= 3ll * p.experts * tile_m;
+}
+
+// Whether a stage multiplies two consecutive blocks of an expert in one workgroup.  Stage 1 with one-byte weights always does with blocks of up to 32 rows (64 tokens x
+// top-8 on 32 experts, blocks of 16: 107 -> 92 us).  The other stages stream half the bytes and have fewer workgroups from the start: they do with blocks of 16 where
+// most experts have two and the pairs still make three workgroups a CU (us single / paired, weights in memory, 32 experts, 4096 x 1536: int4 stage 1 64 tokens x
+// top-8 46.5 / 41.7, 96 53.9 / 41.7, but 51 42.4 / 41.8; 128 experts, 2048 x 512, 256 tokens 36.1 / 31.6, 204 29.8 / 31.3; stage 2 fp8 51 tokens 40.7 / 35.4, 64 41.3 /
+// 36.2, 96 45.5 / 41.1, int4 64 26.7 / 24.8, 96 36.0 / 28.3, but K = 512 33.9 / 34.4, two workgroups a CU 17.3 / 18.9, one 18.8 / 20.8).
+template <int KIND, int STAGE>
+bool takes_pairs(const MoeParams& p, int block_m) {
+    if (!p.pair_blocks || block_m > 32) return false;
+    if (STAGE == 1 && KIND != KIND_INT8W4) return true;
+    const int64_t pairs = (int64_t)p.tokens * p.topk, rows = 16ll * p.experts, tn = STAGE == 1 ? 64 : 128;
+    if (block_m != 16 || p.by_position || p.experts * ((p.n_out + tn - 1) / tn) < 3ll * psg_cu_count()) return false;
+    return STAGE == 1 ? 10 * pairs >= 9 * rows : p.K >= 1024 && 4 * pairs > 3 * rows;
 }
 
 template <int KIND, int STAGE, int NR>
@@ -376,20 +409,21 @@ hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int bl
     const dim3 grid(nx, blocks + rows.wgs, 1);
 #define PSG_MOE(MR_, CO_)                                                                                \
     {                                                                                                    \
-        constexpr bool kHas = MR_ >= 4 && !(STAGE == 1 && NR == 2);  /* the tiles with a deep build */   \
-        constexpr bool kOnly = MR_ == 4 && CO_ == 2;                 /* ... and with no other */         \
+        constexpr bool kOnly = CO_ == 2 || (MR_ <= 2 && STAGE == 1 && KIND != KIND_INT8W4); /* always deep */ \
+        constexpr bool kNt = MR_ <= 2 || CO_ == 2;                             /* may read W past the caches */ \
         if constexpr (STAGE == 2) {                                                                      \
             if (lists) {                                                                                 \
-                hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, false, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
+                hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, 0, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
                 return hipGetLastError();                                                                \
             }                                                                                            \
         }                                                                                                \
-        if (kHas && (deep || kOnly)) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kHas>), grid, dim3(256), 0, stream, p); \
-        else hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kHas && kOnly>), grid, dim3(256), 0, stream, p); \
+        if (kNt && takes_nt<KIND, STAGE>(p, block_m * CO_)) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kNt ? 2 : 1>), grid, dim3(256), 0, stream, p); \
+        else if (deep || kOnly) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, 1>), grid, dim3(256), 0, stream, p); \
+        else hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kOnly ? 1 : 0>), grid, dim3(256), 0, stream, p); \
         return hipGetLastError();                                                                        \
     }
-    if constexpr (STAGE == 1) {
-        if (pair && block_m == 16) PSG_MOE(2, 2)
+    if (pair && block_m == 16) PSG_MOE(2, 2)
+    if constexpr (STAGE == 1 && KIND != KIND_INT8W4) {
         if (pair && block_m == 32) PSG_MOE(4, 2)
     }
     if (block_m == 16) PSG_MOE(1, 1)
@@ -402,19 +436,12 @@ hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int bl
 
 template <int KIND, int STAGE>
 hipError_t launch_kind(const MoeParams& p, const MoeRowsParams& rows, int block_m, int blocks, hipStream_t stream) {
-    // Stage 1 with one-byte weights multiplies blocks of 16 and 32 rows two at a time where they share an expert (64 tokens x
-    // top-8 on 32 experts, blocks of 16: 107 -> 92 us).  Measured and left alone: stage 2 (34 -> 37 us: its second pass over an
-    // expert's smaller slab already hits in L2, and pairing halves the workgroups in flight) and packed int4 weights (49 -> 50).
-    const bool pair = block_m <= 32 && p.pair_blocks != 0 && STAGE == 1 && KIND != KIND_INT8W4;
-    const int tile_m = pair ? 2 * block_m : block_m;
-    // 128 columns per workgroup when they divide the output; stage 1 (two accumulator sets) only for tiles of up to 32
-    // rows: measured at 4096 tokens x top-8, blocks of 128: stage 1 488 us with 64 columns against 800 with 128, stage 2
-    // 442 against 412 (stage 2 with 256 columns: 805 with one workgroup per CU, 492 when held to two)
-    // ... and only when that still leaves several workgroups per CU: a workgroup streams its slab at the pace its loads in
-    // flight allow, so a decode-sized stage 1 (64 tokens x top-8 on 32 experts: at most 63 blocks x 12 column tiles) is faster
-    // with twice as many workgroups of half the width
-    const long wgs128 = (long)blocks / (pair ? 2 : 1) * (long)(p.n_out / 128);
-    if (p.n_out % 128 == 0 && (STAGE == 2 || (tile_m <= 32 && wgs128 >= 1024))) return launch_nr<KIND, STAGE, 2>(p, rows, block_m, blocks, pair, stream);
+    const bool pair = takes_pairs<KIND, STAGE>(p, block_m);
+    // Stage 2 on 128 columns per workgroup where they divide the output, stage 1, which has two accumulator sets, on 64: measured at 4096 tokens x top-8, blocks of 128: stage 1 488 us with
+    // 64 columns against 800 with 128, stage 2 442 against 412 (stage 2 with 256 columns: 805 with one workgroup per CU, 492 when held to two).
+    if constexpr (STAGE == 2) {
+        if (p.n_out % 128 == 0) return launch_nr<KIND, STAGE, 2>(p, rows, block_m, blocks, pair, stream);
+    }
     return launch_nr<KIND, STAGE, 1>(p, rows, block_m, blocks, pair, stream);
 }
 
