@@ -83,7 +83,8 @@ __device__ __forceinline__ int quant_silu_mul(const v4f g0, const v4f g1, const 
 // LDS with the same scale rule as the output (kernels/moe/mxfp_moe/gemm1.py:324-412), and no A-side scales are read.  (A variant
 // that first quantised all K elements of the 16 rows into LDS and then ran the K loop without barriers measured slower: 16 tokens
 // x top-8 on 32 experts 38.9 us against 35.4, 64 tokens 42.2 against 41.)
-template <int AF, int MR, int STAGE, bool IQ = false>
+// NT: W past the caches (takes_nt)
+template <int AF, int MR, int STAGE, bool IQ, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 4 ? 2 : 1))) k_moe_mx(MoeMxParams p, MoeRowsParams rows) {
     static_assert(MR % 2 == 0 || MR == 1, "scale chunks cover 32 rows; a single 16-row block picks its half at run time");
     static_assert(!IQ || (MR == 1 && STAGE == 1 && AF == MXF_FP4), "inline quantisation: 16-row blocks of stage 1");
@@ -199,7 +200,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     auto load_b = [&](int kt, v4i* dst) {
         const bool ok = kt < KT;
 #pragma unroll
-        for (int ni = 0; ni < NR; ni++) dst[ni] = buf_load16(rb, ok ? boff[ni] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
+        for (int ni = 0; ni < NR; ni++) dst[ni] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)(ok ? boff[ni] : 0xFFFFFFF0u), (int)(ok ? (uint32_t)kt * 1024u : 0u), NT ? 2 : 0);
     };
     int sav[2][SC], sbv[2][NR / 2];
     auto load_sc = [&](int kc, int* sa_dst, int* sb_dst) {
@@ -234,9 +235,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     // set SET; requests the operands of step kt + PF and the scales of the next chunk, stages the A rows of step kt + 1
     auto step = [&](int kt, auto KHP, auto SETP, auto WSP) __attribute__((always_inline)) {
         constexpr int KH = decltype(KHP)::value, SET = decltype(SETP)::value, WS = decltype(WSP)::value;
+        if constexpr (KH == 0) load_sc((kt >> 1) + 1, sav[SET ^ 1], sbv[SET ^ 1]);  // (in front: loads return in order, and these are needed a step earlier)
         load_a(kt + PF, areg[(WS + PF) % RING]);
         load_b(kt + PF, bw[(WS + PF) % RING]);
-        if constexpr (KH == 0) load_sc((kt >> 1) + 1, sav[SET ^ 1], sbv[SET ^ 1]);
         const int* sa_cur = sav[SET];
         const int* sb_cur = sbv[SET];
         static_for<MR>([&](auto MI) {
@@ -480,6 +481,15 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
 // accumulators, so one workgroup per CU would run with nothing to overlap its loads and its epilogue with (measured, 4096
 // tokens x top-8 on 32 experts, 4096 x 1536, operands three steps ahead in both: stage 1 364 us with 128-row tiles against 292 with
 // 64-row tiles, stage 2 with the atomic epilogue 655 against 393, one row per sorted position 271 against 225).
+// Whether a stage on blocks of 16 or 32 rows reads W past the caches (non-temporal): where an expert's rows mostly make one block (the sorted list has room for the pairs and
+// a block of every expert) and the weights are too many to stay in the last-level cache between two layers.  us plain / non-temporal, weights in memory, stages 1 and 2, 32 experts,
+// 4096 x 1536: 8 tokens x top-8 38.4 / 35.6 and 23.4 / 21.6, 64 40.0 / 36.8 and 28.3 / 25.7, 40 in blocks of 16 42.0 / 39.3 and 26.1 / 23.5; 64 experts, 2048 x 768, 128 x
+// top-4 22.9 / 21.4 and 17.5 / 16.7; 128 experts, 2048 x 512, 300 x top-8 35.6 / 33.9 and 32.8 / 32.0; but 192 tokens (one and a half blocks an expert) 53.8 / 57.9 and 34.1 / 34.6.
+bool takes_nt(const MoeMxParams& p, int stage, int tile_m) {
+    const int64_t rows_e = stage == 1 ? 2ll * p.n_out : p.n_out, bytes = p.experts * rows_e * p.K / 2;
+    return bytes >= 48000000 && 4ll * p.sorted_size <= 7ll * p.experts * tile_m;
+}
+
 template <int AF, int STAGE>
 hipError_t launch_rows(MoeMxParams p, MoeRowsParams rows, int block_m, int blocks, hipStream_t stream) {
     p.eshift = block_m == 128 ? 1 : 0;
@@ -505,13 +515,20 @@ hipError_t launch_rows(MoeMxParams p, MoeRowsParams rows, int block_m, int block
     p.quad_tiles = !p.by_expert && p.n_tiles % 4 == 0 && p.n_tiles % 8 != 0;
     const unsigned row_blocks = (unsigned)(blocks << p.eshift);
     const dim3 grid((unsigned)(p.by_expert ? p.n_groups * 8 : p.n_tiles) * (p.quad_tiles ? (row_blocks + 1) / 2 * 2 : row_blocks) + (unsigned)rows.wgs);
+    const bool nt = block_m <= 32 && takes_nt(p, STAGE, block_m);
+#define PSG_GO(AF_, MR_, IQ_)                                                                                                                 \
+    {                                                                                                                                         \
+        if (MR_ <= 2 && nt) hipLaunchKernelGGL((k_moe_mx<AF_, MR_, STAGE, IQ_, MR_ <= 2>), grid, dim3(256), 0, stream, p, rows); \
+        else hipLaunchKernelGGL((k_moe_mx<AF_, MR_, STAGE, IQ_, false>), grid, dim3(256), 0, stream, p, rows);                         \
+        return hipGetLastError();                                                                                                             \
+    }
     if (block_m == 16) {
-        if constexpr (STAGE == 2) hipLaunchKernelGGL((k_moe_mx<MXF_FP4, 1, 2>), grid, dim3(256), 0, stream, p, rows);
-        else if constexpr (AF == MXF_FP4) hipLaunchKernelGGL((k_moe_mx<MXF_FP4, 1, 1, true>), grid, dim3(256), 0, stream, p, rows);
+        if constexpr (STAGE == 2) PSG_GO(MXF_FP4, 1, false)
+        else if constexpr (AF == MXF_FP4) PSG_GO(MXF_FP4, 1, true)
         else return hipErrorInvalidValue;
-    } else if (block_m == 32) hipLaunchKernelGGL((k_moe_mx<AF, 2, STAGE>), grid, dim3(256), 0, stream, p, rows);
-    else hipLaunchKernelGGL((k_moe_mx<AF, 4, STAGE>), grid, dim3(256), 0, stream, p, rows);
-    return hipGetLastError();
+    } else if (block_m == 32) PSG_GO(AF, 2, false)
+    else PSG_GO(AF, 4, false)
+#undef PSG_GO
 }
 
 }  // namespace

@@ -394,3 +394,43 @@ def test_blocks_of_128_on_large_tiles_equal_the_small_ones(tokens, model_dim, in
         for got, want, name in zip(run(0, dt), run(4, dt), ("codes", "scales", "rows")):
             assert torch.equal(got, want), (name, dt)
         assert (got[(nv + 63) // 64 * 64:] == torch.tensor(7.0, dtype=dt).view(torch.int16).item()).all()
+
+
+# ---- blocks of 16 and 32 rows whose weights are read past the caches (48 MB of them and more, where the list has room for little more than a block an expert): the same bits as with
+# a list that has room for twice as much, whose weights are read as usual.
+@pytest.mark.parametrize("bm,a_fmt", [(16, "bf16"), (32, "fp4"), (32, "fp8")])
+@pytest.mark.parametrize("model_dim,inter", [(2304, 3584), (3584, 2304)])
+def test_weights_read_past_the_caches_give_the_same_bits(bm, a_fmt, model_dim, inter):
+    dev, experts, tokens, topk = torch.device("cuda"), 12, 17, 2
+    g = torch.Generator(device=dev).manual_seed(bm + inter)
+    u8 = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
+    sc = lambda n: torch.randint(118, 130, (n,), generator=g, device=dev, dtype=torch.uint8)
+    rng = np.random.default_rng(bm)
+    ids = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int32)
+    sid, sw, se, npp = O.moe_sorting(ids, rng.uniform(0.1, 1.0, size=(tokens, topk)).astype(np.float32), experts, bm)
+    nv, most = int(npp[0]), 2 * experts * bm
+    assert 4 * nv <= 7 * experts * bm
+    sid, sw, se = (np.concatenate([v[:n], np.full(most, fill, v.dtype)])[:m] for v, n, m, fill in
+                   ((sid, nv, most, tokens), (sw, nv, most, 0), (se, nv // bm, most // bm, 0)))
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    x = torch.randn(tokens, model_dim, generator=g, device=dev).bfloat16()
+    # fp8 codes without the two NaNs
+    a = u8(tokens, model_dim) & 0xBF if a_fmt == "fp8" else u8(tokens, model_dim // 2)
+    w1, w2 = u8(experts * 2 * inter, model_dim // 2), u8(experts * model_dim, inter // 2)
+    sa, s1, s2 = sc(most * (model_dim // 32)), sc(experts * 2 * inter * (model_dim // 32)), sc(experts * model_dim * (inter // 32))
+    nvt = torch.tensor([nv], dtype=torch.int32, device=dev)
+
+    def run(rows):
+        codes = torch.full((rows, inter // 2), 0x77, dtype=torch.uint8, device=dev)
+        hs = torch.full(((rows + 31) // 32 * 32 * (inter // 32),), 0x77, dtype=torch.uint8, device=dev)
+        kw = dict(sorted_expert_ids=t(se[:rows // bm]), cumsum_tensor=nvt, BM=bm, NE=experts, D_HIDDEN=model_dim, D_INTER=inter, topk=topk)
+        flydsl_mxfp4_gemm1(a_quant=a, a_scale_sorted_shuffled=sa, w1_u8=w1, w1_scale_u8=s1, m_indices=t(sid[:rows]), inter_sorted_quant=codes, inter_sorted_shuffled_scale=hs,
+                           hidden_states=x, n_tokens=tokens, inline_quant=bm == 16, a_dtype="fp4" if bm == 16 else a_fmt, **kw)
+        flat = torch.full((rows, model_dim), 7.0, dtype=torch.bfloat16, device=dev)
+        flydsl_mxfp4_gemm2(inter_sorted_quant=codes, inter_sorted_shuffled_scale=hs, w2_u8=w2, w2_scale_u8=s2, sorted_token_ids=t(sid[:rows]), sorted_weights=t(sw[:rows]),
+                           flat_out=flat, M_logical=tokens, max_sorted=rows, epilog="nonatomic", **kw)
+        torch.cuda.synchronize()
+        return codes[:nv], hs[:nv // 32 * 32 * (inter // 32)], flat[:nv].view(torch.int16)
+
+    for got, want, name in zip(run(nv), run(most), ("codes", "scales", "rows")):
+        assert torch.equal(got, want), name
