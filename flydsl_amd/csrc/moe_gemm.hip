@@ -367,15 +367,15 @@ bool takes_deep(const MoeParams& p, int block_m, int blocks, int nx) {
 }
 
 // Whether a stage on tiles of up to 32 rows, or on two paired blocks of 32, reads W past the caches (non-temporal): where an expert's rows mostly make one tile, so that nothing
-// is read twice, and the weights are too many to stay in the last-level cache between two layers.  Streamed like this they come at 5.5 to 6.6 TB/s
+// is read twice, and the weights of both stages together are more than the last-level cache holds (256 MB).  Streamed like this they come at 5.5 to 6.6 TB/s
 // instead of 5.0 to 6.0, us plain / non-temporal, weights in memory: stage 1, 32 experts, 4096 x 1536, fp8 8 tokens x top-8 64.9 / 59.2, 64 75.3 / 67.9, 96 75.8 /
 // 68.5; blocks of 32 110 80.7 / 73.0, 192 80.3 / 73.1; int4 8 tokens 35.6 / 32.7; 64 experts, 2048 x 768, 128 x top-4 39.1 / 35.9.  Stage 2 8 tokens 33.3 / 30.5, 128 x top-4 23.4 /
-// 21.3, but 96 x top-8 in blocks of 16 (one and a half tiles an expert) 45.6 / 50.9, 100 x top-6 on 16, 3072 x 512 11.6 / 12.3; and 33 MB of weights 10.9 / 11.2, from the
-// last-level cache, which keeps nothing that was read like this, 7.6 / 10.2.
+// 21.3, but 96 x top-8 in blocks of 16 (one and a half tiles an expert) 45.6 / 50.9, 100 x top-6 on 16, 3072 x 512 11.6 / 12.3.  The
+// cache keeps nothing that was read like this: a layer of 226 MB (128 experts, 2304 x 256, 160 x top-8) took 73.7 / 69.4 from memory, 60.8 / 68.9 from the cache.
 template <int KIND, int STAGE>
 bool takes_nt(const MoeParams& p, int tile_m) {
     const int64_t rows_e = STAGE == 1 ? 2ll * p.n_out : p.n_out, bytes = (p.experts * rows_e * p.K) >> (KIND == KIND_INT8W4 ? 1 : 0);
-    return bytes >= 48000000 && 4ll * p.tokens * p.topk <= 3ll * p.experts * tile_m;
+    return bytes * (STAGE == 1 ? 3 : 6) >= 2ll * (256 << 20) && 4ll * p.tokens * p.topk <= 3ll * p.experts * tile_m;
 }
 
 // Whether a stage multiplies two consecutive blocks of an expert in one workgroup.  Stage 1 with one-byte weights always does with blocks of up to 32 rows (64 tokens x

@@ -482,12 +482,12 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
 // tokens x top-8 on 32 experts, 4096 x 1536, operands three steps ahead in both: stage 1 364 us with 128-row tiles against 292 with
 // 64-row tiles, stage 2 with the atomic epilogue 655 against 393, one row per sorted position 271 against 225).
 // Whether a stage on blocks of 16 or 32 rows reads W past the caches (non-temporal): where an expert's rows mostly make one block (the sorted list has room for the pairs and
-// a block of every expert) and the weights are too many to stay in the last-level cache between two layers.  us plain / non-temporal, weights in memory, stages 1 and 2, 32 experts,
+// a block of every expert) and the weights of both stages together are more than the last-level cache holds (256 MB; what is read like this doesn't stay there).  us plain / non-temporal, weights in memory, stages 1 and 2, 32 experts,
 // 4096 x 1536: 8 tokens x top-8 38.4 / 35.6 and 23.4 / 21.6, 64 40.0 / 36.8 and 28.3 / 25.7, 40 in blocks of 16 42.0 / 39.3 and 26.1 / 23.5; 64 experts, 2048 x 768, 128 x
 // top-4 22.9 / 21.4 and 17.5 / 16.7; 128 experts, 2048 x 512, 300 x top-8 35.6 / 33.9 and 32.8 / 32.0; but 192 tokens (one and a half blocks an expert) 53.8 / 57.9 and 34.1 / 34.6.
 bool takes_nt(const MoeMxParams& p, int stage, int tile_m) {
     const int64_t rows_e = stage == 1 ? 2ll * p.n_out : p.n_out, bytes = p.experts * rows_e * p.K / 2;
-    return bytes >= 48000000 && 4ll * p.sorted_size <= 7ll * p.experts * tile_m;
+    return bytes * (stage == 1 ? 3 : 6) >= 2ll * (256 << 20) && 4ll * p.sorted_size <= 7ll * p.experts * tile_m;
 }
 
 template <int AF, int STAGE>

@@ -396,12 +396,12 @@ def test_blocks_of_128_on_large_tiles_equal_the_small_ones(tokens, model_dim, in
         assert (got[(nv + 63) // 64 * 64:] == torch.tensor(7.0, dtype=dt).view(torch.int16).item()).all()
 
 
-# ---- blocks of 16 and 32 rows whose weights are read past the caches (48 MB of them and more, where the list has room for little more than a block an expert): the same bits as with
+# ---- blocks of 16 and 32 rows whose weights are read past the caches (more of them than these hold, where the list has room for little more than a block an expert): the same bits as with
 # a list that has room for twice as much, whose weights are read as usual.
 @pytest.mark.parametrize("bm,a_fmt", [(16, "bf16"), (32, "fp4"), (32, "fp8")])
 @pytest.mark.parametrize("model_dim,inter", [(2304, 3584), (3584, 2304)])
 def test_weights_read_past_the_caches_give_the_same_bits(bm, a_fmt, model_dim, inter):
-    dev, experts, tokens, topk = torch.device("cuda"), 12, 17, 2
+    dev, experts, tokens, topk = torch.device("cuda"), 24, 17, 2
     g = torch.Generator(device=dev).manual_seed(bm + inter)
     u8 = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
     sc = lambda n: torch.randint(118, 130, (n,), generator=g, device=dev, dtype=torch.uint8)
