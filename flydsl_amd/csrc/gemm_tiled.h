@@ -399,14 +399,13 @@ k_a8w8_tiled(A8W8Params p) {
             step(kt + 1, std::integral_constant<int, 1>{});
         }
     } else {
-        // four register sets: steps past the end are skipped (the condition is uniform over the workgroup) instead of run on
-        // zero operands; with 16 steps per workgroup three idle steps would be a fifth of the loop
-        for (int kt = kt_begin; kt < kt_end; kt += 4) {
-            step(kt, std::integral_constant<int, 0>{});
-            if (kt + 1 < kt_end) step(kt + 1, std::integral_constant<int, 1>{});
-            if (kt + 2 < kt_end) step(kt + 2, std::integral_constant<int, 2>{});
-            if (kt + 3 < kt_end) step(kt + 3, std::integral_constant<int, 3>{});
-        }
+        // four register sets: whole rounds without a condition, so that the compiler's count of the loads on their way is exact (with one between the steps it takes
+        // every step for the possible last one), then the steps that are left
+        int kt = kt_begin;
+        for (; kt + 4 <= kt_end; kt += 4) static_for<4>([&](auto I) { step(kt + decltype(I)::value, I); });
+        static_for<3>([&](auto I) {
+            if (kt + decltype(I)::value < kt_end) step(kt + decltype(I)::value, I);
+        });
     }
 
     // epilogue operands, fetched in one batch (one memory latency for the whole tile, not one per fragment)
