@@ -136,7 +136,10 @@ __global__ void __launch_bounds__(256, 2) k_moe_pair(MoeParams p, MoeRowsParams 
                 const int t = (int)(id & 0xFFFFFFu), s = (int)(id >> 24);
                 if (t < p.tokens && s < p.topk && n_st < p.n_out) {
                     const size_t orow = STAGE == 2 && p.by_position ? (size_t)(blk * TM + r) : (size_t)t * p.topk + s;
-                    *reinterpret_cast<v4i*>(static_cast<uint16_t*>(p.out) + orow * (size_t)p.n_out + n_st) = *reinterpret_cast<const v4i*>(lds + r * ROWB + (((g ^ r) & (GR - 1)) << 4));
+                    const v4i v = *reinterpret_cast<const v4i*>(lds + r * ROWB + (((g ^ r) & (GR - 1)) << 4));
+                    v4i* o = reinterpret_cast<v4i*>(static_cast<uint16_t*>(p.out) + orow * (size_t)p.n_out + n_st);
+                    if (STAGE == 2 && p.by_position) __builtin_nontemporal_store(v, o);  // read once, by k_moe_rows_add
+                    else *o = v;
                 }
             }
         } else {

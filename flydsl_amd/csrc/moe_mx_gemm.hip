@@ -470,7 +470,10 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     const int q = half * 64 * 32 + i * 256 + tid, r = q >> 5, g = q & 31;
-                    *reinterpret_cast<v4i*>(out + ((size_t)blk * TM + r) * N + n0 + g * 8) = *reinterpret_cast<const v4i*>(lds + r * 512 + (((g ^ r) & 31) << 4));
+                    const v4i v = *reinterpret_cast<const v4i*>(lds + r * 512 + (((g ^ r) & 31) << 4));
+                    v4i* o = reinterpret_cast<v4i*>(out + ((size_t)blk * TM + r) * N + n0 + g * 8);
+                    if (p.atomic == 2) __builtin_nontemporal_store(v, o);  // read once, by k_moe_rows_add
+                    else *o = v;
                 }
             }
         });

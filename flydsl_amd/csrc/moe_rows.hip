@@ -5,6 +5,9 @@
 // model 4096, i.e. 268 MB of additions: fp8 stage 2 434 us, MX-FP4 436), a store and a read of the same rows at 5.  So `topk`
 // additions per output element become one; that one stays atomic, because launches on other streams may be adding into `out` too.
 //
+// The rows are written once and read once, non-temporally on both sides (stages on 128-row tiles), so that they don't push the operands out of the caches: MX stage 2 and the sum, us before / now,
+// 4096 tokens x top-8 on 32 experts, 4096 x 1536 236 / 213 (weights in the last-level cache 236 / 175), inter 512 on 64 experts 177 / 159, 1024 tokens 73.3 / 72.0; with one side alone 218 and 223.
+//
 // Which sorted rows belong to a token is found on the device, by workgroups beside the stage's tiles (moe_rows_index_share) or in launches in front, so any sorted
 // list the atomic epilogue accepts works here: rows are entered into a list of `topk` places per token, and rows that do not fit (a
 // list that names a token more often than topk times) are chained behind its last entry.
@@ -62,7 +65,7 @@ __global__ void __launch_bounds__(256) k_moe_rows_add(MoeRowsParams p, int chunk
 #pragma unroll
             for (int j = 0; j < DWORDS; j++) {
                 const int c = c0 + j * 256;
-                v[k][j] = rows[base + (c < dws ? c : 0)];
+                v[k][j] = __builtin_nontemporal_load(&rows[base + (c < dws ? c : 0)]);
             }
         }
 #pragma unroll
