@@ -26,8 +26,6 @@
 
 namespace {
 
-constexpr uint32_t OOB = 0xFFFFFFF0u;  // byte offset past every buffer bound: the load returns 0 without a memory access
-
 template <int KIND>
 struct Acc {
     using type = v4f;

@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(256) k_mx_generic(MxGenParams p) {
         for (int j = 0; j < A_LOADS; j++) {
             const int c = tid + 256 * j, row = c / CPR, kc = c % CPR;
             const bool ok = row < TM && kt < kt_end;
-            dst[j] = buf_load16(ra, ok ? (uint32_t)row * a_rs + (uint32_t)kc * 16u : 0xFFFFFFF0u, ok ? (uint32_t)kt * AB : 0u);
+            dst[j] = buf_load16(ra, ok ? (uint32_t)row * a_rs + (uint32_t)kc * 16u : OOB, ok ? (uint32_t)kt * AB : 0u);
         }
     };
     auto store_a = [&](int stage, const v4i* src) {
@@ -101,12 +101,12 @@ __global__ void __launch_bounds__(256) k_mx_generic(MxGenParams p) {
             const bool ok = kt < kt_end;
             v8i v = {0, 0, 0, 0, 0, 0, 0, 0};
             if constexpr (BF == MXF_FP4) {
-                const v4i x = buf_load16(rb, ok ? (uint32_t)lane * 16u + (uint32_t)ni * 16u * b_row_bytes : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
+                const v4i x = buf_load16(rb, ok ? (uint32_t)lane * 16u + (uint32_t)ni * 16u * b_row_bytes : OOB, ok ? (uint32_t)kt * 1024u : 0u);
                 v = __builtin_shufflevector(x, x, 0, 1, 2, 3, -1, -1, -1, -1);
             } else {
                 const uint32_t voff = (uint32_t)lane * 16u + (uint32_t)ni * 16u * b_row_bytes;
-                const v4i x0 = buf_load16(rb, ok ? voff : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
-                const v4i x1 = buf_load16(rb, ok ? voff + 1024u : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
+                const v4i x0 = buf_load16(rb, ok ? voff : OOB, ok ? (uint32_t)kt * 2048u : 0u);
+                const v4i x1 = buf_load16(rb, ok ? voff + 1024u : OOB, ok ? (uint32_t)kt * 2048u : 0u);
                 v = __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
             }
             dst[ni] = v;
@@ -117,9 +117,9 @@ __global__ void __launch_bounds__(256) k_mx_generic(MxGenParams p) {
     auto load_sc = [&](int kc, int* sa_dst, int* sb_dst) {
         const bool ok = kc < (kt_end >> 1);
 #pragma unroll
-        for (int q = 0; q < MR / 2; q++) sa_dst[q] = buf_load4(rsa, ok ? (uint32_t)q * sa_cs + (uint32_t)lane * 4u : 0xFFFFFFF0u, ok ? (uint32_t)kc * 256u : 0u);
+        for (int q = 0; q < MR / 2; q++) sa_dst[q] = buf_load4(rsa, ok ? (uint32_t)q * sa_cs + (uint32_t)lane * 4u : OOB, ok ? (uint32_t)kc * 256u : 0u);
 #pragma unroll
-        for (int q = 0; q < NR / 2; q++) sb_dst[q] = buf_load4(rsb, ok ? (uint32_t)q * chunk_bytes + (uint32_t)lane * 4u : 0xFFFFFFF0u, ok ? (uint32_t)kc * 256u : 0u);
+        for (int q = 0; q < NR / 2; q++) sb_dst[q] = buf_load4(rsb, ok ? (uint32_t)q * chunk_bytes + (uint32_t)lane * 4u : OOB, ok ? (uint32_t)kc * 256u : 0u);
     };
     auto read_frag = [&](int stage, int mi) {
         const int row = mi * 16 + li;

@@ -88,18 +88,18 @@ __global__ void __launch_bounds__(NW * 64) k_mx_smallm(MxGenParams p) {
                 for (int kh = 0; kh < 2; kh++)
 #pragma unroll
                     for (int l = 0; l < AL; l++)
-                        aq[u][mb][kh][l] = buf_load16(ra, ok ? a_voff + (uint32_t)mb * 16u * a_rs : 0xFFFFFFF0u, (so * 2u + (uint32_t)kh) * (uint32_t)AB);
+                        aq[u][mb][kh][l] = buf_load16(ra, ok ? a_voff + (uint32_t)mb * 16u * a_rs : OOB, (so * 2u + (uint32_t)kh) * (uint32_t)AB);
         }
 #pragma unroll
-        for (int mc = 0; mc < MC; mc++) sav[u][mc] = buf_load4(rsa, ok ? (uint32_t)mc * sa_cs + (uint32_t)lane * 4u : 0xFFFFFFF0u, so * 256u);
-        sbv[u] = buf_load4(rsb, ok ? (uint32_t)lane * 4u : 0xFFFFFFF0u, so * 256u);
+        for (int mc = 0; mc < MC; mc++) sav[u][mc] = buf_load4(rsa, ok ? (uint32_t)mc * sa_cs + (uint32_t)lane * 4u : OOB, so * 256u);
+        sbv[u] = buf_load4(rsb, ok ? (uint32_t)lane * 4u : OOB, so * 256u);
 #pragma unroll
         for (int nb = 0; nb < 2; nb++)
 #pragma unroll
             for (int kh = 0; kh < 2; kh++)
 #pragma unroll
                 for (int l = 0; l < BL; l++)
-                    bq[u][nb][kh][l] = buf_load16_nt(rb, ok ? (uint32_t)lane * 16u + (uint32_t)nb * 16u * b_row_bytes + (uint32_t)l * 1024u : 0xFFFFFFF0u, (so * 2u + (uint32_t)kh) * (16u * BB));
+                    bq[u][nb][kh][l] = buf_load16_nt(rb, ok ? (uint32_t)lane * 16u + (uint32_t)nb * 16u * b_row_bytes + (uint32_t)l * 1024u : OOB, (so * 2u + (uint32_t)kh) * (16u * BB));
         // keep the machine scheduler from sinking these loads below later code to save registers
         __builtin_amdgcn_sched_barrier(0);
     };

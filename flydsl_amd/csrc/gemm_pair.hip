@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(256, 2) k_pair(A8W8Params p) {
             for (int i = half * 8; i < half * 8 + 8; i++) {
                 const int r = r0 + i * 8;
                 const v4i v = *reinterpret_cast<const v4i*>(lds + r * 512 + ((g ^ (r & 15)) << 4));
-                __builtin_amdgcn_raw_buffer_store_b128((v4u)v, rc, (int)(n_st < p.N ? c_off + (uint32_t)i * c_step : 0xFFFFFFF0u), 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128((v4u)v, rc, (int)(n_st < p.N ? c_off + (uint32_t)i * c_step : OOB), 0, 0);
             }
         });
     }

@@ -214,7 +214,7 @@ k_a8w8_tiled(A8W8Params p) {
         const uint32_t k0 = (uint32_t)kt * TK;
         const bool in_k = kt < kt_end && (k0 + (uint32_t)a_kc * 16u) < (uint32_t)K;
         const uint32_t off = a_goff0 + (uint32_t)j * (uint32_t)RPP * (uint32_t)K + k0;
-        dst = buf_load16(ra, in_k ? off : 0xFFFFFFF0u, 0);
+        dst = buf_load16(ra, in_k ? off : OOB, 0);
     };
     auto store_a1 = [&](int stage, int j, const v4i& src) {
         *reinterpret_cast<v4i*>(&lds[stage][lds_off(a_row0 + RPP * j, a_kc)]) = src;
@@ -226,9 +226,9 @@ k_a8w8_tiled(A8W8Params p) {
         const bool has = kt < kt_end;
         const uint32_t soff = has ? (uint32_t)(KIND == KIND_MXFP4 ? kt : (kt >> 1)) * 256u : 0u;
         if (q < MP) {
-            sa_dst[q] = buf_load4(rsa, has ? (uint32_t)q * chunk_bytes + (uint32_t)lane * 4u : 0xFFFFFFF0u, soff);
+            sa_dst[q] = buf_load4(rsa, has ? (uint32_t)q * chunk_bytes + (uint32_t)lane * 4u : OOB, soff);
         } else {
-            sb_dst[q - MP] = buf_load4(rsb, has ? (uint32_t)(q - MP) * chunk_bytes + (uint32_t)lane * 4u : 0xFFFFFFF0u, soff);
+            sb_dst[q - MP] = buf_load4(rsb, has ? (uint32_t)(q - MP) * chunk_bytes + (uint32_t)lane * 4u : OOB, soff);
         }
     };
     // W addressing.  Preshuffled: lane l reads bytes [16l, 16l+16) of the 1 KB block (n-block, 64-byte K block).
@@ -241,7 +241,7 @@ k_a8w8_tiled(A8W8Params p) {
         const int ni = W4 ? idx : idx >> 1, half = W4 ? 0 : idx & 1;
         const bool has = kt < kt_end && (kt * TK + half * 64) < K;
         const uint32_t voff = b_lane_off + (uint32_t)ni * 16u * (uint32_t)KW;
-        const v4i v = buf_load16(rb, has ? voff : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
+        const v4i v = buf_load16(rb, has ? voff : OOB, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
         if (half) hi[ni] = v; else lo[ni] = v;
     };
     auto read_frag = [&](int stage, int mi, v4i& flo, v4i& fhi) {

@@ -151,7 +151,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
         const uint32_t dst = lds_base + (uint32_t)(stage * STAGE + (wave * A_DMA + j) * 1024);
         if constexpr (decltype(CHK)::value) {
             const bool in_k = kt < kt_end && (uint32_t)(kt * TK + a_kc[j & 1] * 16) < (uint32_t)K;
-            dma16(ra, dst, in_k ? a_voff[j] : 0xFFFFFFF0u, kt < kt_end ? (uint32_t)kt * TK : 0u);
+            dma16(ra, dst, in_k ? a_voff[j] : OOB, kt < kt_end ? (uint32_t)kt * TK : 0u);
         } else {
             dma16(ra, dst, a_voff[j], (uint32_t)kt * TK);
         }
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
     auto dma_sc = [&](int kt, int slot, int which) __attribute__((always_inline)) {
         const bool has = kt < kt_end;
         const uint32_t dst = lds_base + (uint32_t)(NS * STAGE + slot * SC_SLOT + which * 2048 + wave * 256);
-        dma4(which ? rsb : rsa, dst, has ? (uint32_t)lane * 4u : 0xFFFFFFF0u, has ? (uint32_t)(kt >> 1) * 256u : 0u);
+        dma4(which ? rsb : rsa, dst, has ? (uint32_t)lane * 4u : OOB, has ? (uint32_t)(kt >> 1) * 256u : 0u);
     };
     auto read_sc = [&](int slot, int q, int* sa_dst, int* sb_dst) __attribute__((always_inline)) {
         if (q < MP) sa_dst[q] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + q * 256 + lane * 4);
@@ -173,7 +173,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
         const int ni = W4 ? idx : idx >> 1, half = W4 ? 0 : idx & 1;
         const bool has = !decltype(CHK)::value || (kt < kt_end && (kt * TK + half * 64) < K);
         const uint32_t voff = b_lane_off + (uint32_t)ni * 16u * (uint32_t)KW;
-        const v4i v = buf_load16(rb, has ? voff : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
+        const v4i v = buf_load16(rb, has ? voff : OOB, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
         if (half) hi[ni] = v; else lo[ni] = v;
     };
     // fragment (16 rows x 2 x 16 bytes of K) of m-block mi from a stage: row mi*16 + li, chunks lg and 4 + lg; the swizzle
@@ -436,7 +436,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
 #pragma unroll
             for (int i = half * (TM / 32); i < (half + 1) * (TM / 32); i++) {
                 const v4i v = *reinterpret_cast<const v4i*>(src + i * 16 * ROWB);
-                __builtin_amdgcn_raw_buffer_store_b128((v4u)v, rc, (int)(n_st < p.N ? c_off + (uint32_t)i * c_step : 0xFFFFFFF0u), 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128((v4u)v, rc, (int)(n_st < p.N ? c_off + (uint32_t)i * c_step : OOB), 0, 0);
             }
         });
     }

@@ -9,7 +9,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc_uniform(const void* 
     const uint64_t b = (uint64_t)(uintptr_t)base;
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)(bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes));
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readfirstlane((int)rsrc_bytes(bytes));
     return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>((uintptr_t)(((uint64_t)hi << 32) | lo)), 0, (int)n, 0x00020000);
 }
 

@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
             const int n = n0 + (ni * 4 + wave) * 16;                  // first column of the block: the four wavefronts of pass ni
                                                                       // cover 64 consecutive columns
             const int nb = (n + s * p.n_out) >> 4;
-            b_voff[s][ni] = n < p.n_out ? ((uint32_t)nb * 16u * (uint32_t)K + (uint32_t)lane * 16u) >> WSH : 0xFFFFFFF0u;
+            b_voff[s][ni] = n < p.n_out ? ((uint32_t)nb * 16u * (uint32_t)K + (uint32_t)lane * 16u) >> WSH : OOB;
         }
 
     uint32_t a_voff[A_LOADS];
@@ -136,7 +136,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
 #pragma unroll
         for (int j = 0; j < A_LOADS; j++) {
             const bool ok = kt < KT;
-            areg[set][j] = buf_load16(ra, ok ? a_voff[j] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 128u : 0u);
+            areg[set][j] = buf_load16(ra, ok ? a_voff[j] : OOB, ok ? (uint32_t)kt * 128u : 0u);
         }
     };
     auto store_a = [&](int stage, int set) {
@@ -158,11 +158,11 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
             for (int ni = 0; ni < NR; ni++) {
                 const bool ok = kt < KT;
                 if constexpr (W4) {
-                    blo[set][s][ni] = w8(ok ? b_voff[s][ni] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
-                    bhi[set][s][ni] = w8(ok ? b_voff[s][ni] + 512u : 0xFFFFFFF0u, ok ? (uint32_t)kt * 1024u : 0u);
+                    blo[set][s][ni] = w8(ok ? b_voff[s][ni] : OOB, ok ? (uint32_t)kt * 1024u : 0u);
+                    bhi[set][s][ni] = w8(ok ? b_voff[s][ni] + 512u : OOB, ok ? (uint32_t)kt * 1024u : 0u);
                 } else {
-                    blo[set][s][ni] = w16(ok ? b_voff[s][ni] : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
-                    bhi[set][s][ni] = w16(ok ? b_voff[s][ni] + 1024u : 0xFFFFFFF0u, ok ? (uint32_t)kt * 2048u : 0u);
+                    blo[set][s][ni] = w16(ok ? b_voff[s][ni] : OOB, ok ? (uint32_t)kt * 2048u : 0u);
+                    bhi[set][s][ni] = w16(ok ? b_voff[s][ni] + 1024u : OOB, ok ? (uint32_t)kt * 2048u : 0u);
                 }
             }
     };
@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     for (int j = 0; j < A_LOADS; j++) {
         const int c = tid + 256 * j, row = c >> 3, kc = c & 7;
         const int xr = row < BM ? x_row(row) : -1;
-        a_voff[j] = xr >= 0 ? (uint32_t)xr * (uint32_t)K + (uint32_t)kc * 16u : 0xFFFFFFF0u;
+        a_voff[j] = xr >= 0 ? (uint32_t)xr * (uint32_t)K + (uint32_t)kc * 16u : OOB;
         a_ldsoff[j] = row < BM ? moe_lds_off(row, kc) : -1;
     }
     static_for<DEEP ? 3 : 1>([&](auto I) { load_a(decltype(I)::value, decltype(I)::value); });

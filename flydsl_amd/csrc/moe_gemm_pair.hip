@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_pair(MoeParams p, MoeRowsParams 
     for (int j = 0; j < 4; j++) {
         const int row = (wave * 4 + j) * 8 + (lane >> 3), q = blk * TM + row;
         const int xr = x_row(q < p.sorted_size ? p.sorted_ids[q] : p.tokens);
-        a_voff[j] = xr >= 0 ? (uint32_t)xr * (uint32_t)K + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16) : 0xFFFFFFF0u;
+        a_voff[j] = xr >= 0 ? (uint32_t)xr * (uint32_t)K + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16) : OOB;
     }
     // W: the wavefront's four 16-row blocks, in stage 1 two of gate and two of up rows; a block past the width reads zeros
     const int rows_e = STAGE == 1 ? 2 * p.n_out : p.n_out;
@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_pair(MoeParams p, MoeRowsParams 
     for (int ni = 0; ni < NR; ni++) {
         const int col = STAGE == 1 ? n0 + wave * 32 + (ni & 1) * 16 : n0 + (wave * NR + ni) * 16;
         const int row = STAGE == 1 && ni >= 2 ? p.n_out + col : col;
-        b_voff[ni] = col < p.n_out ? (uint32_t)row * (uint32_t)K + (uint32_t)lane * 16u : 0xFFFFFFF0u;
+        b_voff[ni] = col < p.n_out ? (uint32_t)row * (uint32_t)K + (uint32_t)lane * 16u : OOB;
     }
     if (tid < TM) {
         const int q = blk * TM + tid, id = q < p.sorted_size ? p.sorted_ids[q] : p.tokens, xr = x_row(id);

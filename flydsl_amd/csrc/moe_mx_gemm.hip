@@ -178,7 +178,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     auto load_a = [&](int kt, v4i* dst) {
         const bool ok = kt < KT;
 #pragma unroll
-        for (int j = 0; j < A_LOADS; j++) dst[j] = buf_load16(ra, ok ? arow[j] : 0xFFFFFFF0u, ok ? (uint32_t)kt * A_STEP : 0u);
+        for (int j = 0; j < A_LOADS; j++) dst[j] = buf_load16(ra, ok ? arow[j] : OOB, ok ? (uint32_t)kt * A_STEP : 0u);
     };
     auto store_a = [&](int stage, const v4i* src) {
         if constexpr (IQ) {
@@ -200,16 +200,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     auto load_b = [&](int kt, v4i* dst) {
         const bool ok = kt < KT;
 #pragma unroll
-        for (int ni = 0; ni < NR; ni++) dst[ni] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)(ok ? boff[ni] : 0xFFFFFFF0u), (int)(ok ? (uint32_t)kt * 1024u : 0u), NT ? 2 : 0);
+        for (int ni = 0; ni < NR; ni++) dst[ni] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)(ok ? boff[ni] : OOB), (int)(ok ? (uint32_t)kt * 1024u : 0u), NT ? 2 : 0);
     };
     int sav[2][SC], sbv[2][NR / 2];
     auto load_sc = [&](int kc, int* sa_dst, int* sb_dst) {
         const bool ok = kc < (KT >> 1);
 #pragma unroll
         for (int q = 0; q < SC; q++)
-            sa_dst[q] = IQ ? 0 : buf_load4(rsa, ok ? (uint32_t)q * chunk_bytes + (uint32_t)lane * 4u : 0xFFFFFFF0u, ok ? (uint32_t)kc * 256u : 0u) >> sa_shift;
+            sa_dst[q] = IQ ? 0 : buf_load4(rsa, ok ? (uint32_t)q * chunk_bytes + (uint32_t)lane * 4u : OOB, ok ? (uint32_t)kc * 256u : 0u) >> sa_shift;
 #pragma unroll
-        for (int q = 0; q < NR / 2; q++) sb_dst[q] = buf_load4(rsb, ok ? sboff[q] : 0xFFFFFFF0u, ok ? (uint32_t)kc * 256u : 0u);
+        for (int q = 0; q < NR / 2; q++) sb_dst[q] = buf_load4(rsb, ok ? sboff[q] : OOB, ok ? (uint32_t)kc * 256u : 0u);
     };
     auto read_frag = [&](int stage, int mi) {
         const int row = mi * 16 + li;
@@ -268,7 +268,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     for (int j = 0; j < A_LOADS; j++) {
         // IQ: thread t takes 8 bf16 (16 bytes) of row t / 16: four neighbouring lanes hold one 32-element group
         const int c = tid + 256 * j, row = IQ ? c >> 4 : c / CPR, kc = IQ ? c & 15 : c % CPR;
-        arow[j] = 0xFFFFFFF0u;
+        arow[j] = OOB;
         if (row < TM) {
             const int src = STAGE == 1 ? (p.sorted_ids[blk * TM + row] & 0xFFFFFF) : blk * TM + row;
             if (src < a_rows) arow[j] = (uint32_t)src * a_src_bytes + (uint32_t)kc * 16u;
@@ -399,7 +399,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
     for (int j = 0; j < 4; j++) {
         const int row = (wave * 4 + j) * 8 + (lane >> 3);
         const int src = STAGE == 1 ? (p.sorted_ids[blk * TM + row] & 0xFFFFFF) : blk * TM + row;
-        a_voff[j] = src < a_rows ? (uint32_t)src * row_bytes + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16) : 0xFFFFFFF0u;
+        a_voff[j] = src < a_rows ? (uint32_t)src * row_bytes + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) * 16) : OOB;
     }
     // W: the wavefront's four 16-row blocks; in stage 1 two of gate and two of up rows, so it owns whole 32-column quantisation groups
 #pragma unroll

@@ -62,13 +62,13 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
     constexpr int N_DMA = MX ? 5 : 4;
     auto dma = [&](int kt, int stage, int j, auto CHK) __attribute__((always_inline)) {
         const bool has = !decltype(CHK)::value || kt < KT, in = !decltype(CHK)::value || kt * TK + a_kc[j & 1] * 16 < K;
-        if (j < 4) dma16(ra, lds_base + (uint32_t)(stage * STAGE + (wave * 4 + j) * 1024), in ? a_voff[j < 4 ? j : 0] : 0xFFFFFFF0u, has ? (uint32_t)kt * TK : 0u);
-        else dma16(rs, sc_dst + (uint32_t)(stage * SC_SLOT), has ? s_voff : 0xFFFFFFF0u, has ? (uint32_t)kt * 256u : 0u);
+        if (j < 4) dma16(ra, lds_base + (uint32_t)(stage * STAGE + (wave * 4 + j) * 1024), in ? a_voff[j < 4 ? j : 0] : OOB, has ? (uint32_t)kt * TK : 0u);
+        else dma16(rs, sc_dst + (uint32_t)(stage * SC_SLOT), has ? s_voff : OOB, has ? (uint32_t)kt * 256u : 0u);
     };
     v4i bw[4][NR];
     auto load_w = [&](int kt, int half, int ni, v4i* dst, auto CHK) __attribute__((always_inline)) {
         const bool has = !decltype(CHK)::value || kt * TK + half * 64 < K;
-        dst[ni] = buf_load16(rb, has ? b_voff[ni] : 0xFFFFFFF0u, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
+        dst[ni] = buf_load16(rb, has ? b_voff[ni] : OOB, has ? (uint32_t)kt * b_step + (uint32_t)half * b_half : 0u);
     };
     const int f_base[2] = {li * TK + ((lg ^ ((li >> 1) & 7)) << 4), li * TK + (((4 + lg) ^ ((li >> 1) & 7)) << 4)};
     constexpr int AHEAD = 2;  // blocks of four MFMAs that an A fragment is read ahead

@@ -18,9 +18,14 @@ enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_BIAS_RELU = 2, EPI_BIAS_SILU = 3, EPI_BIA
 // what a kernel writes: the scaled/activated C, or the raw accumulators
 enum { STORE_C = 0, STORE_ACC = 1, STORE_C_GENERIC = 2 };
 
-// Raw buffer resource over [base, base+bytes): loads past the end return 0, stores past it are dropped.
+// Byte offset past every descriptor's bound, to which the kernels redirect accesses that are not to happen.
+constexpr uint32_t OOB = 0xFFFFFFF0u;
+
+// Raw buffer resource over [base, base+bytes): loads past the end return 0, stores past it are dropped.  Over more than 4 GiB it ends at OOB, so that this offset
+// lies outside there too (with 2^32 - 1 as the bound it was 16 bytes of a later row).
+__device__ __forceinline__ uint32_t rsrc_bytes(uint64_t bytes) { return bytes > OOB ? OOB : (uint32_t)bytes; }
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint64_t bytes) {
-    uint32_t n = bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes;
+    const uint32_t n = rsrc_bytes(bytes);
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)n, 0x00020000);
 }
 
