@@ -539,7 +539,7 @@ hipError_t launch_shape(const A8W8Params& p, int tile_m, int tile_n, hipStream_t
         PSG_CASE(8, 8, 2)
     }
     if (p.wave_layout == 8) {  // eight wavefronts side by side along N: 256x256 tile, every W fragment loaded once
-        if (tile_m == 256 && tile_n == 256) return launch_tiled8<KIND, STORE>(p, stream);
+        if (tile_m == 256 && tile_n == 256 && c_in_descriptor(p, 256)) return launch_tiled8<KIND, STORE>(p, stream);
     }
     if constexpr (KIND != KIND_MXFP8) {
         // few tiles (p.ksplit = 3: the planner's mark for launches of at most two workgroups per CU): W fetched three steps ahead
@@ -558,7 +558,7 @@ hipError_t launch_shape(const A8W8Params& p, int tile_m, int tile_n, hipStream_t
     PSG_CASE(8, 8, 1)
     // the 128x256 tile of the 8- and 16-bit kinds has a kernel of its own too (gemm_pair.hip)
     if constexpr (KIND != KIND_MXFP8) {
-        if (tile_m == 128 && tile_n == 256) return psg_launch_pair(p, KIND, STORE, stream);
+        if (tile_m == 128 && tile_n == 256) return c_in_descriptor(p, 128) ? psg_launch_pair(p, KIND, STORE, stream) : launch_one<KIND, 4, 4, 1, STORE>(p, stream);
     }
     PSG_CASE(4, 4, 1)
     PSG_CASE(2, 4, 1)

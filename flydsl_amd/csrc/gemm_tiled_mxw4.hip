@@ -7,8 +7,9 @@ namespace {
 
 template <int KIND, int STORE>
 hipError_t launch_w4(const A8W8Params& p, int tile_m, int tile_n, hipStream_t stream) {
-    if (tile_m == 256 && tile_n == 256) return launch_tiled8<KIND, STORE>(p, stream);
-    if (tile_m == 128 && tile_n == 256) return launch_one<KIND, 8, 4, 1, STORE>(p, stream);
+    const bool large = tile_m == 256 && tile_n == 256;
+    if (large && c_in_descriptor(p, 256)) return launch_tiled8<KIND, STORE>(p, stream);
+    if (large || (tile_m == 128 && tile_n == 256)) return launch_one<KIND, 8, 4, 1, STORE>(p, stream);
     if (tile_m == 64 && tile_n == 256) return launch_one<KIND, 4, 4, 1, STORE>(p, stream);
     if (tile_m == 32 && tile_n == 256) return launch_one<KIND, 2, 4, 1, STORE>(p, stream);
     if (tile_m == 64 && tile_n == 128) return launch_one<KIND, 4, 2, 1, STORE>(p, stream);

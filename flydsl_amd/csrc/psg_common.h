@@ -146,6 +146,10 @@ struct A8W8Params {
     const uint8_t* mx_sb;  // MXFP4 only: shuffled e8m0 [N, K/32]
 };
 
+// Whether a tile of `tile_m` rows can store C by one descriptor (256x256 of eight wavefronts, the 128x256 tiles of pair_loop.h): all its rows within 32 bits of its first one, i.e. up
+// to 8.4 and 16.8 million columns (W may have 2^26 rows).  Wider problems run on tiles that store by 64-bit addresses.
+inline bool c_in_descriptor(const A8W8Params& p, int tile_m) { return (uint64_t)tile_m * (uint64_t)p.N * 2ull <= OOB; }
+
 struct MxParams {
     void* c;
     const uint8_t* a;    // [M,K/2]

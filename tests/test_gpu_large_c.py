@@ -70,3 +70,10 @@ def test_half_steps_past_a_row_of_more_than_4_gib_of_a_read_zero(tile):
     want = torch.full((M,), K * 0.25, device="cuda").bfloat16()
     want[at // K] = float("inf")
     assert torch.equal(c, want[:, None].expand(M, N))
+
+
+# 2^25 columns: 64 MiB a row of C, so that a tile of 128 rows spans 8 GiB
+@pytest.mark.parametrize("kind,tile,M,N,K", [("int8", (128, 256), 128, 1 << 25, 64), ("bf16", (128, 256), 100, 1 << 25, 32), ("int8", (256, 256), 200, (1 << 24) + 16, 64),
+                                             ("fp4", (128, 256), 128, (1 << 25) - 32, 256)])
+def test_rows_further_apart_than_32_bits(kind, tile, M, N, K):
+    _compare(kind, tile, M, N, K)
