@@ -3,12 +3,15 @@
 // Bound: MFMA at the clock the power limit leaves, and for short K the start and the end of a tile.  us, 256x256 tiles of eight wavefronts / these, weights in
 // memory: 4096x7168x2048 42.9 / 39.4, 4096x4096x4096 38.8 / 36.9, 8192x8192x1024 59.6 / 50.9, 6000x3584x4608 68 / 54, 8192x4096x8192 128.6 / 123.1, each in
 // its best tile order; 128x256 tiles of one workgroup a CU / these: 1000x7168x2048 15.4 / 13.1.
+// Scales off 16 bytes (three DMAs of a wavefront a step instead of one) cost 0 to 5 %; us 256x256 tiles / 64x256 tiles / these: 4096x7168x2048 44.6 / 51.4 / 41.3, 8192x4096x8192 126 /
+// 163 / 121, 1024x8192x8192 41.1 / 52.6 / 37.1, 300x28672x1024 16.0 / 17.9 / 15.9.
 #include "pair_loop.h"
 
 namespace {
 
 // STORE_ACC: raw accumulators of the K range blockIdx.y -> slice blockIdx.y of p.c ([splits][M][N] floats)
-template <int STORE, int OUT>
+// SCB: bytes of scales a lane fetches, 16 or, where they are not on 16 bytes, 4
+template <int STORE, int OUT, int SCB>
 __global__ void __launch_bounds__(256, 2) k_mx_pair(A8W8Params p) {
     constexpr int MR = MxPair::MR, NR = MxPair::NR, TM = MxPair::TM, TN = MxPair::TN;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[MxPair::LDS_BYTES];
@@ -35,14 +38,19 @@ __global__ void __launch_bounds__(256, 2) k_mx_pair(A8W8Params p) {
     }
 #pragma unroll
     for (int ni = 0; ni < NR; ni++) b_voff[ni] = (uint32_t)(wave * NR + ni) * 16u * row_bytes + (uint32_t)lane * 16u;
-    const bool a_side = wave == 0 || wave == 3;
-    const int chunks = a_side ? ((p.M + 31) >> 5) - (m0 >> 5) : (p.N >> 5) - (n0 >> 5);
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc_uniform((a_side ? p.mx_sa + (uint64_t)(m0 >> 5) * chunk_bytes : p.mx_sb + (uint64_t)(n0 >> 5) * chunk_bytes) + (uint32_t)at * 256u,
-                                                        (uint64_t)chunks * chunk_bytes - (uint32_t)at * 256u);
-    const uint32_t s_voff = (uint32_t)((a_side ? 0 : (wave - 1) * 4) + (lane >> 4)) * chunk_bytes + (uint32_t)(lane & 15) * 16u;
+    const uint8_t *sa = p.mx_sa + (uint64_t)(m0 >> 5) * chunk_bytes + (uint32_t)at * 256u, *sb = p.mx_sb + (uint64_t)(n0 >> 5) * chunk_bytes + (uint32_t)at * 256u;
+    const uint64_t sa_bytes = (uint64_t)(((p.M + 31) >> 5) - (m0 >> 5)) * chunk_bytes - (uint32_t)at * 256u, sb_bytes = (uint64_t)((p.N >> 5) - (n0 >> 5)) * chunk_bytes - (uint32_t)at * 256u;
 
     v4f acc[MR][NR];
-    pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, KT * TK, wave, lane, 2048u, 1024u, rs, s_voff, wave * 2, wave * 2 + 1);
+    if constexpr (SCB == 16) {
+        const bool a_side = wave == 0 || wave == 3;
+        const uint32_t s_voff = (uint32_t)((a_side ? 0 : (wave - 1) * 4) + (lane >> 4)) * chunk_bytes + (uint32_t)(lane & 15) * 16u;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc_uniform(a_side ? sa : sb, a_side ? sa_bytes : sb_bytes);
+        pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, KT * TK, wave, lane, 2048u, 1024u, rs, rs, s_voff, wave * 2, wave * 2 + 1);
+    } else {
+        pair_loop<KIND_MXFP4, 4>(acc, lds, ra, a_voff, rb, b_voff, KT * TK, wave, lane, 2048u, 1024u, make_rsrc_uniform(sa, sa_bytes), make_rsrc_uniform(sb, sb_bytes),
+                                 (uint32_t)wave * chunk_bytes + (uint32_t)lane * 4u, wave * 2, wave * 2 + 1, chunk_bytes);
+    }
 
     if constexpr (STORE == STORE_ACC) {
         static_for<MR>([&](auto MI) {
@@ -83,15 +91,21 @@ __global__ void __launch_bounds__(256, 2) k_mx_pair(A8W8Params p) {
     }
 }
 
+template <int SCB>
+void go(const A8W8Params& p, int store, dim3 grid, hipStream_t stream) {
+    if (store == STORE_ACC) hipLaunchKernelGGL((k_mx_pair<STORE_ACC, OUT_BF16, SCB>), grid, dim3(256), 0, stream, p);
+    else if (p.out == OUT_BF16) hipLaunchKernelGGL((k_mx_pair<STORE_C, OUT_BF16, SCB>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((k_mx_pair<STORE_C, OUT_FP16, SCB>), grid, dim3(256), 0, stream, p);
+}
+
 }  // namespace
 
-// store: STORE_ACC (p.splits slices) or C in p.out; the scale pointers 16-byte aligned
+// store: STORE_ACC (p.splits slices) or C in p.out
 hipError_t psg_launch_mx_pair(const A8W8Params& p, int store, hipStream_t stream) {
     A8W8Params q = p;
     q.splits = store == STORE_ACC && p.splits > 1 ? p.splits : 1;
     const dim3 grid((unsigned)(((p.M + MxPair::TM - 1) / MxPair::TM) * ((p.N + MxPair::TN - 1) / MxPair::TN)), (unsigned)q.splits);
-    if (store == STORE_ACC) hipLaunchKernelGGL((k_mx_pair<STORE_ACC, OUT_BF16>), grid, dim3(256), 0, stream, q);
-    else if (p.out == OUT_BF16) hipLaunchKernelGGL((k_mx_pair<STORE_C, OUT_BF16>), grid, dim3(256), 0, stream, q);
-    else hipLaunchKernelGGL((k_mx_pair<STORE_C, OUT_FP16>), grid, dim3(256), 0, stream, q);
+    if ((reinterpret_cast<uintptr_t>(p.mx_sa) | reinterpret_cast<uintptr_t>(p.mx_sb)) % 16 == 0) go<16>(q, store, grid, stream);
+    else go<4>(q, store, grid, stream);
     return hipGetLastError();
 }

@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(256, 2) k_pair(A8W8Params p) {
     if constexpr (BIAS) s_bias[tid] = p.epi != EPI_NONE ? p.bias[n0 + tid < p.N ? n0 + tid : p.N - 1] : 0;
 
     acc_t acc[MR][NR];
-    pair_loop<KIND>(acc, lds, ra, a_voff, rb, b_voff, (int)kn, wave, lane, b_step, b_half, ra);
+    pair_loop<KIND>(acc, lds, ra, a_voff, rb, b_voff, (int)kn, wave, lane, b_step, b_half, ra, ra);
 
     if constexpr (STORE == STORE_ACC) {
         static_for<MR>([&](auto MI) {

@@ -8,9 +8,9 @@ namespace {
 template <int STORE>
 hipError_t launch_fp4(const A8W8Params& p, int tile_m, int tile_n, hipStream_t stream) {
     constexpr int KIND = KIND_MXFP4;
-    // there is one large tile, whichever is asked for; it fetches the scales 16 bytes a lane
+    // there is one large tile, whichever is asked for
     const bool large = (tile_m == 256 && tile_n == 256) || (tile_m == 128 && (tile_n == 256 || tile_n == 512));
-    if (large && c_in_descriptor(p, 128) && (reinterpret_cast<uintptr_t>(p.mx_sa) | reinterpret_cast<uintptr_t>(p.mx_sb)) % 16 == 0) return psg_launch_mx_pair(p, STORE, stream);
+    if (large && c_in_descriptor(p, 128)) return psg_launch_mx_pair(p, STORE, stream);
     if (large || (tile_m == 64 && tile_n == 256)) return launch_one<KIND, 4, 4, 1, STORE>(p, stream);
     if (tile_m == 32 && tile_n == 256) return launch_one<KIND, 2, 4, 1, STORE>(p, stream);
     if (tile_m == 64 && tile_n == 128) return launch_one<KIND, 4, 2, 1, STORE>(p, stream);

@@ -88,7 +88,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_pair(MoeParams p, MoeRowsParams 
     }
 
     acc_t acc[MR][NR];
-    pair_loop<KIND>(acc, lds, ra, a_voff, rb, b_voff, K, wave, lane, 2048u, 1024u, ra);
+    pair_loop<KIND>(acc, lds, ra, a_voff, rb, b_voff, K, wave, lane, 2048u, 1024u, ra, ra);
 
     // ---- 16-bit rows through LDS (16-byte granules XORed with the row), in halves, then out row by row ----
     constexpr int ROWB = TN * 2, GR = ROWB / 16, RPP = 256 / GR;  // bytes and granules of a staged row, rows of a store pass

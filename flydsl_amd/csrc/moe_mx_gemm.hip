@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
     }
 
     v4f acc[MR][NR];
-    pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, p.K >> 1, wave, lane, 2048u, 1024u, rs, s_voff, STAGE == 1 ? wave : wave * 2, STAGE == 1 ? wave + 4 : wave * 2 + 1);
+    pair_loop<KIND_MXFP4>(acc, lds, ra, a_voff, rb, b_voff, p.K >> 1, wave, lane, 2048u, 1024u, rs, rs, s_voff, STAGE == 1 ? wave : wave * 2, STAGE == 1 ? wave + 4 : wave * 2 + 1);
 
     // rows past the last 64 in use are not written
     const int end = (used + 63) / 64 * 64 - blk * TM, live = end < TM ? end : TM;

@@ -8,7 +8,8 @@
 //     half-step register sets; two whole-step sets need the same 64 registers and are ahead by half as much.  (fp8, whose MFMA takes both
 //     halves, has those: a step ahead.)
 //   * The scale dwords of a step, 4 chunks of 256 bytes on the A side and 8 on the W side, are one 16-byte DMA of three of the wavefronts: a DMA
-//     takes 64 lanes anywhere, so 16 lanes bring a chunk and one instruction four of them.
+//     takes 64 lanes anywhere, so 16 lanes bring a chunk and one instruction four of them.  Scales that are not on 16 bytes come 4 bytes a lane, a chunk an instruction, three
+//     of every wavefront (SCB = 4).
 //   * At most one memory instruction stands behind an MFMA: what is issued between two of them in a row, the matrix cores wait for (one
 //     workgroup alone on a CU, zero operands: 1,580 core cycles a step with the instructions in front of each block of four MFMAs, 1,450 like
 //     this; 1,088 is what 64 MFMAs take).
@@ -38,14 +39,16 @@ using MxPair = Pair<KIND_MXFP4>;
 //            16-byte piece (lane % 8) ^ (row / 2 % 8); out of the descriptor's bounds for a row that reads as zero
 //   b_voff   this lane's offsets into `rb` of the wavefront's four 16-row blocks, b_step and b_half from a step and a half step to the next (2048 and 1024 in the
 //            preshuffled order)
-// fp4 only (rs: any descriptor otherwise):
+// fp4 only (rs and rs_w: any descriptors otherwise):
 //   s_voff   this lane's offset into `rs`, the scales of wavefront 0 and 3: A side, 1 and 2: W side chunks 0..3 and 4..7 of the tile: chunk
 //            lane / 16, 16-byte piece lane % 16
 //   chunk0/1 which of the eight W-side chunks belong to the wavefront's blocks 0, 1 and 2, 3
-template <int KIND, class ACC>
+//   SCB = 4: `rs` the A side, s_voff chunk `wave` of it, 4-byte piece `lane`; `rs_w` the W side, in chunks of chunk_bytes (SCB = 16: any descriptor)
+template <int KIND, int SCB = 16, class ACC>
 __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const __amdgpu_buffer_rsrc_t ra, const uint32_t (&a_voff)[4],
                                           const __amdgpu_buffer_rsrc_t rb, const uint32_t (&b_voff)[4], const int K, const int wave, const int lane,
-                                          const uint32_t b_step, const uint32_t b_half, const __amdgpu_buffer_rsrc_t rs, const uint32_t s_voff = 0, const int chunk0 = 0, const int chunk1 = 0) {
+                                          const uint32_t b_step, const uint32_t b_half, const __amdgpu_buffer_rsrc_t rs, const __amdgpu_buffer_rsrc_t rs_w,
+                                          const uint32_t s_voff = 0, const int chunk0 = 0, const int chunk1 = 0, const uint32_t chunk_bytes = 0) {
     using P = Pair<KIND>;
     constexpr int MR = P::MR, NR = P::NR, NS = P::NS, STAGE = P::STAGE, SC_SLOT = P::SC_SLOT;
     constexpr bool MX = KIND == KIND_MXFP4, WHOLE = KIND == KIND_FP8;  // WHOLE: an MFMA takes both halves of a step
@@ -58,12 +61,17 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
     // (wavefront 3 brings the bytes of wavefront 0 once more: all of them count the same number of DMAs)
     const uint32_t sc_dst = lds_base + (uint32_t)(NS * STAGE) + (uint32_t)(wave == 3 ? 0 : wave) * 1024u;
 
-    // DMA j of step kt: 0..3 A, 4 scales.  Without CHK the step is known to be before the end
-    constexpr int N_DMA = MX ? 5 : 4;
+    // DMA j of step kt: 0..3 A, from 4 on scales.  Without CHK the step is known to be before the end
+    constexpr int N_DMA = !MX ? 4 : SCB == 16 ? 5 : 7;
     auto dma = [&](int kt, int stage, int j, auto CHK) __attribute__((always_inline)) {
         const bool has = !decltype(CHK)::value || kt < KT, in = !decltype(CHK)::value || kt * TK + a_kc[j & 1] * 16 < K;
         if (j < 4) dma16(ra, lds_base + (uint32_t)(stage * STAGE + (wave * 4 + j) * 1024), in ? a_voff[j < 4 ? j : 0] : OOB, has ? (uint32_t)kt * TK : 0u);
-        else dma16(rs, sc_dst + (uint32_t)(stage * SC_SLOT), has ? s_voff : OOB, has ? (uint32_t)kt * 256u : 0u);
+        else if (SCB == 16) dma16(rs, sc_dst + (uint32_t)(stage * SC_SLOT), has ? s_voff : OOB, has ? (uint32_t)kt * 256u : 0u);
+        else if (j == 4) dma4(rs, lds_base + (uint32_t)(NS * STAGE + stage * SC_SLOT + wave * 256), has ? s_voff : OOB, has ? (uint32_t)kt * 256u : 0u);
+        else {
+            const int ch = j == 5 ? chunk0 : chunk1;
+            dma4(rs_w, lds_base + (uint32_t)(NS * STAGE + stage * SC_SLOT + 1024 + ch * 256), has ? (uint32_t)ch * chunk_bytes + (uint32_t)lane * 4u : OOB, has ? (uint32_t)kt * 256u : 0u);
+        }
     };
     v4i bw[4][NR];
     auto load_w = [&](int kt, int half, int ni, v4i* dst, auto CHK) __attribute__((always_inline)) {
@@ -128,9 +136,10 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
                 // for W let as many instructions be on their way as there are W loads behind the awaited one, DMAs among them: in each half the DMAs
                 // go first, and both halves have some.
                 if constexpr (ni == 2) {
-                    if constexpr (b >= 1 && b < 4) dma(kt + 3, (S + 3) % NS, b - 1, CHK);
+                    constexpr int FROM = N_DMA == 7 ? 0 : 1, LOW = 4 - FROM;  // block of the first DMA in a half; DMAs in the lower one
+                    if constexpr (b >= FROM && b < 4) dma(kt + 3, (S + 3) % NS, b - FROM, CHK);
                     if constexpr (b >= 4 && b < 8) load_w(kt + 1, 1, b - 4, bw[(2 * S + 3) % 4], CHK);
-                    if constexpr (b >= 9 && b < (MX ? 11 : 10)) dma(kt + 3, (S + 3) % NS, b - 6, CHK);
+                    if constexpr (b >= 8 + FROM && b < 8 + FROM + N_DMA - LOW) dma(kt + 3, (S + 3) % NS, b - 8 - FROM + LOW, CHK);
                     if constexpr (b >= 11 && b < 15) load_w(kt + 2, 0, b - 11, bw[(2 * S + 4) % 4], CHK);
                 }
                 __builtin_amdgcn_sched_barrier(0);

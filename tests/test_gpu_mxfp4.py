@@ -149,8 +149,8 @@ def test_mxfp4_strided_batched_default_strides():
 
 
 # ---- the 128x256 tile (two workgroups a CU): the same accumulator bits as the 64x256 tile, which has the same K order, at one to nine K steps, either side of a
-# tile's rows and columns, 32 columns, over K splits of uneven length (one of them empty), in both output types; with scales off 16 bytes
-# the call runs on 64x256 tiles
+# tile's rows and columns, 32 columns, over K splits of uneven length (one of them empty), in both output types; with scales on 16
+# bytes, which one instruction a step fetches, and off them (fetched 4 bytes a lane)
 @pytest.mark.parametrize("M,N,K", [(1, 32, 256), (127, 256, 512), (128, 288, 768), (129, 544, 1024), (255, 224, 1280), (385, 1056, 1792), (64, 480, 2048), (300, 512, 2304)])
 def test_large_tile_equals_the_64_row_tile(M, N, K):
     from kernels.gemm.mxfp4_preshuffle import launch_gemm
