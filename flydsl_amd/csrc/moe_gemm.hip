@@ -15,6 +15,7 @@
 // (v_j & 15) | (v_{j+4} << 4) (tests/kernels/test_moe_gemm_2stage.py:64-80 of the reference), so a lane's 16-byte piece
 // of a fragment is 8 bytes at half the offset; it is unpacked with the reference's sign-extending mask-and-multiply
 // (kernels/common/mma/mfma_preshuffle_pipeline.py:225-238) into the same int8 fragment and multiplied by the int8 MFMA.
+#include "moe_blocks.h"
 #include "moe_rows.h"
 #include "psg_common.h"
 
@@ -58,11 +59,11 @@ __device__ __forceinline__ float silu(float g) { return g / (1.0f + __expf(-g));
 // from the start of each run of equal expert ids: the workgroup of the second block of a pair ends at once, and the
 // first one treats the second half of its tile as padding when the run ends there.
 // AHEAD: 0 = operands a step ahead; 1 = three steps (the rule and its figures: takes_deep; a stage by rows never, having more workgroups than that); 2 = three steps,
-// and W past the caches (takes_nt).
+// and W past the caches where a tile is the only one to read it (takes_nt, moe_reads_once).
 // ROWS = MoeRowsParams: the down stage by rows, whose first `rows.wgs` rows of the grid make the lists of the tokens' rows.  A build of
 // its own: the decode layers, which add directly, lost 0.4 to 0.8 us of 55 to 140 to the longer arguments and the branch.
 template <int KIND, int MR, int NR, int STAGE, int CO, int AHEAD, class... ROWS>
-__global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AHEAD != 2 || KIND == KIND_INT8W4 ? 1 : MR <= 2 ? 4 : 3))) k_moe_gemm(MoeParams p, ROWS... rows) {
     using acc_t = typename MoeAcc<KIND>::type;
     constexpr int BM = 16 * MR, TN = 64 * NR;
     constexpr int BLK = BM / CO;                        // rows of one block of the sorted list
@@ -71,7 +72,6 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     constexpr bool W4 = KIND == KIND_INT8W4;           // packed int4 weights
     constexpr int WSH = W4 ? 1 : 0;                    // weight byte offsets are halved
     constexpr bool DEEP = AHEAD != 0;
-    constexpr int W_CACHE = AHEAD == 2 ? 2 : 0;        // cache policy of a W load: nt or none
     __shared__ __attribute__((aligned(16))) uint8_t lds[2][BM * 128];
     __shared__ int ids[BM];
     __shared__ float s_sx[BM], s_rw[BM];  // per tile row: scale of its x row and routing weight, fetched before the K loop
@@ -90,6 +90,14 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     }
     const int n0 = (int)blockIdx.x * TN;
     const int used = p.num_valid[0];
+    // what is looked at of the list's experts, in one go
+    MoeNeighbours around;
+    int back = 0;  // of block blk - 1 - lane
+    if constexpr (AHEAD == 2) around = moe_neighbours(p.expert_ids, (int)gridDim.y, blk, CO, lane);
+    if constexpr (CO == 2) back = p.expert_ids[blk - 1 - lane > 0 ? blk - 1 - lane : 0];
+    auto sorted_row = [&]() { return tid < BM && blk * BLK + tid < p.sorted_size ? p.sorted_ids[blk * BLK + tid] : p.tokens; };  // past the list = a padding row
+    int my_id = 0;
+    if constexpr (AHEAD == 2) my_id = sorted_row();
     if (blk * BLK >= used) return;                     // uniform: blocks past the sorted rows in use
     const int e = p.expert_ids[blk];
     if (e < 0 || e >= p.experts) return;               // uniform: a block without an expert
@@ -99,7 +107,8 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
         int before = 0;
         for (int base = blk - 1; base >= 0; base -= 64) {
             const int j = base - lane;
-            const unsigned long long same = __ballot(j >= 0 && p.expert_ids[j] == e);
+            const int v = base == blk - 1 ? back : p.expert_ids[j > 0 ? j : 0];
+            const unsigned long long same = __ballot(j >= 0 && v == e);
             const int run = same == ~0ull ? 64 : __builtin_ctzll(~same);
             before += run;
             if (run < 64) break;
@@ -149,9 +158,10 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
     constexpr int WPF = DEEP ? 3 : 1;
     constexpr int NWS = WPF + 1;
     wreg_t blo[NWS][NSET][NR], bhi[NWS][NSET][NR];
-    auto w8 = [&](uint32_t voff, uint32_t soff) { return (v2i)__builtin_amdgcn_raw_buffer_load_b64(rb, (int)voff, (int)soff, W_CACHE); };
-    auto w16 = [&](uint32_t voff, uint32_t soff) { return (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)voff, (int)soff, W_CACHE); };
-    auto load_b = [&](int kt, int set) {
+    auto load_b = [&](int kt, int set, auto NTP) __attribute__((always_inline)) {
+        constexpr int POLICY = decltype(NTP)::value ? 2 : 0;  // non-temporal or none
+        auto w8 = [&](uint32_t voff, uint32_t soff) { return (v2i)__builtin_amdgcn_raw_buffer_load_b64(rb, (int)voff, (int)soff, POLICY); };
+        auto w16 = [&](uint32_t voff, uint32_t soff) { return (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)voff, (int)soff, POLICY); };
 #pragma unroll
         for (int s = 0; s < NSET; s++)
 #pragma unroll
@@ -185,11 +195,11 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
 #pragma unroll
             for (int ni = 0; ni < NR; ni++) acc[mi][s][ni] = (acc_t){0, 0, 0, 0};
 
-    auto step = [&](int kt, auto SP, auto WP) __attribute__((always_inline)) {
+    auto step = [&](int kt, auto SP, auto WP, auto NTP) __attribute__((always_inline)) {
         constexpr int S = decltype(SP)::value;    // LDS stage of this step's A tile
         constexpr int WS = decltype(WP)::value;   // register set of this step's W fragments
         load_a(kt + (DEEP ? 3 : 1), DEEP ? (WS + 3) % NAS : 0);
-        load_b(kt + WPF, (WS + WPF) % NWS);
+        load_b(kt + WPF, (WS + WPF) % NWS, NTP);
         // packed int4: this step's fragments unpacked once, in front of the row blocks that share them
         v4i ulo[W4 ? NSET : 1][W4 ? NR : 1], uhi[W4 ? NSET : 1][W4 ? NR : 1];
         if constexpr (W4) {
@@ -228,51 +238,60 @@ __global__ void __launch_bounds__(256) k_moe_gemm(MoeParams p, ROWS... rows) {
         __syncthreads();
     };
 
-    // W first: its addresses need only the expert, so these requests are in flight while the sorted row list is fetched
-    static_for<WPF>([&](auto I) { load_b(decltype(I)::value, decltype(I)::value); });
-    if (tid < BM) {
-        const int q = blk * BLK + tid;
-        ids[tid] = (tid < rows_live && q < p.sorted_size) ? p.sorted_ids[q] : p.tokens;  // past the list or the pair = a padding row
-    }
-    __syncthreads();
+    // the product, W past the caches (NTP) or through them
+    auto product = [&](auto NTP) __attribute__((always_inline)) {
+        // W first: its addresses need only the expert, so these requests are in flight while the sorted row list is fetched (which is here already where W waited for the
+        // experts of the list)
+        static_for<WPF>([&](auto I) { load_b(decltype(I)::value, decltype(I)::value, NTP); });
+        if constexpr (AHEAD != 2) my_id = sorted_row();
+        if (tid < BM) ids[tid] = tid < rows_live ? my_id : p.tokens;  // past the pair = a padding row
+        __syncthreads();
 
-    // row of x (and of its scale) a tile row reads, or -1 for a padding row
-    auto x_row = [&](int r) {
-        const uint32_t sid = (uint32_t)ids[r];
-        const int t = (int)(sid & 0xFFFFFFu), s = (int)(sid >> 24);
-        if (t >= p.tokens || s >= p.topk) return -1;
-        if constexpr (STAGE == 1) return p.x_slot_major ? s * p.tokens + t : t;
-        return t * p.topk + s;
-    };
-    // the epilogue's per-row factors now, so that their memory latency runs under the K loop (whose barriers also make them
-    // visible to every wavefront)
-    if (tid < BM) {
-        const int xr = x_row(tid);
-        s_sx[tid] = xr >= 0 ? p.sx[xr] : 0.f;
-        s_rw[tid] = (p.doweight && xr >= 0) ? p.sorted_w[blk * BLK + tid] : 1.0f;
-    }
+        // row of x (and of its scale) a tile row reads, or -1 for a padding row
+        auto x_row = [&](int r) {
+            const uint32_t sid = (uint32_t)ids[r];
+            const int t = (int)(sid & 0xFFFFFFu), s = (int)(sid >> 24);
+            if (t >= p.tokens || s >= p.topk) return -1;
+            if constexpr (STAGE == 1) return p.x_slot_major ? s * p.tokens + t : t;
+            return t * p.topk + s;
+        };
+        // the epilogue's per-row factors now, so that their memory latency runs under the K loop (whose barriers also make them
+        // visible to every wavefront)
+        if (tid < BM) {
+            const int xr = x_row(tid);
+            s_sx[tid] = xr >= 0 ? p.sx[xr] : 0.f;
+            s_rw[tid] = (p.doweight && xr >= 0) ? p.sorted_w[blk * BLK + tid] : 1.0f;
+        }
 
 #pragma unroll
-    for (int j = 0; j < A_LOADS; j++) {
-        const int c = tid + 256 * j, row = c >> 3, kc = c & 7;
-        const int xr = row < BM ? x_row(row) : -1;
-        a_voff[j] = xr >= 0 ? (uint32_t)xr * (uint32_t)K + (uint32_t)kc * 16u : OOB;
-        a_ldsoff[j] = row < BM ? moe_lds_off(row, kc) : -1;
-    }
-    static_for<DEEP ? 3 : 1>([&](auto I) { load_a(decltype(I)::value, decltype(I)::value); });
-    store_a(0, 0);
-    __syncthreads();
-    // unrolled over lcm(2 LDS stages, NWS register sets) steps so that both indices are compile-time
-    constexpr int UN = NWS % 2 == 0 ? NWS : 2 * NWS;
-    int kt0 = 0;
-    if constexpr (DEEP)  // whole rounds without a condition: the compiler's count of the loads on their way is then exact
-        for (; kt0 + UN <= KT; kt0 += UN)
-            static_for<UN>([&](auto I) { step(kt0 + decltype(I)::value, std::integral_constant<int, decltype(I)::value & 1>{}, std::integral_constant<int, decltype(I)::value % NWS>{}); });
-    for (; kt0 < KT; kt0 += UN) {
-        static_for<UN>([&](auto I) {
-            constexpr int i = decltype(I)::value;
-            if (kt0 + i < KT) step(kt0 + i, std::integral_constant<int, i & 1>{}, std::integral_constant<int, i % NWS>{});
-        });
+        for (int j = 0; j < A_LOADS; j++) {
+            const int c = tid + 256 * j, row = c >> 3, kc = c & 7;
+            const int xr = row < BM ? x_row(row) : -1;
+            a_voff[j] = xr >= 0 ? (uint32_t)xr * (uint32_t)K + (uint32_t)kc * 16u : OOB;
+            a_ldsoff[j] = row < BM ? moe_lds_off(row, kc) : -1;
+        }
+        static_for<DEEP ? 3 : 1>([&](auto I) { load_a(decltype(I)::value, decltype(I)::value); });
+        store_a(0, 0);
+        __syncthreads();
+        // unrolled over lcm(2 LDS stages, NWS register sets) steps so that both indices are compile-time
+        constexpr int UN = NWS % 2 == 0 ? NWS : 2 * NWS;
+        int kt0 = 0;
+        if constexpr (DEEP)  // whole rounds without a condition: the compiler's count of the loads on their way is then exact
+            for (; kt0 + UN <= KT; kt0 += UN)
+                static_for<UN>([&](auto I) { step(kt0 + decltype(I)::value, std::integral_constant<int, decltype(I)::value & 1>{}, std::integral_constant<int, decltype(I)::value % NWS>{}, NTP); });
+        for (; kt0 < KT; kt0 += UN) {
+            static_for<UN>([&](auto I) {
+                constexpr int i = decltype(I)::value;
+                if (kt0 + i < KT) step(kt0 + i, std::integral_constant<int, i & 1>{}, std::integral_constant<int, i % NWS>{}, NTP);
+            });
+        }
+    };
+    if constexpr (AHEAD == 2) {
+        const int n = (used + BLK - 1) / BLK;
+        if (moe_reads_once(around, p.expert_ids, n < (int)gridDim.y ? n : (int)gridDim.y, blk, CO, e, p.experts, p.cached, lane)) product(std::true_type{});
+        else product(std::false_type{});
+    } else {
+        product(std::false_type{});
     }
 
     // Epilogue, one pass per ni (64 consecutive columns of the tile): every lane finishes its own fragments (rows
@@ -372,10 +391,13 @@ bool takes_deep(const MoeParams& p, int block_m, int blocks, int nx) {
 // 68.5; blocks of 32 110 80.7 / 73.0, 192 80.3 / 73.1; int4 8 tokens 35.6 / 32.7; 64 experts, 2048 x 768, 128 x top-4 39.1 / 35.9.  Stage 2 8 tokens 33.3 / 30.5, 128 x top-4 23.4 /
 // 21.3, but 96 x top-8 in blocks of 16 (one and a half tiles an expert) 45.6 / 50.9, 100 x top-6 on 16, 3072 x 512 11.6 / 12.3.  The
 // cache keeps nothing that was read like this: a layer of 226 MB (128 experts, 2304 x 256, 160 x top-8) took 73.7 / 69.4 from memory, 60.8 / 68.9 from the cache.
-template <int KIND, int STAGE>
+// That is the rule for the routings that a call can have; which tiles of its own do is for the workgroups to say (moe_reads_once), because a router that prefers some experts leaves the others'
+// weights unread, so that what is read fits the cache, and gives the busy ones several tiles.  Layers, us through the caches / past them everywhere / as it is, weights in memory; in the
+// cache, expert preferences N(0, 4^2) beside N(0, 1) logits, 32 experts, 4096 x 1536, top-8, fp8: 64 tokens 94.2 / 96.8 / 89.0; 71.3 / 92.9 / 72.5, 96 98.2 / 102.8 / 94.8; 79.8 / 101.5 / 80.3,
+// int4 64 74.0 / 72.5 / 72.9; 58.3 / 69.6 / 59.0; 64 experts, 2048 x 2048, 128 x top-4 56.9 / 62.8 / 57.5; 45.3 / 56.0 / 44.0.  Without preferences within 0.5 % of past them everywhere.
+template <int STAGE>
 bool takes_nt(const MoeParams& p, int tile_m) {
-    const int64_t rows_e = STAGE == 1 ? 2ll * p.n_out : p.n_out, bytes = (p.experts * rows_e * p.K) >> (KIND == KIND_INT8W4 ? 1 : 0);
-    return bytes * (STAGE == 1 ? 3 : 6) >= 2ll * (256 << 20) && 4ll * p.tokens * p.topk <= 3ll * p.experts * tile_m;
+    return p.experts > p.cached && 4ll * p.tokens * p.topk <= 3ll * p.experts * tile_m;
 }
 
 // Whether a stage multiplies two consecutive blocks of an expert in one workgroup.  Stage 1 with one-byte weights always does with blocks of up to 32 rows (64 tokens x
@@ -393,9 +415,10 @@ bool takes_pairs(const MoeParams& p, int block_m) {
 }
 
 template <int KIND, int STAGE, int NR>
-hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int blocks, bool pair, hipStream_t stream) {
+hipError_t launch_nr(MoeParams p, MoeRowsParams rows, int block_m, int blocks, bool pair, hipStream_t stream) {
     const unsigned nx = (unsigned)((p.n_out + 64 * NR - 1) / (64 * NR));
     rows.wgs = 0;
+    p.cached = moe_experts_cached(STAGE, ((STAGE == 1 ? 2ll * p.n_out : p.n_out) * p.K) >> (KIND == KIND_INT8W4 ? 1 : 0));
     // rows of the grid for the lists, as far as it has any left (65535 of them)
     const int list_rows = (int)((ROWS_INDEX_WGS + nx - 1) / nx);
     const bool lists = STAGE == 2 && p.by_position && rows.sorted_size <= moe_rows_share_max(block_m) && blocks + list_rows <= 65535;
@@ -417,7 +440,7 @@ hipError_t launch_nr(const MoeParams& p, MoeRowsParams rows, int block_m, int bl
                 return hipGetLastError();                                                                \
             }                                                                                            \
         }                                                                                                \
-        if (kNt && takes_nt<KIND, STAGE>(p, block_m * CO_)) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kNt ? 2 : 1>), grid, dim3(256), 0, stream, p); \
+        if (kNt && takes_nt<STAGE>(p, block_m * CO_)) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kNt ? 2 : 1>), grid, dim3(256), 0, stream, p); \
         else if (deep || kOnly) hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, 1>), grid, dim3(256), 0, stream, p); \
         else hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, kOnly ? 1 : 0>), grid, dim3(256), 0, stream, p); \
         return hipGetLastError();                                                                        \
@@ -512,5 +535,20 @@ hipError_t psg_launch_moe_reduce(const void* x, void* y, int tokens, int topk, i
     const size_t quads = (size_t)tokens * (size_t)(dim >> 2);
     hipLaunchKernelGGL(k_moe_reduce, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, static_cast<const uint16_t*>(x),
                        static_cast<uint16_t*>(y), tokens, topk, dim, out_dtype, mask, ids, experts);
+    return hipGetLastError();
+}
+
+// What moe_reads_once says of every block of a list, by one wavefront each (for tests)
+namespace {
+__global__ void __launch_bounds__(64) k_moe_reads_once(const int32_t* expert_ids, int blocks, int used, int per_tile, int experts, int cached, int32_t* out) {
+    const int blk = (int)blockIdx.x, lane = (int)threadIdx.x, e = expert_ids[blk];
+    const bool counts = blk < used && (unsigned)e < (unsigned)experts;
+    const int once = moe_reads_once(moe_neighbours(expert_ids, blocks, blk, per_tile, lane), expert_ids, used, blk, per_tile, e, experts, cached, lane);
+    if (lane == 0) out[blk] = counts ? once : -1;
+}
+}  // namespace
+
+hipError_t psg_launch_moe_reads_once(const int32_t* expert_ids, int blocks, int used, int per_tile, int experts, int cached, int32_t* out, hipStream_t stream) {
+    hipLaunchKernelGGL(k_moe_reads_once, dim3((unsigned)blocks), dim3(64), 0, stream, expert_ids, blocks, used, per_tile, experts, cached, out);
     return hipGetLastError();
 }

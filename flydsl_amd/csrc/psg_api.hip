@@ -15,6 +15,7 @@
 
 hipError_t psg_launch_a8w8_tiled(const A8W8Params& p, int kind, int store, int tile_m, int tile_n, hipStream_t stream);
 hipError_t psg_launch_a8w8_stream(const A8W8Params& p, int kind, int store, hipStream_t stream);
+hipError_t psg_launch_moe_reads_once(const int32_t* expert_ids, int blocks, int used, int per_tile, int experts, int cached, int32_t* out, hipStream_t stream);
 hipError_t psg_launch_moe_gemm(const MoeParams& p, const MoeRowsParams& rows, int kind, int stage, int block_m, int blocks, hipStream_t stream);
 hipError_t psg_launch_moe_mx_gemm(const MoeMxParams& p, const MoeRowsParams& rows, int a_format, int stage, int block_m, int blocks, hipStream_t stream);
 hipError_t psg_launch_moe_mx_scale_sort(const void* scale, const int32_t* sorted_ids, const int32_t* num_valid, void* out, int tokens, int topk, int cols,
@@ -725,6 +726,16 @@ int psg_debug_tile_order(int32_t tiles_m, int32_t tiles_n, int32_t group_m, int3
         return fail(PSG_E_SHAPE, "need tiles_m, tiles_n, group_m >= 1 and at most 2^24 tiles");
     const hipError_t e = psg_launch_tile_order(tiles_m, tiles_n, group_m, out, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "psg_debug_tile_order launch");
+    g_err[0] = 0;
+    return 0;
+}
+
+int psg_debug_moe_reads_once(const int32_t* expert_ids, int32_t blocks, int32_t used, int32_t per_tile, int32_t experts, int32_t cached, int32_t* out, void* stream) {
+    if (!expert_ids || !out) return fail(PSG_E_NULL, "expert_ids and out must be non-NULL");
+    if (blocks < 1 || blocks > (1 << 20) || used < 0 || used > blocks || (per_tile != 1 && per_tile != 2) || experts < 1 || cached < 0)
+        return fail(PSG_E_SHAPE, "need 1 <= blocks <= 2^20, 0 <= used <= blocks, per_tile 1 or 2, experts >= 1, cached >= 0");
+    const hipError_t e = psg_launch_moe_reads_once(expert_ids, blocks, used, per_tile, experts, cached, out, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(e, "psg_debug_moe_reads_once launch");
     g_err[0] = 0;
     return 0;
 }

@@ -203,6 +203,7 @@ struct MoeParams {
     int blocks;                 // set by the launcher of the 128x256 tiles: entries of expert_ids
     int by_position;            // stage 2 without accumulate: one row per sorted position instead of one per (token, slot)
     int pair_blocks;            // blocks of 16 / 32 rows: multiply two consecutive blocks of one expert in one workgroup
+    int cached;                 // set by the launcher of the builds that may read W past the caches: experts whose weights these hold
 };
 
 // Arguments of the MX (fp4 weights, e8m0 scales per 32 K elements) MoE grouped GEMMs over sorted token blocks.

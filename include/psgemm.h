@@ -25,6 +25,8 @@
  *   psg_tile_coords     the workgroup-id -> tile remap xcd_remap_bx_by
  *                       kernels/common/mma/mfma_preshuffle_pipeline.py:685-729 (host evaluation of the function the
  *                       tiled kernel uses); psg_debug_tile_order runs the same function on the device
+ *   psg_debug_moe_reads_once
+ *                       no counterpart: which tiles of a MoE stage read their weights past the caches
  *   psg_gemm_a8w8_static, psg_init, psg_static_scratch_bytes
  *                       no counterpart in the reference: for callers that cannot allocate (see below)
  *   psg_moe_gemm        kernels/moe/moe_gemm_2stage/gemm1.py, gemm2.py (launch_moe_gemm1 / launch_moe_gemm2), fp8 and int8
@@ -205,6 +207,11 @@ void psg_tile_coords(int32_t id, int32_t tiles_m, int32_t tiles_n, int32_t group
 
 /* Evaluates the same function on the device for every id: out[2*id] = tm, out[2*id+1] = tn (int32 [tiles_m*tiles_n*2]). */
 int psg_debug_tile_order(int32_t tiles_m, int32_t tiles_n, int32_t group_m, int32_t *out, void *stream);
+
+/* How the MoE stages on small blocks read the weights, for tests: out[i] = 1 where the tile of `per_tile` (1 or 2) blocks from block i on reads them past the
+ * caches, 0 where through them, -1 where the block has no expert or is not one of the `used` ones.  expert_ids int32 [blocks]; `cached` experts' weights fit the
+ * last-level cache. */
+int psg_debug_moe_reads_once(const int32_t *expert_ids, int32_t blocks, int32_t used, int32_t per_tile, int32_t experts, int32_t cached, int32_t *out, void *stream);
 
 /* Same mainloop, but writes the raw accumulators [M,N] (int32 for int8, fp32 for fp8) to `acc`
  * instead of C.  c, scale_a, scale_b, bias are ignored. */

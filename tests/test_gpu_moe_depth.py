@@ -58,3 +58,26 @@ def test_depths(stage, block, tokens, topk, experts, n_out, kind, steps):
     else:
         # half a unit in the last place of bf16, and the fp32 exponential and division
         assert ((out.double() - want).abs() <= (2.0 ** -8 + 2.0 ** -18) * want.abs() + 1e-30).all()
+
+
+@pytest.mark.parametrize("per_tile", [1, 2])
+@pytest.mark.parametrize("runs,unused", [([1] * 20, 0), ([1] * 20, 1), ([3, 1, 2, 1, 4], 0), ([3, 1, 2, 1, 4], 2), ([1] * 64, 0), ([1] * 65, 0), ([2] * 64, 0), ([1, 2] * 43, 0), ([1, 2] * 43, 3),
+                                         ([1] * 300, 0), ([5] + [1] * 200 + [64, 1, 1], 0), ([7], 0), ([2, 2], 4)])
+def test_the_only_tile_of_an_expert_reads_past_the_caches(runs, unused, per_tile):
+    """... and only where more experts have rows than the caches hold: over runs of blocks, some without an expert, the last ones not in use."""
+    from flydsl_amd import _lib
+
+    experts, handle = len(runs) + 5, _lib.lib()
+    ids = [e if e % 7 != 3 else (-1 if e % 2 else experts + 2) for e, n in enumerate(runs) for _ in range(n)]
+    used = len(ids) - unused
+    seen = len({e for e in ids[:used] if 0 <= e < experts})
+    t = torch.tensor(ids, dtype=torch.int32, device="cuda")
+    for cached in (0, max(seen - 1, 0), seen):
+        want = []
+        for i, e in enumerate(ids):
+            alone = (i == 0 or ids[i - 1] != e) and not (i + per_tile < used and ids[i + per_tile] == e)
+            want.append(-1 if i >= used or not 0 <= e < experts else int(alone and seen > cached))
+        out = torch.full((len(ids),), -5, dtype=torch.int32, device="cuda")
+        rc = handle.psg_debug_moe_reads_once(t.data_ptr(), len(ids), used, per_tile, experts, cached, out.data_ptr(), _lib.stream_handle(None))
+        assert rc == 0, handle.psg_last_error()
+        assert out.tolist() == want, cached
