@@ -393,8 +393,8 @@ bool takes_deep(const MoeParams& p, int block_m, int blocks, int nx) {
 // cache keeps nothing that was read like this: a layer of 226 MB (128 experts, 2304 x 256, 160 x top-8) took 73.7 / 69.4 from memory, 60.8 / 68.9 from the cache.
 // That is the rule for the routings that a call can have; which tiles of its own do is for the workgroups to say (moe_reads_once), because a router that prefers some experts leaves the others'
 // weights unread, so that what is read fits the cache, and gives the busy ones several tiles.  Layers, us through the caches / past them everywhere / as it is, weights in memory; in the
-// cache, expert preferences N(0, 4^2) beside N(0, 1) logits, 32 experts, 4096 x 1536, top-8, fp8: 64 tokens 94.2 / 96.8 / 89.0; 71.3 / 92.9 / 72.5, 96 98.2 / 102.8 / 94.8; 79.8 / 101.5 / 80.3,
-// int4 64 74.0 / 72.5 / 72.9; 58.3 / 69.6 / 59.0; 64 experts, 2048 x 2048, 128 x top-4 56.9 / 62.8 / 57.5; 45.3 / 56.0 / 44.0.  Without preferences within 0.5 % of past them everywhere.
+// cache, expert preferences N(0, 4^2) beside N(0, 1) logits, 32 experts, 4096 x 1536, top-8, fp8: 64 tokens 94.8 / 96.8 / 89.5; 70.9 / 92.9 / 69.3, 96 98.4 / 102.8 / 91.2; 80.6 / 101.5 / 76.1,
+// int4 64 74.0 / 72.5 / 70.6; 58.1 / 69.6 / 56.6; 64 experts, 2048 x 2048, 128 x top-4 56.9 / 62.8 / 52.8; 45.5 / 56.0 / 42.9.  Without preferences within 0.5 % of past them everywhere.
 template <int STAGE>
 bool takes_nt(const MoeParams& p, int tile_m) {
     return p.experts > p.cached && 4ll * p.tokens * p.topk <= 3ll * p.experts * tile_m;

@@ -14,6 +14,7 @@
 // Operands are swapped (src0 = W, src1 = A) so a lane ends up with 4 consecutive columns of one row.  Four wavefronts side
 // by side along N; each covers 64 W rows: in stage 1 32 gate rows and the 32 up rows of the same columns, so a wavefront
 // owns whole 32-column quantisation groups.
+#include "moe_blocks.h"
 #include "moe_rows.h"
 #include "pair_loop.h"
 
@@ -83,7 +84,7 @@ __device__ __forceinline__ int quant_silu_mul(const v4f g0, const v4f g1, const 
 // LDS with the same scale rule as the output (kernels/moe/mxfp_moe/gemm1.py:324-412), and no A-side scales are read.  (A variant
 // that first quantised all K elements of the 16 rows into LDS and then ran the K loop without barriers measured slower: 16 tokens
 // x top-8 on 32 experts 38.9 us against 35.4, 64 tokens 42.2 against 41.)
-// NT: W past the caches (takes_nt)
+// NT: W past the caches where a tile is the only one to read it (takes_nt, moe_reads_once)
 template <int AF, int MR, int STAGE, bool IQ, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 4 ? 2 : 1))) k_moe_mx(MoeMxParams p, MoeRowsParams rows) {
     static_assert(MR % 2 == 0 || MR == 1, "scale chunks cover 32 rows; a single 16-row block picks its half at run time");
@@ -129,7 +130,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
         n_tile = wg % p.n_tiles;
     }
     // the quad order rounds the row blocks up to an even number: the odd one out has no entry in expert_ids
-    if ((blk >> p.eshift) >= p.blocks || blk * TM >= p.num_valid[0]) return;
+    if ((blk >> p.eshift) >= p.blocks) return;
+    // the row of `a` behind each of the thread's pieces; IQ: thread t takes 8 bf16 (16 bytes) of row t / 16: four neighbouring lanes hold one 32-element group
+    int src[A_LOADS];
+    auto piece_row = [&](int j) { return ((int)threadIdx.x + 256 * j) / (IQ ? 16 : CPR); };
+    auto find_rows = [&]() {
+#pragma unroll
+        for (int j = 0; j < A_LOADS; j++) src[j] = STAGE != 1 ? blk * TM + piece_row(j) : piece_row(j) < TM ? p.sorted_ids[blk * TM + piece_row(j)] & 0xFFFFFF : 0;
+    };
+    // the list's experts that decide how W is read, and with them what else depends on nothing but the block
+    MoeNeighbours around;
+    if constexpr (NT) {
+        around = moe_neighbours(p.expert_ids, p.blocks, blk, 1, (int)threadIdx.x & 63);  // (blocks of TM rows)
+        find_rows();
+    }
+    const int used = p.num_valid[0];
+    if (blk * TM >= used) return;
     const int e = p.expert_ids[blk >> p.eshift];
     if ((unsigned)e >= (unsigned)p.experts) return;
     if (p.by_expert) n_tile += (wg - e * p.n_tiles) & 7;
@@ -197,10 +213,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
         }
     };
     v4i bw[RING][NR];
-    auto load_b = [&](int kt, v4i* dst) {
+    auto load_b = [&](int kt, v4i* dst, auto NTP) __attribute__((always_inline)) {
         const bool ok = kt < KT;
 #pragma unroll
-        for (int ni = 0; ni < NR; ni++) dst[ni] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)(ok ? boff[ni] : OOB), (int)(ok ? (uint32_t)kt * 1024u : 0u), NT ? 2 : 0);
+        for (int ni = 0; ni < NR; ni++) dst[ni] = (v4i)__builtin_amdgcn_raw_buffer_load_b128(rb, (int)(ok ? boff[ni] : OOB), (int)(ok ? (uint32_t)kt * 1024u : 0u), decltype(NTP)::value ? 2 : 0);
     };
     int sav[2][SC], sbv[2][NR / 2];
     auto load_sc = [&](int kc, int* sa_dst, int* sb_dst) {
@@ -233,11 +249,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
 
     // One K step of parity KH (= 128-K half of the current scale chunk): MFMAs on LDS stage KH, W set WS = kt % RING and scale
     // set SET; requests the operands of step kt + PF and the scales of the next chunk, stages the A rows of step kt + 1
-    auto step = [&](int kt, auto KHP, auto SETP, auto WSP) __attribute__((always_inline)) {
+    auto step = [&](int kt, auto KHP, auto SETP, auto WSP, auto NTP) __attribute__((always_inline)) {
         constexpr int KH = decltype(KHP)::value, SET = decltype(SETP)::value, WS = decltype(WSP)::value;
         if constexpr (KH == 0) load_sc((kt >> 1) + 1, sav[SET ^ 1], sbv[SET ^ 1]);  // (in front: loads return in order, and these are needed a step earlier)
         load_a(kt + PF, areg[(WS + PF) % RING]);
-        load_b(kt + PF, bw[(WS + PF) % RING]);
+        load_b(kt + PF, bw[(WS + PF) % RING], NTP);
         const int* sa_cur = sav[SET];
         const int* sb_cur = sbv[SET];
         static_for<MR>([&](auto MI) {
@@ -261,31 +277,34 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2 % RING>;
     using I3 = std::integral_constant<int, 3 % RING>;
-    // the first W fragments are requested before the list of sorted rows is fetched: they only depend on the expert
+    // the product, W past the caches (NTP) or through them
+    auto product = [&](auto NTP) __attribute__((always_inline)) {
+        // the first W fragments are requested before the list of sorted rows is fetched: they only depend on the expert
 #pragma unroll
-    for (int i = 0; i < PF; i++) load_b(i, bw[i]);
+        for (int i = 0; i < PF; i++) load_b(i, bw[i], NTP);
+        if constexpr (!NT) find_rows();
 #pragma unroll
-    for (int j = 0; j < A_LOADS; j++) {
-        // IQ: thread t takes 8 bf16 (16 bytes) of row t / 16: four neighbouring lanes hold one 32-element group
-        const int c = tid + 256 * j, row = IQ ? c >> 4 : c / CPR, kc = IQ ? c & 15 : c % CPR;
-        arow[j] = OOB;
-        if (row < TM) {
-            const int src = STAGE == 1 ? (p.sorted_ids[blk * TM + row] & 0xFFFFFF) : blk * TM + row;
-            if (src < a_rows) arow[j] = (uint32_t)src * a_src_bytes + (uint32_t)kc * 16u;
+        for (int j = 0; j < A_LOADS; j++) arow[j] = piece_row(j) < TM && src[j] < a_rows ? (uint32_t)src[j] * a_src_bytes + (uint32_t)(tid & ((IQ ? 16 : CPR) - 1)) * 16u : OOB;
+#pragma unroll
+        for (int i = 0; i < PF; i++) load_a(i, areg[i]);
+        load_sc(0, sav[0], sbv[0]);
+        store_a(0, areg[0]);
+        __syncthreads();
+        for (int kt = 0; kt < KT; kt += 4) {  // two scale chunks per trip, so every register index is a constant
+            step(kt, I0{}, I0{}, I0{}, NTP);
+            step(kt + 1, I1{}, I0{}, I1{}, NTP);
+            if (kt + 2 < KT) {
+                step(kt + 2, I0{}, I1{}, I2{}, NTP);
+                step(kt + 3, I1{}, I1{}, I3{}, NTP);
+            }
         }
-    }
-#pragma unroll
-    for (int i = 0; i < PF; i++) load_a(i, areg[i]);
-    load_sc(0, sav[0], sbv[0]);
-    store_a(0, areg[0]);
-    __syncthreads();
-    for (int kt = 0; kt < KT; kt += 4) {  // two scale chunks per trip, so every register index is a constant
-        step(kt, I0{}, I0{}, I0{});
-        step(kt + 1, I1{}, I0{}, I1{});
-        if (kt + 2 < KT) {
-            step(kt + 2, I0{}, I1{}, I2{});
-            step(kt + 3, I1{}, I1{}, I3{});
-        }
+    };
+    if constexpr (NT) {
+        const int n = (used + TM - 1) / TM;
+        if (moe_reads_once(around, p.expert_ids, n < p.blocks ? n : p.blocks, blk, 1, e, p.experts, p.cached, lane)) product(std::true_type{});
+        else product(std::false_type{});
+    } else {
+        product(std::false_type{});
     }
 
     if constexpr (STAGE == 1) {
@@ -480,19 +499,19 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
     }
 }
 
-// Blocks of 128 sorted rows that k_moe_mx_pair does not take run as two workgroups of 64 rows each: a 128-row tile needs every register of the wavefront for its
-// accumulators, so one workgroup per CU would run with nothing to overlap its loads and its epilogue with (measured, 4096
-// tokens x top-8 on 32 experts, 4096 x 1536, operands three steps ahead in both: stage 1 364 us with 128-row tiles against 292 with
-// 64-row tiles, stage 2 with the atomic epilogue 655 against 393, one row per sorted position 271 against 225).
 // Whether a stage on blocks of 16 or 32 rows reads W past the caches (non-temporal): where an expert's rows mostly make one block (the sorted list has room for the pairs and
 // a block of every expert) and the weights of both stages together are more than the last-level cache holds (256 MB; what is read like this doesn't stay there).  us plain / non-temporal, weights in memory, stages 1 and 2, 32 experts,
 // 4096 x 1536: 8 tokens x top-8 38.4 / 35.6 and 23.4 / 21.6, 64 40.0 / 36.8 and 28.3 / 25.7, 40 in blocks of 16 42.0 / 39.3 and 26.1 / 23.5; 64 experts, 2048 x 768, 128 x
 // top-4 22.9 / 21.4 and 17.5 / 16.7; 128 experts, 2048 x 512, 300 x top-8 35.6 / 33.9 and 32.8 / 32.0; but 192 tokens (one and a half blocks an expert) 53.8 / 57.9 and 34.1 / 34.6.
-bool takes_nt(const MoeMxParams& p, int stage, int tile_m) {
-    const int64_t rows_e = stage == 1 ? 2ll * p.n_out : p.n_out, bytes = p.experts * rows_e * p.K / 2;
-    return bytes * (stage == 1 ? 3 : 6) >= 2ll * (256 << 20) && 4ll * p.sorted_size <= 7ll * p.experts * tile_m;
-}
+// The rule for the routings that a call can have; which tiles of its own do is for the workgroups to say (moe_reads_once).  Layers, us through the caches / past them everywhere / as it is, weights
+// in memory; in the cache, expert preferences N(0, 4^2) beside N(0, 1) logits: 32 experts, 4096 x 1536, 64 tokens x top-8 66.2 / 64.6 / 65.9; 52.7 / 60.9 / 52.2, 40 in blocks of 16 55.7 / 53.8 /
+// 54.2; 42.3 / 50.7 / 42.1; 128 experts, 2048 x 768, 100 x top-8 43.6 / 48.2 / 43.0; 43.5 / 46.3 / 43.3.  Without preferences within 0.1 % of past them everywhere, 128 experts 1 %.
+bool takes_nt(const MoeMxParams& p, int tile_m) { return p.experts > p.cached && 4ll * p.sorted_size <= 7ll * p.experts * tile_m; }
 
+// Blocks of 128 sorted rows that k_moe_mx_pair does not take run as two workgroups of 64 rows each: a 128-row tile needs every register of the wavefront for its
+// accumulators, so one workgroup per CU would run with nothing to overlap its loads and its epilogue with (measured, 4096
+// tokens x top-8 on 32 experts, 4096 x 1536, operands three steps ahead in both: stage 1 364 us with 128-row tiles against 292 with
+// 64-row tiles, stage 2 with the atomic epilogue 655 against 393, one row per sorted position 271 against 225).
 template <int AF, int STAGE>
 hipError_t launch_rows(MoeMxParams p, MoeRowsParams rows, int block_m, int blocks, hipStream_t stream) {
     p.eshift = block_m == 128 ? 1 : 0;
@@ -518,7 +537,8 @@ hipError_t launch_rows(MoeMxParams p, MoeRowsParams rows, int block_m, int block
     p.quad_tiles = !p.by_expert && p.n_tiles % 4 == 0 && p.n_tiles % 8 != 0;
     const unsigned row_blocks = (unsigned)(blocks << p.eshift);
     const dim3 grid((unsigned)(p.by_expert ? p.n_groups * 8 : p.n_tiles) * (p.quad_tiles ? (row_blocks + 1) / 2 * 2 : row_blocks) + (unsigned)rows.wgs);
-    const bool nt = block_m <= 32 && takes_nt(p, STAGE, block_m);
+    p.cached = moe_experts_cached(STAGE, (STAGE == 1 ? 2ll * p.n_out : p.n_out) * p.K / 2);
+    const bool nt = block_m <= 32 && takes_nt(p, block_m);
 #define PSG_GO(AF_, MR_, IQ_)                                                                                                                 \
     {                                                                                                                                         \
         if (MR_ <= 2 && nt) hipLaunchKernelGGL((k_moe_mx<AF_, MR_, STAGE, IQ_, MR_ <= 2>), grid, dim3(256), 0, stream, p, rows); \

@@ -231,6 +231,7 @@ struct MoeMxParams {
     int by_expert;              // set by the launcher: workgroup ids are mapped to XCDs by (expert, column tile)
     int quad_tiles;             // set by the launcher: workgroup ids are mapped to XCDs by (row block parity, column tile % 4)
     int blocks;                 // set by the launcher: entries of expert_ids (a workgroup id past the last block leaves at once)
+    int cached;                 // set by the launcher: experts whose weights the caches hold
 };
 
 // Arguments of the device-side expert sorter (the step in front of the MoE grouped GEMMs).

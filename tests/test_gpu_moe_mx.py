@@ -396,17 +396,22 @@ def test_blocks_of_128_on_large_tiles_equal_the_small_ones(tokens, model_dim, in
         assert (got[(nv + 63) // 64 * 64:] == torch.tensor(7.0, dtype=dt).view(torch.int16).item()).all()
 
 
-# ---- blocks of 16 and 32 rows whose weights are read past the caches (more of them than these hold, where the list has room for little more than a block an expert): the same bits as with
-# a list that has room for twice as much, whose weights are read as usual.
+# ---- blocks of 16 and 32 rows in the build that may read weights past the caches (more of them than these hold, where the list has room for little more than a block an expert): the same bits
+# as with a list that has room for twice as much, whose weights are read as usual.  17 tokens reach 18 of 24 experts, whose weights fit the caches: all tiles read as usual.  Else all do: those
+# with one block read past the caches, those with two (all tokens' first choice is one of two experts) as usual.
 @pytest.mark.parametrize("bm,a_fmt", [(16, "bf16"), (32, "fp4"), (32, "fp8")])
-@pytest.mark.parametrize("model_dim,inter", [(2304, 3584), (3584, 2304)])
-def test_weights_read_past_the_caches_give_the_same_bits(bm, a_fmt, model_dim, inter):
-    dev, experts, tokens, topk = torch.device("cuda"), 24, 17, 2
+@pytest.mark.parametrize("model_dim,inter,tokens", [(2304, 3584, 17), (3584, 2304, 17), (2304, 3584, 110), (3584, 2304, 110)])
+def test_weights_read_past_the_caches_give_the_same_bits(bm, a_fmt, model_dim, inter, tokens):
+    dev, experts, topk = torch.device("cuda"), 24, 2
     g = torch.Generator(device=dev).manual_seed(bm + inter)
     u8 = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
     sc = lambda n: torch.randint(118, 130, (n,), generator=g, device=dev, dtype=torch.uint8)
     rng = np.random.default_rng(bm)
-    ids = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int32)
+    if tokens == 17:
+        ids = np.stack([rng.permutation(experts)[:topk] for _ in range(tokens)]).astype(np.int32)
+    else:
+        ids = np.stack([np.arange(tokens) % 2 * 9, 10 + np.arange(tokens) % 14], 1).astype(np.int32)
+        ids[:16, 0] = np.arange(16) // 2 + 1  # experts 1 to 8
     sid, sw, se, npp = O.moe_sorting(ids, rng.uniform(0.1, 1.0, size=(tokens, topk)).astype(np.float32), experts, bm)
     nv, most = int(npp[0]), 2 * experts * bm
     assert 4 * nv <= 7 * experts * bm
