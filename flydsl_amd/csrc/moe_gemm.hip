@@ -434,7 +434,7 @@ hipError_t launch_nr(MoeParams p, MoeRowsParams rows, int block_m, int blocks, b
     {                                                                                                    \
         constexpr bool kOnly = CO_ == 2 || (MR_ <= 2 && STAGE == 1 && KIND != KIND_INT8W4); /* always deep */ \
         constexpr bool kNt = MR_ <= 2 || CO_ == 2;                             /* may read W past the caches */ \
-        if constexpr (STAGE == 2) {                                                                      \
+        if constexpr (STAGE == 2 && CO_ == 1) {  /* (a stage by rows takes no pairs) */                   \
             if (lists) {                                                                                 \
                 hipLaunchKernelGGL((k_moe_gemm<KIND, MR_, NR, STAGE, CO_, 0, MoeRowsParams>), grid, dim3(256), 0, stream, p, rows); \
                 return hipGetLastError();                                                                \
