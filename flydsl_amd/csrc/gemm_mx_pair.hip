@@ -15,6 +15,7 @@ template <int STORE, int OUT, int SCB>
 __global__ void __launch_bounds__(256, 2) k_mx_pair(A8W8Params p) {
     constexpr int MR = MxPair::MR, NR = MxPair::NR, TM = MxPair::TM, TN = MxPair::TN;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[MxPair::LDS_BYTES];
+    static_assert(MxPair::fits(0), "two workgroups a CU");
     const int tid = threadIdx.x;
     const int wave = wave_id();
     const int lane = tid & 63, li = lane & 15, lg = lane >> 4;

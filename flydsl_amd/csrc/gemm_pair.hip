@@ -18,6 +18,7 @@ __global__ void __launch_bounds__(256, 2) k_pair(A8W8Params p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[P::LDS_BYTES];
     __shared__ float s_a[SCALED ? TM : 1], s_b[SCALED ? TN : 1];
     __shared__ __attribute__((aligned(8))) uint16_t s_bias[BIAS ? TN : 1];
+    static_assert(P::fits(TM * 4 + TN * 6), "two workgroups a CU");
     const int tid = threadIdx.x;
     const int wave = wave_id();
     const int lane = tid & 63, li = lane & 15, lg = lane >> 4;

@@ -28,6 +28,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_pair(MoeParams p, MoeRowsParams 
     __shared__ __attribute__((aligned(1024))) uint8_t lds[P::LDS_BYTES];
     __shared__ int ids[TM];
     __shared__ float s_sx[TM], s_rw[TM], s_sw[256];  // per row: scale of its x row, routing weight; per weight row of the tile: scale
+    static_assert(P::fits(TM * 12 + 256 * 4), "two workgroups a CU");
 
     if constexpr (STAGE == 2) {
         if ((int)blockIdx.x < rows.wgs) {

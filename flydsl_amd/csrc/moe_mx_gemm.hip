@@ -385,6 +385,7 @@ __global__ void __launch_bounds__(256, 2) k_moe_mx_pair(MoeMxParams p, MoeRowsPa
     constexpr int TN = STAGE == 1 ? 128 : 256;  // output columns
     __shared__ __attribute__((aligned(1024))) uint8_t lds[MxPair::LDS_BYTES];
     __shared__ float s_w[STAGE == 2 ? TM : 1];
+    static_assert(MxPair::fits(TM * 4), "two workgroups a CU");
 
     if constexpr (STAGE == 2) {
         if ((int)blockIdx.x < rows.wgs) {

@@ -1,5 +1,6 @@
-// Mainloop of the 128x256 tile that runs two workgroups per CU (gfx950), for fp4 operands with e8m0 scales on both sides, fp8 and int8: the dense
-// MXFP4 GEMM (gemm_mx_pair.hip) and the stages of both MoE pairs on blocks of 128 sorted rows (moe_mx_gemm.hip, moe_gemm_pair.hip).
+// Mainloop of the 128x256 tile that runs two workgroups per CU (gfx950), for fp4 operands with e8m0 scales on both sides, fp8, int8, fp16 and bf16: the dense
+// MXFP4 GEMM (gemm_mx_pair.hip), that of the 8- and 16-bit kinds (gemm_pair.hip) and the stages of both MoE pairs on blocks of 128 sorted rows (moe_mx_gemm.hip,
+// moe_gemm_pair.hip).
 //
 // Four wavefronts side by side along N, each 128 rows x 64 weight rows (128 accumulator registers a lane), 128 bytes of K a step:
 //   * A goes global -> LDS by DMA into four stages of 16 KB (rows of 128 bytes, 16-byte pieces XORed with row / 2), requested three steps
@@ -29,7 +30,8 @@ struct Pair {
     static constexpr int STAGE = TM * TK;         // bytes of one A stage
     static constexpr int SC_SLOT = KIND == KIND_MXFP4 ? 12 * 256 : 0;  // scale dwords of a step
     static constexpr int LDS_BYTES = NS * (STAGE + SC_SLOT);
-    static_assert(2 * LDS_BYTES + 2048 <= 160 * 1024, "two workgroups a CU, with 1 KB each for what a kernel adds");
+    // two workgroups a CU, with `more` bytes each for what a kernel adds
+    static constexpr bool fits(int more) { return 2 * (LDS_BYTES + more) <= 160 * 1024; }
 };
 using MxPair = Pair<KIND_MXFP4>;
 

@@ -305,7 +305,7 @@ double widest_gap(int tiles_m, int tiles_n, int g) {
 // is the least for its L2 to fetch.  But where its range starts, every XCD asks for one panel of W and stores to one range of columns, and with eight many
 // problems have all of them start at the same column tile or at two (whenever num / 8 is a multiple of half a group): they then walk
 // the columns side by side, and the rows of C, a power of two apart, meet in a few memory channels.  So the group of about that size is taken
-// whose starts lie apart (us in groups of 8 / as chosen here: // fp8 8192x4096x4096 111.2 / 107.8, 8192x8192x1024 87.2 / 79.0, 4096x7168x2048 58.8 / 56.0, 4096x6144x4096 93.9 / 89.9; int8 8192x8192x1024 92.1 / 82.7; bf16
+// whose starts lie apart (us in groups of 8 / as chosen here: fp8 8192x4096x4096 111.2 / 107.8, 8192x8192x1024 87.2 / 79.0, 4096x7168x2048 58.8 / 56.0, 4096x6144x4096 93.9 / 89.9; int8 8192x8192x1024 92.1 / 82.7; bf16
 // 8192x4096x2048 111.5 / 108.6; fp4 8192x8192x1024 65.4 / 58.1, 4221x7744x1536 49.9 / 45.7; over 40 drawn sizes, few of which are aligned like that,
 // 0.98 to 1.10 and 1.004 on average).
 // Only where A, W and C fit the last-level cache together: beyond, XCDs that walk side by side read a panel of W from memory once (int8
