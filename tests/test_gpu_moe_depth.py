@@ -1,6 +1,6 @@
 """The builds of the MoE stages that ask for their operands one and three steps ahead, on both sides of the rule that chooses them and on every remainder of
-the K steps by the four register sets; blocks of 16 and 32 rows with weights read past the caches (more than these hold) and, from three workgroups a CU on, two blocks of an expert
-at a time in every stage.  Whole numbers as operands and powers of two as scales: the sums are exact, stage 2 is one rounding of them."""
+the K steps by the four register sets; blocks of 16 and 32 rows with weights read past the caches (more than these hold) and, from three workgroups a CU on, two blocks of 16 rows of an
+expert at a time in every stage, through the caches and past them.  Whole numbers as operands and powers of two as scales: the sums are exact, stage 2 is one rounding of them."""
 
 import pytest
 import torch
@@ -9,12 +9,15 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(64, 130, 2, 4, 64), (128, 300, 3, 4, 192), (128, 290, 1, 2, 128), (64, 700, 2, 4, 4096), (128, 900, 2, 4, 4160), (32, 130, 2, 4, 192),
           (16, 40, 2, 4, 192), (16, 12, 3, 8, 128)]
+# Two blocks of 16 rows a workgroup, rows an expert: 12.5 stage 1 of one-byte weights and every stage 2, 15 stage 1 of int4 weights too, at most 24 past the caches where the
+# weights are more than these hold (stage 1 and 2, fp8: from 8 steps on; int4: from 9, an odd number of which stage 1 doubles), 25 through them
+PAIRED = [(16, 200, 2, 32, 4096), (16, 240, 2, 32, 4096), (16, 400, 2, 32, 4096)]
 STREAMED = [(16, 20, 2, 32, 4160, 13), (16, 20, 2, 32, 4160, 14), (16, 20, 2, 32, 4160, 15), (16, 20, 2, 32, 4160, 16), (32, 60, 2, 32, 4160, 14), (32, 60, 2, 32, 4160, 15)]
 
 
 @pytest.mark.parametrize("kind", ["fp8", "int8", "int4"])
 @pytest.mark.parametrize("block,tokens,topk,experts,n_out,steps", [s + (k,) for s in SHAPES for k in (1, 2, 3, 4, 5, 6, 7, 8, 11) if s[4] < 4000 or k <= 4]
-                         + STREAMED + [(16, 200, 2, 32, 4096, k) for k in (8, 9, 10, 11)])
+                         + STREAMED + [s + (k,) for s in PAIRED for k in (8, 9, 10, 11)])
 @pytest.mark.parametrize("stage", [1, 2])
 def test_depths(stage, block, tokens, topk, experts, n_out, kind, steps):
     from flydsl_amd import layout

@@ -352,12 +352,13 @@ def test_unbuilt_variants_raise_like_the_reference():
 
 
 # ---- blocks of 128 rows on the 128x256 tiles: from 160 tiles on (five eighths of 256 CUs), with scales on 16 bytes.  The 64-row workgroups, which calls with scales off 16
-# bytes keep, accumulate in the same K order: the same bits everywhere, at one to nine K steps, with cut last blocks, blocks of masked
-# experts, blocks past num_valid and a num_valid that ends inside a block (in the middle of one 64 rows are not written).
-@pytest.mark.parametrize("tokens,model_dim,inter,experts,topk,cut,mask", [
-    (700, 256, 2304, 3, 2, 0, False), (650, 2304, 512, 7, 4, 0, True), (333, 1280, 1024, 9, 5, 64, False), (1030, 1024, 256, 4, 3, 128, True),
-    (2600, 256, 256, 5, 4, 64, False), (300, 512, 1536, 20, 2, 0, True)])
-def test_blocks_of_128_on_large_tiles_equal_the_small_ones(tokens, model_dim, inter, experts, topk, cut, mask):
+# bytes keep, accumulate in the same K order: the same bits everywhere.  `large`: the stages that are above the line, stage 1 at one to nine K steps (model_dim / 256), stage 2
+# at one to nine (inter / 256), either with cut last blocks, blocks of masked experts, blocks past num_valid and a num_valid that ends inside a block (in the middle of one 64 rows are not written).
+@pytest.mark.parametrize("tokens,model_dim,inter,experts,topk,cut,mask,large", [
+    (700, 256, 2304, 3, 2, 0, False, (1,)), (650, 2304, 512, 7, 4, 0, True, (2,)), (333, 1280, 1024, 9, 5, 64, False, (1,)), (1030, 2048, 768, 4, 3, 128, True, (1, 2)),
+    (2600, 256, 256, 5, 4, 64, False, (1,)), (300, 512, 1536, 20, 2, 0, True, (1,)), (650, 2304, 256, 7, 4, 64, False, (2,)), (900, 1536, 1280, 6, 5, 64, True, (1, 2)),
+    (700, 2304, 2304, 3, 4, 64, True, (1, 2)), (520, 2048, 1024, 9, 5, 128, False, (1, 2))])
+def test_blocks_of_128_on_large_tiles_equal_the_small_ones(tokens, model_dim, inter, experts, topk, cut, mask, large):
     bm, dev = 128, torch.device("cuda")
     g = torch.Generator(device=dev).manual_seed(tokens)
     u8 = lambda *shape: torch.randint(0, 256, shape, generator=g, device=dev, dtype=torch.uint8)
@@ -372,8 +373,8 @@ def test_blocks_of_128_on_large_tiles_equal_the_small_ones(tokens, model_dim, in
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
     sid, sw, se, nvt = t(sid[:rows]), t(sw[:rows]), t(se), torch.tensor([nv], dtype=torch.int32, device=dev)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    for tiles in (rows // bm * (inter // 128), rows // bm * (model_dim // 256)):
-        assert tiles * 8 >= 5 * cus or tiles * 8 < 4 * cus  # on either side of the line, and not by a hair
+    for stage, tiles in ((1, rows // bm * (inter // 128)), (2, rows // bm * (model_dim // 256))):
+        assert (tiles * 8 >= 5 * cus) == (stage in large)
     a, w1, w2 = u8(tokens, model_dim // 2), u8(experts * 2 * inter, model_dim // 2), u8(experts * model_dim, inter // 2)
     sa, s1, s2 = sc(rows * (model_dim // 32)), sc(experts * 2 * inter * (model_dim // 32)), sc(experts * model_dim * (inter // 32))
 

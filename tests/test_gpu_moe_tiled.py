@@ -1,6 +1,5 @@
-"""The 256-row tiles of the MoE stages against the 128-row kernel: the same sums in the same order, so the same bits.  The lists
-are hand-made: runs of one, two, three and many blocks of an expert, runs cut up so that there are more tiles than a grouped list
-of that length can have, more than 512 blocks, blocks without an expert, and blocks past the rows in use; the widths leave the last
+"""The 128x256 tiles of the MoE stages on blocks of 128 rows against the kernel of the smaller tiles: the same sums in the same order, so the same bits.  The lists
+are hand-made: runs of one, two, three and many blocks of an expert, more than 512 blocks, blocks without an expert, and blocks past the rows in use; the widths leave the last
 column tile partly filled, the K extents cover one step up to more than the pipeline holds."""
 
 import pytest
@@ -26,15 +25,15 @@ def _launch(stage, kind, out_dtype, x, w, sx, sw, ids, eids, wts, used, tokens, 
     ("fp8", 2, 5904, 640, [3, 1, 2, 7, 3], torch.float16),
     ("int8", 1, 3072, 896, [8, 5, 4], torch.float16),
     ("int8", 2, 6144, 1152, [2, 2, 9, 3], torch.bfloat16),
-    ("fp8", 2, 2816, 256, [1] * 40, torch.bfloat16),        # every run odd: the grid's bound is exceeded, workgroups take a second tile
+    ("fp8", 2, 2816, 256, [1] * 40, torch.bfloat16),        # another expert for every block
     ("fp8", 1, 1920, 256, [301, 230, 9], torch.bfloat16),    # 540 blocks
 ])
-def test_same_bits_as_the_128_row_kernel(kind, stage, n_out, K, runs, out_dtype):
+def test_same_bits_as_the_smaller_tiles(kind, stage, n_out, K, runs, out_dtype):
     g = torch.Generator(device="cuda").manual_seed(n_out + K)
     dev = dict(device="cuda")
     experts = 4
     blocks = sum(runs)
-    tokens, topk = blocks * 128 // 2 + 3, 2  # enough rows per expert for the 256-row tiles
+    tokens, topk = blocks * 128 // 2 + 3, 2  # enough rows per expert for the 128x256 tiles
     eids = []
     for i, n in enumerate(runs):
         eids += [i % experts if i != 3 else experts + 1] * n  # run 3 has no expert

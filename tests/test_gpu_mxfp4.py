@@ -60,6 +60,7 @@ def test_mxfp4_small_m(M, N, K):
         assert np.allclose(acc, want, rtol=1e-5, atol=1e-5 * np.abs(want).max())
 
 
+# (256, 256) stands for a caller's wish: the largest tile that is built, 128x256, answers it
 @pytest.mark.parametrize("tile", [(256, 256), (128, 256), (64, 256), (32, 256), (64, 128), (32, 128)])
 @pytest.mark.parametrize("M,N,K", [(64, 512, 512), (133, 288, 768), (300, 1056, 256)])
 def test_mxfp4_tiled_shapes(tile, M, N, K):
@@ -73,10 +74,10 @@ def test_mxfp4_tiled_shapes(tile, M, N, K):
     assert np.allclose(acc, want, rtol=1e-5, atol=1e-5 * np.abs(want).max())
 
 
-# ---- the 256x256 tile of eight wavefronts (A and the scale dwords by LDS DMA), which the planner only takes for problems that
-# fill the GPU: forced here on ragged shapes (rows and scale chunks past M, columns past N in the last tile, one to nine K steps)
+# ---- the largest tile (128x256, A and the scale dwords by LDS DMA), asked for as 256x256 with and without a wavefront layout, which fp4 has one of:
+# ragged shapes (rows and scale chunks past M, columns past N in the last tile, one to nine K steps)
 @pytest.mark.parametrize("M,N,K", [(64, 512, 512), (133, 288, 768), (300, 1056, 256), (257, 32, 1280), (700, 544, 2304)])
-def test_mxfp4_eight_wavefront_tile_ragged(M, N, K):
+def test_mxfp4_largest_tile_ragged(M, N, K):
     d = make_mxfp4(M, N, K, seed=M + K)
     ref = O.run_torch_w4(d["a_q"].numpy(), d["b_q"].numpy(), d["sa"].numpy(), d["sb"].numpy())
     want = C.mxfp4(d["a_q"].numpy(), d["b_shuf"].numpy(), d["sa_shuf"].numpy(), d["sb_shuf"].numpy(), M, N, K)["out_f32"]
@@ -86,8 +87,9 @@ def test_mxfp4_eight_wavefront_tile_ragged(M, N, K):
         assert (c[M:] == SENTINEL).all()
         acc = _run(d, M, N, K, force_path=1, tile=(256, 256), acc=True, wave_layout=8)
         assert np.allclose(acc, want, rtol=1e-5, atol=1e-5 * np.abs(want).max())
-    # the same K order as the four-wavefront build of the tile: the same accumulator bits
-    assert np.array_equal(acc, _run(d, M, N, K, force_path=1, tile=(256, 256), acc=True, wave_layout=0))
+    # the same K order as the 64x256 tile: the same accumulator bits
+    for other in ((256, 256), (64, 256)):
+        assert np.array_equal(acc, _run(d, M, N, K, force_path=1, tile=other, acc=True, wave_layout=0))
 
 
 def test_mxfp4_config5_prefill():
