@@ -310,7 +310,9 @@ double widest_gap(int tiles_m, int tiles_n, int g) {
 // 0.98 to 1.10 and 1.004 on average).
 // Only where A, W and C fit the last-level cache together: beyond, XCDs that walk side by side read a panel of W from memory once (int8
 // 4096x28672x8192 714 in groups of 8 or 6, four or three starts, 728 to 732 with 7, 9 or 11, eight).  A last group of one M-tile
-// reads all of W for it (fp8 4096x8192x2048, 16 M-tiles, 64 / 71 in groups of 8 / 5).  Up to a tile a CU all of them are at work at once in any order (fp8
+// reads all of W for it (fp8 4096x8192x2048, 16 M-tiles, 64 / 71 in groups of 8 / 5), and so does one of less than half the size behind a single whole one, with W in memory (12 to 14
+// M-tiles, us in groups of 8 / 9 to 11, from memory: fp8 1506x12800x2432 48.8 / 52.1, 1460x13696x2176 46.1 / 49.5, fp4 1532x12736x1280 24.3 / 26.4, bf16 1536x6656x1280 31.1 / 34.4; 2 % over 40
+// such problems, 1 % from the cache).  Behind two whole ones it does not (fp4 2048x9728x3072, 16 M-tiles, 42.2 / 37.4 in groups of 8 / 7).  Up to a tile a CU all of them are at work at once in any order (fp8
 // 4096x4096x7168, 256 tiles, 87 / 89).
 int tile_group(int hint, int M, int N, Tile t, double bytes) {
     if (hint > 0) return hint;
@@ -319,7 +321,8 @@ int tile_group(int hint, int M, int N, Tile t, double bytes) {
     int best = 8;
     double gap = 2;
     for (const int g : {8, 7, 9, 6, 10, 11, 5}) {
-        if (tiles_m > g && tiles_m % g == 1) continue;
+        const int last = tiles_m % g;
+        if (tiles_m > g && (last == 1 || (g != 8 && tiles_m < 2 * g && 2 * last < g))) continue;
         const double d = widest_gap(tiles_m, tiles_n, g);
         if (d < gap - 0.02) {
             gap = d;
