@@ -226,17 +226,20 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
 // 30.1 / 22.4, 1416x3136x5568 41.8 / 31.2; fp8 137x16656x1152 13.5 / 10.8; bf16 3156x1536x2752 39.1 / 28.7, 643x9088x1344 25.0 / 18.4.
 // Two tiles are left out where they read W from memory more often than the estimate sees (us, W in memory): 64x256 up to 128 rows, where one row of 128x128 tiles does
 // (64x256 / 128x128: fp8 96x28672x4096 33.0 / 31.4, bf16 80x26624x1280 20.7 / 19.8, 128x28672x4096 59.5 / 54.1), and 64x64 on long rows (64x64 / 128x128: fp8
-// 302x5872x9920 43.4 / 38.6, bf16 302x5872x6208 50.6 / 45.7).
+// 302x5872x9920 43.4 / 38.6, bf16 302x5872x6208 50.6 / 45.7).  Up to a 128x128 tile a CU the 256 columns wide ones don't come into question either: on the short rows that are left there (longer ones
+// are split or have fixed tiles) their estimates lie beside that of 128x128, but not their times (us chosen before / 128x128, W in memory: bf16 1182x3200x960 14.4 / 12.6, 2557x1248x1088 15.2 / 13.7,
+// 915x3872x704 11.7 / 10.7; of 190 drawn problems this changes 12, by 0.85 to 1.01).
 Tile pick_plain_tile(int M, int N, int kbytes, bool wide, bool long_rows) {
     static const TileCost costs8[] = {{256, 256, 8, 1, 0.0, 6.7, {0, 1.25}}, {128, 256, 4, 2, 4.8, 0.2, {0, 0.75, 1.60}}, {128, 128, 4, 2, 5.7, 0.0, {0, 0.47, 0.99}},
                                       {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};
     static const TileCost costs16[] = {{256, 256, 8, 1, 0.0, 5.1, {0, 1.26}}, {128, 256, 4, 2, 2.7, 0.0, {0, 0.71, 1.54}}, {128, 128, 4, 2, 4.8, 0.0, {0, 0.51, 0.94}},
                                        {64, 64, 4, 5, 2.4, 0.0, {0, 0.33, 0.43, 0.64, 0.91, 0.99}}, {64, 256, 4, 2, 3.3, 0.0, {0, 0.60, 1.08}}};
     const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;
+    const bool one_each = (long)((M + 127) / 128) * (long)((N + 127) / 128) <= psg_cu_count();
     double best = 1e30;
     Tile t{};
     for (const TileCost& c : wide ? costs16 : costs8) {
-        if ((c.m == 64 && c.n == 256 && M <= 128) || (c.n == 64 && long_rows)) continue;
+        if ((c.m == 64 && c.n == 256 && M <= 128) || (c.n == 64 && long_rows) || (c.n == 256 && one_each)) continue;
         const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
         if (us < best) {
             best = us;
@@ -250,6 +253,9 @@ Tile pick_plain_tile(int M, int N, int kbytes, bool wide, bool long_rows) {
 // fp8 x fp8 the score's unless an estimate is 6 % below that of the score's tile.
 // fp4: on 410 timed problems, weights in memory and in the last-level cache, the estimates are 6 to 10 % off (r.m.s.) and the tile they choose takes 0.2 % longer
 // than the best of the five, at worst 7 %.
+// Where 64x128 tiles come one to a CU and 32x128 tiles would come two to some, the latter are left out, because reading W once more costs more than the estimate sees (us 32x128 / 64x128, W in
+// memory; in the cache: 113x10720x1792 8.5 / 7.7; 6.9 / 6.6, 187x7360x1536 7.3 / 6.8; 6.0 / 5.9, 539x3328x1280 6.9 / 6.5; 6.1 / 6.0, 40x20480x2048 8.7 / 8.0; 6.8 / 6.5; fifteen of 260 drawn problems,
+// 3.3 and 2.3 % faster), but for rows of up to 1024 elements and few tiles above the CUs (315x3264x1024, 260 tiles, 5.2 / 5.5; with 320 40x20480x1024 6.1 / 5.8).
 // fp8: with most weights in memory the estimates are 10 to 13 % off, so the score's tile stays where they are close: at 3 % twelve of 115 drawn
 // problems, those between the two lines, took 2 % longer on average (590x14048x10496 154 instead of 126); of the 115 34 take another tile, 10 % faster and three
 // 4 to 7 % slower (us score / estimate 600x7680x3840 35.8 / 38.2).
@@ -267,10 +273,13 @@ Tile pick_mx_tile(int M, int N, int kbytes, int formats) {
                                        {64, 128, 4, 3, 3.4, 1.0, {0, 0.34, 0.49, 0.68}},    {32, 128, 4, 4, 3.1, 0.5, {0, 0.28, 0.35, 0.49, 0.60}}};
     const double mem = ((double)M * kbytes + (double)N * (formats == MX_W4 ? kbytes / 2 : kbytes) + 2.0 * M * N) / 4.3e6;
     const Tile scored = formats == MX_FP8 ? pick_tile(M, N, true, 0, 0) : Tile{};
+    const long cus = psg_cu_count(), n128 = (N + 127) / 128, tiles32 = (M + 31) / 32 * n128;
+    const bool no32 = formats == MX_FP4 && (M + 63) / 64 * n128 <= cus && tiles32 > cus && (kbytes > 512 || tiles32 * 5 > cus * 6);
     double best = 1e30, kept = 1e30;
     Tile t = scored;
     auto consider = [&](const auto& costs) {
         for (const TileCost& c : costs) {
+            if (no32 && c.m == 32 && c.n == 128) continue;
             const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
             if (formats == MX_FP8 && c.m == scored.m && c.n == scored.n) kept = us;
             if (us < best) {
