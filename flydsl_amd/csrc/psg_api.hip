@@ -644,7 +644,11 @@ int run_a8w8(const psg_a8w8_args* a, void* out, int store, void* stream) {
         // steps ahead run (ksplit doubles as that mark for the tiled kernel); reserved = 7 keeps the one-step builds (tests)
         const long wgs = (long)((a->M + t.m - 1) / t.m) * (long)((a->N + t.n - 1) / t.n) * splits;
         const int steps_per_wg = ((kbytes + 127) / 128 + splits - 1) / splits;
-        if (wgs <= 512 && steps_per_wg >= 6 && a->reserved != 7) p.ksplit = 3;
+        // Not so one row of 64x64 tiles, more than one to a CU: from memory both builds are as fast, from the last-level cache the one-step build is (us three steps / one, memory; cache: int8
+        // 35x17056x12096 60.3 / 58.5; 46.4 / 37.3, 64x24576x4096 24.5 / 25.0; 19.3 / 18.0, fp8 46x19456x7424 38.5 / 38.7; 28.9 / 24.9, bf16 44x17632x1472 16.6 / 16.8; 13.3 / 11.6; but with four rows
+        // of tiles 200x8192x8192 32.9 / 38.0; 28.3 / 26.8).
+        const bool one_row = t.m == 64 && t.n == 64 && a->M <= 64 && splits == 1 && wgs > psg_cu_count();
+        if (wgs <= 512 && steps_per_wg >= 6 && a->reserved != 7 && (forced || !one_row)) p.ksplit = 3;
         if (splits > 1) {
             A8W8Params part = p;
             part.c = a->workspace;
