@@ -92,9 +92,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AHEAD 
     const int used = p.num_valid[0];
     // what is looked at of the list's experts, in one go
     MoeNeighbours around;
-    int back = 0;  // of block blk - 1 - lane
+    int back = 0;  // of block blk - 1 - lane (not in the builds that look at nothing else: it takes four of their registers, and the pairs of 16 a wavefront)
     if constexpr (AHEAD == 2) around = moe_neighbours(p.expert_ids, (int)gridDim.y, blk, CO, lane);
-    if constexpr (CO == 2) back = p.expert_ids[blk - 1 - lane > 0 ? blk - 1 - lane : 0];
+    if constexpr (CO == 2 && AHEAD == 2) back = p.expert_ids[blk - 1 - lane > 0 ? blk - 1 - lane : 0];
     auto sorted_row = [&]() { return tid < BM && blk * BLK + tid < p.sorted_size ? p.sorted_ids[blk * BLK + tid] : p.tokens; };  // past the list = a padding row
     int my_id = 0;
     if constexpr (AHEAD == 2) my_id = sorted_row();
@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AHEAD 
         int before = 0;
         for (int base = blk - 1; base >= 0; base -= 64) {
             const int j = base - lane;
-            const int v = base == blk - 1 ? back : p.expert_ids[j > 0 ? j : 0];
+            const int v = AHEAD == 2 && base == blk - 1 ? back : p.expert_ids[j > 0 ? j : 0];
             const unsigned long long same = __ballot(j >= 0 && v == e);
             const int run = same == ~0ull ? 64 : __builtin_ctzll(~same);
             before += run;
@@ -158,6 +158,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AHEAD 
     constexpr int WPF = DEEP ? 3 : 1;
     constexpr int NWS = WPF + 1;
     wreg_t blo[NWS][NSET][NR], bhi[NWS][NSET][NR];
+    __builtin_assume(KT > 0);  // (otherwise the first loads stand behind branches)
     auto load_b = [&](int kt, int set, auto NTP) __attribute__((always_inline)) {
         constexpr int POLICY = decltype(NTP)::value ? 2 : 0;  // non-temporal or none
         auto w8 = [&](uint32_t voff, uint32_t soff) { return (v2i)__builtin_amdgcn_raw_buffer_load_b64(rb, (int)voff, (int)soff, POLICY); };

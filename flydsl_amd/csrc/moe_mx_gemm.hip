@@ -155,6 +155,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     const int lane = tid & 63, li = lane & 15, lg = lane >> 4;
     const int n0 = n_tile * TN;
     const int KT = p.K >> 7;  // 128-element steps (even: K % 256 == 0)
+    if constexpr (!NT) __builtin_assume(KT > 1);  // (otherwise the first loads stand behind branches; the builds that look at the list lose a wavefront a SIMD to it)
     const uint32_t a_row_bytes = AF == MXF_FP4 ? (uint32_t)p.K >> 1 : (uint32_t)p.K;
     const uint32_t b_row_bytes = (uint32_t)p.K >> 1;
     const uint32_t chunk_bytes = (uint32_t)(p.K >> 8) * 256u;  // one 32-row chunk of shuffled scales
