@@ -145,7 +145,7 @@ struct Tile {
     int waves;  // wavefronts per workgroup: 4 (side by side along N, or 2x2) or 8 (side by side along N)
 };
 
-// Tile by score: what the split rules below start from, and the tile of an fp8 x fp8 problem unless an estimate is better (other problems whose K isn't split take
+// Tile by score: what the split rules below start from (the MX table's 256x256 stands for two of the 128x256 tiles that fp4 runs), and the tile of an fp8 x fp8 problem unless an estimate is better (other problems whose K isn't split take
 // the smallest estimate).  Each shape has a measured relative efficiency at full occupancy; the score multiplies it by how evenly the tiles fill the CUs'
 // workgroup slots and by the fraction of each tile that is not padding.
 Tile pick_tile(int M, int N, bool mx, int hint_m, int hint_n) {
@@ -220,9 +220,9 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
     return c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
 }
 
-// Tile of an 8- or 16-bit problem whose K isn't split: the one with the smallest estimate.  On 299 timed problems (33 to 8192 rows, weights in memory and in the
-// last-level cache) that are neither split nor streamed, the estimates are 7 to 11 % off (r.m.s.) and the chosen tile takes 0.7 % longer than the best of the five, at
-// worst 10 % (fp8 4197x1088x11904 79 on 128x256, 72 on 128x128).  us by the tiles' scores, with the 128x256 tile of that time / by estimate: int8 813x7600x3136
+// Tile of an 8- or 16-bit problem whose K isn't split: the one with the smallest estimate.  On 310 drawn problems (weights in memory and in the
+// last-level cache, profiles/tile_times.csv) the estimates are 9 to 12 % off (r.m.s.) and the chosen tile takes 1 % longer than the best of the five; the 128x256 tile, which reads W from the
+// cache fastest, waits for it from memory (fp8 4197x1088x11904 64 on 128x256, 71 on 128x128 from the cache, 76 and 71 from memory).  us by the tiles' scores, with the 128x256 tile of that time / by estimate: int8 813x7600x3136
 // 30.1 / 22.4, 1416x3136x5568 41.8 / 31.2; fp8 137x16656x1152 13.5 / 10.8; bf16 3156x1536x2752 39.1 / 28.7, 643x9088x1344 25.0 / 18.4.
 // Two tiles are left out where they read W from memory more often than the estimate sees (us, W in memory): 64x256 up to 128 rows, where one row of 128x128 tiles does
 // (64x256 / 128x128: fp8 96x28672x4096 33.0 / 31.4, bf16 80x26624x1280 20.7 / 19.8, 128x28672x4096 59.5 / 54.1), and 64x64 on long rows (64x64 / 128x128: fp8
@@ -251,8 +251,8 @@ Tile pick_plain_tile(int M, int N, int kbytes, bool wide, bool long_rows) {
 
 // Tile of an MX problem whose K isn't split (kbytes: of a row of A): of an fp4 x fp4 or fp8 / fp6 x fp4 problem the one with the smallest estimated time; of
 // fp8 x fp8 the score's unless an estimate is 6 % below that of the score's tile.
-// fp4: on 410 timed problems, weights in memory and in the last-level cache, the estimates are 6 to 10 % off (r.m.s.) and the tile they choose takes 0.2 % longer
-// than the best of the five, at worst 7 %.
+// fp4: on 260 drawn problems, weights in memory and in the last-level cache (profiles/tile_times.csv), the estimates are 8 to 11 % off (r.m.s.) and the tile they choose takes 0.3 % longer
+// than the best of the five, at worst 8 %.
 // Where 64x128 tiles come one to a CU and 32x128 tiles would come two to some, the latter are left out, because reading W once more costs more than the estimate sees (us 32x128 / 64x128, W in
 // memory; in the cache: 113x10720x1792 8.5 / 7.7; 6.9 / 6.6, 187x7360x1536 7.3 / 6.8; 6.0 / 5.9, 539x3328x1280 6.9 / 6.5; 6.1 / 6.0, 40x20480x2048 8.7 / 8.0; 6.8 / 6.5; fifteen of 260 drawn problems,
 // 3.3 and 2.3 % faster), but for rows of up to 1024 elements and few tiles above the CUs (315x3264x1024, 260 tiles, 5.2 / 5.5; with 320 40x20480x1024 6.1 / 5.8).
