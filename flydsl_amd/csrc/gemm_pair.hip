@@ -66,11 +66,8 @@ __global__ void __launch_bounds__(256, 2) k_pair(A8W8Params p) {
             }
         });
     } else {
-        // C through LDS as whole rows (512 bytes, 16-byte granules XORed with the row), in halves: the stores of one are under way while the other is
-        // converted.  Rows >= M lie behind the descriptor's bound, granules past N are redirected there.
-        const int g = tid & 31, r0 = tid >> 5, n_st = n0 + g * 8;
+        // C through LDS, in halves: the stores of one are under way while the other is converted
         const __amdgpu_buffer_rsrc_t rc = make_rsrc(static_cast<uint16_t*>(p.c) + (size_t)m0 * (size_t)p.N, (uint64_t)(p.M - m0) * (uint64_t)p.N * 2ull);
-        const uint32_t c_off = ((uint32_t)r0 * (uint32_t)p.N + (uint32_t)n_st) * 2u, c_step = 16u * (uint32_t)p.N;
         v4f sb_v[NR], bias_v[NR] = {};
 #pragma unroll
         for (int ni = 0; ni < NR; ni++) {
@@ -94,17 +91,12 @@ __global__ void __launch_bounds__(256, 2) k_pair(A8W8Params p) {
                             const v4f sb = sb_v[ni];
                             x = (v4f){((float)r[0] * sa) * sb[0], ((float)r[1] * sa) * sb[1], ((float)r[2] * sa) * sb[2], ((float)r[3] * sa) * sb[3]};
                         }
-                        *reinterpret_cast<v2i*>(lds + (mi * 16 + li) * 512 + (((((wave * NR + ni) * 2 + (lg >> 1)) ^ li) & 31) << 4) + (lg & 1) * 8) = finish4(x, bias_v[ni]);
+                        *reinterpret_cast<v2i*>(pair_c_at(lds, mi, wave * NR + ni, li, lg)) = finish4(x, bias_v[ni]);
                     });
                 });
             });
             __syncthreads();
-#pragma unroll
-            for (int i = half * 8; i < half * 8 + 8; i++) {
-                const int r = r0 + i * 8;
-                const v4i v = *reinterpret_cast<const v4i*>(lds + r * 512 + ((g ^ (r & 15)) << 4));
-                __builtin_amdgcn_raw_buffer_store_b128((v4u)v, rc, (int)(n_st < p.N ? c_off + (uint32_t)i * c_step : OOB), 0, 0);
-            }
+            pair_store_rows(lds, half, rc, n0, p.N, tid);
         });
     }
 }

@@ -208,4 +208,19 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
     asm volatile("s_nop 15\n\ts_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// A tile of 16-bit C on its way through LDS, as whole rows of 512 bytes, 16-byte granules XORed with the row: where a lane's four columns of row 16 mi + li in the 16-column block `nb` go
+__device__ __forceinline__ uint8_t* pair_c_at(uint8_t* lds, int mi, int nb, int li, int lg) { return lds + (mi * 16 + li) * 512 + ((((nb * 2 + (lg >> 1)) ^ li) & 31) << 4) + (lg & 1) * 8; }
+
+// ... and its rows of half `half`, out by all lanes.  `rc` is C from the tile's first row on: rows past the last lie behind its bound, granules past N are redirected there.
+__device__ __forceinline__ void pair_store_rows(const uint8_t* lds, int half, const __amdgpu_buffer_rsrc_t rc, int n0, int N, int tid) {
+    const int g = tid & 31, r0 = tid >> 5, n = n0 + g * 8;
+    const uint32_t off = ((uint32_t)r0 * (uint32_t)N + (uint32_t)n) * 2u, step = 16u * (uint32_t)N;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int i = half * 8 + j, r = r0 + i * 8;
+        const v4i v = *reinterpret_cast<const v4i*>(lds + r * 512 + ((g ^ (r & 15)) << 4));
+        __builtin_amdgcn_raw_buffer_store_b128((v4u)v, rc, (int)(n < N ? off + (uint32_t)i * step : OOB), 0, 0);
+    }
+}
+
 }  // namespace
