@@ -14,6 +14,12 @@
 //   * At most one memory instruction stands behind an MFMA: what is issued between two of them in a row, the matrix cores wait for (one
 //     workgroup alone on a CU, zero operands: 1,580 core cycles a step with the instructions in front of each block of four MFMAs, 1,450 like
 //     this; 1,088 is what 64 MFMAs take).
+//   * Every MFMA has one of its operands in common with the one in front of it, A or W, because at the power limit what the operands' change costs is clock (a
+//     loop of nothing but MFMAs on random data, eight A and four W fragments, us with all W for one A fragment after the other / as here / with both operands changing every
+//     time: fp4 3620 / 3508 / 3710, int8 3160 / 3070 / 3290, bf16 3180 / 3090 / 3280, fp8 3000 / 2970 / 3100).  Eight products of two A and four W fragments in a row like a
+//     snake; fp8, whose fragments have no registers for two of A and the next two, back through W in every other m-block.  us before / now: fp4 4096x7168x2048 36.1 / 35.5,
+//     8192x4096x8192 116.0 / 114.7; bf16 1500x5264x4096 48.5 / 47.5, fp16 49.5 / 48.4; int8 1500x11264x4096 66.2 / 65.3; fp8 the same 66.9 / 66.7; MX layer of 4096 tokens x top-8
+//     457 / 452, int8 735 / 729.  The order of an accumulator's own sums is the same.
 // Two workgroups on a CU take 2,600 to 3,000 cycles for a step of both, the 256x256 tile of eight wavefronts (gemm_tiled8.h) 2,850 to 3,100 for as much
 // work; but they are not in step with each other, so that the start and the end of one, 7 of the 18 us of a tile with K = 2048, stand beside
 // MFMAs of the other.
@@ -92,21 +98,21 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
         else sbv[set][q < 4 ? 0 : q - 4] = *reinterpret_cast<const int*>(lds_x + slot * SC_SLOT + 1024 + (q == 4 ? chunk0 : chunk1) * 256 + lane * 4);
     };
 
-    // fp8: eight m-blocks of four MFMAs of 32 cycles; the DMAs of step kt + 3, then the W fragments of the next step into the other set, early in
+    // fp8: eight m-blocks of four MFMAs of 32 cycles, back through W in every other one; the DMAs of step kt + 3, then the W fragments of the next step into the other set, early in
     // the step, the A fragments an m-block ahead
     auto whole_step = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
         constexpr int S = decltype(SP)::value, B0 = 2 * (S & 1), B1 = 2 - B0;  // sets of W: halves B0, B0 + 1 and B1, B1 + 1
         static_for<MR>([&](auto MI) {
             constexpr int mi = decltype(MI)::value, f = 2 * (mi & 1), fn = 2 - f;
             static_for<NR>([&](auto NI) {
-                constexpr int ni = decltype(NI)::value, slot = mi * NR + ni;
+                constexpr int at = decltype(NI)::value, ni = mi & 1 ? NR - 1 - at : at, slot = mi * NR + at;
                 const v8i a = {fr[f][0], fr[f][1], fr[f][2], fr[f][3], fr[f + 1][0], fr[f + 1][1], fr[f + 1][2], fr[f + 1][3]};
                 const v8i b = {bw[B0][ni][0], bw[B0][ni][1], bw[B0][ni][2], bw[B0][ni][3], bw[B0 + 1][ni][0], bw[B0 + 1][ni][1], bw[B0 + 1][ni][2], bw[B0 + 1][ni][3]};
                 if constexpr (WHOLE) mfma_f8(acc[mi][ni], b, a);
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (ni < 2) {
-                    if constexpr (mi + 1 < MR) read_frag(S, ni, mi + 1, fr[fn + ni]);
-                    else read_frag((S + 1) % NS, ni, 0, fr[fn + ni]);
+                if constexpr (at < 2) {
+                    if constexpr (mi + 1 < MR) read_frag(S, at, mi + 1, fr[fn + at]);
+                    else read_frag((S + 1) % NS, at, 0, fr[fn + at]);
                 }
                 if constexpr (slot >= 3 && slot < 7) dma(kt + 3, (S + 3) % NS, slot - 3, CHK);
                 if constexpr (slot >= 7 && slot < 15) load_w(kt + 1, slot & 1, (slot - 7) / 2, bw[B1 + (slot & 1)], CHK);
@@ -116,28 +122,31 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NR + N_DMA + 2 * NR) : "memory");
     };
 
-    // Step kt (kt % 4 = S): sixteen blocks of four MFMAs, eight m-blocks of the lower half of K and eight of the upper.  A's stage and scales of the step
+    // Step kt (kt % 4 = S): sixteen blocks of four MFMAs, m-blocks by twos, eight of the lower half of K and eight of the upper.  A's stage and scales of the step
     // have landed for everybody a step ago, so its first fragments and scales were read before the barrier in front of it.
     auto half_steps = [&](int kt, auto SP, auto CHK) __attribute__((always_inline)) {
         constexpr int S = decltype(SP)::value, SS = S & 1;
         static_for<16>([&](auto BI) {
-            constexpr int b = decltype(BI)::value, half = b >> 3, mi = b & 7, nb = b + AHEAD;
+            constexpr int b = decltype(BI)::value, half = b >> 3;
             static_for<NR>([&](auto NI) {
-                constexpr int ni = decltype(NI)::value;
-                if constexpr (MX) mfma_mx<half, ni & 1, mi & 1>(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3], sbv[SS][ni / 2], sav[SS][mi / 2]);
-                else if constexpr (KIND == KIND_INT8) mfma_i8(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
-                else if constexpr (KIND == KIND_BF16) mfma_bf16(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
-                else if constexpr (KIND == KIND_FP16) mfma_f16(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[b & 3]);
+                constexpr int at = decltype(NI)::value;
+                // two blocks: the products of two A fragments with all of W
+                constexpr int q = (b & 1) * 4 + at, fb = (b & 14) + (((q + 1) >> 1) & 1), mi = fb & 7, ni = b & 2 ? NR - 1 - (q >> 1) : q >> 1;
+                if constexpr (MX) mfma_mx<half, ni & 1, mi & 1>(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[fb & 3], sbv[SS][ni / 2], sav[SS][mi / 2]);
+                else if constexpr (KIND == KIND_INT8) mfma_i8(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[fb & 3]);
+                else if constexpr (KIND == KIND_BF16) mfma_bf16(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[fb & 3]);
+                else if constexpr (KIND == KIND_FP16) mfma_f16(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[fb & 3]);
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (ni == 0) {
+                if constexpr ((b & 1) == 0 && at < 2) {
+                    constexpr int nb = b + 2 + at;
                     if constexpr (nb < 16) read_frag(S, nb >> 3, nb & 7, fr[nb & 3]);
                     else read_frag((S + 1) % NS, 0, nb - 16, fr[nb & 3]);
                 }
-                if constexpr (MX && ni == 1 && b >= 10) read_sc((S + 1) % NS, b - 10, SS ^ 1);
+                if constexpr (MX && at == 3 && b >= 10) read_sc((S + 1) % NS, b - 10, SS ^ 1);
                 // The DMAs of step kt + 3 and the W fragments three half steps ahead.  The compiler counts only the loads it knows, W's, so its waits
                 // for W let as many instructions be on their way as there are W loads behind the awaited one, DMAs among them: in each half the DMAs
                 // go first, and both halves have some.
-                if constexpr (ni == 2) {
+                if constexpr (at == 2) {
                     constexpr int FROM = N_DMA == 7 ? 0 : 1, LOW = 4 - FROM;  // block of the first DMA in a half; DMAs in the lower one
                     if constexpr (b >= FROM && b < 4) dma(kt + 3, (S + 3) % NS, b - FROM, CHK);
                     if constexpr (b >= 4 && b < 8) load_w(kt + 1, 1, b - 4, bw[(2 * S + 3) % 4], CHK);
