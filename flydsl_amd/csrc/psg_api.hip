@@ -229,16 +229,28 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
 // 302x5872x9920 43.4 / 38.6, bf16 302x5872x6208 50.6 / 45.7).  Up to a 128x128 tile a CU the 256 columns wide ones don't come into question either: on the short rows that are left there (longer ones
 // are split or have fixed tiles) their estimates lie beside that of 128x128, but not their times (us chosen before / 128x128, W in memory: bf16 1182x3200x960 14.4 / 12.6, 2557x1248x1088 15.2 / 13.7,
 // 915x3872x704 11.7 / 10.7; of 190 drawn problems this changes 12, by 0.85 to 1.01).
-Tile pick_plain_tile(int M, int N, int kbytes, bool wide, bool long_rows) {
+// int8 and the 16-bit kinds have fits of their own for the two large tiles since these share operands between MFMAs, which the 128x256 tile gains more from (64 to 110 problems of
+// each kind drawn for the fit and as many others, W rotated over three sets): the chosen tile takes 0.4 % (int8) and 0.6 % (16 bits) longer than the best where it took 1.3 %; of 409 problems 88 go from
+// 256x256 to 128x256, 5 % and 4 % faster on average (us 256x256 / 128x256: bf16 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104,
+// 4693x22320x3840 346 / 311), one more than 5 % slower (int8 3337x21488x13248 770 / 822, with 285 MB of W).  They don't see W read from memory by few rows of tiles, so 256x256 tiles that make one round of the CUs, more than half
+// full, are kept where 128x256 ones make no more than one and a half, or have up to 1536 rows to share W (us 256x256 / 128x256: int8 362x24768x12480 140 / 173, 701x14736x6656 0.87, 1680x5568x8000 76 / 83,
+// bf16 1108x11056x7040 0.92; but 4096x4096x7168, 256 and 512 tiles, 88.0 / 85.9 and 174 / 166).
+Tile pick_plain_tile(int M, int N, int kbytes, int kind, bool long_rows) {
     static const TileCost costs8[] = {{256, 256, 8, 1, 0.0, 6.7, {0, 1.25}}, {128, 256, 4, 2, 4.8, 0.2, {0, 0.75, 1.60}}, {128, 128, 4, 2, 5.7, 0.0, {0, 0.47, 0.99}},
                                       {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};
-    static const TileCost costs16[] = {{256, 256, 8, 1, 0.0, 5.1, {0, 1.26}}, {128, 256, 4, 2, 2.7, 0.0, {0, 0.71, 1.54}}, {128, 128, 4, 2, 4.8, 0.0, {0, 0.51, 0.94}},
+    static const TileCost costsi[] = {{256, 256, 8, 1, 1.6, 7.7, {0, 1.38}}, {128, 256, 4, 2, 4.2, 0.3, {0, 0.70, 1.53}}, {128, 128, 4, 2, 5.7, 0.0, {0, 0.47, 0.99}},
+                                      {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};
+    static const TileCost costs16[] = {{256, 256, 8, 1, 0.0, 3.6, {0, 1.39}}, {128, 256, 4, 2, 1.3, 0.1, {0, 0.70, 1.46}}, {128, 128, 4, 2, 4.8, 0.0, {0, 0.51, 0.94}},
                                        {64, 64, 4, 5, 2.4, 0.0, {0, 0.33, 0.43, 0.64, 0.91, 0.99}}, {64, 256, 4, 2, 3.3, 0.0, {0, 0.60, 1.08}}};
+    if (kind != KIND_FP8) {
+        const long cus = psg_cu_count(), t256 = (long)((M + 255) / 256) * (long)((N + 255) / 256), t128 = (long)((M + 127) / 128) * (long)((N + 255) / 256);
+        if (t256 <= cus && t256 * 20 > cus * 11 && t128 > cus && (t128 * 2 < cus * 3 || M <= 1536)) return {256, 256, 8};
+    }
     const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;
     const bool one_each = (long)((M + 127) / 128) * (long)((N + 127) / 128) <= psg_cu_count();
     double best = 1e30;
     Tile t{};
-    for (const TileCost& c : wide ? costs16 : costs8) {
+    for (const TileCost& c : kind == KIND_FP8 ? costs8 : kind == KIND_INT8 ? costsi : costs16) {
         if ((c.m == 64 && c.n == 256 && M <= 128) || (c.n == 64 && long_rows) || (c.n == 256 && one_each)) continue;
         const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
         if (us < best) {
@@ -458,7 +470,7 @@ struct Plan {
     int splits;
 };
 // wide: 16-bit operands
-Plan plan_tiled(int M, int N, int kbytes, bool mx, bool wide) {
+Plan plan_tiled(int M, int N, int kbytes, bool mx, int kind) {
     // more columns than the streaming kernel takes in one round: 64x64 tiles, unsplit (these problems have no workspace)
     if (!mx && stream_holds(M, N, kbytes) && N > 32 * psg_cu_count()) return {Tile{64, 64, 4}, 1};
     Tile t = pick_tile(M, N, mx, 0, 0);
@@ -478,7 +490,7 @@ Plan plan_tiled(int M, int N, int kbytes, bool mx, bool wide) {
     // N=8192 22.0 against 23.7; M=384, N=8192, 768 tiles: 28.0 against 26.5, so the larger tile is kept there)
     if (!mx && steps >= 8 && steps < 48 && tiles64 <= 600) t = Tile{64, 64, 4}, fixed = true;
     const int splits = mx && mx_small_holds(M, N, kbytes * 2) ? 1 : pick_splits(M, N, kbytes, t);
-    if (splits == 1 && !fixed) t = mx ? pick_mx_tile(M, N, kbytes, MX_FP4) : pick_plain_tile(M, N, kbytes, wide, long_rows);
+    if (splits == 1 && !fixed) t = mx ? pick_mx_tile(M, N, kbytes, MX_FP4) : pick_plain_tile(M, N, kbytes, kind, long_rows);
     return {t, splits};
 }
 
@@ -630,7 +642,7 @@ int run_a8w8(const psg_a8w8_args* a, void* out, int store, void* stream) {
         e = psg_launch_a8w8_stream(p, kind, store, static_cast<hipStream_t>(stream));
     } else {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
-        const Plan plan = plan_tiled(a->M, a->N, kbytes, false, kind == KIND_FP16 || kind == KIND_BF16);
+        const Plan plan = plan_tiled(a->M, a->N, kbytes, false, kind);
         const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : plan.t;
         p.ksplit = 1;
         // wavefront layout of the 256x256 tile: the planner's choice, or forced (2 = 2x2, 8 = 1x8) by tests / tuning
@@ -689,7 +701,7 @@ uint64_t psg_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t in_dtype) 
     const bool mx = in_dtype == 4;  // MXFP4 (psg_gemm_mxfp4)
     const int kbytes = mx ? K / 2 : ((in_dtype == PSG_IN_FP16 || in_dtype == PSG_IN_BF16) ? K * 2 : K);
     if (mx ? mx_takes_small(M, N, K) : takes_stream(M, N, kbytes)) return 0;  // the small-M kernels reduce inside their workgroups
-    return splitk_bytes(M, N, plan_tiled(M, N, kbytes, mx, false).splits);
+    return splitk_bytes(M, N, plan_tiled(M, N, kbytes, mx, KIND_FP8).splits);
 }
 
 int psg_gemm_a8w8(const psg_a8w8_args* args, void* stream) {
@@ -917,7 +929,7 @@ static int mx_common(const psg_mxfp4_args* a, void* out, int store, void* stream
         e = psg_launch_mxfp4_smallm(p, store, nw, static_cast<hipStream_t>(stream));
     } else {
         const bool forced = a->force_path == 1 && a->tile_m > 0 && a->tile_n > 0;
-        const Plan plan = plan_tiled(a->M, a->N, a->K / 2, true, false);
+        const Plan plan = plan_tiled(a->M, a->N, a->K / 2, true, KIND_MXFP4);
         const Tile t = forced ? Tile{a->tile_m, a->tile_n, 4} : plan.t;
         int splits = forced ? (a->tile_k >= 1 && a->tile_k <= 16 ? a->tile_k : 1) : plan.splits;
         if (store != STORE_C || !a->workspace || !aligned(a->workspace, 16) || a->workspace_bytes < splitk_bytes(a->M, a->N, splits)) splits = 1;
