@@ -85,6 +85,9 @@ __device__ __forceinline__ int quant_silu_mul(const v4f g0, const v4f g1, const 
 // that first quantised all K elements of the 16 rows into LDS and then ran the K loop without barriers measured slower: 16 tokens
 // x top-8 on 32 experts 38.9 us against 35.4, 64 tokens 42.2 against 41.)
 // NT: W past the caches where a tile is the only one to read it (takes_nt, moe_reads_once)
+// Stage 2's end is as long as its chain of latencies, and with two workgroups a CU that end together nothing hides it: fetched row by row behind the loop, the tokens and weights
+// of 32 rows took it 3 to 4 us, so they come into LDS beside the first operands, and the rows leave several at a time.  Layers, us before / now: 64 tokens x top-8 on 32 experts,
+// 4096 x 1536, 75.2 / 71.3; 40 in blocks of 16 67.2 / 65.2; 102 x top-4 on 64, 2560 x 1024, 79.7 / 71.6; 300 x top-8 on 128, 2048 x 512, 90.3 / 79.9; 247 x top-2 on 16, 3840 x 256, 37.7 / 32.8.
 template <int AF, int MR, int STAGE, bool IQ, bool NT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 4 ? 2 : 1))) k_moe_mx(MoeMxParams p, MoeRowsParams rows) {
     static_assert(MR % 2 == 0 || MR == 1, "scale chunks cover 32 rows; a single 16-row block picks its half at run time");
@@ -102,6 +105,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
     __shared__ __attribute__((aligned(16))) uint8_t lds_raw[LDS_BYTES];
     __shared__ uint8_t iq_scale[2][IQ ? 64 : 1];   // IQ: scale byte of (row, 32-element group) of each LDS stage
     uint8_t(*lds)[TM * AB] = reinterpret_cast<uint8_t(*)[TM * AB]>(lds_raw);
+    __shared__ int s_tok[STAGE == 2 ? TM : 1];     // stage 2: token and routing weight of the block's rows, fetched beside the first operands
+    __shared__ float s_rw[STAGE == 2 ? TM : 1];
 
     if constexpr (STAGE == 2) {
         if ((int)blockIdx.x < rows.wgs) {
@@ -286,9 +291,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
         if constexpr (!NT) find_rows();
 #pragma unroll
         for (int j = 0; j < A_LOADS; j++) arow[j] = piece_row(j) < TM && src[j] < a_rows ? (uint32_t)src[j] * a_src_bytes + (uint32_t)(tid & ((IQ ? 16 : CPR) - 1)) * 16u : OOB;
+        int tok = 0;
+        float rw = 1.0f;
+        if (STAGE == 2 && p.atomic && tid < TM) {
+            tok = p.sorted_ids[blk * TM + tid] & 0xFFFFFF;
+            rw = p.sorted_w[blk * TM + tid];
+        }
 #pragma unroll
         for (int i = 0; i < PF; i++) load_a(i, areg[i]);
         load_sc(0, sav[0], sbv[0]);
+        if (STAGE == 2 && tid < TM) {
+            s_tok[tid] = tok;
+            s_rw[tid] = rw;
+        }
         store_a(0, areg[0]);
         __syncthreads();
         for (int kt = 0; kt < KT; kt += 4) {  // two scale chunks per trip, so every register index is a constant
@@ -344,7 +359,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
 #pragma unroll
         for (int mi = 0; mi < MR; mi++) {
             const int r = mi * 16 + li;
-            const float wgt = p.atomic ? p.sorted_w[blk * TM + r] : 1.0f;
+            const float wgt = s_rw[r];
 #pragma unroll
             for (int ni = 0; ni < NR; ni++) {
                 const int cb = ((wave * NR + ni) * 16 + lg * 4) * 2;
@@ -354,20 +369,40 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MR <= 
             }
         }
         __syncthreads();
+        // some trips together, so that a row's token and values come out of LDS beside those of others
         if (p.atomic == 1) {
-            for (int q = tid; q < TM * 128; q += 256) {
-                const int r = q >> 7, cb = (q & 127) * 4;
-                const int t = p.sorted_ids[blk * TM + r] & 0xFFFFFF;
-                if (t >= p.tokens) continue;
-                const int bits = *reinterpret_cast<const int*>(lds_raw + r * 512 + ((((cb >> 4) ^ r) & 31) << 4) + (cb & 15));
-                uint16_t* o = out + (size_t)t * N + n0 + (cb >> 1);
-                if (p.out_dtype == OUT_BF16) atomic_add2<OUT_BF16>(o, bits);
-                else atomic_add2<OUT_FP16>(o, bits);
+            constexpr int B = 8;
+            const int cb = (tid & 127) * 4, g = cb >> 4;
+            uint16_t* const o = out + n0 + (cb >> 1);
+#pragma unroll
+            for (int i = 0; i < TM / 2; i += B) {
+                int t[B], bits[B];
+#pragma unroll
+                for (int j = 0; j < B; j++) {
+                    const int r = (i + j) * 2 + (tid >> 7);
+                    t[j] = s_tok[r];
+                    bits[j] = *reinterpret_cast<const int*>(lds_raw + r * 512 + (((g ^ r) & 31) << 4) + (cb & 15));
+                }
+#pragma unroll
+                for (int j = 0; j < B; j++) {
+                    if (t[j] >= p.tokens) continue;
+                    if (p.out_dtype == OUT_BF16) atomic_add2<OUT_BF16>(o + (size_t)t[j] * N, bits[j]);
+                    else atomic_add2<OUT_FP16>(o + (size_t)t[j] * N, bits[j]);
+                }
             }
         } else {
-            for (int q = tid; q < TM * 32; q += 256) {
-                const int r = q >> 5, g = q & 31;
-                *reinterpret_cast<v4i*>(out + ((size_t)blk * TM + r) * N + n0 + g * 8) = *reinterpret_cast<const v4i*>(lds_raw + r * 512 + (((g ^ r) & 31) << 4));
+            constexpr int B = TM / 8 < 4 ? TM / 8 : 4;
+            const int g = tid & 31;
+#pragma unroll
+            for (int i = 0; i < TM / 8; i += B) {
+                v4i v[B];
+#pragma unroll
+                for (int j = 0; j < B; j++) {
+                    const int r = (i + j) * 8 + (tid >> 5);
+                    v[j] = *reinterpret_cast<const v4i*>(lds_raw + r * 512 + (((g ^ r) & 31) << 4));
+                }
+#pragma unroll
+                for (int j = 0; j < B; j++) *reinterpret_cast<v4i*>(out + ((size_t)blk * TM + (i + j) * 8 + (tid >> 5)) * N + n0 + g * 8) = v[j];
             }
         }
     }
