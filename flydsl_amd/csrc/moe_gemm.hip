@@ -336,27 +336,57 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AHEAD 
         });
         __syncthreads();
         const bool atomic = STAGE == 2 && p.accumulate;
-        const int unit = atomic ? 4 : 16;                      // bytes one thread moves per trip
-        const int upr = row_bytes / unit;                      // units per row
-        for (int q = tid; q < BM * upr; q += 256) {
-            const int r = q / upr, cb = (q % upr) * unit;
-            const int n = n0 + ni * 64 + cb / esize;
-            const uint32_t sid = (uint32_t)ids[r];
-            const int t = (int)(sid & 0xFFFFFFu), slot = (int)(sid >> 24);
-            if (t < p.tokens && slot < p.topk && n < p.n_out) {
-                const uint8_t* src = stage + r * row_bytes + ((((cb >> 4) ^ r) & gmask) << 4) + (cb & 15);
-                const size_t orow = atomic ? (size_t)t : p.by_position ? (size_t)(blk * BLK + r) : (size_t)t * p.topk + slot;
-                uint8_t* o = static_cast<uint8_t*>(p.out) + (orow * (size_t)p.n_out + n) * esize;
-                if (!atomic) {
-                    *reinterpret_cast<v4i*>(o) = *reinterpret_cast<const v4i*>(src);
-                } else if (f32_out) {
-                    unsafeAtomicAdd(reinterpret_cast<float*>(o), *reinterpret_cast<const float*>(src));
-                } else if (p.out_dtype == OUT_FP16) {
-                    __builtin_amdgcn_global_atomic_fadd_v2f16((__attribute__((address_space(1))) v2h*)o, *reinterpret_cast<const v2h*>(src));
-                } else {
-                    __builtin_amdgcn_global_atomic_fadd_v2bf16((__attribute__((address_space(1))) v2b*)o, *reinterpret_cast<const v2b*>(src));
+        // trips of the workgroup over the pass, 4 or 16 bytes a thread; four of them together (two on larger tiles, whose builds it would cost a wavefront a SIMD), so that their row ids and values come out of LDS side by side
+        // (and no division where the units of a row are a power of two; layers, us before / now: fp8 64 tokens x top-8 on 32 experts, 4096 x 1536, 120.7 / 119.8, 98 x top-4 on 8, 1280 x
+        // 1024, 31.3 / 29.1, 433 x top-2 on 16, 4096 x 1792, 103.0 / 100.7; int8 226 x top-4 on 32, 1280 x 768, 45.2 / 44.1; int4 2000 x top-8, 4096 x 1536, 475 / 470)
+        auto walk = [&](auto SH, auto&& put) __attribute__((always_inline)) {
+            constexpr int sh = decltype(SH)::value, TRIPS = ((BM << sh) + 255) / 256;  // log2 of the units of a row
+            const int unit_sh = (f32_out ? 8 : 7) - sh, cb = (tid & ((1 << sh) - 1)) << unit_sh, n = n0 + ni * 64 + (cb >> (f32_out ? 2 : 1));
+            constexpr int MOST = MR <= 2 ? 4 : 2;
+            static_for<(TRIPS + MOST - 1) / MOST>([&](auto I) {
+                constexpr int at = decltype(I)::value * MOST, B = TRIPS - at < MOST ? TRIPS - at : MOST;
+                uint32_t sid[B];
+                const uint8_t* src[B];
+#pragma unroll
+                for (int j = 0; j < B; j++) {
+                    const int r = (tid >> sh) + ((at + j) * 256 >> sh);
+                    sid[j] = r < BM ? (uint32_t)ids[r] : 0xFFFFFFu;
+                    src[j] = stage + r * row_bytes + ((((cb >> 4) ^ r) & gmask) << 4) + (cb & 15);
                 }
-            }
+                put(sid, src, n, at, std::integral_constant<int, B>{});
+            });
+        };
+        auto live = [&](uint32_t sid, int n) { return (int)(sid & 0xFFFFFFu) < p.tokens && (int)(sid >> 24) < p.topk && n < p.n_out; };
+        if (!atomic) {
+            walk(std::integral_constant<int, 3>{}, [&](const auto& sid, const auto& src, int n, int at, auto B) __attribute__((always_inline)) {
+                v4i v[decltype(B)::value];
+#pragma unroll
+                for (int j = 0; j < decltype(B)::value; j++) v[j] = *reinterpret_cast<const v4i*>(src[j]);
+#pragma unroll
+                for (int j = 0; j < decltype(B)::value; j++) {
+                    const size_t t = sid[j] & 0xFFFFFFu, orow = p.by_position ? (size_t)(blk * BLK + (tid >> 3) + (at + j) * 32) : t * p.topk + (sid[j] >> 24);
+                    if (live(sid[j], n)) *reinterpret_cast<v4i*>(static_cast<uint16_t*>(p.out) + orow * (size_t)p.n_out + n) = v[j];
+                }
+            });
+        } else if (f32_out) {
+            walk(std::integral_constant<int, 6>{}, [&](const auto& sid, const auto& src, int n, int, auto B) __attribute__((always_inline)) {
+#pragma unroll
+                for (int j = 0; j < decltype(B)::value; j++)
+                    if (live(sid[j], n)) unsafeAtomicAdd(static_cast<float*>(p.out) + (size_t)(sid[j] & 0xFFFFFFu) * (size_t)p.n_out + n, *reinterpret_cast<const float*>(src[j]));
+            });
+        } else {
+            walk(std::integral_constant<int, 5>{}, [&](const auto& sid, const auto& src, int n, int, auto B) __attribute__((always_inline)) {
+                int v[decltype(B)::value];
+#pragma unroll
+                for (int j = 0; j < decltype(B)::value; j++) v[j] = *reinterpret_cast<const int*>(src[j]);
+#pragma unroll
+                for (int j = 0; j < decltype(B)::value; j++) {
+                    if (!live(sid[j], n)) continue;
+                    uint16_t* o = static_cast<uint16_t*>(p.out) + (size_t)(sid[j] & 0xFFFFFFu) * (size_t)p.n_out + n;
+                    if (p.out_dtype == OUT_FP16) __builtin_amdgcn_global_atomic_fadd_v2f16((__attribute__((address_space(1))) v2h*)o, __builtin_bit_cast(v2h, v[j]));
+                    else __builtin_amdgcn_global_atomic_fadd_v2bf16((__attribute__((address_space(1))) v2b*)o, __builtin_bit_cast(v2b, v[j]));
+                }
+            });
         }
         if constexpr (ni + 1 < NR) __syncthreads();
     });
