@@ -57,6 +57,7 @@ EXPORTS = (
     "psg_gemm_a8w8_static",
     "psg_tile_coords",
     "psg_debug_tile_order",
+    "psg_debug_plan",
     "psg_debug_moe_reads_once",
     "psg_moe_gemm",
     "psg_moe_mx_gemm",
@@ -256,6 +257,8 @@ def lib() -> ctypes.CDLL:
     handle.psg_tile_coords.argtypes = [ctypes.c_int32] * 4 + [ctypes.POINTER(ctypes.c_int32)] * 2
     handle.psg_debug_tile_order.restype = ctypes.c_int
     handle.psg_debug_tile_order.argtypes = [ctypes.c_int32] * 3 + [ctypes.c_void_p, ctypes.c_void_p]
+    handle.psg_debug_plan.restype = ctypes.c_int
+    handle.psg_debug_plan.argtypes = [ctypes.c_int32] * 4 + [ctypes.POINTER(ctypes.c_int32)] * 3
     handle.psg_debug_moe_reads_once.restype = ctypes.c_int
     handle.psg_debug_moe_reads_once.argtypes = [ctypes.c_void_p] + [ctypes.c_int32] * 5 + [ctypes.c_void_p, ctypes.c_void_p]
     handle.psg_moe_reduce_masked.restype = ctypes.c_int

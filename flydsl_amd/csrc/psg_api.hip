@@ -225,16 +225,27 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
 // cache fastest, waits for it from memory (fp8 4197x1088x11904 64 on 128x256, 71 on 128x128 from the cache, 76 and 71 from memory).  us by the tiles' scores, with the 128x256 tile of that time / by estimate: int8 813x7600x3136
 // 30.1 / 22.4, 1416x3136x5568 41.8 / 31.2; fp8 137x16656x1152 13.5 / 10.8; bf16 3156x1536x2752 39.1 / 28.7, 643x9088x1344 25.0 / 18.4.
 // Two tiles are left out where they read W from memory more often than the estimate sees (us, W in memory): 64x256 up to 128 rows, where one row of 128x128 tiles does
-// (64x256 / 128x128: fp8 96x28672x4096 33.0 / 31.4, bf16 80x26624x1280 20.7 / 19.8, 128x28672x4096 59.5 / 54.1), and 64x64 on long rows (64x64 / 128x128: fp8
+// (64x256 / 128x128: fp8 96x28672x4096 33.0 / 31.4, bf16 80x26624x1280 20.7 / 19.8, 128x28672x4096 59.5 / 54.1), and with nine rows of tiles where tile_group makes groups of eight, the ninth with all of W to itself (64x256 /
+// 128x256: int8 550x14144x13312 161 / 125, 528x26176x8128 184 / 138, bf16 556x26928x4480 215 / 153, fp8 540x26688x11648 275 / 200; the 256x256 tile is faster too), and 64x64 on long rows (64x64 / 128x128: fp8
 // 302x5872x9920 43.4 / 38.6, bf16 302x5872x6208 50.6 / 45.7).  Up to a 128x128 tile a CU the 256 columns wide ones don't come into question either: on the short rows that are left there (longer ones
 // are split or have fixed tiles) their estimates lie beside that of 128x128, but not their times (us chosen before / 128x128, W in memory: bf16 1182x3200x960 14.4 / 12.6, 2557x1248x1088 15.2 / 13.7,
 // 915x3872x704 11.7 / 10.7; of 190 drawn problems this changes 12, by 0.85 to 1.01).
-// int8 and the 16-bit kinds have fits of their own for the two large tiles since these share operands between MFMAs, which the 128x256 tile gains more from (64 to 110 problems of
-// each kind drawn for the fit and as many others, W rotated over three sets): the chosen tile takes 0.4 % (int8) and 0.6 % (16 bits) longer than the best where it took 1.3 %; of 409 problems 88 go from
-// 256x256 to 128x256, 5 % and 4 % faster on average (us 256x256 / 128x256: bf16 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104,
-// 4693x22320x3840 346 / 311), one more than 5 % slower (int8 3337x21488x13248 770 / 822, with 285 MB of W).  They don't see W read from memory by few rows of tiles, so 256x256 tiles that make one round of the CUs, more than half
-// full, are kept where 128x256 ones make no more than one and a half, or have up to 1536 rows to share W (us 256x256 / 128x256: int8 362x24768x12480 140 / 173, 701x14736x6656 0.87, 1680x5568x8000 76 / 83,
-// bf16 1108x11056x7040 0.92; but 4096x4096x7168, 256 and 512 tiles, 88.0 / 85.9 and 174 / 166).
+// int8 and the 16-bit kinds have fits of their own for the two large tiles since these share operands between MFMAs, which the 128x256 tile gains more from (us 256x256 / 128x256: bf16
+// 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104, 4693x22320x3840 346 / 311).  What these don't see: keeps_256 below.
+// Whether 256x256 tiles are kept although the estimate of the 128x256 tile is the smallest.
+// They are where they make one round of the CUs, more than half full, and 128x256 tiles would come two to some CUs: with few rows of tiles to share W those wait for it from memory. How much the estimates
+// have to say then depends on the rows (524 problems, both tiles timed with W in memory and in the cache; time of 128x256 over that of 256x256 where the estimates are at most 12 % apart, memory; cache: int8 up to
+// 768 rows 1.16; 1.00, up to 1536 1.13; 0.98, beyond 0.99; 0.98, but at less than one and a half of the smaller tiles a CU 1.01; 1.02; 16 bits 1.14; 0.98, 1.08; 0.98, 0.97; 0.96, 0.98; 1.00). Further apart 128x256 is the better one from
+// some 12 to 18 % on (int8 650x11920x832 17.5 / 16.9), and on rows of up to 1 KB always (bf16 2863x4096x192 11.8 / 10.9).  Of the 524 the tile so chosen takes 0.1 % longer than the better of the two, none is slower both ways.
+// The other tiles, where one of them has the smallest estimate, stay (256x256 / the smallest estimate's, memory; cache: int8 838x9248x7296 71.4 / 63.9; 68.5 / 58.6 on 128x128, bf16 826x9360x1088 27.2 / 26.4; 26.3 / 22.4 on
+// 64x256; 64 problems 1.01; 1.19).
+bool keeps_256(int M, int N, int kbytes, bool wide, double us256, double us128) {
+    const long cus = psg_cu_count(), t256 = (long)((M + 255) / 256) * (long)((N + 255) / 256), t128 = (long)((M + 127) / 128) * (long)((N + 255) / 256);
+    const bool one_round = t256 <= cus && t256 * 20 > cus * 11 && t128 > cus;
+    if (!one_round || kbytes <= 1024 || (M > 1536 && (wide || t128 * 2 >= cus * 3))) return false;
+    return us128 > (wide ? 0.86 : M <= 768 ? 0.82 : M <= 1536 ? 0.88 : 0.92) * us256;
+}
+
 Tile pick_plain_tile(int M, int N, int kbytes, int kind, bool long_rows) {
     static const TileCost costs8[] = {{256, 256, 8, 1, 0.0, 6.7, {0, 1.25}}, {128, 256, 4, 2, 4.8, 0.2, {0, 0.75, 1.60}}, {128, 128, 4, 2, 5.7, 0.0, {0, 0.47, 0.99}},
                                       {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};
@@ -242,22 +253,21 @@ Tile pick_plain_tile(int M, int N, int kbytes, int kind, bool long_rows) {
                                       {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};
     static const TileCost costs16[] = {{256, 256, 8, 1, 0.0, 3.6, {0, 1.39}}, {128, 256, 4, 2, 1.3, 0.1, {0, 0.70, 1.46}}, {128, 128, 4, 2, 4.8, 0.0, {0, 0.51, 0.94}},
                                        {64, 64, 4, 5, 2.4, 0.0, {0, 0.33, 0.43, 0.64, 0.91, 0.99}}, {64, 256, 4, 2, 3.3, 0.0, {0, 0.60, 1.08}}};
-    if (kind != KIND_FP8) {
-        const long cus = psg_cu_count(), t256 = (long)((M + 255) / 256) * (long)((N + 255) / 256), t128 = (long)((M + 127) / 128) * (long)((N + 255) / 256);
-        if (t256 <= cus && t256 * 20 > cus * 11 && t128 > cus && (t128 * 2 < cus * 3 || M <= 1536)) return {256, 256, 8};
-    }
     const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;
     const bool one_each = (long)((M + 127) / 128) * (long)((N + 127) / 128) <= psg_cu_count();
-    double best = 1e30;
+    const bool ninth = M > 512 && M <= 576 && (double)(M + (double)N) * kbytes + 2.0 * M * N > 200e6;
+    double best = 1e30, us256 = 0;
     Tile t{};
     for (const TileCost& c : kind == KIND_FP8 ? costs8 : kind == KIND_INT8 ? costsi : costs16) {
-        if ((c.m == 64 && c.n == 256 && M <= 128) || (c.n == 64 && long_rows) || (c.n == 256 && one_each)) continue;
+        if ((c.m == 64 && c.n == 256 && (M <= 128 || ninth)) || (c.n == 64 && long_rows) || (c.n == 256 && one_each)) continue;
         const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
+        if (c.m == 256) us256 = us;
         if (us < best) {
             best = us;
             t = {c.m, c.n, c.waves};
         }
     }
+    if (kind != KIND_FP8 && t.m == 128 && t.n == 256 && keeps_256(M, N, kbytes, kind != KIND_INT8, us256, best)) t = {256, 256, 8};
     return t;
 }
 
@@ -619,6 +629,8 @@ int check_moe_gating(const psg_moe_gating_args* a, bool need_outputs, MoeGatingP
     return 0;
 }
 
+constexpr int kKinds[4] = {KIND_INT8, KIND_FP8, KIND_FP16, KIND_BF16};  // by PSG_IN_*
+
 int run_a8w8(const psg_a8w8_args* a, void* out, int store, void* stream) {
     A8W8Params p{};
     p.c = out;
@@ -633,8 +645,7 @@ int run_a8w8(const psg_a8w8_args* a, void* out, int store, void* stream) {
     p.epi = a->epilogue;
     p.out = a->out_dtype;
     p.b_rowmajor = a->b_layout;
-    const int kinds[4] = {KIND_INT8, KIND_FP8, KIND_FP16, KIND_BF16};
-    const int kind = kinds[a->in_dtype];
+    const int kind = kKinds[a->in_dtype];
     const int kbytes = (kind == KIND_FP16 || kind == KIND_BF16) ? a->K * 2 : a->K;
     const bool small = a->force_path == 2 || (a->force_path == 0 && takes_stream(a->M, a->N, kbytes));
     hipError_t e;
@@ -754,6 +765,22 @@ int psg_debug_tile_order(int32_t tiles_m, int32_t tiles_n, int32_t group_m, int3
         return fail(PSG_E_SHAPE, "need tiles_m, tiles_n, group_m >= 1 and at most 2^24 tiles");
     const hipError_t e = psg_launch_tile_order(tiles_m, tiles_n, group_m, out, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "psg_debug_tile_order launch");
+    g_err[0] = 0;
+    return 0;
+}
+
+int psg_debug_plan(int32_t M, int32_t N, int32_t K, int32_t in_dtype, int32_t* tile_m, int32_t* tile_n, int32_t* splits) {
+    if (!tile_m || !tile_n || !splits) return fail(PSG_E_NULL, "tile_m, tile_n and splits must be non-NULL");
+    if (in_dtype < PSG_IN_INT8 || in_dtype > PSG_IN_BF16) return fail(PSG_E_DTYPE, "in_dtype %d unknown", in_dtype);
+    const int kind = kKinds[in_dtype], eb = kind == KIND_FP16 || kind == KIND_BF16 ? 2 : 1;
+    if (M < 1 || M > 65536 || N < 16 || K < 1 || (uint64_t)N * (uint64_t)K * eb > 0xFFFFFFFFull)
+        return fail(PSG_E_SHAPE, "M=%d outside [1, 65536], N=%d below 16, K=%d below 1 or W above 4 GiB", M, N, K);
+    const int kbytes = K * eb;
+    const bool small = takes_stream(M, N, kbytes);
+    const Plan plan = small ? Plan{Tile{0, 0, 0}, 1} : plan_tiled(M, N, kbytes, false, kind);
+    *tile_m = plan.t.m;
+    *tile_n = plan.t.n;
+    *splits = plan.splits;
     g_err[0] = 0;
     return 0;
 }

@@ -25,6 +25,7 @@
  *   psg_tile_coords     the workgroup-id -> tile remap xcd_remap_bx_by
  *                       kernels/common/mma/mfma_preshuffle_pipeline.py:685-729 (host evaluation of the function the
  *                       tiled kernel uses); psg_debug_tile_order runs the same function on the device
+ *   psg_debug_plan      no counterpart: the tile and the K splits that psg_gemm_a8w8 gives a problem
  *   psg_debug_moe_reads_once
  *                       no counterpart: which tiles of a MoE stage read their weights past the caches
  *   psg_gemm_a8w8_static, psg_init, psg_static_scratch_bytes
@@ -207,6 +208,10 @@ void psg_tile_coords(int32_t id, int32_t tiles_m, int32_t tiles_n, int32_t group
 
 /* Evaluates the same function on the device for every id: out[2*id] = tm, out[2*id+1] = tn (int32 [tiles_m*tiles_n*2]). */
 int psg_debug_tile_order(int32_t tiles_m, int32_t tiles_n, int32_t group_m, int32_t *out, void *stream);
+
+/* What psg_gemm_a8w8 does with a problem whose path, tile and splits the caller leaves open (in_dtype as there), on a GPU of 256 CUs where there is none: *tile_m x *tile_n (0 x 0: the
+ * streaming kernel) and the number of K splits, which it makes if the workspace for them is there.  For tests.  Host function. */
+int psg_debug_plan(int32_t M, int32_t N, int32_t K, int32_t in_dtype, int32_t *tile_m, int32_t *tile_n, int32_t *splits);
 
 /* How the MoE stages on small blocks read the weights, for tests: out[i] = 1 where the tile of `per_tile` (1 or 2) blocks from block i on reads them past the
  * caches, 0 where through them, -1 where the block has no expert or is not one of the `used` ones.  expert_ids int32 [blocks]; `cached` experts' weights fit the
