@@ -220,6 +220,24 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
     return c.start + std::sqrt(std::sqrt(us * us * us * us + mem * mem * mem * mem));
 }
 
+// Whether 256x256 tiles are kept although the estimate of the 128x256 tile is the smallest: the estimates don't see W read from memory by few rows of tiles, for which the 128x256 tile has too few bytes on their way.
+// One round: where 256x256 tiles make one round of the CUs, more than half full, and 128x256 tiles would come two to some CUs.  How much the estimates
+// have to say then depends on the rows that share W (524 problems, both tiles timed with W in memory and in the cache; time of 128x256 over that of 256x256 where the estimates are at most 12 % apart, memory; cache: int8 up to
+// 768 rows 1.16; 1.00, up to 1536 1.13; 0.98, beyond 0.99; 0.98, but at less than one and a half of the smaller tiles a CU 1.01; 1.02; 16 bits 1.14; 0.98, 1.08; 0.98, 0.97; 0.96, 0.98; 1.00). Further apart 128x256 is the better one from
+// some 12 to 18 % on (int8 650x11920x832 17.5 / 16.9), and on rows of up to 1 KB always (bf16 2863x4096x192 11.8 / 10.9).  Of the 524 the tile so chosen takes 0.1 % longer than the better of the two, none is slower both ways.
+// The other tiles, where one of them has the smallest estimate, stay (256x256 / the smallest estimate's, memory; cache: int8 838x9248x7296 71.4 / 63.9; 68.5 / 58.6 on 128x128, bf16 826x9360x1088 27.2 / 26.4; 26.3 / 22.4 on
+// 64x256; 64 problems 1.01; 1.19).
+// W beyond the last-level cache (256 MB, of which A and C take some): W comes from memory then in every pass.  Where the estimates are at most 7 % apart 128x256 takes 1.03 of the time in int8, 1.06 in 16 bits up to 2048 rows
+// (102 problems; 76 drawn afterwards 1.02 and 1.04; us 256x256 / 128x256: int8 3337x21488x13248 771 / 817, 2985x23344x13632 777 / 832, bf16 1113x23744x8320 363 / 408, 1270x22928x7552 343 / 391); with more rows 16 bits are level (16 problems 0.97 to 1.07). With 200 to
+// 240 MB of W there is no difference (0.99), further apart 128x256 is the better one (int8 2624x25376x8384 491 / 482, bf16 1953x27936x4032 368 / 338).
+bool keeps_256(int M, int N, int kbytes, bool wide, double us256, double us128) {
+    const long cus = psg_cu_count(), t256 = (long)((M + 255) / 256) * (long)((N + 255) / 256), t128 = (long)((M + 127) / 128) * (long)((N + 255) / 256);
+    if ((double)N * kbytes > 240e6 && (!wide || M <= 2048) && us128 > 0.93 * us256) return true;
+    const bool one_round = t256 <= cus && t256 * 20 > cus * 11 && t128 > cus;
+    if (!one_round || kbytes <= 1024 || (M > 1536 && (wide || t128 * 2 >= cus * 3))) return false;
+    return us128 > (wide ? 0.86 : M <= 768 ? 0.82 : M <= 1536 ? 0.88 : 0.92) * us256;
+}
+
 // Tile of an 8- or 16-bit problem whose K isn't split: the one with the smallest estimate.  On 310 drawn problems (weights in memory and in the
 // last-level cache, profiles/tile_times.csv) the estimates are 9 to 12 % off (r.m.s.) and the chosen tile takes 1 % longer than the best of the five; the 128x256 tile, which reads W from the
 // cache fastest, waits for it from memory (fp8 4197x1088x11904 64 on 128x256, 71 on 128x128 from the cache, 76 and 71 from memory).  us by the tiles' scores, with the 128x256 tile of that time / by estimate: int8 813x7600x3136
@@ -231,21 +249,7 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
 // are split or have fixed tiles) their estimates lie beside that of 128x128, but not their times (us chosen before / 128x128, W in memory: bf16 1182x3200x960 14.4 / 12.6, 2557x1248x1088 15.2 / 13.7,
 // 915x3872x704 11.7 / 10.7; of 190 drawn problems this changes 12, by 0.85 to 1.01).
 // int8 and the 16-bit kinds have fits of their own for the two large tiles since these share operands between MFMAs, which the 128x256 tile gains more from (us 256x256 / 128x256: bf16
-// 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104, 4693x22320x3840 346 / 311).  What these don't see: keeps_256 below.
-// Whether 256x256 tiles are kept although the estimate of the 128x256 tile is the smallest.
-// They are where they make one round of the CUs, more than half full, and 128x256 tiles would come two to some CUs: with few rows of tiles to share W those wait for it from memory. How much the estimates
-// have to say then depends on the rows (524 problems, both tiles timed with W in memory and in the cache; time of 128x256 over that of 256x256 where the estimates are at most 12 % apart, memory; cache: int8 up to
-// 768 rows 1.16; 1.00, up to 1536 1.13; 0.98, beyond 0.99; 0.98, but at less than one and a half of the smaller tiles a CU 1.01; 1.02; 16 bits 1.14; 0.98, 1.08; 0.98, 0.97; 0.96, 0.98; 1.00). Further apart 128x256 is the better one from
-// some 12 to 18 % on (int8 650x11920x832 17.5 / 16.9), and on rows of up to 1 KB always (bf16 2863x4096x192 11.8 / 10.9).  Of the 524 the tile so chosen takes 0.1 % longer than the better of the two, none is slower both ways.
-// The other tiles, where one of them has the smallest estimate, stay (256x256 / the smallest estimate's, memory; cache: int8 838x9248x7296 71.4 / 63.9; 68.5 / 58.6 on 128x128, bf16 826x9360x1088 27.2 / 26.4; 26.3 / 22.4 on
-// 64x256; 64 problems 1.01; 1.19).
-bool keeps_256(int M, int N, int kbytes, bool wide, double us256, double us128) {
-    const long cus = psg_cu_count(), t256 = (long)((M + 255) / 256) * (long)((N + 255) / 256), t128 = (long)((M + 127) / 128) * (long)((N + 255) / 256);
-    const bool one_round = t256 <= cus && t256 * 20 > cus * 11 && t128 > cus;
-    if (!one_round || kbytes <= 1024 || (M > 1536 && (wide || t128 * 2 >= cus * 3))) return false;
-    return us128 > (wide ? 0.86 : M <= 768 ? 0.82 : M <= 1536 ? 0.88 : 0.92) * us256;
-}
-
+// 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104, 4693x22320x3840 346 / 311).  What these don't see: keeps_256.
 Tile pick_plain_tile(int M, int N, int kbytes, int kind, bool long_rows) {
     static const TileCost costs8[] = {{256, 256, 8, 1, 0.0, 6.7, {0, 1.25}}, {128, 256, 4, 2, 4.8, 0.2, {0, 0.75, 1.60}}, {128, 128, 4, 2, 5.7, 0.0, {0, 0.47, 0.99}},
                                       {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};

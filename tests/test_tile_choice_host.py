@@ -33,6 +33,15 @@ def test_large_tile_of_one_round(kind, M, N, K, rows):
     assert _plan(kind, M, N, K) == (rows, 256, 1)
 
 
+@pytest.mark.parametrize("kind,M,N,K,rows", [
+    ("int8", 3337, 21488, 13248, 256), ("int8", 2985, 23344, 13632, 256), ("int8", 3195, 20832, 14272, 256), ("bf16", 1113, 23744, 8320, 256), ("bf16", 1270, 22928, 7552, 256), ("fp16", 947, 28352, 8192, 256),
+    ("int8", 4704, 18800, 12736, 128), ("int8", 4704, 18800, 12800, 256),  # 239.4 and 240.6 MB of W
+    ("bf16", 2048, 20496, 5888, 256), ("bf16", 2049, 20496, 5888, 128),
+    ("int8", 2624, 25376, 8384, 128), ("bf16", 1953, 27936, 4032, 128)])
+def test_weights_beyond_the_last_level_cache(kind, M, N, K, rows):
+    assert _plan(kind, M, N, K) == (rows, 256, 1)
+
+
 @pytest.mark.parametrize("kind,M,N,K,tile", [("int8", 550, 14144, 12288, (64, 256)), ("int8", 550, 14144, 13312, (256, 256)), ("fp8", 540, 26688, 11648, (128, 256)),
                                              ("bf16", 556, 26928, 4480, (128, 256))])
 def test_nine_rows_of_tiles_in_groups_of_eight(kind, M, N, K, tile):
