@@ -33,6 +33,12 @@ def test_large_tile_of_one_round(kind, M, N, K, rows):
     assert _plan(kind, M, N, K) == (rows, 256, 1)
 
 
+@pytest.mark.parametrize("kind,M,N,K,rows", [("int8", 463, 17184, 4800, 256), ("int8", 463, 17104, 4800, 128), ("int8", 733, 11632, 4032, 256), ("int8", 733, 11456, 4032, 128), ("bf16", 511, 17664, 2496, 256),
+                                             ("fp16", 720, 11696, 4352, 256), ("int8", 800, 8944, 6016, 128)])
+def test_few_rows_of_tiles_on_little_more_than_half_of_the_cus(kind, M, N, K, rows):
+    assert _plan(kind, M, N, K) == (rows, 256, 1)
+
+
 @pytest.mark.parametrize("kind,M,N,K,rows", [
     ("int8", 3337, 21488, 13248, 256), ("int8", 2985, 23344, 13632, 256), ("int8", 3195, 20832, 14272, 256), ("bf16", 1113, 23744, 8320, 256), ("bf16", 1270, 22928, 7552, 256), ("fp16", 947, 28352, 8192, 256),
     ("int8", 4704, 18800, 12736, 128), ("int8", 4704, 18800, 12800, 256),  # 239.4 and 240.6 MB of W
