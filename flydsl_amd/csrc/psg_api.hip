@@ -251,6 +251,8 @@ bool keeps_256(int M, int N, int kbytes, bool wide, double us256, double us128) 
 // 915x3872x704 11.7 / 10.7; of 190 drawn problems this changes 12, by 0.85 to 1.01).
 // int8 and the 16-bit kinds have fits of their own for the two large tiles since these share operands between MFMAs, which the 128x256 tile gains more from (us 256x256 / 128x256: bf16
 // 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104, 4693x22320x3840 346 / 311).  What these don't see: keeps_256.
+// Up to a 128x256 tile a CU the 16-bit fit, made where they come in rounds, has their start 1.4 us too early, so that they replaced 64x256 tiles on short rows (us 64x256 / 128x256, memory; cache: fp16 264x11872x1152
+// 17.0 / 18.2; 13.6 / 14.6, 161x20640x1152 18.6 / 19.4; 14.2 / 15.3; 46 problems 1.03; 1.03).
 Tile pick_plain_tile(int M, int N, int kbytes, int kind, bool long_rows) {
     static const TileCost costs8[] = {{256, 256, 8, 1, 0.0, 6.7, {0, 1.25}}, {128, 256, 4, 2, 4.8, 0.2, {0, 0.75, 1.60}}, {128, 128, 4, 2, 5.7, 0.0, {0, 0.47, 0.99}},
                                       {64, 64, 4, 5, 3.2, 0.0, {0, 0.30, 0.45, 0.67, 0.95, 1.06}}, {64, 256, 4, 2, 4.6, 0.9, {0, 0.55, 1.10}}};
@@ -260,12 +262,13 @@ Tile pick_plain_tile(int M, int N, int kbytes, int kind, bool long_rows) {
                                        {64, 64, 4, 5, 2.4, 0.0, {0, 0.33, 0.43, 0.64, 0.91, 0.99}}, {64, 256, 4, 2, 3.3, 0.0, {0, 0.60, 1.08}}};
     const double mem = ((double)(M + N) * kbytes + 2.0 * M * N) / 4.3e6;
     const bool one_each = (long)((M + 127) / 128) * (long)((N + 127) / 128) <= psg_cu_count();
+    const bool few = kind != KIND_FP8 && kind != KIND_INT8 && (long)((M + 127) / 128) * (long)((N + 255) / 256) <= psg_cu_count();
     const bool ninth = M > 512 && M <= 576 && (double)(M + (double)N) * kbytes + 2.0 * M * N > 200e6;
     double best = 1e30, us256 = 0;
     Tile t{};
     for (const TileCost& c : kind == KIND_FP8 ? costs8 : kind == KIND_INT8 ? costsi : costs16) {
         if ((c.m == 64 && c.n == 256 && (M <= 128 || ninth)) || (c.n == 64 && long_rows) || (c.n == 256 && one_each)) continue;
-        const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem);
+        const double us = tile_us(c, M, N, (kbytes + 127) / 128, mem) + (few && c.m == 128 && c.n == 256 ? 1.4 : 0);
         if (c.m == 256) us256 = us;
         if (us < best) {
             best = us;

@@ -54,6 +54,13 @@ def test_nine_rows_of_tiles_in_groups_of_eight(kind, M, N, K, tile):
     assert _plan(kind, M, N, K) == (*tile, 1)
 
 
+@pytest.mark.parametrize("kind,M,N,K,tile", [
+    ("fp16", 264, 11872, 1152, (64, 256)), ("bf16", 161, 20640, 1152, (64, 256)), ("bf16", 394, 8432, 1152, (64, 256)), ("bf16", 301, 11376, 1408, (64, 256)),  # at most one 128x256 tile a CU
+    ("bf16", 703, 23456, 1792, (128, 256)), ("fp16", 909, 16400, 1536, (128, 256))])  # more
+def test_16_bits_around_a_128x256_tile_a_cu(kind, M, N, K, tile):
+    assert _plan(kind, M, N, K) == (*tile, 1)
+
+
 def test_what_the_query_refuses():
     out = [ctypes.byref(ctypes.c_int32()) for _ in range(3)]
     h = _lib.lib()
