@@ -224,8 +224,8 @@ double tile_us(const TileCost& c, int M, int N, double steps, double mem) {
 // One round: where 256x256 tiles make one round of the CUs, more than half full, and 128x256 tiles would come two to some CUs (up to 768 rows from 136 tiles on: with 136 to 140 of them 128x256 takes 1.13 of the time from memory and
 // 0.98 from the cache in int8, 1.14 and 0.97 in 16 bits, us 256x256 / 128x256 from memory int8 463x17184x4800 54.1 / 63.9).  How much the estimates
 // have to say then depends on the rows that share W (524 problems, both tiles timed with W in memory and in the cache; time of 128x256 over that of 256x256 where the estimates are at most 12 % apart, memory; cache: int8 up to
-// 768 rows 1.16; 1.00, up to 1536 1.13; 0.98, beyond 0.99; 0.98, but at less than one and a half of the smaller tiles a CU 1.01; 1.02; 16 bits 1.14; 0.98, 1.08; 0.98, 0.97; 0.96, 0.98; 1.00). Further apart 128x256 is the better one from
-// some 12 to 18 % on (int8 650x11920x832 17.5 / 16.9), and on rows of up to 1 KB always (bf16 2863x4096x192 11.8 / 10.9).  Of the 524 the tile so chosen takes 0.1 % longer than the better of the two, none is slower both ways.
+// 768 rows 1.16; 1.00, up to 1536 1.13; 0.98, beyond 0.99; 0.98, but at less than one and a half of the smaller tiles a CU 1.01; 1.02; 16 bits 1.14; 0.98, 1.08; 0.98, 0.97; 0.96, 0.98; 1.00). Further apart 128x256 is the better one
+// from some 14 to 18 % on (int8 650x11920x832 17.5 / 16.9; but 1261x8480x1856, 14 % apart, 27.5 / 31.1 from memory, 26.5 / 25.9 from the cache), and on rows of up to 1 KB always (bf16 2863x4096x192 11.8 / 10.9).  Of the 524 the tile so chosen takes 0.1 % longer than the better of the two, none is slower both ways.
 // The other tiles, where one of them has the smallest estimate, stay (256x256 / the smallest estimate's, memory; cache: int8 838x9248x7296 71.4 / 63.9; 68.5 / 58.6 on 128x128, bf16 826x9360x1088 27.2 / 26.4; 26.3 / 22.4 on
 // 64x256; 64 problems 1.01; 1.19).
 // W beyond the last-level cache (256 MB, of which A and C take some): W comes from memory then in every pass.  Where the estimates are at most 7 % apart 128x256 takes 1.03 of the time in int8, 1.06 in 16 bits up to 2048 rows
@@ -236,7 +236,7 @@ bool keeps_256(int M, int N, int kbytes, bool wide, double us256, double us128) 
     if ((double)N * kbytes > 240e6 && (!wide || M <= 2048) && us128 > 0.93 * us256) return true;
     const bool one_round = t256 <= cus && t256 * 100 > cus * (M <= 768 ? 53 : 55) && t128 > cus;
     if (!one_round || kbytes <= 1024 || (M > 1536 && (wide || t128 * 2 >= cus * 3))) return false;
-    return us128 > (wide ? 0.86 : M <= 768 ? 0.82 : M <= 1536 ? 0.88 : 0.92) * us256;
+    return us128 > (wide ? 0.86 : M <= 1536 ? 0.82 : 0.92) * us256;
 }
 
 // Tile of an 8- or 16-bit problem whose K isn't split: the one with the smallest estimate.  On 310 drawn problems (weights in memory and in the

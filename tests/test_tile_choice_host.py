@@ -26,7 +26,7 @@ def test_smaller_tiles_of_the_smallest_estimate_stay(kind, M, N, K, tile):
 @pytest.mark.parametrize("kind,M,N,K,rows", [
     ("int8", 1024, 9024, 4096, 256), ("int8", 1024, 8960, 4096, 128),  # 144 and 140 of 256 CUs
     ("int8", 1536, 6016, 4096, 256), ("int8", 1537, 5888, 4096, 128), ("int8", 1537, 6656, 4096, 256), ("bf16", 1536, 6016, 4096, 256), ("bf16", 1537, 6016, 4096, 128),  # rows that share W
-    ("int8", 768, 12288, 2048, 256), ("int8", 769, 11000, 2048, 128),
+    ("int8", 768, 12288, 2048, 256), ("int8", 1261, 8480, 1856, 256), ("int8", 941, 10048, 1856, 256), ("int8", 902, 10192, 1088, 128),
     ("int8", 1920, 6400, 6144, 256), ("int8", 2048, 6016, 6144, 128), ("int8", 2048, 6144, 4096, 128), ("bf16", 2048, 6144, 4096, 128),  # one and a half 128x256 tiles a CU: 375, 384
     ("int8", 1638, 5824, 704, 128), ("int8", 829, 10224, 832, 128), ("bf16", 2863, 4096, 192, 128), ("fp16", 717, 12320, 256, 128)])  # short rows
 def test_large_tile_of_one_round(kind, M, N, K, rows):
