@@ -88,6 +88,7 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
     };
     const int f_base[2] = {li * TK + ((lg ^ ((li >> 1) & 7)) << 4), li * TK + (((4 + lg) ^ ((li >> 1) & 7)) << 4)};
     constexpr int AHEAD = 2;  // blocks of four MFMAs that an A fragment is read ahead
+    static_assert(AHEAD == 2, "a ring of four: two fragments at work, the two behind them on their way");
     v4i fr[4];
     auto read_frag = [&](int stage, int half, int mi, v4i& dst) __attribute__((always_inline)) {
         dst = *reinterpret_cast<const v4i*>(&lds[stage * STAGE + mi * 16 * TK + f_base[half]]);
@@ -138,7 +139,7 @@ __device__ __forceinline__ void pair_loop(ACC (&acc)[8][4], uint8_t* lds, const 
                 else if constexpr (KIND == KIND_FP16) mfma_f16(acc[mi][ni], bw[(2 * S + half) % 4][ni], fr[fb & 3]);
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr ((b & 1) == 0 && at < 2) {
-                    constexpr int nb = b + 2 + at;
+                    constexpr int nb = b + AHEAD + at;
                     if constexpr (nb < 16) read_frag(S, nb >> 3, nb & 7, fr[nb & 3]);
                     else read_frag((S + 1) % NS, 0, nb - 16, fr[nb & 3]);
                 }
