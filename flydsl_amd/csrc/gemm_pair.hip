@@ -3,7 +3,7 @@
 // Bound: MFMA at the clock the power limit leaves; on long rows the 256x256 tile (gemm_tiled8.h), which moves two thirds of the bytes, is as fast or faster, on short
 // ones, where a tile's start and end count, and for problems of few 256x256 tiles this one.  us, 256x256 tiles / 128x256 tiles with A through registers / these: fp8
 // 8192x4096x4096 106.7 / 121.4 / 107.8, 8192x8192x1024 78.9 / 85.1 / 69.3, 1024x8192x2048 25.6 / 22.3 / 19.5, 1500x11264x4096 86.1 / 84.9 / 71.8, 5120x5120x8320
-// 170 / 201 / 181; int8 4096x8192x2048 65.2 / 67.9 / 60.4, 4096x28672x8192 701 / 720 / 688; bf16 1500x5264x4096 84.4 / 64.6 / 57.7, 5133x5120x8320 348 / 371 / 346.
+// 170 / 201 / 181; int8 4096x8192x2048 65.2 / 67.9 / 60.4, 4096x28672x8192 701 / 720 / 688 (the estimates of pick_plain_tile see it the other way round, 674 / 692, and take the larger tile); bf16 1500x5264x4096 84.4 / 64.6 / 57.7, 5133x5120x8320 348 / 371 / 346.
 // Same bits.
 #include "pair_loop.h"
 

@@ -228,8 +228,9 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
             __builtin_amdgcn_sched_barrier(0);
             const v4i alo = flo[mi % FRAG_BUFS], ahi = fhi[mi % FRAG_BUFS];
             if constexpr (KIND == KIND_INT8) {
-                // Back through the W fragments in every other m-block, and the halves of K in the other order there (the sums are exact in any): an MFMA has
-                // an operand in common with the one in front of it, which costs less power (pair_loop.h).  4096x28672x8192 698 -> 686 us, 8192x4096x4096 106.5 -> 104.6.
+                // Back through the W fragments in every other m-block, and the halves of K in the other order there (the sums are exact in any): three MFMAs of four have
+                // an operand in common with the one in front of them, which costs less power (pair_loop.h); between the halves of an m-block both change, and the last
+                // accumulator of the first half is the first of the second, two MFMAs in a row.  4096x28672x8192 698 -> 686 us, 8192x4096x4096 106.5 -> 104.6.
 #pragma unroll
                 for (int ni = 0; ni < NR; ni++) mfma_i8(acc[mi][ni], mi & 1 ? bhi[SB][ni] : blo[SB][ni], mi & 1 ? ahi : alo);
 #pragma unroll
@@ -264,7 +265,7 @@ __global__ void __launch_bounds__(WAVES * 64, 1) k_tiled_dma(A8W8Params p) {
                 });
             } else {
                 const v8i af = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1], ahi[2], ahi[3]};
-                // as above: 8192x4096x4096 99.7 -> 99.0 us, 8192x8192x8192 380 -> 377 (bf16 and fp16, whose sums are not exact, keep the lower half of K first and gain nothing)
+                // Back through W as above, so that only the first MFMA of a step shares nothing: 8192x4096x4096 99.7 -> 99.0 us, 8192x8192x8192 380 -> 377 (bf16 and fp16, whose sums are not exact, keep the lower half of K first and gain nothing)
 #pragma unroll
                 for (int at = 0; at < NR; at++) {
                     const int ni = mi & 1 ? NR - 1 - at : at;

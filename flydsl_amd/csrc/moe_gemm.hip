@@ -337,7 +337,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(AHEAD 
         __syncthreads();
         const bool atomic = STAGE == 2 && p.accumulate;
         // trips of the workgroup over the pass, 4 or 16 bytes a thread; four of them together (two on larger tiles, whose builds it would cost a wavefront a SIMD), so that their row ids and values come out of LDS side by side
-        // (and no division where the units of a row are a power of two; layers, us before / now: fp8 64 tokens x top-8 on 32 experts, 4096 x 1536, 120.7 / 119.8, 98 x top-4 on 8, 1280 x
+        // (and shifts instead of a division for every unit, the units of a row being a power of two known at build time; layers, us before / now: fp8 64 tokens x top-8 on 32 experts, 4096 x 1536, 120.7 / 119.8, 98 x top-4 on 8, 1280 x
         // 1024, 31.3 / 29.1, 433 x top-2 on 16, 4096 x 1792, 103.0 / 100.7; int8 226 x top-4 on 32, 1280 x 768, 45.2 / 44.1; int4 2000 x top-8, 4096 x 1536, 475 / 470)
         auto walk = [&](auto SH, auto&& put) __attribute__((always_inline)) {
             constexpr int sh = decltype(SH)::value, TRIPS = ((BM << sh) + 255) / 256;  // log2 of the units of a row

@@ -14,7 +14,7 @@
 //   * At most one memory instruction stands behind an MFMA: what is issued between two of them in a row, the matrix cores wait for (one
 //     workgroup alone on a CU, zero operands: 1,580 core cycles a step with the instructions in front of each block of four MFMAs, 1,450 like
 //     this; 1,088 is what 64 MFMAs take).
-//   * Every MFMA has one of its operands in common with the one in front of it, A or W, because at the power limit what the operands' change costs is clock (a
+//   * Within a half step (fp8: a step) every MFMA has one of its operands in common with the one in front of it, A or W; where a half begins both change, two of 64 times a step (fp8: one of 32). At the power limit what the operands' change costs is clock (a
 //     loop of nothing but MFMAs on random data, eight A and four W fragments, us with all W for one A fragment after the other / as here / with both operands changing every
 //     time: fp4 3620 / 3508 / 3710, int8 3160 / 3070 / 3290, bf16 3180 / 3090 / 3280, fp8 3000 / 2970 / 3100).  Eight products of two A and four W fragments in a row like a
 //     snake; fp8, whose fragments have no registers for two of A and the next two, back through W in every other m-block.  us before / now: fp4 4096x7168x2048 36.1 / 35.5,

@@ -240,7 +240,7 @@ bool keeps_256(int M, int N, int kbytes, bool wide, double us256, double us128) 
 }
 
 // Tile of an 8- or 16-bit problem whose K isn't split: the one with the smallest estimate.  On 310 drawn problems (weights in memory and in the
-// last-level cache, profiles/tile_times.csv) the estimates are 9 to 12 % off (r.m.s.) and the chosen tile takes 1 % longer than the best of the five; the 128x256 tile, which reads W from the
+// last-level cache, profiles/tile_times.csv) the estimates are 9 to 16 % off (r.m.s.) and the chosen tile takes 0.2 to 1 % longer than the best of the five; the 128x256 tile, which reads W from the
 // cache fastest, waits for it from memory (fp8 4197x1088x11904 64 on 128x256, 71 on 128x128 from the cache, 76 and 71 from memory).  us by the tiles' scores, with the 128x256 tile of that time / by estimate: int8 813x7600x3136
 // 30.1 / 22.4, 1416x3136x5568 41.8 / 31.2; fp8 137x16656x1152 13.5 / 10.8; bf16 3156x1536x2752 39.1 / 28.7, 643x9088x1344 25.0 / 18.4.
 // Two tiles are left out where they read W from memory more often than the estimate sees (us, W in memory): 64x256 up to 128 rows, where one row of 128x128 tiles does
@@ -250,7 +250,7 @@ bool keeps_256(int M, int N, int kbytes, bool wide, double us256, double us128) 
 // are split or have fixed tiles) their estimates lie beside that of 128x128, but not their times (us chosen before / 128x128, W in memory: bf16 1182x3200x960 14.4 / 12.6, 2557x1248x1088 15.2 / 13.7,
 // 915x3872x704 11.7 / 10.7; of 190 drawn problems this changes 12, by 0.85 to 1.01).
 // int8 and the 16-bit kinds have fits of their own for the two large tiles since these share operands between MFMAs, which the 128x256 tile gains more from (us 256x256 / 128x256: bf16
-// 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104, 4693x22320x3840 346 / 311).  What these don't see: keeps_256.
+// 5133x5120x8320 359 / 352, 8192x8192x1024 124 / 113, 5817x21104x1792 370 / 337, int8 8192x4096x4096 110 / 104, 4693x22320x3840 346 / 311).  What these don't see: keeps_256.  Over the 1800 problems of profiles/large_tile_times.csv, most of them drawn on the lines of the rules here and there, the chosen tile takes 1 % longer than the best.
 // Up to a 128x256 tile a CU the 16-bit fit, made where they come in rounds, has their start 1.4 us too early, so that they replaced 64x256 tiles on short rows (us 64x256 / 128x256, memory; cache: fp16 264x11872x1152
 // 17.0 / 18.2; 13.6 / 14.6, 161x20640x1152 18.6 / 19.4; 14.2 / 15.3; 46 problems 1.03; 1.03).
 Tile pick_plain_tile(int M, int N, int kbytes, int kind, bool long_rows) {
@@ -487,7 +487,7 @@ struct Plan {
     Tile t;
     int splits;
 };
-// wide: 16-bit operands
+// kind: of the operands, for the tile where K isn't split (mx: of no account; the splits are the same for all)
 Plan plan_tiled(int M, int N, int kbytes, bool mx, int kind) {
     // more columns than the streaming kernel takes in one round: 64x64 tiles, unsplit (these problems have no workspace)
     if (!mx && stream_holds(M, N, kbytes) && N > 32 * psg_cu_count()) return {Tile{64, 64, 4}, 1};
